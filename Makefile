@@ -35,7 +35,7 @@ oracle/liboracle.so: oracle/vite_oracle.c oracle/vite_oracle.h
 	gcc -O2 -std=gnu99 -Wall -ffp-contract=off -fPIC -shared -o $@ oracle/vite_oracle.c -lm
 
 ref:
-	@if [ -d /root/reference ]; then $(MAKE) -f oracle/Makefile.ref; else echo "reference tree absent: skipping oracle/_ref"; fi
+	@if [ -f /root/reference/main.cpp ]; then $(MAKE) -f oracle/Makefile.ref; else echo "reference tree absent: skipping oracle/_ref"; fi
 
 clean:
 	rm -f $(OBJS) $(LIB) $(HOSTLIB) $(CLI) oracle/liboracle.so
