@@ -140,13 +140,13 @@ static_assert(sizeof(VRec) == 16, "record must be 16 bytes");
 struct MoveArgs {
     const int64_t* offs;
     const DEdge* edges;
-    const int64_t* curr;
+    const int32_t* curr;
     const double* vdeg;
     const double* cdeg;
-    const int64_t* csize;
+    const int32_t* csize;
     const unsigned char* active;  // null when ET is off
     double* frozen;               // null when ET is off
-    int64_t* target;
+    int32_t* target;
     double* cw;
     const double* constant;       // 1/2m: a device scalar, or one per graph of a batch
     unsigned long long* inactive_count;
@@ -154,11 +154,9 @@ struct MoveArgs {
     // iterating (null for a single graph).
     const int32_t* gid;
     const unsigned char* gact;
-    // Structure-of-arrays copy of the edges (32-bit tails, weights) and a 32-bit copy of
-    // currComm, read by the group buckets; null when the build reads the records directly.
+    // Structure-of-arrays copy of the edges (32-bit tails, weights), read by the group buckets.
     const int32_t* tail32;
     const double* wgt;
-    const int32_t* curr32;
     // Records of the same community state (null unless the launch tuning asks for them); the
     // group kernels then read communities, sizes and degrees from them.
     const VRec* rec;
@@ -355,11 +353,6 @@ constexpr int kNch[5] = {2, VT_NCH_G8, VT_NCH_G16, VT_NCH_G32, VT_NCH_G64};
 // one-wave 2048-slot kernel.
 constexpr int32_t kBucketCap[6] = {2 * 4 - 1, VT_NCH_G8 * 8 - 1, VT_NCH_G16 * 16 - 1, VT_NCH_G32 * 32 - 1,
                                    VT_NCH_G64 * 64 - 1, 1023};
-
-#ifndef VT_SPLIT_EDGES
-#define VT_SPLIT_EDGES 1
-#endif
-constexpr bool kSplitEdges = VT_SPLIT_EDGES;
 
 #ifndef VT_DPP_ARGMAX
 #define VT_DPP_ARGMAX 1
@@ -562,8 +555,7 @@ __device__ __forceinline__ VHeader<BATCH> load_header(const MoveArgs& a, int32_t
         h.e0 = a.offs[v];
         h.deg = live ? (int32_t)(a.offs[v + 1] - h.e0) : -1;
         if constexpr (REC) h.cc = a.rec[v].comm;
-        else if constexpr (kSplitEdges) h.cc = a.curr32[v];
-        else h.cc = (int32_t)a.curr[v];
+        else h.cc = a.curr[v];
         h.kv = a.vdeg[v];
         if constexpr (BATCH) {
             const int32_t gg = a.gid[v];
@@ -605,13 +597,8 @@ __device__ __forceinline__ void row_issue_edges(const MoveArgs& a, const VHeader
         r.t[u] = -1;
         r.w[u] = 0.0;
         if (r.ok[u]) {
-            if constexpr (kSplitEdges) {
-                r.t[u] = a.tail32[j];
-                r.w[u] = a.wgt[j];
-            } else {
-                r.t[u] = reinterpret_cast<const int32_t*>(a.edges)[4 * j];
-                r.w[u] = reinterpret_cast<const double*>(a.edges)[2 * j + 1];
-            }
+            r.t[u] = a.tail32[j];
+            r.w[u] = a.wgt[j];
         }
     }
 }
@@ -624,8 +611,7 @@ __device__ __forceinline__ void row_issue_gathers(const MoveArgs& a, int32_t v, 
         r.c[u] = 0;
         if (r.ok[u]) {
             if constexpr (REC) r.c[u] = a.rec[r.t[u]].comm;
-            else if constexpr (kSplitEdges) r.c[u] = a.curr32[r.t[u]];
-            else r.c[u] = reinterpret_cast<const int32_t*>(a.curr)[2 * (int64_t)r.t[u]];
+            else r.c[u] = a.curr[r.t[u]];
         }
         r.self[u] = r.ok[u] && r.t[u] == v;
     }
@@ -1142,7 +1128,7 @@ __global__ void __launch_bounds__(64) k_move_hbm(MoveArgs a, const int32_t* __re
 template <class K>
 __global__ void k_hub_keys(const int32_t* __restrict__ hubs, int32_t nh, const int64_t* __restrict__ hoffs,
                            const int64_t* __restrict__ offs, const int32_t* __restrict__ tail32,
-                           const int32_t* __restrict__ curr32, int cbits, K* __restrict__ keys,
+                           const int32_t* __restrict__ curr, int cbits, K* __restrict__ keys,
                            uint32_t* __restrict__ vals)
 {
     const int64_t total = hoffs[nh];
@@ -1160,7 +1146,7 @@ __global__ void k_hub_keys(const int32_t* __restrict__ hubs, int32_t nh, const i
             int32_t j = lo;
             while (hoffs[j + 1] <= q) j++;  // hoffs[nh] = total > q
             const int64_t k = offs[hubs[j]] + (q - hoffs[j]);
-            keys[q] = ((K)j << cbits) | (K)(uint32_t)curr32[tail32[k]];
+            keys[q] = ((K)j << cbits) | (K)(uint32_t)curr[tail32[k]];
             vals[q] = (uint32_t)k;
         }
     }
@@ -1171,14 +1157,14 @@ __global__ void k_hub_keys(const int32_t* __restrict__ hubs, int32_t nh, const i
 template <class K>
 __global__ void k_hub_keys_rows(const int32_t* __restrict__ hubs, int32_t nh, const int64_t* __restrict__ hoffs,
                                 const int64_t* __restrict__ offs, const int32_t* __restrict__ tail32,
-                                const int32_t* __restrict__ curr32, int cbits, K* __restrict__ keys,
+                                const int32_t* __restrict__ curr, int cbits, K* __restrict__ keys,
                                 uint32_t* __restrict__ vals)
 {
     for (int32_t j = blockIdx.x; j < nh; j += gridDim.x) {
         const int64_t q0 = hoffs[j], n = hoffs[j + 1] - q0, e0 = offs[hubs[j]];
         for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
             const int64_t k = e0 + i;
-            keys[q0 + i] = ((K)j << cbits) | (K)(uint32_t)curr32[tail32[k]];
+            keys[q0 + i] = ((K)j << cbits) | (K)(uint32_t)curr[tail32[k]];
             vals[q0 + i] = (uint32_t)k;
         }
     }
@@ -1534,15 +1520,15 @@ __global__ void __launch_bounds__(64 * kFoldWaveRows) k_row_fold_wave(const int6
 }
 
 __global__ void k_init(int64_t nv, const double* __restrict__ vdeg, double* __restrict__ cdeg,
-                       int64_t* __restrict__ csize, int64_t* __restrict__ past, int64_t* __restrict__ curr,
-                       int64_t* __restrict__ target, unsigned char* __restrict__ active, double* __restrict__ frozen,
+                       int32_t* __restrict__ csize, int32_t* __restrict__ past, int32_t* __restrict__ curr,
+                       int32_t* __restrict__ target, unsigned char* __restrict__ active, double* __restrict__ frozen,
                        double* __restrict__ p_curr, double* __restrict__ p_prev)
 {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nv; i += (int64_t)gridDim.x * blockDim.x) {
         cdeg[i] = vdeg[i];
         csize[i] = 1;
-        past[i] = i;
-        curr[i] = i;
+        past[i] = (int32_t)i;
+        curr[i] = (int32_t)i;
         target[i] = 0;
         if (active) {
             active[i] = 1;
@@ -1601,8 +1587,8 @@ __global__ void k_key_histogram(const uint32_t* __restrict__ keys, int64_t n, in
 
 // Movers in processing order: a vertex that was processed (active, or ET off) and whose
 // target differs from its community contributes two delta events (louvain.cpp:2343-2359).
-__global__ void k_mover_flags(const int32_t* __restrict__ order, int64_t n, const int64_t* __restrict__ target,
-                              const int64_t* __restrict__ curr, const unsigned char* __restrict__ active,
+__global__ void k_mover_flags(const int32_t* __restrict__ order, int64_t n, const int32_t* __restrict__ target,
+                              const int32_t* __restrict__ curr, const unsigned char* __restrict__ active,
                               int32_t* __restrict__ flags)
 {
     for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < n; p += (int64_t)gridDim.x * blockDim.x) {
@@ -1629,8 +1615,8 @@ __global__ void k_scan_total(const int32_t* __restrict__ flags, const int32_t* _
 }
 
 __global__ void k_emit_events(const int32_t* __restrict__ order, int64_t n, const int32_t* __restrict__ flags,
-                              const int32_t* __restrict__ pos, const int64_t* __restrict__ target,
-                              const int64_t* __restrict__ curr, uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
+                              const int32_t* __restrict__ pos, const int32_t* __restrict__ target,
+                              const int32_t* __restrict__ curr, uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
                               unsigned long long* __restrict__ long_runs)
 {
     if (blockIdx.x == 0 && threadIdx.x == 0) *long_runs = 0;  // k_fold_events marks long runs
@@ -1647,10 +1633,10 @@ __global__ void k_emit_events(const int32_t* __restrict__ order, int64_t n, cons
 
 // One sorted event's contribution: +k_v when v arrives in the event's community c (its target
 // is c), -k_v when it leaves (a - x == a + (-x) exactly); s = +-1, the member-count change.
-__device__ __forceinline__ double event_delta(uint32_t c, uint32_t v, const int64_t* __restrict__ target,
+__device__ __forceinline__ double event_delta(uint32_t c, uint32_t v, const int32_t* __restrict__ target,
                                               const double* __restrict__ vdeg, int& s)
 {
-    const bool in = (uint64_t)target[v] == (uint64_t)c;
+    const bool in = (uint32_t)target[v] == c;
     const double k = vdeg[v];
     s = in ? 1 : -1;
     return in ? k : -k;
@@ -1666,9 +1652,9 @@ __device__ __forceinline__ double event_delta(uint32_t c, uint32_t v, const int6
 constexpr int64_t kFoldLongRun = 1024;
 
 __global__ void k_fold_events(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ vals,
-                              const int64_t* __restrict__ target, const double* __restrict__ vdeg, int64_t n,
+                              const int32_t* __restrict__ target, const double* __restrict__ vdeg, int64_t n,
                               const int64_t* __restrict__ d_movers, double* __restrict__ cdeg,
-                              int64_t* __restrict__ csize, uint32_t none, unsigned long long* __restrict__ long_runs)
+                              int32_t* __restrict__ csize, uint32_t none, unsigned long long* __restrict__ long_runs)
 {
     if (d_movers) n = 2 * d_movers[0];
     for (int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; j < n; j += (int64_t)gridDim.x * blockDim.x) {
@@ -1681,9 +1667,9 @@ __global__ void k_fold_events(const uint32_t* __restrict__ keys, const uint32_t*
         // the community's counters, read before the run so their (random) loads overlap
         // the run's; no other run touches community c
         const double deg0 = cdeg[c];
-        const int64_t size0 = csize[c];
+        const int32_t size0 = csize[c];
         double acc = 0.0;
-        int64_t cnt = 0;
+        int32_t cnt = 0;
         int64_t k = j;
         // keys ascend, so keys[k + 3] == c means keys[k..k+3] all are c
         for (; k + 4 <= n && keys[k + 3] == c; k += 4) {
@@ -1715,10 +1701,10 @@ __global__ void k_fold_events(const uint32_t* __restrict__ keys, const uint32_t*
 // member-count changes are integers, summed in any order.
 __global__ void __launch_bounds__(256) k_fold_events_long(const uint32_t* __restrict__ keys,
                                                           const uint32_t* __restrict__ vals,
-                                                          const int64_t* __restrict__ target,
+                                                          const int32_t* __restrict__ target,
                                                           const double* __restrict__ vdeg, int64_t n,
                                                           const int64_t* __restrict__ d_movers,
-                                                          double* __restrict__ cdeg, int64_t* __restrict__ csize,
+                                                          double* __restrict__ cdeg, int32_t* __restrict__ csize,
                                                           uint32_t none, const unsigned long long* __restrict__ long_runs)
 {
     if (*long_runs == 0) return;  // k_fold_events found none (the common case)
@@ -1737,7 +1723,7 @@ __global__ void __launch_bounds__(256) k_fold_events_long(const uint32_t* __rest
             const int64_t j0 = base + __builtin_ctzll(sm);
             const uint32_t c = keys[j0];
             double acc = 0.0;
-            int64_t cnt = 0;
+            int32_t cnt = 0;
             for (int64_t k = j0;; k += 64) {
                 const int64_t idx = k + lane;
                 const bool in = idx < n && keys[idx] == c;
@@ -1775,32 +1761,32 @@ __global__ void k_modularity(const double* __restrict__ sums, const double* __re
 // ET types 1/3 rotation (louvain.cpp:173-183): the freeze test parses as
 // ((target == curr) == past), a bool against a community id; vertices that fail it
 // rotate even when already frozen.
-__global__ void k_rotate_et1(int64_t nv, int num_iters, int64_t* __restrict__ past, int64_t* __restrict__ curr,
-                             int64_t* __restrict__ target, unsigned char* __restrict__ active)
+__global__ void k_rotate_et1(int64_t nv, int num_iters, int32_t* __restrict__ past, int32_t* __restrict__ curr,
+                             int32_t* __restrict__ target, unsigned char* __restrict__ active)
 {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nv; i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t t = target[i], c = curr[i], p = past[i];
-        if (num_iters > 2 && (int64_t)(t == c) == p) active[i] = 0;
+        const int32_t t = target[i], c = curr[i], p = past[i];
+        if (num_iters > 2 && (int32_t)(t == c) == p) active[i] = 0;
         else { past[i] = c; curr[i] = t; target[i] = p; }
     }
 }
 
 // ET types 2/4 rotation (louvain.cpp:380-400); the caller swaps p_curr/p_prev afterwards.
-__global__ void k_rotate_et2(int64_t nv, int num_iters, double one_minus_delta, int64_t* __restrict__ past,
-                             int64_t* __restrict__ curr, int64_t* __restrict__ target,
+__global__ void k_rotate_et2(int64_t nv, int num_iters, double one_minus_delta, int32_t* __restrict__ past,
+                             int32_t* __restrict__ curr, int32_t* __restrict__ target,
                              unsigned char* __restrict__ active, double* __restrict__ p_curr,
                              const double* __restrict__ p_prev)
 {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nv; i += (int64_t)gridDim.x * blockDim.x) {
         if (!active[i]) continue;
-        const int64_t c = curr[i], p = past[i];
+        const int32_t c = curr[i], p = past[i];
         bool act = true;
         if (num_iters > 2 && c == p) {
             const double pc = p_prev[i] * one_minus_delta;
             p_curr[i] = pc;
             if (pc <= 0.02) { active[i] = 0; act = false; }
         }
-        if (act) { const int64_t t = target[i]; past[i] = c; curr[i] = t; target[i] = p; }
+        if (act) { const int32_t t = target[i]; past[i] = c; curr[i] = t; target[i] = p; }
     }
 }
 
@@ -1855,23 +1841,33 @@ __global__ void __launch_bounds__(256) k_split_fold(const int64_t* __restrict__ 
     }
 }
 
+// A caller's 64-bit ids or sizes, saturated (a size beyond 32 bits stays larger than 1).
 __global__ void k_narrow_ids(const int64_t* __restrict__ src, int64_t n, int32_t* __restrict__ dst)
 {
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t x = src[i];
+        dst[i] = x > INT32_MAX ? INT32_MAX : x < INT32_MIN ? INT32_MIN : (int32_t)x;
+    }
+}
+
+// The phase's 32-bit ids as the boundary's 64-bit ones.
+__global__ void k_widen_ids(const int32_t* __restrict__ src, int64_t n, int64_t* __restrict__ dst)
+{
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        dst[i] = (int32_t)src[i];
+        dst[i] = src[i];
 }
 
 // Records of vertices 0..n-1, or of the listed vertices live[0..n-1] (a batch's graphs still
 // iterating: the sweep reads no other records).
-__global__ void k_pack_records(const int64_t* __restrict__ curr, const int64_t* __restrict__ csize,
+__global__ void k_pack_records(const int32_t* __restrict__ curr, const int32_t* __restrict__ csize,
                                const double* __restrict__ cdeg, int64_t n, const int32_t* __restrict__ live,
                                VRec* __restrict__ rec)
 {
     for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < n; p += (int64_t)gridDim.x * blockDim.x) {
         const int64_t i = live ? live[p] : p;
         VRec r;
-        r.comm = (int32_t)curr[i];
-        r.size = (int32_t)csize[i];
+        r.comm = curr[i];
+        r.size = csize[i];
         r.deg = cdeg[i];
         rec[i] = r;
     }
@@ -1892,8 +1888,8 @@ __global__ void k_seg_constant(const double* __restrict__ sums, int32_t ng, doub
 // A batch vertex moves when its graph is still iterating and its target differs.  Flags are
 // per position of the live list (the vertices of the graphs iterating at the last relist, in
 // vertex order), so the scan and the events follow vertex order.
-__global__ void k_batch_flags(int64_t n, const int32_t* __restrict__ live, const int64_t* __restrict__ target,
-                              const int64_t* __restrict__ curr, const int32_t* __restrict__ gid,
+__global__ void k_batch_flags(int64_t n, const int32_t* __restrict__ live, const int32_t* __restrict__ target,
+                              const int32_t* __restrict__ curr, const int32_t* __restrict__ gid,
                               const unsigned char* __restrict__ gact, int32_t* __restrict__ flags)
 {
     for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < n; p += (int64_t)gridDim.x * blockDim.x) {
@@ -1949,19 +1945,16 @@ __global__ void k_batch_decide(int32_t ng, const double* __restrict__ sums, cons
 }
 
 // past <- curr <- target for the graphs that continue (louvain.cpp:565-570), over the live
-// list; the 32-bit copy of currComm the sweep reads (curr32) is kept equal to curr here.
+// list.
 __global__ void k_batch_rotate(int64_t n, const int32_t* __restrict__ live, const int32_t* __restrict__ gid,
-                               const unsigned char* __restrict__ grot, int64_t* __restrict__ past,
-                               int64_t* __restrict__ curr, const int64_t* __restrict__ target,
-                               int32_t* __restrict__ curr32)
+                               const unsigned char* __restrict__ grot, int32_t* __restrict__ past,
+                               int32_t* __restrict__ curr, const int32_t* __restrict__ target)
 {
     for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < n; p += (int64_t)gridDim.x * blockDim.x) {
         const int32_t v = live[p];
         if (!grot[gid[v]]) continue;
-        const int64_t t = target[v];
         past[v] = curr[v];
-        curr[v] = t;
-        if (curr32) curr32[v] = (int32_t)t;
+        curr[v] = target[v];
     }
 }
 
@@ -1993,7 +1986,9 @@ struct Phase {
     const vt_graph* g;
     int64_t nv;
     bool et = false;
-    DBuf<int64_t> past, curr, target, csize;
+    // Community ids and sizes are 32-bit here (nv < 2^31): the partition is widened for the
+    // caller at the end of the phase.
+    DBuf<int32_t> past, curr, target, csize;
     DBuf<double> vdeg, cdeg, cw, frozen, pa, pb;
     DBuf<unsigned char> active;
     DBuf<int32_t> lists;     // vertices grouped by (color, degree bucket), vertex order inside
@@ -2014,40 +2009,32 @@ struct Phase {
     const int32_t* gid = nullptr;
     const unsigned char* gact = nullptr;
     double* gconst = nullptr;
-    // Narrow copies read by the group buckets: edges split once per phase, currComm
-    // narrowed before every sweep (it changes between sweeps).
-    DBuf<int32_t> tail32, curr32;
+    // The edges split into 32-bit tails and weights, once per phase (the group buckets read them).
+    DBuf<int32_t> tail32;
     DBuf<double> wgt;
     DBuf<VRec> rec;  // community records, rebuilt before every sweep when the tuning asks
-    // A batch narrows currComm once and keeps curr32 current in its rotation (narrow_once);
-    // its records are packed for the live list only (pack_live, pack_n) when set.
-    bool narrow_once = false, narrowed = false;
+    // A batch packs its records for the live list only (pack_live, pack_n) when set.
     const int32_t* pack_live = nullptr;
     int64_t pack_n = 0;
 
     Phase(vt_ctx* c, const vt_graph* gr) : ctx(c), g(gr), nv(gr->nv) {}
 
-    void prepare_narrow()
+    void prepare_sweep()
     {
-        if constexpr (!kSplitEdges) return;
         if (!tail32.p) {
             const size_t ne1 = (size_t)std::max<int64_t>(g->ne, 1);
             tail32 = DBuf<int32_t>(ctx, ne1);
             wgt = DBuf<double>(ctx, ne1);
-            curr32 = DBuf<int32_t>(ctx, (size_t)std::max<int64_t>(nv, 1));
             if (g->ne)
                 VT_LAUNCH(ctx, "split_edges", k_split_edges, grid_for(g->ne, 256, 16384), 256, 0,
                           (const DEdge*)g->edges, g->ne, tail32.p, wgt.p);
         }
-        if (nv && !(narrow_once && narrowed))
-            VT_LAUNCH(ctx, "narrow_curr", k_narrow_ids, grid_for(nv, 256, 8192), 256, 0, (const int64_t*)curr.p, nv, curr32.p);
-        narrowed = true;
         if (ctx->tuning.vertex_records && nv) {
             if (!rec.p) rec = DBuf<VRec>(ctx, (size_t)nv);
             const int64_t n = pack_live ? pack_n : nv;
             if (n)
-                VT_LAUNCH(ctx, "pack_records", k_pack_records, grid_for(n, 256, 8192), 256, 0, (const int64_t*)curr.p,
-                          (const int64_t*)csize.p, (const double*)cdeg.p, n, pack_live, rec.p);
+                VT_LAUNCH(ctx, "pack_records", k_pack_records, grid_for(n, 256, 8192), 256, 0, (const int32_t*)curr.p,
+                          (const int32_t*)csize.p, (const double*)cdeg.p, n, pack_live, rec.p);
         }
     }
 
@@ -2068,10 +2055,10 @@ struct Phase {
     {
         et = with_et;
         const size_t n = (size_t)std::max<int64_t>(nv, 1);
-        past = DBuf<int64_t>(ctx, n);
-        curr = DBuf<int64_t>(ctx, n);
-        target = DBuf<int64_t>(ctx, n);
-        csize = DBuf<int64_t>(ctx, n);
+        past = DBuf<int32_t>(ctx, n);
+        curr = DBuf<int32_t>(ctx, n);
+        target = DBuf<int32_t>(ctx, n);
+        csize = DBuf<int32_t>(ctx, n);
         vdeg = DBuf<double>(ctx, n);
         cdeg = DBuf<double>(ctx, n);
         cw = DBuf<double>(ctx, n);
@@ -2088,13 +2075,12 @@ struct Phase {
 
     void init_state(bool with_et)
     {
-        if (kSplitEdges && !tail32.p && nv && g->ne <= 48 * nv && g->max_degree <= kSfTile) {
+        if (!tail32.p && nv && g->ne <= 48 * nv && g->max_degree <= kSfTile) {
             // short rows (a row's fold is one thread's, so no long ones): the split copy the
             // local move reads and the degrees in one pass
             const size_t ne1 = (size_t)std::max<int64_t>(g->ne, 1);
             tail32 = DBuf<int32_t>(ctx, ne1);
             wgt = DBuf<double>(ctx, ne1);
-            curr32 = DBuf<int32_t>(ctx, (size_t)nv);
             VT_LAUNCH(ctx, "split_fold", k_split_fold, grid_for(nv, kSfRows, 65536), 256, 0, g->offs, g->edges, nv,
                       tail32.p, wgt.p, vdeg.p);
         } else if (nv && nv < 65536 && g->ne > 48 * nv) {  // few, long rows: a thread per row would leave the GPU idle
@@ -2261,7 +2247,6 @@ struct Phase {
         a.gact = gact;
         a.tail32 = tail32.p;
         a.wgt = wgt.p;
-        a.curr32 = curr32.p;
         a.rec = (ctx->tuning.vertex_records && rec.p) ? rec.p : nullptr;
         return a;
     }
@@ -2274,7 +2259,6 @@ struct Phase {
     template <class K>
     void hub_sweep(const MoveArgs& a, const ColorSweep& cs, int64_t total, int cbits, int kbits)
     {
-        static_assert(kSplitEdges, "the hub keys read the 32-bit tail and community copies");
         const int32_t nh = (int32_t)cs.hub_n;
         // many hubs, none holding much of the work (the coarse levels): a workgroup per hub
         // sorts its segment and moves it; otherwise (BA's level 0: a few hundred or thousand
@@ -2303,10 +2287,10 @@ struct Phase {
             const char* kname = sizeof(K) == 4 ? "hub_keys32" : "hub_keys64";
             if (many)
                 VT_LAUNCH(ctx, kname, k_hub_keys_rows<K>, (unsigned)std::min<int64_t>(nh, 16384), 256, 0, hubs, nh, hoffs,
-                          (const int64_t*)g->offs, (const int32_t*)tail32.p, (const int32_t*)curr32.p, cbits, k0, v0);
+                          (const int64_t*)g->offs, (const int32_t*)tail32.p, (const int32_t*)curr.p, cbits, k0, v0);
             else
                 VT_LAUNCH(ctx, kname, k_hub_keys<K>, grid_for(total, 256, 16384), 256, 0, hubs, nh, hoffs,
-                          (const int64_t*)g->offs, (const int32_t*)tail32.p, (const int32_t*)curr32.p, cbits, k0, v0);
+                          (const int64_t*)g->offs, (const int32_t*)tail32.p, (const int32_t*)curr.p, cbits, k0, v0);
             bool alt = false;
             if (many) {
                 // each hub's entries are already together: sort each hub's segment by the
@@ -2352,7 +2336,7 @@ struct Phase {
 
     void sweep(const ColorSweep& cs)
     {
-        prepare_narrow();
+        prepare_sweep();
         const MoveArgs a = move_args();
         if (cs.lpv_n) {
             const int64_t nblk = std::min<int64_t>((cs.lpv_n + 63) / 64, 16384);
@@ -2406,7 +2390,7 @@ struct Phase {
     // Folds the sweep's moves into localCinfo in processing order, with no host read: the
     // mover count stays on the device (the scan's total sizes the event sort and folds) and
     // is added to iscal[1], the iteration's movers, which the host reads with Q.
-    void apply_moves(const int32_t* order, int64_t n, double* dst_cdeg, int64_t* dst_csize)
+    void apply_moves(const int32_t* order, int64_t n, double* dst_cdeg, int32_t* dst_csize)
     {
         if (n == 0) return;
         int32_t* flags = (int32_t*)scratch(ctx, "mv_flags", 4 * (size_t)n);
@@ -2444,13 +2428,13 @@ struct Phase {
     // is given.
     // The long-run flag (ucount[1]) was cleared by the emission of these events.
     void fold_events(const uint32_t* ks, const uint32_t* vs, int64_t ne, uint32_t none, double* dst_cdeg,
-                     int64_t* dst_csize, const int64_t* d_movers = nullptr)
+                     int32_t* dst_csize, const int64_t* d_movers = nullptr)
     {
-        VT_LAUNCH(ctx, "fold_events", k_fold_events, grid_for(ne, 256, 16384), 256, 0, ks, vs, (const int64_t*)target.p,
+        VT_LAUNCH(ctx, "fold_events", k_fold_events, grid_for(ne, 256, 16384), 256, 0, ks, vs, (const int32_t*)target.p,
                   (const double*)vdeg.p, ne, d_movers, dst_cdeg, dst_csize, none, ucount.p + 1);
         if (ne >= kFoldLongRun)
             VT_LAUNCH(ctx, "fold_events_long", k_fold_events_long, grid_for(ne, 256, 4096), 256, 0, ks, vs,
-                      (const int64_t*)target.p, (const double*)vdeg.p, ne, d_movers, dst_cdeg, dst_csize, none,
+                      (const int32_t*)target.p, (const double*)vdeg.p, ne, d_movers, dst_cdeg, dst_csize, none,
                       (const unsigned long long*)(ucount.p + 1));
     }
 
@@ -2590,8 +2574,8 @@ double phase_end(vt_ctx* ctx, vt_phase* st, int64_t* cvect_out, int32_t* iters_o
     vt_graph* g = st->g;
     const int64_t nv = g->nv;
     if (!g->part) g->part = (int64_t*)dalloc(ctx, 8 * (size_t)std::max<int64_t>(nv, 1));
-    d2d(ctx, g->part, ph.past.p, 8 * (size_t)nv);
-    if (cvect_out) d2h(ctx, cvect_out, ph.past.p, 8 * (size_t)nv);
+    VT_LAUNCH(ctx, "widen_part", k_widen_ids, grid_for(nv, 256, 8192), 256, 0, (const int32_t*)ph.past.p, nv, g->part);
+    if (cvect_out) d2h(ctx, cvect_out, g->part, 8 * (size_t)nv);
     sync(ctx);
     if (iters_out) *iters_out = st->numIters;
     return st->prevMod;
@@ -2690,7 +2674,6 @@ void batch_phase(vt_ctx* ctx, vt_graph* u, const int32_t* d_gid, const SegSums& 
         sync(ctx);
     };
     build_live();
-    ph.narrow_once = true;  // k_batch_rotate keeps curr32 equal to curr from here on
     ph.pack_live = live.p;
     ph.pack_n = nlive;
 
@@ -2704,12 +2687,12 @@ void batch_phase(vt_ctx* ctx, vt_graph* u, const int32_t* d_gid, const SegSums& 
         ph.sweep(ph.sweeps[0]);
         if (nlive) {
             VT_LAUNCH(ctx, "batch_flags", k_batch_flags, grid_for(nlive, 256, 8192), 256, 0, nlive,
-                      (const int32_t*)live.p, (const int64_t*)ph.target.p, (const int64_t*)ph.curr.p, d_gid,
+                      (const int32_t*)live.p, (const int32_t*)ph.target.p, (const int32_t*)ph.curr.p, d_gid,
                       (const unsigned char*)gact.p, mflags);
             dev_scan_i32(ctx, mflags, mpos, d_nlive, nlive, d_movers, "bmv_part");
             VT_LAUNCH(ctx, "emit_events", k_emit_events, grid_for(nlive, 256, 8192), 256, 0, (const int32_t*)live.p,
-                      nlive, (const int32_t*)mflags, (const int32_t*)mpos, (const int64_t*)ph.target.p,
-                      (const int64_t*)ph.curr.p, k0, v0, ph.ucount.p + 1);
+                      nlive, (const int32_t*)mflags, (const int32_t*)mpos, (const int32_t*)ph.target.p,
+                      (const int32_t*)ph.curr.p, k0, v0, ph.ucount.p + 1);
         } else {
             dzero(ctx, d_movers, 8);  // every graph has left: no events
         }
@@ -2724,7 +2707,7 @@ void batch_phase(vt_ctx* ctx, vt_graph* u, const int32_t* d_gid, const SegSums& 
         if (nlive)
             VT_LAUNCH(ctx, "batch_rotate", k_batch_rotate, grid_for(nlive, 256, 8192), 256, 0, nlive,
                       (const int32_t*)live.p, d_gid, (const unsigned char*)grot.p, ph.past.p, ph.curr.p,
-                      (const int64_t*)ph.target.p, ph.curr32.p);
+                      (const int32_t*)ph.target.p);
     };
 
     hipGraphExec_t gexec = nullptr;
@@ -2804,7 +2787,7 @@ void batch_phase(vt_ctx* ctx, vt_graph* u, const int32_t* d_gid, const SegSums& 
     }
     release();
     if (!u->part) u->part = (int64_t*)dalloc(ctx, 8 * (size_t)std::max<int64_t>(nv, 1));
-    d2d(ctx, u->part, ph.past.p, 8 * (size_t)nv);
+    VT_LAUNCH(ctx, "widen_part", k_widen_ids, grid_for(nv, 256, 8192), 256, 0, (const int32_t*)ph.past.p, nv, u->part);
     q_out.assign((size_t)ng, 0.0);
     iters_out.assign((size_t)ng, 0);
     d2h(ctx, q_out.data(), gprev.p, 8 * (size_t)ng);
@@ -3086,11 +3069,17 @@ int vt_phase_get_state(vt_ctx* ctx, const vt_phase* st, int64_t* curr, int64_t* 
         VT_HIP(ctx, hipSetDevice(ctx->device));
         const Phase& ph = st->ph;
         const size_t b8 = 8 * (size_t)ph.nv;
-        if (curr) d2h(ctx, curr, ph.curr.p, b8);
-        if (csize) d2h(ctx, csize, ph.csize.p, b8);
+        DBuf<int64_t> wide(ctx, (size_t)std::max<int64_t>(ph.nv, 1));
+        auto ids = [&](int64_t* dst, const int32_t* src) {
+            if (!dst) return;
+            VT_LAUNCH(ctx, "widen_ids", k_widen_ids, grid_for(ph.nv, 256, 8192), 256, 0, src, ph.nv, wide.p);
+            d2h(ctx, dst, wide.p, b8);
+        };
+        ids(curr, ph.curr.p);
+        ids(csize, ph.csize.p);
+        ids(target, ph.target.p);
         if (cdeg) d2h(ctx, cdeg, ph.cdeg.p, b8);
         if (vdeg) d2h(ctx, vdeg, ph.vdeg.p, b8);
-        if (target) d2h(ctx, target, ph.target.p, b8);
         if (cw) d2h(ctx, cw, ph.cw.p, b8);
         if (constant) d2h(ctx, constant, ph.scal.p + 2, 8);
     });
@@ -3147,23 +3136,32 @@ int vt_sweep(vt_ctx* ctx, const vt_graph* g, const int64_t* curr, const int64_t*
         Phase ph(ctx, g);
         ph.alloc(false);
         const size_t b8 = 8 * (size_t)nv;
-        h2d(ctx, ph.curr.p, curr, b8);
-        h2d(ctx, ph.csize.p, csize, b8);
+        DBuf<int64_t> wide(ctx, (size_t)std::max<int64_t>(nv, 1));
+        auto ids = [&](const int64_t* src, int32_t* dst) {
+            h2d(ctx, wide.p, src, b8);
+            VT_LAUNCH(ctx, "narrow_ids", k_narrow_ids, grid_for(nv, 256, 8192), 256, 0, (const int64_t*)wide.p, nv, dst);
+        };
+        auto ids_out = [&](int64_t* dst, const int32_t* src) {
+            VT_LAUNCH(ctx, "widen_ids", k_widen_ids, grid_for(nv, 256, 8192), 256, 0, src, nv, wide.p);
+            d2h(ctx, dst, wide.p, b8);
+        };
+        ids(curr, ph.curr.p);
+        ids(csize, ph.csize.p);
         h2d(ctx, ph.cdeg.p, cdeg, b8);
         h2d(ctx, ph.vdeg.p, vdeg, b8);
         h2d(ctx, ph.constant(), &constant, 8);
         ph.build_lists(nullptr, 1, false);
         ph.sweep(ph.sweeps[0]);
-        if (target_out) d2h(ctx, target_out, ph.target.p, b8);
+        if (target_out) ids_out(target_out, ph.target.p);
         if (cw_out) d2h(ctx, cw_out, ph.cw.p, b8);
         if (dsize_out || ddeg_out) {
             DBuf<double> dd(ctx, (size_t)std::max<int64_t>(nv, 1));
-            DBuf<int64_t> ds(ctx, (size_t)std::max<int64_t>(nv, 1));
+            DBuf<int32_t> ds(ctx, (size_t)std::max<int64_t>(nv, 1));
             dzero(ctx, dd.p, b8);
-            dzero(ctx, ds.p, b8);
+            dzero(ctx, ds.p, 4 * (size_t)nv);
             ph.apply_moves(nullptr, nv, dd.p, ds.p);
             if (ddeg_out) d2h(ctx, ddeg_out, dd.p, b8);
-            if (dsize_out) d2h(ctx, dsize_out, ds.p, b8);
+            if (dsize_out) ids_out(dsize_out, ds.p);
         }
         sync(ctx);
     });
