@@ -203,6 +203,13 @@ void d2h(vt_ctx* ctx, void* dst, const void* src, size_t bytes)
     }
     ctx->stage_off = 0;  // the stream has drained: every staged copy has run
 }
+// Pinned host memory a kernel writes an iteration's scalars to (64 bytes): they are there when
+// the stream has drained, with no copy queued behind the kernel.
+double* mail(vt_ctx* ctx)
+{
+    if (!ctx->mail) VT_HIP(ctx, hipHostMalloc((void**)&ctx->mail, 64, hipHostMallocDefault));
+    return ctx->mail;
+}
 void d2d(vt_ctx* ctx, void* dst, const void* src, size_t bytes)
 {
     if (bytes) VT_HIP(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, ctx->stream));
@@ -293,7 +300,7 @@ __global__ void __launch_bounds__(kSumBlock) k_sum2_final(const double2* __restr
 
 // The blocking of an n-element tree sum: at most kSumGrid blocks, four strides of 256
 // elements per block at least.  A function of n alone.
-static void sum2_plan(int64_t n, int64_t* grid_out, int64_t* chunk_out)
+void sum2_plan(int64_t n, int64_t* grid_out, int64_t* chunk_out)
 {
     int64_t grid = (n + 4 * kSumBlock - 1) / (4 * kSumBlock);
     if (grid < 1) grid = 1;
@@ -692,6 +699,7 @@ int vt_ctx_destroy(vt_ctx* ctx)
     for (auto e : ctx->event_pool) (void)hipEventDestroy(e);
     (void)hipStreamDestroy(ctx->stream);
     if (ctx->stage) (void)hipHostFree(ctx->stage);
+    if (ctx->mail) (void)hipHostFree(ctx->mail);
     delete ctx;
     return VT_OK;
 }

@@ -63,6 +63,7 @@ struct vt_ctx {
     // ring restarts whenever the stream has drained (sync, d2h).
     unsigned char* stage = nullptr;
     size_t stage_off = 0;
+    double* mail = nullptr;  // pinned: Q and the movers of an iteration (vt::mail)
     // sweep launch shape (performance only: every setting gives the same results)
     vt_tuning tuning = {{7, 15, 31, 63, 127, 1023}, 16384};  // replaced by default_tuning() at creation
 };
@@ -158,6 +159,7 @@ void sync(vt_ctx* ctx);
 void h2d(vt_ctx* ctx, void* dst, const void* src, size_t bytes);
 void d2h(vt_ctx* ctx, void* dst, const void* src, size_t bytes);
 void d2d(vt_ctx* ctx, void* dst, const void* src, size_t bytes);
+double* mail(vt_ctx* ctx);
 void dzero(vt_ctx* ctx, void* dst, size_t bytes);
 
 inline unsigned grid_for(int64_t n, int block, int64_t cap = 1 << 20)
@@ -204,6 +206,7 @@ __device__ __forceinline__ double readlane_f64(double x, int j)
 // ---- device primitives (vt_prims.hip) -------------------------------------------------
 // Deterministic fixed-order sums: every block reduces a fixed contiguous chunk with a
 // fixed tree; block partials are reduced by one block in index order.
+void sum2_plan(int64_t n, int64_t* grid_out, int64_t* chunk_out);  // tree_sum2's blocking, of n alone
 void tree_sum2(vt_ctx* ctx, const double* a, const double* b_sq, int64_t n, double* d_out2);
 void seq_sum2(vt_ctx* ctx, const double* a, const double* b_sq, int64_t n, double* d_out2);
 // The same sums per graph of a batch of disjoint graphs (vertex ranges voff[g]..voff[g+1]),

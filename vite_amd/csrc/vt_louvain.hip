@@ -1744,17 +1744,532 @@ __global__ void __launch_bounds__(256) k_fold_events_long(const uint32_t* __rest
     }
 }
 
+// ---- event folds without a sort (graphs of at most kEvVerts vertices) ------------------------
+// The same per-community folds in fewer launches.  The radix sort's three kernels per digit
+// and the flags, scan and emission are thirteen launches of a few microseconds each, whatever
+// the event count; here every community's events are counted with atomics, placed by a
+// running cursor in any order, and each run, a handful of events, is put in processing order
+// by whoever folds it: a thread (up to 8 events, a register sorting network), a wave (up to
+// 64, a bitonic sort over its lanes), or a workgroup (longer: a bit per possible event in
+// LDS, which bounds kEvVerts).  An event is its position in processing order with the
+// departure bit below it, so ascending events are the order in which one thread of the
+// reference applies them, and the folds are those of k_fold_events.
+#ifndef VT_EV_VERTS
+#define VT_EV_VERTS 524288
+#endif
+constexpr int64_t kEvVerts = VT_EV_VERTS;
+constexpr uint32_t kEvRunThread = 8;
+constexpr uint32_t kEvRunWave = 64;
+
+struct MoverArgs {
+    const int32_t* order;  // processing order, or null for vertex order
+    int64_t n;             // positions
+    const int32_t* target;
+    const int32_t* curr;
+    const unsigned char* active;  // null when ET is off
+};
+
+// Whether position p moves (k_mover_flags' rule), its vertex and its two communities.
+__device__ __forceinline__ bool mover_at(const MoverArgs& m, int64_t p, int32_t& v, int32_t& t, int32_t& c)
+{
+    v = m.order ? m.order[p] : (int32_t)p;
+    t = m.target[v];
+    c = m.curr[v];
+    return t != c && !(m.active && !m.active[v]);
+}
+
+// ctl: [0] the running cursor, [1] the long runs' count, [2] the medium runs' count.
+__global__ void __launch_bounds__(256) k_ev_count(MoverArgs m, uint32_t* __restrict__ cnt, uint2* __restrict__ rank,
+                                                  uint32_t* __restrict__ ctl, unsigned long long* __restrict__ movers)
+{
+    if (blockIdx.x == 0 && threadIdx.x == 0) ctl[0] = ctl[1] = ctl[2] = 0;
+    unsigned mine = 0;
+    for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < m.n; p += (int64_t)gridDim.x * blockDim.x) {
+        int32_t v, t, c;
+        if (!mover_at(m, p, v, t, c)) continue;
+        uint2 r;
+        r.x = atomicAdd(&cnt[t], 1u);
+        r.y = atomicAdd(&cnt[c], 1u);
+        rank[p] = r;
+        mine++;
+    }
+    for (int o = 32; o > 0; o >>= 1) mine += __shfl_xor(mine, o);
+    __shared__ unsigned s_wave[4];
+    if ((threadIdx.x & 63) == 0) s_wave[threadIdx.x >> 6] = mine;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        mine = s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
+        if (mine) atomicAdd(movers, (unsigned long long)mine);
+    }
+}
+
+// Each community's place in the event array, one cursor update per workgroup of 1024 (one per
+// wave of 64 queued at the cursor: 17.5 us at n = 131072 against 5), and the lists of the runs
+// that are more than a thread's.
+__global__ void __launch_bounds__(1024) k_ev_alloc(int64_t nv, const uint32_t* __restrict__ cnt, uint32_t* __restrict__ base,
+                                                   uint32_t* __restrict__ ctl, int32_t* __restrict__ longs,
+                                                   int32_t* __restrict__ mids)
+{
+    __shared__ uint32_t s_wave[16];
+    __shared__ uint32_t s_base;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int64_t c0 = blockIdx.x * (int64_t)1024; c0 < nv; c0 += (int64_t)gridDim.x * 1024) {
+        const int64_t c = c0 + threadIdx.x;
+        const uint32_t s = c < nv ? cnt[c] : 0;
+        uint32_t x = s;
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(x, o);
+            if (lane >= o) x += y;
+        }
+        if (lane == 63) s_wave[w] = x;
+        __syncthreads();
+        uint32_t before = 0, all = 0;
+        for (int k = 0; k < 16; k++) {
+            if (k < w) before += s_wave[k];
+            all += s_wave[k];
+        }
+        if (threadIdx.x == 0) s_base = all ? atomicAdd(&ctl[0], all) : 0;
+        __syncthreads();
+        if (s) base[c] = s_base + before + x - s;
+        auto list = [&](bool in, uint32_t* count, int32_t* ids) {  // one cursor update per wave
+            const unsigned long long b = __ballot(in);
+            if (!b) return;
+            uint32_t at = 0;
+            if (lane == 0) at = atomicAdd(count, (uint32_t)__popcll(b));
+            at = __shfl(at, 0);
+            if (in) ids[at + __popcll(b & ((1ull << lane) - 1))] = (int32_t)c;
+        };
+        list(s > kEvRunWave, &ctl[1], longs);
+        list(s > kEvRunThread && s <= kEvRunWave, &ctl[2], mids);
+    }
+}
+
+__global__ void k_ev_scatter(MoverArgs m, const uint32_t* __restrict__ base, const uint2* __restrict__ rank,
+                             uint32_t* __restrict__ ev)
+{
+    for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < m.n; p += (int64_t)gridDim.x * blockDim.x) {
+        int32_t v, t, c;
+        if (!mover_at(m, p, v, t, c)) continue;
+        const uint2 r = rank[p];
+        ev[base[t] + r.x] = (uint32_t)p << 1;
+        ev[base[c] + r.y] = (uint32_t)p << 1 | 1u;
+    }
+}
+
+__device__ __forceinline__ double event_weight(uint32_t e, const int32_t* __restrict__ order, const double* __restrict__ vdeg)
+{
+    const int32_t p = (int32_t)(e >> 1);
+    const double k = vdeg[order ? order[p] : p];
+    return (e & 1u) ? -k : k;
+}
+
+// The fold of `s` values held by the lanes of a wave in lane order (lanes past s: -0.0).
+__device__ __forceinline__ double wave_fold(double acc, double d, int s)
+{
+    for (int u = 0; u < s; u += 8)
+#pragma unroll
+        for (int k = 0; k < 8; k++) acc = acc + readlane_f64(d, u + k);
+    return acc;
+}
+
+__device__ __forceinline__ void order2(uint32_t& a, uint32_t& b)
+{
+    const uint32_t lo = min(a, b), hi = max(a, b);
+    a = lo;
+    b = hi;
+}
+
+// The short runs by a thread each, then the medium ones, from their list, by a wave each (a
+// wave taking those among its own 64 communities instead held the launch for 117 us on BA
+// n = 131000, whose busy communities have neighbouring ids).
+__global__ void __launch_bounds__(256) k_ev_fold(int64_t nv, uint32_t* __restrict__ cnt, const uint32_t* __restrict__ base,
+                                                 const uint32_t* __restrict__ ctl, const int32_t* __restrict__ mids,
+                                                 const uint32_t* __restrict__ ev, const int32_t* __restrict__ order,
+                                                 const double* __restrict__ vdeg, double* __restrict__ cdeg,
+                                                 int32_t* __restrict__ csize)
+{
+    for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < nv; c += (int64_t)gridDim.x * blockDim.x) {
+        const uint32_t s = cnt[c];
+        if (s && s <= kEvRunThread) {
+            const uint32_t b = base[c];
+            uint32_t e[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) e[k] = (uint32_t)k < s ? ev[b + k] : 0xffffffffu;
+            if (s > 1) {  // Batcher's network for 8
+                order2(e[0], e[1]); order2(e[2], e[3]); order2(e[4], e[5]); order2(e[6], e[7]);
+                order2(e[0], e[2]); order2(e[1], e[3]); order2(e[4], e[6]); order2(e[5], e[7]);
+                order2(e[1], e[2]); order2(e[5], e[6]);
+                order2(e[0], e[4]); order2(e[1], e[5]); order2(e[2], e[6]); order2(e[3], e[7]);
+                order2(e[2], e[4]); order2(e[3], e[5]);
+                order2(e[1], e[2]); order2(e[3], e[4]); order2(e[5], e[6]);
+            }
+            double d[8];
+            int change = 0;
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                d[k] = -0.0;  // leaves any sum unchanged
+                if ((uint32_t)k < s) {
+                    d[k] = event_weight(e[k], order, vdeg);
+                    change += (e[k] & 1u) ? -1 : 1;
+                }
+            }
+            double acc = 0.0;
+#pragma unroll
+            for (int k = 0; k < 8; k++) acc = acc + d[k];
+            cdeg[c] = cdeg[c] + acc;
+            csize[c] += change;
+            cnt[c] = 0;
+        }
+    }
+    const int lane = threadIdx.x & 63;
+    const uint32_t nm = ctl[2];
+    for (uint32_t i = blockIdx.x * 4 + (threadIdx.x >> 6); i < nm; i += gridDim.x * 4) {
+        const int32_t c = mids[i];
+        const int s = (int)cnt[c];
+        uint32_t e = lane < s ? ev[base[c] + lane] : 0xffffffffu;
+        for (int k = 2; k <= 64; k <<= 1)
+            for (int o = k >> 1; o > 0; o >>= 1) {
+                const uint32_t x = __shfl_xor(e, o);
+                const bool keep_min = ((lane & k) == 0) == ((lane & o) == 0);
+                e = keep_min ? min(e, x) : max(e, x);
+            }
+        const bool in = lane < s;
+        const double acc = wave_fold(0.0, in ? event_weight(e, order, vdeg) : -0.0, s);
+        const int left = __popcll(__ballot(in && (e & 1u)));
+        if (lane == 0) {
+            cdeg[c] = cdeg[c] + acc;
+            csize[c] += s - 2 * left;
+            cnt[c] = 0;
+        }
+    }
+}
+
+// The long runs, a workgroup each: the run's events set their bits in LDS, every thread reads
+// back a stretch of the bits, and a scan of the threads' counts gives each its place in the
+// sorted run, which overwrites the unsorted one; wave 0 then folds it.
+__global__ void __launch_bounds__(256) k_ev_fold_long(MoverArgs m, const uint32_t* __restrict__ ctl,
+                                                      const int32_t* __restrict__ longs, uint32_t* __restrict__ cnt,
+                                                      const uint32_t* __restrict__ base, uint32_t* __restrict__ ev,
+                                                      const double* __restrict__ vdeg, double* __restrict__ cdeg,
+                                                      int32_t* __restrict__ csize)
+{
+    __shared__ uint32_t bits[2 * kEvVerts / 32];
+    __shared__ uint32_t s_wave[4];
+    const uint32_t nl = ctl[1];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int per = (int)((2 * m.n + 32 * 256 - 1) / (32 * 256));  // words per thread
+    for (uint32_t i = blockIdx.x; i < nl; i += gridDim.x) {
+        const int32_t c = longs[i];
+        const uint32_t s = cnt[c], b = base[c];
+        for (int k = threadIdx.x; k < per * 256; k += 256) bits[k] = 0;
+        __syncthreads();
+        for (uint32_t k = threadIdx.x; k < s; k += 256) {
+            const uint32_t e = ev[b + k];
+            atomicOr(&bits[e >> 5], 1u << (e & 31));
+        }
+        __syncthreads();
+        uint32_t sum = 0;
+        for (int k = 0; k < per; k++) sum += __popc(bits[threadIdx.x * per + k]);
+        uint32_t inc = sum;
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(inc, o);
+            if (lane >= o) inc += y;
+        }
+        if (lane == 63) s_wave[w] = inc;
+        __syncthreads();
+        uint32_t at = b + inc - sum;
+        for (int k = 0; k < w; k++) at += s_wave[k];
+        for (int k = 0; k < per; k++)
+            for (uint32_t x = bits[threadIdx.x * per + k]; x; x &= x - 1)
+                ev[at++] = (uint32_t)(threadIdx.x * per + k) * 32 + (uint32_t)__builtin_ctz(x);
+        __syncthreads();
+        if (w == 0) {
+            double acc = 0.0;
+            int change = 0;
+            for (uint32_t k = 0; k < s; k += 64) {
+                const bool in = k + lane < s;
+                const uint32_t e = in ? ev[b + k + lane] : 0;
+                const int here = (int)min(s - k, 64u);
+                acc = wave_fold(acc, in ? event_weight(e, m.order, vdeg) : -0.0, here);
+                change += here - 2 * __popcll(__ballot(in && (e & 1u)));
+            }
+            if (lane == 0) {
+                cdeg[c] = cdeg[c] + acc;
+                csize[c] += change;
+                cnt[c] = 0;
+            }
+        }
+        __syncthreads();  // the bits are reused
+    }
+}
+
+// ---- the end of an iteration in one workgroup (graphs of at most kTailVerts vertices) --------
+// Small graphs and the coarse levels of large ones spend their time in launches, not in work:
+// the event folds above are five launches and the modularity two, each a few microseconds for
+// a few thousand vertices.  Here one workgroup counts, places and folds the events in LDS and
+// forms the modularity, in the order and with the trees of the separate kernels.
+constexpr int kTailVerts = 8192;
+constexpr int kTailBlock = 1024;
+constexpr int kTailRun = 24;  // events a thread orders by insertion; longer runs take a wave each
+
+struct TailArgs {
+    MoverArgs m;
+    int32_t nv;
+    const double* vdeg;
+    double* cdeg;
+    int32_t* csize;
+    unsigned long long* movers;  // the iteration's movers so far
+    // the modularity (cw null: folds only); the sums go to sums[0..1], Q and the movers to out
+    const double* cw;
+    const double* constant;
+    int64_t chunk;  // tree_sum2's blocking of nv elements
+    int32_t blocks;
+    double* sums;
+    double* out;
+};
+
+__global__ void __launch_bounds__(kTailBlock) k_tail_small(TailArgs a)
+{
+    __shared__ uint32_t cur[kTailVerts];     // events per community, then the end of its run so far
+    __shared__ uint16_t ev[2 * kTailVerts];  // runs of positions, top bit: departure
+    __shared__ uint16_t lt[kTailVerts], lc[kTailVerts];
+    __shared__ uint16_t s_long[2 * kTailVerts / kTailRun];
+    __shared__ uint32_t s_wave[kTailBlock / 64];
+    __shared__ uint32_t s_nlong;
+    __shared__ double s_part[2][kTailVerts / (4 * 256)];
+    constexpr uint16_t kNone = 0xffff;
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int n = (int)a.m.n;
+    for (int c = t; c < a.nv; c += kTailBlock) cur[c] = 0;
+    if (t == 0) s_nlong = 0;
+    __syncthreads();
+    unsigned mine = 0;
+    for (int p = t; p < n; p += kTailBlock) {
+        int32_t v, tg, c;
+        const bool mv = mover_at(a.m, p, v, tg, c);
+        lt[p] = mv ? (uint16_t)tg : kNone;
+        lc[p] = mv ? (uint16_t)c : kNone;
+        if (mv) {
+            atomicAdd(&cur[tg], 1u);
+            atomicAdd(&cur[c], 1u);
+            mine++;
+        }
+    }
+    for (int o = 32; o > 0; o >>= 1) mine += __shfl_xor(mine, o);
+    if (lane == 0) s_wave[w] = mine;
+    __syncthreads();
+    unsigned moved = 0;
+    for (int k = 0; k < kTailBlock / 64; k++) moved += s_wave[k];
+    __syncthreads();
+    if (moved) {  // uniform
+        // exclusive scan of the counts: thread t takes kTailVerts / kTailBlock consecutive ones
+        constexpr int kPer = kTailVerts / kTailBlock;
+        uint32_t x[kPer], sum = 0;
+#pragma unroll
+        for (int k = 0; k < kPer; k++) {
+            const int c = t * kPer + k;
+            x[k] = c < a.nv ? cur[c] : 0;
+            sum += x[k];
+        }
+        uint32_t inc = sum;
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(inc, o);
+            if (lane >= o) inc += y;
+        }
+        if (lane == 63) s_wave[w] = inc;
+        __syncthreads();
+        uint32_t run = inc - sum;
+        for (int k = 0; k < w; k++) run += s_wave[k];
+#pragma unroll
+        for (int k = 0; k < kPer; k++) {
+            const int c = t * kPer + k;
+            if (c < a.nv) cur[c] = run;
+            run += x[k];
+        }
+        __syncthreads();
+        for (int p = t; p < n; p += kTailBlock) {
+            if (lt[p] == kNone) continue;
+            ev[atomicAdd(&cur[lt[p]], 1u)] = (uint16_t)p;
+            ev[atomicAdd(&cur[lc[p]], 1u)] = (uint16_t)(p | 0x8000);
+        }
+        __syncthreads();
+        for (int c = t; c < a.nv; c += kTailBlock) {
+            const uint32_t b = c ? cur[c - 1] : 0, s = cur[c] - b;
+            if (s == 0) continue;
+            if (s > (uint32_t)kTailRun) {
+                s_long[atomicAdd(&s_nlong, 1u)] = (uint16_t)c;
+                continue;
+            }
+            for (uint32_t k = 1; k < s; k++) {  // by position
+                const uint16_t e = ev[b + k];
+                uint32_t j = k;
+                while (j > 0 && (ev[b + j - 1] & 0x7fff) > (e & 0x7fff)) {
+                    ev[b + j] = ev[b + j - 1];
+                    j--;
+                }
+                ev[b + j] = e;
+            }
+            double acc = 0.0;
+            int change = 0;
+            for (uint32_t k = 0; k < s; k++) {
+                const uint16_t e = ev[b + k];
+                const int p = e & 0x7fff;
+                const double kv = a.vdeg[a.m.order ? a.m.order[p] : p];
+                acc = acc + ((e & 0x8000) ? -kv : kv);
+                change += (e & 0x8000) ? -1 : 1;
+            }
+            a.cdeg[c] = a.cdeg[c] + acc;
+            a.csize[c] += change;
+        }
+        __syncthreads();
+        // long runs: a wave meets the community's events in order by walking the positions
+        for (uint32_t i = w; i < s_nlong; i += kTailBlock / 64) {
+            const int c = s_long[i];
+            double acc = 0.0;
+            int change = 0;
+            for (int p0 = 0; p0 < n; p0 += 64) {
+                const int p = p0 + lane;
+                const bool in = p < n && lt[p] == c, out = p < n && lc[p] == c;
+                const unsigned long long hits = __ballot(in || out);
+                if (!hits) continue;
+                double d = 0.0;
+                if (in || out) {
+                    d = a.vdeg[a.m.order ? a.m.order[p] : p];
+                    d = in ? d : -d;
+                }
+                for (unsigned long long h = hits; h; h &= h - 1) acc = acc + readlane_f64(d, __builtin_ctzll(h));
+                change += __popcll(hits) - 2 * __popcll(__ballot(out));
+            }
+            if (lane == 0) {
+                a.cdeg[c] = a.cdeg[c] + acc;
+                a.csize[c] += change;
+            }
+        }
+        if (t == 0) *a.movers += moved;
+        __syncthreads();
+    }
+    if (!a.cw) return;
+    // tree_sum2's blocks of 256 threads, four at a time, in ev's space
+    double* sa = (double*)ev;
+    double* sb = sa + kTailBlock;
+    const int sub = t & 255;
+    for (int b0 = 0; b0 < a.blocks; b0 += kTailBlock / 256) {
+        const int b = b0 + (t >> 8);
+        const int64_t lo = (int64_t)b * a.chunk;
+        const int64_t hi = b < a.blocks ? min(lo + a.chunk, (int64_t)a.nv) : lo;
+        double xa = 0.0, xb = 0.0;
+        for (int64_t i = lo + sub; i < hi; i += 256) {
+            xa = xa + a.cw[i];
+            const double v = a.cdeg[i];
+            xb = xb + v * v;
+        }
+        sa[t] = xa;
+        sb[t] = xb;
+        __syncthreads();
+        for (int h = 128; h > 0; h >>= 1) {
+            if (sub < h) {
+                sa[t] = sa[t] + sa[t + h];
+                sb[t] = sb[t] + sb[t + h];
+            }
+            __syncthreads();
+        }
+        if (sub == 0 && b < a.blocks) {
+            s_part[0][b] = sa[t];
+            s_part[1][b] = sb[t];
+        }
+        __syncthreads();
+    }
+    if (t == 0) {
+        // k_sum2_final's halving tree over the (at most 8) partials; its other entries are zeros
+        double r[2];
+        for (int q = 0; q < 2; q++) {
+            double y[8];
+            for (int k = 0; k < 8; k++) y[k] = 0.0 + (k < a.blocks ? s_part[q][k] : 0.0);
+            for (int h = 4; h > 0; h >>= 1)
+                for (int k = 0; k < h; k++) y[k] = y[k] + y[k + h];
+            r[q] = y[0];
+            a.sums[q] = y[0];
+        }
+        const double c = a.constant[0];
+        a.out[0] = fabs((r[0] * c) - (r[1] * c * c));
+        ((unsigned long long*)a.out)[1] = *a.movers;
+        *a.movers = 0;
+    }
+}
+
 // currMod = |e_xx*c - a2_x*c*c| (louvain.cpp:2518-2524).
-// movers (or null): the iteration's mover count, copied to movers_out so that one read
-// returns it with the value.
+// movers (or null): the iteration's mover count, copied to q[1] so that one read returns it
+// with the value, and cleared for the next iteration.
 __global__ void k_modularity(const double* __restrict__ sums, const double* __restrict__ constant,
-                             double* __restrict__ q, const int64_t* __restrict__ movers,
-                             int64_t* __restrict__ movers_out)
+                             double* __restrict__ q, int64_t* __restrict__ movers)
 {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
         const double c = constant[0];
         q[0] = fabs((sums[0] * c) - (sums[1] * c * c));
-        if (movers) movers_out[0] = movers[0];
+        if (movers) {
+            ((int64_t*)q)[1] = movers[0];
+            movers[0] = 0;
+        }
+    }
+}
+
+// tree_sum2 and k_modularity in one launch: the block that finishes last reduces the blocks'
+// partial sums as k_sum2_final does (the same trees, so the same bits).  out (pinned host
+// memory) receives Q and the iteration's movers; done counts the finished blocks and is left 0.
+__global__ void __launch_bounds__(256) k_modularity_tree(const double* __restrict__ cw, const double* __restrict__ cdeg,
+                                                         int64_t n, int64_t chunk, double2* __restrict__ part,
+                                                         uint32_t* __restrict__ done, const double* __restrict__ constant,
+                                                         double* __restrict__ sums, unsigned long long* __restrict__ movers,
+                                                         double* __restrict__ out)
+{
+    __shared__ double sa[256], sb[256];
+    __shared__ bool s_last;
+    const int t = threadIdx.x;
+    auto reduce = [&](double xa, double xb) {
+        sa[t] = xa;
+        sb[t] = xb;
+        __syncthreads();
+        for (int h = 128; h > 0; h >>= 1) {
+            if (t < h) {
+                sa[t] = sa[t] + sa[t + h];
+                sb[t] = sb[t] + sb[t + h];
+            }
+            __syncthreads();
+        }
+    };
+    const int64_t lo = (int64_t)blockIdx.x * chunk;
+    const int64_t hi = (lo + chunk < n) ? lo + chunk : n;
+    double xa = 0.0, xb = 0.0;
+    for (int64_t i = lo + t; i < hi; i += 256) {
+        xa = xa + cw[i];
+        const double v = cdeg[i];
+        xb = xb + v * v;
+    }
+    reduce(xa, xb);
+    if (t == 0) {
+        part[blockIdx.x] = make_double2(sa[0], sb[0]);
+        __threadfence();  // the partial is visible to whoever sees the count
+        s_last = atomicAdd(done, 1u) + 1 == gridDim.x;
+    }
+    __syncthreads();
+    if (!s_last) return;
+    __threadfence();
+    xa = 0.0;
+    xb = 0.0;
+    for (unsigned i = t; i < gridDim.x; i += 256) {
+        const double2 x = part[i];
+        xa = xa + x.x;
+        xb = xb + x.y;
+    }
+    reduce(xa, xb);
+    if (t == 0) {
+        sums[0] = sa[0];
+        sums[1] = sb[0];
+        const double c = constant[0];
+        out[0] = fabs((sa[0] * c) - (sb[0] * c * c));
+        ((unsigned long long*)out)[1] = *movers;
+        *movers = 0;
+        *done = 0;
     }
 }
 
@@ -1993,9 +2508,12 @@ struct Phase {
     DBuf<unsigned char> active;
     DBuf<int32_t> lists;     // vertices grouped by (color, degree bucket), vertex order inside
     DBuf<int32_t> corder;    // vertices by color, vertex order inside (event order for color modes)
-    DBuf<double> scal;       // [0..1] sums, [2] constant, [3] q, [4] the iteration's movers (int64 bits)
-    DBuf<int64_t> iscal;     // [0] movers of the last apply, [1] of the iteration, [2] scan length
+    DBuf<double> scal;       // [0..1] sums, [2] constant
+    DBuf<int64_t> iscal;     // [0] movers of the last apply, [1] of the iteration (cleared with Q), [2] scan length
+    // [0] frozen vertices, [1] the long-run flag, [2..3] the event cursor and the long and
+    // medium runs (32 bits each), [4] finished blocks of the modularity (32 bits)
     DBuf<unsigned long long> ucount;
+    DBuf<uint32_t> ev_cnt;   // events per community, zero between uses
     std::vector<ColorSweep> sweeps;      // per color (one entry in plain/vorder)
     std::vector<int64_t> color_ptr;      // colorPtr (louvain.cpp:647-661)
     int64_t hub_cap = 0;
@@ -2049,7 +2567,6 @@ struct Phase {
 
     double* sums() { return scal.p; }
     double* constant() { return scal.p + 2; }
-    double* q() { return scal.p + 3; }
 
     void alloc(bool with_et)
     {
@@ -2070,7 +2587,9 @@ struct Phase {
         }
         scal = DBuf<double>(ctx, 8);
         iscal = DBuf<int64_t>(ctx, 4);
-        ucount = DBuf<unsigned long long>(ctx, 4);
+        ucount = DBuf<unsigned long long>(ctx, 5);
+        dzero(ctx, iscal.p, 32);
+        dzero(ctx, ucount.p, 40);
     }
 
     void init_state(bool with_et)
@@ -2388,11 +2907,45 @@ struct Phase {
     }
 
     // Folds the sweep's moves into localCinfo in processing order, with no host read: the
-    // mover count stays on the device (the scan's total sizes the event sort and folds) and
-    // is added to iscal[1], the iteration's movers, which the host reads with Q.
+    // mover count stays on the device and is added to iscal[1], the iteration's movers, which
+    // the host reads with Q.  Three forms with the same folds, by the vertex count: one
+    // workgroup; counted and placed with atomics; a radix sort, whose passes stream where the
+    // atomics of millions of events would not.
     void apply_moves(const int32_t* order, int64_t n, double* dst_cdeg, int32_t* dst_csize)
     {
         if (n == 0) return;
+        unsigned long long* movers = (unsigned long long*)(iscal.p + 1);
+        const MoverArgs m{order, n, target.p, curr.p, et ? active.p : nullptr};
+        if (nv <= kTailVerts) {
+            TailArgs a = tail_args(m, dst_cdeg, dst_csize);
+            a.cw = nullptr;
+            VT_LAUNCH(ctx, "tail", k_tail_small, 1, kTailBlock, 0, a);
+            return;
+        }
+        if (nv <= kEvVerts) {
+            if (!ev_cnt.p) {
+                ev_cnt = DBuf<uint32_t>(ctx, (size_t)nv);  // zero between uses
+                dzero(ctx, ev_cnt.p, 4 * (size_t)nv);
+            }
+            uint32_t* base = (uint32_t*)scratch(ctx, "ev_base", 4 * (size_t)nv);
+            uint2* rank = (uint2*)scratch(ctx, "ev_rank", 8 * (size_t)n);
+            uint32_t* ev = (uint32_t*)scratch(ctx, "ev_k0", 8 * (size_t)n);
+            int32_t* longs = (int32_t*)scratch(ctx, "ev_longs", 4 * (size_t)(2 * n / kEvRunWave + 1));
+            int32_t* mids = (int32_t*)scratch(ctx, "ev_mids", 4 * (size_t)(2 * n / kEvRunThread + 1));
+            uint32_t* ctl = (uint32_t*)(ucount.p + 2);
+            VT_LAUNCH(ctx, "ev_count", k_ev_count, grid_for(n, 256, 4096), 256, 0, m, ev_cnt.p, rank, ctl, movers);
+            VT_LAUNCH(ctx, "ev_alloc", k_ev_alloc, grid_for(nv, 1024, 4096), 1024, 0, nv, (const uint32_t*)ev_cnt.p, base, ctl,
+                      longs, mids);
+            VT_LAUNCH(ctx, "ev_scatter", k_ev_scatter, grid_for(n, 256, 4096), 256, 0, m, (const uint32_t*)base,
+                      (const uint2*)rank, ev);
+            VT_LAUNCH(ctx, "ev_fold", k_ev_fold, grid_for(nv, 256, 4096), 256, 0, nv, ev_cnt.p, (const uint32_t*)base,
+                      (const uint32_t*)ctl, (const int32_t*)mids, (const uint32_t*)ev, order, (const double*)vdeg.p, dst_cdeg,
+                      dst_csize);
+            VT_LAUNCH(ctx, "ev_fold_long", k_ev_fold_long, (unsigned)std::min<int64_t>(2 * n / kEvRunWave + 1, 512), 256, 0, m,
+                      (const uint32_t*)ctl, (const int32_t*)longs, ev_cnt.p, (const uint32_t*)base, ev,
+                      (const double*)vdeg.p, dst_cdeg, dst_csize);
+            return;
+        }
         int32_t* flags = (int32_t*)scratch(ctx, "mv_flags", 4 * (size_t)n);
         int32_t* pos = (int32_t*)scratch(ctx, "mv_pos", 4 * (size_t)n);
         int64_t* d_movers = iscal.p;
@@ -2411,6 +2964,25 @@ struct Phase {
         const bool alt = dev_sort_pairs_u32(ctx, k0, v0, k1, v1, d_movers, 2, ne, (int)bits_for(nv > 1 ? nv - 1 : 1));
         fold_events(alt ? k1 : k0, alt ? v1 : v0, ne, 0xFFFFFFFFu, dst_cdeg, dst_csize, d_movers);
         VT_LAUNCH(ctx, "count_movers", k_add_i64, 1, 64, 0, iscal.p + 1, (const int64_t*)d_movers);
+    }
+
+    TailArgs tail_args(const MoverArgs& m, double* dst_cdeg, int32_t* dst_csize)
+    {
+        TailArgs a;
+        a.m = m;
+        a.nv = (int32_t)nv;
+        a.vdeg = vdeg.p;
+        a.cdeg = dst_cdeg;
+        a.csize = dst_csize;
+        a.movers = (unsigned long long*)(iscal.p + 1);
+        a.cw = cw.p;
+        a.constant = constant();
+        int64_t blocks = 0;
+        sum2_plan(nv, &blocks, &a.chunk);
+        a.blocks = (int32_t)blocks;
+        a.sums = sums();
+        a.out = mail(ctx);
+        return a;
     }
 
     // The iteration's mover count: read with Q by modularity(), else from the device.
@@ -2438,16 +3010,33 @@ struct Phase {
                       (const unsigned long long*)(ucount.p + 1));
     }
 
-    double modularity(int flags)
+    // The end of an iteration: the moves from `order` (n of them; n = 0: already applied) and
+    // the modularity, whose kernel writes Q and the movers to pinned host memory.
+    double finish(const int32_t* order, int64_t n, int flags)
     {
-        if (flags & VT_FLAG_SEQUENTIAL_SUMS) seq_sum2(ctx, cw.p, cdeg.p, nv, sums());
-        else tree_sum2(ctx, cw.p, cdeg.p, nv, sums());
-        VT_LAUNCH(ctx, "modularity", k_modularity, 1, 64, 0, (const double*)sums(), (const double*)constant(), q(),
-                  (const int64_t*)(iscal.p + 1), (int64_t*)(scal.p + 4));
-        double qm[2];  // Q and the movers' bits, one read
-        d2h(ctx, qm, q(), 16);
-        std::memcpy(&movers_read, &qm[1], 8);
-        return qm[0];
+        const bool seq = (flags & VT_FLAG_SEQUENTIAL_SUMS) != 0;
+        double* out = mail(ctx);
+        if (nv <= kTailVerts && nv && !seq) {
+            const MoverArgs m{order, n, target.p, curr.p, et ? active.p : nullptr};
+            VT_LAUNCH(ctx, "tail", k_tail_small, 1, kTailBlock, 0, tail_args(m, cdeg.p, csize.p));
+        } else {
+            apply_moves(order, n, cdeg.p, csize.p);
+            if (seq) {
+                seq_sum2(ctx, cw.p, cdeg.p, nv, sums());
+                VT_LAUNCH(ctx, "modularity", k_modularity, 1, 64, 0, (const double*)sums(), (const double*)constant(), out,
+                          iscal.p + 1);
+            } else {
+                int64_t grid = 0, chunk = 0;
+                sum2_plan(nv, &grid, &chunk);
+                double2* part = (double2*)scratch(ctx, "sum2_part", sizeof(double2) * 1024);
+                VT_LAUNCH(ctx, "modularity", k_modularity_tree, (unsigned)grid, 256, 0, (const double*)cw.p,
+                          (const double*)cdeg.p, nv, chunk, part, (uint32_t*)(ucount.p + 4), (const double*)constant(),
+                          sums(), (unsigned long long*)(iscal.p + 1), out);
+            }
+        }
+        sync(ctx);
+        std::memcpy(&movers_read, &out[1], 8);
+        return out[0];
     }
 };
 
@@ -2519,7 +3108,6 @@ void phase_step(vt_ctx* ctx, vt_phase* st)
     const int64_t nv = ph.nv;
     st->numIters++;
     if (ph.et) dzero(ctx, ph.ucount.p, 8);
-    dzero(ctx, ph.iscal.p + 1, 8);  // the iteration's movers
     ph.movers_read = -1;
     if (st->mode == VT_MODE_COLOR) {
         for (int64_t ci = 0; ci < p.num_color; ci++) {
@@ -2541,10 +3129,9 @@ void phase_step(vt_ctx* ctx, vt_phase* st)
             return;
         }
     }
-    if (st->mode == VT_MODE_PLAIN) ph.apply_moves(nullptr, nv, ph.cdeg.p, ph.csize.p);
-    else if (st->mode == VT_MODE_VORDER) ph.apply_moves(ph.corder.p, nv, ph.cdeg.p, ph.csize.p);
-
-    st->currMod = ph.modularity(p.flags);
+    // the colors' moves are applied by now; the others' are here
+    if (st->mode == VT_MODE_COLOR) st->currMod = ph.finish(nullptr, 0, p.flags);
+    else st->currMod = ph.finish(st->mode == VT_MODE_VORDER ? ph.corder.p : nullptr, nv, p.flags);
     ctx->trace_q.push_back(st->currMod);
     ctx->trace_moves.push_back(ph.iteration_movers());
     if ((st->currMod - st->prevMod) < p.thresh) { st->done = true; return; }
@@ -3180,7 +3767,7 @@ int vt_modularity(vt_ctx* ctx, int64_t nv, const double* cw, const double* cdeg,
         if (flags & VT_FLAG_SEQUENTIAL_SUMS) seq_sum2(ctx, a.p, b.p, nv, s.p);
         else tree_sum2(ctx, a.p, b.p, nv, s.p);
         VT_LAUNCH(ctx, "modularity", k_modularity, 1, 64, 0, (const double*)s.p, (const double*)(s.p + 2), s.p + 3,
-                  (const int64_t*)nullptr, (int64_t*)nullptr);
+                  (int64_t*)nullptr);
         double q = 0;
         d2h(ctx, &q, s.p + 3, 8);
         if (q_out) *q_out = q;
