@@ -183,9 +183,9 @@ struct MemberRows {
 };
 
 constexpr int kCfWaves = 4;
-// The fold's (and the overflow emission's) blocks are one wave each: a block holds its
-// resources until its last wave ends, and the waves of a block take communities of very
-// different sizes, so 4-wave blocks left about half of the resident-wave slots idle.
+// The fold's blocks are one wave each: a block holds its resources until its last wave ends,
+// and the waves of a block take communities of very different sizes, so 4-wave blocks left
+// about half of the resident-wave slots idle.
 constexpr int kFoldWaves = 1;
 constexpr int kCfLog = 8;
 constexpr int kCfCap = 1 << kCfLog;       // table slots per wave
@@ -326,66 +326,56 @@ __global__ void __launch_bounds__(64 * kFoldWaves) k_comm_fold(
     }
 }
 
-// Every entry of the communities that overflowed the table, as ((C1 << bits) | C2, weight),
-// at xoff[C1] + its position in C1's concatenated row.
-// Overflowing communities of more than this many entries (a giant community on a skewed
-// graph) are emitted by every wave of k_ovf_emit_big instead of one wave each: emitting
-// needs no order, and one wave walking such a community held the launch for 4 ms on BA
-// n = 2^22.
-constexpr int64_t kOvfBig = 1 << 16;
+// Work items of segments of very different lengths (a skewed graph's coarse levels have one
+// community with most of the entries): chunk k of segment c, for every segment of at least
+// `min_len` entries, in any order.  A wave or workgroup per segment would leave the chip idle
+// behind the longest: on BA n = 300007 a wave per community emitted in 1.40 ms and 16 lanes per
+// row copied in 1.14 ms what the items do in 0.04 and 0.03 ms.
+struct Item {
+    uint32_t seg, chunk;
+};
+constexpr int64_t kItemLen = 4096;
 
-// The ids of those communities, in any order (their entries' places do not depend on it).
-__global__ void k_ovf_big_list(int64_t nc, const int64_t* __restrict__ xcnt, unsigned long long* __restrict__ count,
-                               int64_t* __restrict__ list)
+__global__ void k_split_items(int64_t n, const int64_t* __restrict__ len, int64_t min_len, uint32_t* __restrict__ count,
+                              Item* __restrict__ items)
 {
-    for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < nc; c += (int64_t)gridDim.x * blockDim.x)
-        if (xcnt[c] > kOvfBig) list[atomicAdd(count, 1ull)] = c;
-}
-
-__global__ void __launch_bounds__(64 * kFoldWaves) k_ovf_emit(
-    int64_t nc, const int64_t* __restrict__ cstart, const int64_t* __restrict__ moff, const int64_t* __restrict__ mrow,
-    const DEdge* __restrict__ edges, const uint32_t* __restrict__ newid,
-    const int64_t* __restrict__ xcnt, const int64_t* __restrict__ xoff, int bits, unsigned long long* __restrict__ keys,
-    double* __restrict__ vals)
-{
-    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    for (int64_t c = (int64_t)blockIdx.x * kFoldWaves + w; c < nc; c += (int64_t)gridDim.x * kFoldWaves) {
-        if (xcnt[c] == 0 || xcnt[c] > kOvfBig) continue;  // k_ovf_emit_big takes the giant ones
-        const MemberRows mr(cstart, moff, mrow, c, lane);
-        const int64_t o = xoff[c] - mr.s0;
-        for (int64_t base = mr.s0; base < mr.s1; base += 64) {
-            const int64_t p = base + lane;
-            const int64_t k = mr.csr_index(p, moff, mrow);
-            if (p < mr.s1) {
-                const DEdge e = edges[k];
-                keys[o + p] = ((unsigned long long)c << bits) | newid[e.tail];
-                vals[o + p] = e.weight;
-            }
+    const int lane = threadIdx.x & 63;
+    for (int64_t c0 = blockIdx.x * (int64_t)blockDim.x + (threadIdx.x & ~63); c0 < n; c0 += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t c = c0 + lane;
+        const int64_t l = c < n ? len[c] : 0;
+        const uint32_t k = l >= min_len ? (uint32_t)((l + kItemLen - 1) / kItemLen) : 0;
+        uint32_t x = k;
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(x, o);
+            if (lane >= o) x += y;
         }
+        uint32_t at = 0;
+        if (lane == 63 && x) at = atomicAdd(count, x);
+        at = __shfl(at, 63) + x - k;
+        for (uint32_t i = 0; i < k; i++) items[at + i] = Item{(uint32_t)c, i};
     }
 }
 
-// The giant overflowing communities: for each listed community, the whole grid deals its
-// 64-entry chunks to the waves; each lane finds its entry's CSR index by a search of the
-// member offsets, as k_ovf_emit does for communities of more than 64 members.
-__global__ void __launch_bounds__(64 * kCfWaves) k_ovf_emit_big(
-    const unsigned long long* __restrict__ count, const int64_t* __restrict__ list, const int64_t* __restrict__ cstart,
+// Every entry of the communities that overflowed the table, as ((C1 << bits) | C2, weight),
+// at xoff[C1] + its position in C1's concatenated row; a wave per item.
+__global__ void __launch_bounds__(64) k_ovf_emit(
+    const uint32_t* __restrict__ count, const Item* __restrict__ items, const int64_t* __restrict__ cstart,
     const int64_t* __restrict__ moff, const int64_t* __restrict__ mrow, const DEdge* __restrict__ edges,
     const uint32_t* __restrict__ newid, const int64_t* __restrict__ xoff, int bits, unsigned long long* __restrict__ keys,
     double* __restrict__ vals)
 {
-    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t wave = (int64_t)blockIdx.x * kCfWaves + w, waves = (int64_t)gridDim.x * kCfWaves;
-    const int64_t nbig = (int64_t)*count;
-    for (int64_t i = 0; i < nbig; i++) {
-        const int64_t c = list[i];
+    const int lane = threadIdx.x;
+    const uint32_t ni = *count;
+    for (uint32_t i = blockIdx.x; i < ni; i += gridDim.x) {
+        const int64_t c = items[i].seg;
         const MemberRows mr(cstart, moff, mrow, c, lane);
         const int64_t o = xoff[c] - mr.s0;
-        const int64_t nchunks = (mr.s1 - mr.s0 + 63) / 64;
-        for (int64_t ch = wave; ch < nchunks; ch += waves) {
-            const int64_t p = mr.s0 + ch * 64 + lane;
+        const int64_t lo = mr.s0 + items[i].chunk * kItemLen;
+        const int64_t hi = lo + kItemLen < mr.s1 ? lo + kItemLen : mr.s1;
+        for (int64_t base = lo; base < hi; base += 64) {
+            const int64_t p = base + lane;
             const int64_t k = mr.csr_index(p, moff, mrow);
-            if (p < mr.s1) {
+            if (p < hi) {
                 const DEdge e = edges[k];
                 keys[o + p] = ((unsigned long long)c << bits) | newid[e.tail];
                 vals[o + p] = e.weight;
@@ -394,14 +384,25 @@ __global__ void __launch_bounds__(64 * kCfWaves) k_ovf_emit_big(
     }
 }
 
+// Runs of at least this many entries are folded by a wave each (k_ext_runs_long): a thread
+// folding the entries between two giant communities held the launch for 3.3 ms on BA n = 300007.
+constexpr int64_t kExtLongRun = 256;
+
 __global__ void k_ext_runs(const unsigned long long* __restrict__ keys, const double* __restrict__ vals,
                            const int64_t* __restrict__ starts, int64_t nu, int bits, uint32_t* __restrict__ rc1,
-                           uint32_t* __restrict__ rc2, double* __restrict__ rw)
+                           uint32_t* __restrict__ rc2, double* __restrict__ rw, uint32_t* __restrict__ nlong,
+                           uint32_t* __restrict__ longs)
 {
     const unsigned long long lomask = (1ull << bits) - 1;
     for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < nu; r += (int64_t)gridDim.x * blockDim.x) {
         const int64_t b = starts[r], e = starts[r + 1];
         const unsigned long long key = keys[b];
+        rc1[r] = (uint32_t)(key >> bits);
+        rc2[r] = (uint32_t)(key & lomask);
+        if (e - b >= kExtLongRun) {
+            longs[atomicAdd(nlong, 1u)] = (uint32_t)r;
+            continue;
+        }
         double acc = vals[b];
         int64_t k = b + 1;
         for (; k + 4 <= e; k += 4) {
@@ -412,9 +413,30 @@ __global__ void k_ext_runs(const unsigned long long* __restrict__ keys, const do
             acc = acc + x3;
         }
         for (; k < e; k++) acc = acc + vals[k];
-        rc1[r] = (uint32_t)(key >> bits);
-        rc2[r] = (uint32_t)(key & lomask);
         rw[r] = acc;
+    }
+}
+
+// The long runs: a wave loads 64 values at a time, the next 64 in flight, and adds them in
+// lane order (from -0.0, so that the first is taken as it is; lanes past the end hold -0.0).
+__global__ void __launch_bounds__(64) k_ext_runs_long(const uint32_t* __restrict__ nlong, const uint32_t* __restrict__ longs,
+                                                      const double* __restrict__ vals, const int64_t* __restrict__ starts,
+                                                      double* __restrict__ rw)
+{
+    const int lane = threadIdx.x;
+    const uint32_t n = *nlong;
+    for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
+        const uint32_t r = longs[i];
+        const int64_t b = starts[r], e = starts[r + 1];
+        double acc = -0.0;
+        double x = b + lane < e ? vals[b + lane] : -0.0;
+        for (int64_t base = b; base < e; base += 64) {
+            const double xn = base + 64 + lane < e ? vals[base + 64 + lane] : -0.0;
+#pragma unroll
+            for (int u = 0; u < 64; u++) acc = acc + readlane_f64(x, u);
+            x = xn;
+        }
+        if (lane == 0) rw[r] = acc;
     }
 }
 
@@ -456,7 +478,10 @@ __global__ void k_ovf_place(const uint32_t* __restrict__ rc1, const uint32_t* __
     }
 }
 
-// Staged rows -> the coarse CSR, one wave per community.
+// Staged rows -> the coarse CSR, 16 lanes per community (coarse rows average a few dozen
+// entries); rows of kCopyLongRow and more are left to k_row_copy_long.
+constexpr int64_t kCopyLongRow = 2048;
+
 __global__ void __launch_bounds__(64 * kCfWaves) k_row_copy(int64_t nc, const int64_t* __restrict__ cstart,
                                                            const int64_t* __restrict__ moff,
                                                            const int64_t* __restrict__ rowlen,
@@ -464,17 +489,37 @@ __global__ void __launch_bounds__(64 * kCfWaves) k_row_copy(int64_t nc, const in
                                                            const uint32_t* __restrict__ rkey,
                                                            const double* __restrict__ rval, DEdge* __restrict__ out)
 {
-    // 16 lanes per community (coarse rows average a few dozen entries)
     constexpr int kLanes = 16;
     const int sub = threadIdx.x % kLanes;
     const int64_t groups = (int64_t)gridDim.x * blockDim.x / kLanes;
     for (int64_t c = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kLanes; c < nc; c += groups) {
         const int64_t s0 = moff[cstart[c]], len = rowlen[c], o = out_offs[c];
+        if (len >= kCopyLongRow) continue;
         for (int64_t i = sub; i < len; i += kLanes) {
             DEdge e;
             e.tail = (int64_t)rkey[s0 + i];
             e.weight = rval[s0 + i];
             out[o + i] = e;
+        }
+    }
+}
+
+__global__ void __launch_bounds__(256) k_row_copy_long(const uint32_t* __restrict__ count, const Item* __restrict__ items,
+                                                       const int64_t* __restrict__ cstart, const int64_t* __restrict__ moff,
+                                                       const int64_t* __restrict__ rowlen, const int64_t* __restrict__ out_offs,
+                                                       const uint32_t* __restrict__ rkey, const double* __restrict__ rval,
+                                                       DEdge* __restrict__ out)
+{
+    const uint32_t ni = *count;
+    for (uint32_t i = blockIdx.x; i < ni; i += gridDim.x) {
+        const uint32_t c = items[i].seg;
+        const int64_t s0 = moff[cstart[c]], len = rowlen[c], o = out_offs[c];
+        const int64_t lo = items[i].chunk * kItemLen, hi = lo + kItemLen < len ? lo + kItemLen : len;
+        for (int64_t k = lo + threadIdx.x; k < hi; k += 256) {
+            DEdge e;
+            e.tail = (int64_t)rkey[s0 + k];
+            e.weight = rval[s0 + k];
+            out[o + k] = e;
         }
     }
 }
@@ -491,31 +536,35 @@ __global__ void k_pair_totals(const int64_t* __restrict__ a, const int64_t* __re
 // right, and each community's runs placed in its staged row.
 static void overflow_rows(vt_ctx* ctx, const vt_graph* g, const uint32_t* newid, int64_t nc, int bits,
                           const int64_t* cstart, const int64_t* mrow, const int64_t* moff, const int64_t* xcnt,
-                          const int64_t* xoff, int64_t nx, uint32_t* rkey, double* rval, int64_t* rowlen)
+                          const int64_t* xoff, int64_t nx, int64_t xmax, uint32_t* rkey, double* rval, int64_t* rowlen)
 {
     const size_t x1 = (size_t)std::max<int64_t>(nx, 1), c1n = (size_t)nc + 1;
     DBuf<unsigned long long> k0(ctx, x1), k1(ctx, x1);
     DBuf<double> v0(ctx, x1), v1(ctx, x1);
-    VT_LAUNCH(ctx, "rb_ovf_emit", k_ovf_emit, grid_for(nc, kFoldWaves, 262144), 64 * kFoldWaves, 0, nc, cstart, moff, mrow,
-              (const DEdge*)g->edges, newid, xcnt, xoff, bits, k0.p, v0.p);
-    if (nx > kOvfBig) {  // a community that big may exist
-        DBuf<unsigned long long> nbig(ctx, 1);
-        DBuf<int64_t> big(ctx, (size_t)std::max<int64_t>(nx / kOvfBig, 1));
-        dzero(ctx, nbig.p, 8);
-        VT_LAUNCH(ctx, "rb_ovf_big_list", k_ovf_big_list, grid_for(nc, 256, 4096), 256, 0, nc, xcnt, nbig.p, big.p);
-        VT_LAUNCH(ctx, "rb_ovf_emit_big", k_ovf_emit_big, 1024, 64 * kCfWaves, 0, (const unsigned long long*)nbig.p,
-                  (const int64_t*)big.p, cstart, moff, mrow, (const DEdge*)g->edges, newid, xoff, bits, k0.p, v0.p);
+    DBuf<uint32_t> counts(ctx, 2);
+    dzero(ctx, counts.p, 8);
+    {
+        // an overflowing community has more than kCfMaxKeys entries
+        const int64_t cap = nx / kCfMaxKeys + nx / kItemLen + 1;
+        DBuf<Item> items(ctx, (size_t)cap);
+        VT_LAUNCH(ctx, "rb_ovf_items", k_split_items, grid_for(nc, 256, 4096), 256, 0, nc, xcnt, (int64_t)1, counts.p,
+                  items.p);
+        // timed under a name of its own where a giant community is among them
+        const char* name = xmax > (1 << 16) ? "rb_ovf_emit_big" : "rb_ovf_emit";
+        VT_LAUNCH(ctx, name, k_ovf_emit, (unsigned)std::min<int64_t>(cap, 65536), 64, 0, (const uint32_t*)counts.p,
+                  (const Item*)items.p, cstart, moff, mrow, (const DEdge*)g->edges, newid, xoff, bits, k0.p, v0.p);
     }
     const unsigned long long* ks = k0.p;
     const double* vs = v0.p;
     if (nx > 1) {
         rocprim::double_buffer<unsigned long long> kb(k0.p, k1.p);
         rocprim::double_buffer<double> vb(v0.p, v1.p);
-        // Many entries per community (the coarse levels, where nearly every community
-        // overflows): each community's entries, already together at xoff[C1], are sorted by C2
-        // alone, a workgroup each; otherwise one sort of every entry by (C1, C2).  Both are
-        // stable, so the order is the same.
-        const bool seg = nx >= 16 * nc;
+        // Many entries per community and none with much of them (the coarse levels, where
+        // nearly every community overflows): each community's entries, already together at
+        // xoff[C1], are sorted by C2 alone, a workgroup each; otherwise one sort of every entry
+        // by (C1, C2).  Both are stable, so the order is the same.  One workgroup sorting a giant
+        // community took 6.8 ms on BA n = 300007, the sort of every entry 0.4 ms.
+        const bool seg = nx >= 16 * nc && 64 * xmax <= nx;
         auto sort = [&](void* tmp, size_t& tb) {
             if (seg)
                 return rocprim::segmented_radix_sort_pairs(tmp, tb, kb, vb, (unsigned)nx, (unsigned)nc, xoff, xoff + 1, 0u,
@@ -546,8 +595,11 @@ static void overflow_rows(vt_ctx* ctx, const vt_graph* g, const uint32_t* newid,
     }
     DBuf<uint32_t> rc1(ctx, (size_t)nu), rc2(ctx, (size_t)nu);
     DBuf<double> rw(ctx, (size_t)nu);
+    DBuf<uint32_t> longs(ctx, (size_t)(nx / kExtLongRun + 1));
     VT_LAUNCH(ctx, "rb_fold", k_ext_runs, grid_for(nu, 256, 16384), 256, 0, ks, vs, (const int64_t*)starts.p, nu, bits,
-              rc1.p, rc2.p, rw.p);
+              rc1.p, rc2.p, rw.p, counts.p + 1, longs.p);
+    VT_LAUNCH(ctx, "rb_fold_long", k_ext_runs_long, (unsigned)std::min<int64_t>(nx / kExtLongRun + 1, 16384), 64, 0,
+              (const uint32_t*)(counts.p + 1), (const uint32_t*)longs.p, vs, (const int64_t*)starts.p, rw.p);
     DBuf<int64_t> run_first(ctx, c1n);
     VT_LAUNCH(ctx, "rb_ovf_rows", k_ovf_rows, grid_for(nc, 256, 16384), 256, 0, nc, xcnt, (const uint32_t*)rc1.p, nu,
               run_first.p, rowlen);
@@ -581,7 +633,7 @@ static vt_graph* rebuild_fold(vt_ctx* ctx, const vt_graph* g, const uint32_t* ne
     // every community's coarse row, staged at its offset in the concatenated rows
     DBuf<uint32_t> rkey(ctx, e1);
     DBuf<double> rval(ctx, e1);
-    DBuf<int64_t> rowlen(ctx, c1n), xcnt(ctx, c1n), out_offs(ctx, c1n), xoff(ctx, c1n), tot(ctx, 3);
+    DBuf<int64_t> rowlen(ctx, c1n), xcnt(ctx, c1n), out_offs(ctx, c1n), xoff(ctx, c1n), tot(ctx, 4);
     dzero(ctx, rowlen.p + nc, 8);
     dzero(ctx, xcnt.p + nc, 8);
     if (nc)
@@ -594,21 +646,22 @@ static vt_graph* rebuild_fold(vt_ctx* ctx, const vt_graph* g, const uint32_t* ne
               tot.p);
     // the coarse graph's largest row is read with its entry count (the overflowing
     // communities' rows are added below, and the count and the largest row read again)
-    auto max_row = [&]() {
-        dzero(ctx, tot.p + 2, 8);
+    auto max_row = [&](const int64_t* offs, int64_t* out) {
         if (nc)
-            VT_LAUNCH(ctx, "max_degree", k_max_degree, grid_for(nc, 256, 512), 256, 0, (const int64_t*)out_offs.p, nc,
-                      (unsigned long long*)(tot.p + 2));
+            VT_LAUNCH(ctx, "max_degree", k_max_degree, grid_for(nc, 256, 512), 256, 0, offs, nc, (unsigned long long*)out);
     };
-    max_row();
-    int64_t totals[3] = {0, 0, 0};
-    d2h(ctx, totals, tot.p, 24);
+    dzero(ctx, tot.p + 2, 16);
+    max_row(out_offs.p, tot.p + 2);
+    max_row(xoff.p, tot.p + 3);
+    int64_t totals[4] = {0, 0, 0, 0};  // entries, overflowing entries, largest row, largest overflowing community
+    d2h(ctx, totals, tot.p, 32);
     if (totals[1]) {
-        overflow_rows(ctx, g, newid, nc, bits, cstart.p, mrow.p, moff.p, xcnt.p, xoff.p, totals[1], rkey.p, rval.p,
-                      rowlen.p);
+        overflow_rows(ctx, g, newid, nc, bits, cstart.p, mrow.p, moff.p, xcnt.p, xoff.p, totals[1], totals[3], rkey.p,
+                      rval.p, rowlen.p);
         exclusive_scan_i64(ctx, rowlen.p, out_offs.p, nc + 1);
         d2d(ctx, tot.p, out_offs.p + nc, 8);
-        max_row();
+        dzero(ctx, tot.p + 2, 8);
+        max_row(out_offs.p, tot.p + 2);
         d2h(ctx, totals, tot.p, 24);
     }
 
@@ -619,6 +672,18 @@ static vt_graph* rebuild_fold(vt_ctx* ctx, const vt_graph* g, const uint32_t* ne
             VT_LAUNCH(ctx, "rb_row_copy", k_row_copy, grid_for(nc, kCfWaves, 65536), 64 * kCfWaves, 0, nc,
                       (const int64_t*)cstart.p, (const int64_t*)moff.p, (const int64_t*)rowlen.p,
                       (const int64_t*)out_offs.p, (const uint32_t*)rkey.p, (const double*)rval.p, out->edges);
+        if (totals[2] >= kCopyLongRow) {
+            const int64_t cap = totals[0] / kCopyLongRow + totals[0] / kItemLen + 1;
+            DBuf<uint32_t> count(ctx, 1);
+            DBuf<Item> items(ctx, (size_t)cap);
+            dzero(ctx, count.p, 4);
+            VT_LAUNCH(ctx, "rb_copy_items", k_split_items, grid_for(nc, 256, 4096), 256, 0, nc, (const int64_t*)rowlen.p,
+                      kCopyLongRow, count.p, items.p);
+            VT_LAUNCH(ctx, "rb_row_copy_long", k_row_copy_long, (unsigned)std::min<int64_t>(cap, 16384), 256, 0,
+                      (const uint32_t*)count.p, (const Item*)items.p, (const int64_t*)cstart.p, (const int64_t*)moff.p,
+                      (const int64_t*)rowlen.p, (const int64_t*)out_offs.p, (const uint32_t*)rkey.p, (const double*)rval.p,
+                      out->edges);
+        }
         out->max_degree = totals[2];
     } catch (...) {
         graph_delete(ctx, out);
