@@ -203,6 +203,102 @@ __device__ __forceinline__ double readlane_f64(double x, int j)
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
+// ---- long left folds --------------------------------------------------------------------
+// A left fold is a chain of dependent adds, one per term.  Where every term and the running sum
+// are whole numbers whose magnitudes total less than 2^53 (the weights and degrees of any
+// unweighted graph, and of all its coarse levels), no add rounds, so the sum in any order is
+// the left fold to the last bit, and the terms are added side by side; otherwise the chain
+// runs in order.  The test is on the values themselves, a chunk of terms at a time.
+__device__ __forceinline__ bool whole_number(double x) { return x == rint(x); }
+
+// acc + f(0) + ... + f(n - 1), left to right, by a wave (n and acc the same in every lane).
+// The next 64 * R terms are in flight while a chunk is added; lanes past the end hold -0.0,
+// which leaves any sum unchanged.  In order, a term is two lane reads and an add.
+template <int R, class F>
+__device__ __forceinline__ double wave_left_fold(double acc, int64_t n, F f)
+{
+    const int lane = threadIdx.x & 63;
+    double x[R], xn[R], part = -0.0, mag = 0.0;
+#pragma unroll
+    for (int r = 0; r < R; r++) x[r] = r * 64 + lane < n ? f((int64_t)(r * 64 + lane)) : -0.0;
+    bool open = false;  // part holds terms not yet in acc
+    auto flush = [&] {
+        for (int o = 32; o > 0; o >>= 1) part = part + __shfl_xor(part, o);
+        acc = acc + part;
+        part = -0.0;
+        mag = 0.0;
+        open = false;
+    };
+    for (int64_t base = 0; base < n; base += 64 * R) {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int64_t i = base + 64 * R + r * 64 + lane;
+            xn[r] = i < n ? f(i) : -0.0;
+        }
+        double s = part, m = mag;
+        bool ok = true;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            ok = ok & whole_number(x[r]);
+            s = s + x[r];
+            m = m + fabs(x[r]);
+        }
+        // 64 lanes of less than 2^45 and an acc below 2^51
+        ok = ok & (m < 0x1p45) & (open | (whole_number(acc) & (fabs(acc) < 0x1p51)));
+        if (__ballot(!ok) == 0) {
+            part = s;
+            mag = m;
+            open = true;
+        } else {
+            if (open) flush();
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                if (base + r * 64 >= n) break;
+#pragma unroll
+                for (int u = 0; u < 64; u++) acc = acc + readlane_f64(x[r], u);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) x[r] = xn[r];
+    }
+    if (open) flush();
+    return acc;
+}
+
+// Where all of f(0) .. f(n - 1) are whole numbers of magnitudes totalling less than 2^51: true,
+// with *sum their sum (-0.0 for n = 0) in every thread; false, and *sum undefined, otherwise.
+// Every thread of a workgroup of B calls it; red: B / 64 doubles of LDS.
+template <int B, int R, class F>
+__device__ __forceinline__ bool block_exact_sum(int64_t n, F f, double* red, double* sum)
+{
+    double part = -0.0, mag = 0.0;
+    bool ok = true;
+    for (int64_t base = 0; base < n; base += B * R) {
+        double x[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int64_t i = base + r * B + threadIdx.x;
+            x[r] = i < n ? f(i) : -0.0;
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            ok = ok & whole_number(x[r]);
+            part = part + x[r];
+            mag = mag + fabs(x[r]);
+        }
+        if (base == 0 && !__syncthreads_and(ok)) return false;  // fractional terms show at once
+    }
+    for (int o = 32; o > 0; o >>= 1) part = part + __shfl_xor(part, o);
+    if (!__syncthreads_and(ok & (mag < 0x1p51 / B))) return false;
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = part;
+    __syncthreads();
+    double t = red[0];
+    for (int w = 1; w < B / 64; w++) t = t + red[w];
+    __syncthreads();  // red may be reused
+    *sum = t;
+    return true;
+}
+
 // ---- device primitives (vt_prims.hip) -------------------------------------------------
 // Deterministic fixed-order sums: every block reduces a fixed contiguous chunk with a
 // fixed tree; block partials are reduced by one block in index order.

@@ -1194,30 +1194,40 @@ __global__ void k_hub_degrees(const int32_t* __restrict__ hubs, int32_t nh, cons
         deg[j] = j < nh ? offs[hubs[j] + 1] - offs[hubs[j]] : 0;
 }
 
-// Left fold of a run's weights: the first as is, or from 0.0 for the vertex's own community
-// (whose counter the reference seeds with 0.0); the self-loop weights folded from 0.0 too.
-__device__ __forceinline__ double hub_run_fold(const DEdge* __restrict__ edges, const uint32_t* __restrict__ vals,
-                                               int64_t b, int64_t e, bool own, int32_t v, double& self)
+// Left fold of a run's weights, the first as is, by one thread.
+__device__ __forceinline__ double hub_run_fold(const double* __restrict__ wgt, const uint32_t* __restrict__ vals, int64_t b,
+                                               int64_t e)
 {
-    double acc = own ? 0.0 : edges[vals[b]].weight;
-    int64_t k = own ? b : b + 1;
+    double acc = wgt[vals[b]];
+    int64_t k = b + 1;
     for (; k + 4 <= e; k += 4) {
-        const DEdge x0 = edges[vals[k]], x1 = edges[vals[k + 1]], x2 = edges[vals[k + 2]], x3 = edges[vals[k + 3]];
-        acc = acc + x0.weight;
-        if (own && x0.tail == v) self = self + x0.weight;
-        acc = acc + x1.weight;
-        if (own && x1.tail == v) self = self + x1.weight;
-        acc = acc + x2.weight;
-        if (own && x2.tail == v) self = self + x2.weight;
-        acc = acc + x3.weight;
-        if (own && x3.tail == v) self = self + x3.weight;
+        const double x0 = wgt[vals[k]], x1 = wgt[vals[k + 1]], x2 = wgt[vals[k + 2]], x3 = wgt[vals[k + 3]];
+        acc = acc + x0;
+        acc = acc + x1;
+        acc = acc + x2;
+        acc = acc + x3;
     }
-    for (; k < e; k++) {
-        const DEdge x = edges[vals[k]];
-        acc = acc + x.weight;
-        if (own && x.tail == v) self = self + x.weight;
-    }
+    for (; k < e; k++) acc = acc + wgt[vals[k]];
     return acc;
+}
+
+// The runs of this many entries and more that a wave's lanes hold (`mine`), one after another by
+// the whole wave; every lane calls it, and a lane with `mine` gets its run's fold in ey.
+constexpr int32_t kHubLongRun = 256;
+// Runs of this many by a workgroup, where their launch has whole tiles of runs to a workgroup.
+constexpr int32_t kHubBlockRun = 8192;
+
+template <int R>
+__device__ __forceinline__ void hub_long_runs(const double* __restrict__ wgt, const uint32_t* __restrict__ vals, bool mine,
+                                              int32_t b, int32_t e, double& ey)
+{
+    for (unsigned long long m = __ballot(mine); m; m &= m - 1) {
+        const int l = __builtin_ctzll(m);
+        const uint32_t* q = vals + __builtin_amdgcn_readlane(b, l);
+        const int64_t n = __builtin_amdgcn_readlane(e, l) - __builtin_amdgcn_readlane(b, l);
+        const double x = wave_left_fold<R>(-0.0, n, [=](int64_t k) { return wgt[q[k]]; });
+        if ((int)(threadIdx.x & 63) == l) ey = x;
+    }
 }
 
 // The hub local move as four flat launches, for sweeps with few hubs or one hub holding much
@@ -1232,34 +1242,84 @@ __device__ __forceinline__ int32_t hub_run_count(const int64_t* __restrict__ hof
     return total ? pos[total - 1] + head[total - 1] : 0;
 }
 
-// Per hub: its own community's run folded from 0.0 with the self-loops (louvain.cpp:2326-2327,
-// 2440-2441), and the argmax cells cleared.
-template <class K>
-__global__ void k_hub_own(MoveArgs a, const int32_t* __restrict__ hubs, int32_t nh, const int64_t* __restrict__ hoffs,
-                          const K* __restrict__ keys, const uint32_t* __restrict__ vals, const int32_t* __restrict__ pos,
-                          const int32_t* __restrict__ head, const int32_t* __restrict__ starts, int cbits,
-                          double* __restrict__ own, unsigned long long* __restrict__ best, int32_t* __restrict__ bestc)
+// The own community's run of hub j folded from 0.0, and its self-loop weights (louvain.cpp:
+// 2326-2327, 2440-2441), by a workgroup: where the weights are whole numbers the run is summed
+// side by side, else wave 0 folds it in order.  A skewed graph's coarse hub has most of its
+// entries in this run: one thread held the launch for 6 ms on BA n = 2^22.  The result is in
+// every thread; lds: kHubBlock / 64 + 2 doubles; R: terms a lane has in flight.
+constexpr int kHubBlock = 256;
+
+template <int R, class K>
+__device__ __forceinline__ void hub_own_fold(const MoveArgs& a, int32_t v, K ckey, int32_t r0, int32_t r1,
+                                             const K* __restrict__ keys, const uint32_t* __restrict__ vals,
+                                             const int32_t* __restrict__ starts, double* lds, double& ecc, double& self)
 {
+    int32_t lo = r0, hi = r1;  // the same in every thread
+    while (lo < hi) {
+        const int32_t mid = (lo + hi) >> 1;
+        if (keys[starts[mid]] < ckey) lo = mid + 1;
+        else hi = mid;
+    }
+    ecc = self = 0.0;
+    if (lo >= r1 || keys[starts[lo]] != ckey) return;  // the same in every thread
+    const uint32_t* q = vals + starts[lo];
+    const int64_t n = starts[lo + 1] - starts[lo];
+    bool loops = false;
+    auto weight = [&](int64_t k) {
+        const uint32_t e = q[k];
+        loops = loops | (a.tail32[e] == v);
+        return a.wgt[e];
+    };
+    double* out = lds + kHubBlock / 64;
+    double sum = 0.0;
+    auto loop_weight = [&](int64_t k) { return a.tail32[q[k]] == v ? a.wgt[q[k]] : -0.0; };
+    if (n > 256 && block_exact_sum<kHubBlock, 2 * R>(n, weight, lds, &sum)) {
+        ecc = 0.0 + sum;
+        if (__syncthreads_or(loops) && block_exact_sum<kHubBlock, 2 * R>(n, loop_weight, lds, &sum)) self = 0.0 + sum;
+        return;
+    }
+    if (threadIdx.x < 64) {
+        ecc = wave_left_fold<R>(0.0, n, weight);
+        if (__ballot(loops)) self = wave_left_fold<R>(0.0, n, loop_weight);
+        if (threadIdx.x == 0) {
+            out[0] = ecc;
+            out[1] = self;
+        }
+    }
+    __syncthreads();
+    ecc = out[0];
+    self = out[1];
+    __syncthreads();  // lds may be reused
+}
+
+// Per hub: the own community's run, and the argmax cells cleared; a workgroup per hub.
+template <class K>
+__global__ void __launch_bounds__(kHubBlock) k_hub_own(MoveArgs a, const int32_t* __restrict__ hubs, int32_t nh,
+                                                       const int64_t* __restrict__ hoffs, const K* __restrict__ keys,
+                                                       const uint32_t* __restrict__ vals, const int32_t* __restrict__ pos,
+                                                       const int32_t* __restrict__ head, const int32_t* __restrict__ starts,
+                                                       int cbits, double* __restrict__ own,
+                                                       unsigned long long* __restrict__ best, int32_t* __restrict__ bestc)
+{
+    __shared__ double s_lds[kHubBlock / 64 + 2];
     const int64_t total = hoffs[nh];
     const int32_t nruns = hub_run_count(hoffs, nh, pos, head);
-    for (int32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < nh; j += gridDim.x * blockDim.x) {
-        best[j] = 0ull;  // the bits of +0.0: only gains > 0 can win
-        bestc[j] = INT_MAX;
+    for (int32_t j = blockIdx.x; j < nh; j += gridDim.x) {
+        if (threadIdx.x == 0) {
+            best[j] = 0ull;  // the bits of +0.0: only gains > 0 can win
+            bestc[j] = INT_MAX;
+        }
         const int32_t v = hubs[j];
         if (a.active && !a.active[v]) continue;
         const int32_t r0 = hoffs[j] < total ? pos[hoffs[j]] : nruns;
         const int32_t r1 = hoffs[j + 1] < total ? pos[hoffs[j + 1]] : nruns;
         const K ckey = ((K)j << cbits) | (K)(uint32_t)a.curr[v];
-        int32_t lo = r0, hi = r1;
-        while (lo < hi) {
-            const int32_t mid = (lo + hi) >> 1;
-            if (keys[starts[mid]] < ckey) lo = mid + 1;
-            else hi = mid;
+        double ecc, self;
+        hub_own_fold<4, K>(a, v, ckey, r0, r1, keys, vals, starts, s_lds, ecc, self);
+        if (threadIdx.x == 0) {
+            own[2 * j] = ecc;
+            own[2 * j + 1] = self;
         }
-        double self = 0.0, ecc = 0.0;
-        if (lo < r1 && keys[starts[lo]] == ckey) ecc = hub_run_fold(a.edges, vals, starts[lo], starts[lo + 1], true, v, self);
-        own[2 * j] = ecc;
-        own[2 * j + 1] = self;
     }
 }
 
@@ -1267,45 +1327,64 @@ __global__ void k_hub_own(MoveArgs a, const int32_t* __restrict__ hubs, int32_t 
 // first as is) and its gain (louvain.cpp:2246-2273); best[j] = the largest positive gain's
 // bits (non-negative doubles order as their bit patterns).
 template <class K>
-__global__ void k_hub_runs(MoveArgs a, const int32_t* __restrict__ hubs, int32_t nh, const int64_t* __restrict__ hoffs,
+__global__ void __launch_bounds__(kHubBlock) k_hub_runs(MoveArgs a, const int32_t* __restrict__ hubs, int32_t nh, const int64_t* __restrict__ hoffs,
                            const K* __restrict__ keys, const uint32_t* __restrict__ vals, const int32_t* __restrict__ pos,
                            const int32_t* __restrict__ head, const int32_t* __restrict__ starts, int cbits,
                            const double* __restrict__ own, double* __restrict__ gains,
                            unsigned long long* __restrict__ best)
 {
+    __shared__ double s_red[kHubBlock / 64], s_ey[kHubBlock];
+    __shared__ int2 s_run[kHubBlock];
     const int32_t nruns = hub_run_count(hoffs, nh, pos, head);
     const double constant = *a.constant;
     const K cmask = (K)(((unsigned long long)1 << cbits) - 1);
     const int lane = threadIdx.x & 63;
-    // whole waves step together (the bound is wave-uniform), so the shuffles see every lane
-    for (int64_t base = blockIdx.x * (int64_t)blockDim.x + (threadIdx.x & ~63); base < nruns;
-         base += (int64_t)gridDim.x * blockDim.x) {
-        const int32_t r = (int32_t)(base + lane);
+    // the workgroup steps together, so the shuffles and barriers see every lane
+    for (int64_t base = blockIdx.x * (int64_t)kHubBlock; base < nruns; base += (int64_t)gridDim.x * kHubBlock) {
+        const int64_t r = base + threadIdx.x;
         const bool valid = r < nruns;
-        int32_t j = -1;
-        double gain = 0.0;
+        int32_t j = -1, c = 0, v = 0, cc = 0, b = 0, e = 0;
+        double gain = 0.0, ey = 0.0;
+        bool other = false;  // a run to fold
         if (valid) {
-            const int32_t b = starts[r], e = starts[r + 1];
+            b = starts[r];
+            e = starts[r + 1];
             const K key = keys[b];
             j = (int32_t)(key >> cbits);
-            const int32_t c = (int32_t)(uint32_t)(key & cmask);
-            const int32_t v = hubs[j];
-            if (!(a.active && !a.active[v])) {
-                const int64_t cc = a.curr[v];
-                if ((int64_t)c != cc) {
-                    double unused = 0.0;
-                    const double ey = hub_run_fold(a.edges, vals, b, e, false, v, unused);
-                    const double kv = a.vdeg[v];
-                    const double eix = own[2 * j] - own[2 * j + 1];
-                    const double ax = a.cdeg[cc] - kv;
-                    const double ay = a.cdeg[c];
-                    gain = 2.0 * (ey - eix) - 2.0 * kv * (ay - ax) * constant;
-                }
-            }
-            gains[r] = gain;
+            c = (int32_t)(uint32_t)(key & cmask);
+            v = hubs[j];
+            cc = a.curr[v];
+            other = !(a.active && !a.active[v]) && c != cc;
         }
+        const int32_t len = e - b;
+        const bool big = other && len >= kHubBlockRun;
+        if (other && len < kHubLongRun) ey = hub_run_fold(a.wgt, vals, b, e);
+        hub_long_runs<4>(a.wgt, vals, other && len >= kHubLongRun && !big, b, e, ey);
+        if (__syncthreads_or(big)) {  // runs between a hub and a giant community: by the workgroup
+            s_run[threadIdx.x] = big ? make_int2(b, e) : make_int2(0, 0);
+            __syncthreads();
+            for (int t = 0; t < kHubBlock; t++) {
+                const int2 q = s_run[t];
+                if (q.x == q.y) continue;
+                auto weight = [&](int64_t k) { return a.wgt[vals[q.x + k]]; };
+                double sum = 0.0;
+                if (!block_exact_sum<kHubBlock, 8>(q.y - q.x, weight, s_red, &sum) && threadIdx.x < 64)
+                    sum = wave_left_fold<4>(-0.0, q.y - q.x, weight);
+                if (threadIdx.x == 0) s_ey[t] = sum;
+            }
+            __syncthreads();
+            if (big) ey = s_ey[threadIdx.x];
+        }
+        if (other) {
+            const double kv = a.vdeg[v];
+            const double eix = own[2 * j] - own[2 * j + 1];
+            const double ax = a.cdeg[cc] - kv;
+            const double ay = a.cdeg[c];
+            gain = 2.0 * (ey - eix) - 2.0 * kv * (ay - ax) * constant;
+        }
+        if (valid) gains[r] = gain;
         // A hub has thousands of runs: when the wave's runs all belong to one hub (lane 0's,
-        // always valid), one atomic carries the wave's largest gain instead of one per run.
+        // valid if any is), one atomic carries the wave's largest gain instead of one per run.
         const unsigned long long gb = gain > 0.0 ? (unsigned long long)__double_as_longlong(gain) : 0ull;
         const int32_t j0 = __shfl(j, 0);
         if (__ballot(valid && j != j0) == 0) {
@@ -1341,19 +1420,21 @@ __global__ void k_hub_pick(const int32_t* __restrict__ pos, const int32_t* __res
 }
 
 // The same move with a workgroup per hub, for sweeps with enough hubs to fill the chip (the
-// coarse levels: thousands of hubs; vt_tuning.hub_block_min sets how many): thread 0 folds the own community's run, the threads take
-// the other runs in turn, and the workgroup reduces their (gain, community) argmax.
-constexpr int kHubBlock = 256;
+// coarse levels: thousands of hubs; vt_tuning.hub_block_min sets how many): the own
+// community's run first, then a thread per other run, the long ones by their wave, and the
+// workgroup reduces the runs' (gain, community) argmax.
 
+// One term in flight per lane in the folds: with four the kernel held 92 registers and 5 waves per
+// SIMD instead of 8, and took 4.6 ms of a run on RGG n = 2^24 instead of 3.5.
 template <class K>
-__global__ void __launch_bounds__(kHubBlock) k_hub_move(MoveArgs a, const int32_t* __restrict__ hubs, int32_t nh,
+__global__ void __launch_bounds__(kHubBlock, 8) k_hub_move(MoveArgs a, const int32_t* __restrict__ hubs, int32_t nh,
                                                         const int64_t* __restrict__ hoffs, const K* __restrict__ keys,
                                                         const uint32_t* __restrict__ vals,
                                                         const int32_t* __restrict__ pos,
                                                         const int32_t* __restrict__ head,
                                                         const int32_t* __restrict__ starts, int cbits)
 {
-    __shared__ double s_ecc, s_self;
+    __shared__ double s_lds[kHubBlock / 64 + 2];
     __shared__ double s_bg[kHubBlock / 64];
     __shared__ int32_t s_bc[kHubBlock / 64];
     unsigned inactive = 0;
@@ -1373,36 +1454,30 @@ __global__ void __launch_bounds__(kHubBlock) k_hub_move(MoveArgs a, const int32_
         const int32_t r0 = hoffs[j] < total ? pos[hoffs[j]] : nruns;
         const int32_t r1 = hoffs[j + 1] < total ? pos[hoffs[j + 1]] : nruns;
         const int64_t cc = a.curr[v];
-        if (threadIdx.x == 0) {
-            const K ckey = ((K)j << cbits) | (K)(uint32_t)cc;
-            int32_t lo = r0, hi = r1;
-            while (lo < hi) {
-                const int32_t mid = (lo + hi) >> 1;
-                if (keys[starts[mid]] < ckey) lo = mid + 1;
-                else hi = mid;
-            }
-            double self = 0.0, ecc = 0.0;
-            if (lo < r1 && keys[starts[lo]] == ckey)
-                ecc = hub_run_fold(a.edges, vals, starts[lo], starts[lo + 1], true, v, self);
-            s_ecc = ecc;
-            s_self = self;
-        }
-        __syncthreads();
-        const double ecc = s_ecc;
+        double ecc, self;
+        hub_own_fold<1, K>(a, v, ((K)j << cbits) | (K)(uint32_t)cc, r0, r1, keys, vals, starts, s_lds, ecc, self);
         const double kv = a.vdeg[v];
-        const double eix = ecc - s_self;
+        const double eix = ecc - self;
         const double ax = a.cdeg[cc] - kv;
         double bg = 0.0;
         int32_t bc = INT_MAX;
-        for (int32_t r = r0 + threadIdx.x; r < r1; r += kHubBlock) {
-            const int32_t b = starts[r], e = starts[r + 1];
-            const int32_t c = (int32_t)(uint32_t)(keys[b] & cmask);
-            if ((int64_t)c == cc) continue;
-            double unused = 0.0;
-            const double ey = hub_run_fold(a.edges, vals, b, e, false, v, unused);
-            const double ay = a.cdeg[c];
-            const double gain = 2.0 * (ey - eix) - 2.0 * kv * (ay - ax) * constant;
-            argmax_take(bg, bc, gain > 0.0 ? gain : 0.0, gain > 0.0 ? c : INT_MAX);
+        for (int32_t rb = r0 + (int32_t)(threadIdx.x & ~63u); rb < r1; rb += kHubBlock) {  // whole waves
+            const int32_t r = rb + (int32_t)(threadIdx.x & 63);
+            int32_t b = 0, e = 0, c = (int32_t)cc;
+            if (r < r1) {
+                b = starts[r];
+                e = starts[r + 1];
+                c = (int32_t)(uint32_t)(keys[b] & cmask);
+            }
+            const bool other = c != (int32_t)cc, lng = e - b >= kHubLongRun;
+            double ey = 0.0;
+            if (other && !lng) ey = hub_run_fold(a.wgt, vals, b, e);
+            hub_long_runs<1>(a.wgt, vals, other && lng, b, e, ey);
+            if (other) {
+                const double ay = a.cdeg[c];
+                const double gain = 2.0 * (ey - eix) - 2.0 * kv * (ay - ax) * constant;
+                argmax_take(bg, bc, gain > 0.0 ? gain : 0.0, gain > 0.0 ? c : INT_MAX);
+            }
         }
         for (int o = 32; o > 0; o >>= 1) argmax_take(bg, bc, __shfl_xor(bg, o), __shfl_xor(bc, o));
         if ((threadIdx.x & 63) == 0) {
@@ -1467,11 +1542,11 @@ __global__ void k_hbm_table_init(int32_t* keys, double* vals, int64_t n)
 // vDegree: left fold of each row's weights from 0.0 in CSR order (distSumVertexDegree,
 // louvain.cpp:2161-2186), one thread per row.  Eight loads are issued ahead of the dependent
 // adds, so a long row (coarse levels, hubs) streams at memory rate instead of one load
-// latency per edge.  Rows of degree >= long_min are left to k_row_fold_wave.
+// latency per edge.  Rows of degree >= long_min are left to k_row_fold_long.
 constexpr int kFoldRows = 256;
 // Rows at least this long get a wave each when a graph has them (a hub of degree 36 K
 // folded by one thread held the whole launch for 3 ms).
-constexpr int64_t kFoldLongRow = 2048;
+constexpr int64_t kFoldLongRow = 512;
 
 __global__ void __launch_bounds__(kFoldRows) k_row_fold(const int64_t* __restrict__ offs, const DEdge* __restrict__ edges,
                                                         int64_t nv, double* __restrict__ vdeg, int64_t long_min)
@@ -1493,29 +1568,55 @@ __global__ void __launch_bounds__(kFoldRows) k_row_fold(const int64_t* __restric
     }
 }
 
-// Long rows (the coarse levels, hubs): one wave per row loads 64 weights at a time with
-// coalesced reads (the next 64 in flight while these are added), and every lane adds them in
-// lane order, each read as a wave-uniform value -- the same left fold as k_row_fold.  Lanes
-// past the row's end hold -0.0, which leaves any sum unchanged.  Rows shorter than long_min
-// are left to k_row_fold.
-constexpr int kFoldWaveRows = 4;
-__global__ void __launch_bounds__(64 * kFoldWaveRows) k_row_fold_wave(const int64_t* __restrict__ offs,
-                                                                     const DEdge* __restrict__ edges, int64_t nv,
-                                                                     double* __restrict__ vdeg, int64_t long_min)
+// The rows of long_min entries and more (hubs, the coarse levels), a wave each, and those of
+// kFoldBlockRow and more a workgroup each where their weights are whole numbers: a skewed
+// graph's giant coarse row (half a million entries) held the launch for 4.5 ms as one wave's
+// chain of lane reads on BA n = 2^22.  A workgroup's rows are gridDim apart, so that hubs
+// with neighbouring ids spread over the chip.
+constexpr int kFoldLongBlock = 256;
+constexpr int64_t kFoldBlockRow = 8192;
+__global__ void __launch_bounds__(kFoldLongBlock) k_row_fold_long(const int64_t* __restrict__ offs,
+                                                                 const DEdge* __restrict__ edges, int64_t nv,
+                                                                 double* __restrict__ vdeg, int64_t long_min)
 {
+    __shared__ int32_t s_row[kFoldLongBlock];
+    __shared__ int32_t s_n, s_big;
+    __shared__ double s_red[kFoldLongBlock / 64];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    for (int64_t i = (int64_t)blockIdx.x * kFoldWaveRows + w; i < nv; i += (int64_t)gridDim.x * kFoldWaveRows) {
-        const int64_t e0 = offs[i], e1 = offs[i + 1];
-        if (e1 - e0 < long_min) continue;  // wave-uniform: i is the same in every lane
-        double acc = 0.0;
-        double x = (e0 + lane < e1) ? edges[e0 + lane].weight : -0.0;
-        for (int64_t base = e0; base < e1; base += 64) {
-            const double xn = (base + 64 + lane < e1) ? edges[base + 64 + lane].weight : -0.0;
-#pragma unroll
-            for (int u = 0; u < 64; u++) acc = acc + readlane_f64(x, u);
-            x = xn;
+    const int64_t step = (int64_t)gridDim.x * kFoldLongBlock;
+    for (int64_t base = 0; base < nv; base += step) {
+        if (threadIdx.x == 0) s_n = s_big = 0;
+        __syncthreads();
+        const int64_t i = base + (int64_t)threadIdx.x * gridDim.x + blockIdx.x;
+        if (i < nv) {
+            const int64_t d = offs[i + 1] - offs[i];
+            if (d >= long_min) {  // the workgroup's rows from the list's end
+                if (d >= kFoldBlockRow) s_row[kFoldLongBlock - 1 - atomicAdd(&s_big, 1)] = (int32_t)i;
+                else s_row[atomicAdd(&s_n, 1)] = (int32_t)i;
+            }
         }
-        if (lane == 0) vdeg[i] = acc;
+        __syncthreads();
+        const int n = s_n, nbig = s_big;
+        for (int k = 0; k < nbig; k++) {
+            const int64_t v = s_row[kFoldLongBlock - 1 - k];
+            const DEdge* e = edges + offs[v];
+            const int64_t d = offs[v + 1] - offs[v];
+            auto weight = [=](int64_t j) { return e[j].weight; };
+            double sum = 0.0;
+            if (block_exact_sum<kFoldLongBlock, 8>(d, weight, s_red, &sum)) {
+                if (threadIdx.x == 0) vdeg[v] = 0.0 + sum;
+            } else if (w == 0) {
+                sum = wave_left_fold<4>(0.0, d, weight);
+                if (lane == 0) vdeg[v] = sum;
+            }
+        }
+        for (int k = w; k < n; k += kFoldLongBlock / 64) {
+            const int64_t v = s_row[k];
+            const DEdge* e = edges + offs[v];
+            const double sum = wave_left_fold<4>(0.0, offs[v + 1] - offs[v], [=](int64_t j) { return e[j].weight; });
+            if (lane == 0) vdeg[v] = sum;
+        }
+        __syncthreads();  // the list is reused
     }
 }
 
@@ -2603,7 +2704,7 @@ struct Phase {
             VT_LAUNCH(ctx, "split_fold", k_split_fold, grid_for(nv, kSfRows, 65536), 256, 0, g->offs, g->edges, nv,
                       tail32.p, wgt.p, vdeg.p);
         } else if (nv && nv < 65536 && g->ne > 48 * nv) {  // few, long rows: a thread per row would leave the GPU idle
-            VT_LAUNCH(ctx, "row_fold", k_row_fold_wave, grid_for(nv, kFoldWaveRows, 65536), 64 * kFoldWaveRows, 0, g->offs,
+            VT_LAUNCH(ctx, "row_fold", k_row_fold_long, grid_for(nv, kFoldLongBlock / 64, 65536), kFoldLongBlock, 0, g->offs,
                       g->edges, nv, vdeg.p, (int64_t)0);
         } else if (nv) {
             // a thread per row, and a wave per row for the rows of kFoldLongRow or more
@@ -2611,7 +2712,7 @@ struct Phase {
             VT_LAUNCH(ctx, "row_fold", k_row_fold, grid_for(nv, kFoldRows, 16384), kFoldRows, 0, g->offs, g->edges, nv,
                       vdeg.p, split ? kFoldLongRow : INT64_MAX);
             if (split)
-                VT_LAUNCH(ctx, "row_fold_long", k_row_fold_wave, grid_for(nv, kFoldWaveRows, 16384), 64 * kFoldWaveRows, 0,
+                VT_LAUNCH(ctx, "row_fold_long", k_row_fold_long, grid_for(nv, kFoldLongBlock, 4096), kFoldLongBlock, 0,
                           g->offs, g->edges, nv, vdeg.p, kFoldLongRow);
         }
         VT_LAUNCH(ctx, "init", k_init, grid_for(nv, 256, 8192), 256, 0, nv, (const double*)vdeg.p, cdeg.p, csize.p, past.p,
@@ -2842,9 +2943,9 @@ struct Phase {
                       nh, hoffs, ks, vs, (const int32_t*)pos, (const int32_t*)head, (const int32_t*)starts, cbits);
             return;
         }
-        VT_LAUNCH(ctx, "hub_own", k_hub_own<K>, grid_for(nh, 64, 4096), 64, 0, a, hubs, nh, hoffs, ks, vs,
+        VT_LAUNCH(ctx, "hub_own", k_hub_own<K>, (unsigned)std::min<int64_t>(nh, 16384), kHubBlock, 0, a, hubs, nh, hoffs, ks, vs,
                   (const int32_t*)pos, (const int32_t*)head, (const int32_t*)starts, cbits, own, best, bestc);
-        VT_LAUNCH(ctx, "hub_runs", k_hub_runs<K>, grid_for(total, 256, 16384), 256, 0, a, hubs, nh, hoffs, ks, vs,
+        VT_LAUNCH(ctx, "hub_runs", k_hub_runs<K>, grid_for(total, kHubBlock, 16384), kHubBlock, 0, a, hubs, nh, hoffs, ks, vs,
                   (const int32_t*)pos, (const int32_t*)head, (const int32_t*)starts, cbits, (const double*)own, gains, best);
         VT_LAUNCH(ctx, "hub_pick", k_hub_pick<K>, grid_for(total, 256, 16384), 256, 0, (const int32_t*)pos,
                   (const int32_t*)head, hoffs, nh, ks, (const int32_t*)starts, cbits, (const double*)gains,

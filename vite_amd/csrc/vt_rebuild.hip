@@ -417,26 +417,17 @@ __global__ void k_ext_runs(const unsigned long long* __restrict__ keys, const do
     }
 }
 
-// The long runs: a wave loads 64 values at a time, the next 64 in flight, and adds them in
-// lane order (from -0.0, so that the first is taken as it is; lanes past the end hold -0.0).
+// The long runs, a wave each (from -0.0, so that the first is taken as it is).
 __global__ void __launch_bounds__(64) k_ext_runs_long(const uint32_t* __restrict__ nlong, const uint32_t* __restrict__ longs,
                                                       const double* __restrict__ vals, const int64_t* __restrict__ starts,
                                                       double* __restrict__ rw)
 {
-    const int lane = threadIdx.x;
     const uint32_t n = *nlong;
     for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
         const uint32_t r = longs[i];
-        const int64_t b = starts[r], e = starts[r + 1];
-        double acc = -0.0;
-        double x = b + lane < e ? vals[b + lane] : -0.0;
-        for (int64_t base = b; base < e; base += 64) {
-            const double xn = base + 64 + lane < e ? vals[base + 64 + lane] : -0.0;
-#pragma unroll
-            for (int u = 0; u < 64; u++) acc = acc + readlane_f64(x, u);
-            x = xn;
-        }
-        if (lane == 0) rw[r] = acc;
+        const double* x = vals + starts[r];
+        const double acc = wave_left_fold<4>(-0.0, starts[r + 1] - starts[r], [=](int64_t k) { return x[k]; });
+        if (threadIdx.x == 0) rw[r] = acc;
     }
 }
 
