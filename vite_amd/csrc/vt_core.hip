@@ -203,11 +203,12 @@ void d2h(vt_ctx* ctx, void* dst, const void* src, size_t bytes)
     }
     ctx->stage_off = 0;  // the stream has drained: every staged copy has run
 }
-// Pinned host memory a kernel writes an iteration's scalars to (64 bytes): they are there when
-// the stream has drained, with no copy queued behind the kernel.
+// Pinned host memory that kernels write a few scalars to (256 bytes; [0, 1]: an iteration's Q and
+// movers, [2]: a phase's whole degrees, [8, 14): a rebuild's totals): they are there when the
+// stream has drained, with no copy queued behind the kernel.
 double* mail(vt_ctx* ctx)
 {
-    if (!ctx->mail) VT_HIP(ctx, hipHostMalloc((void**)&ctx->mail, 64, hipHostMallocDefault));
+    if (!ctx->mail) VT_HIP(ctx, hipHostMalloc((void**)&ctx->mail, 256, hipHostMallocDefault));
     return ctx->mail;
 }
 void d2d(vt_ctx* ctx, void* dst, const void* src, size_t bytes)

@@ -244,7 +244,7 @@ __device__ __forceinline__ double wave_left_fold(double acc, int64_t n, F f)
             m = m + fabs(x[r]);
         }
         // 64 lanes of less than 2^45 and an acc below 2^51
-        ok = ok & (m < 0x1p45) & (open | (whole_number(acc) & (fabs(acc) < 0x1p51)));
+        ok = ok & (m < 0x1p45) & (open || (whole_number(acc) && fabs(acc) < 0x1p51));
         if (__ballot(!ok) == 0) {
             part = s;
             mag = m;
@@ -297,6 +297,28 @@ __device__ __forceinline__ bool block_exact_sum(int64_t n, F f, double* red, dou
     __syncthreads();  // red may be reused
     *sum = t;
     return true;
+}
+
+// Exclusive scan of one value per thread over a workgroup of B; *total = the sum.
+template <int B, class T>
+__device__ __forceinline__ T block_scan(T x, T* s_wave, T* total)
+{
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    T inc = x;
+    for (int o = 1; o < 64; o <<= 1) {
+        const T y = __shfl_up(inc, o);
+        if (lane >= o) inc += y;
+    }
+    if (lane == 63) s_wave[w] = inc;
+    __syncthreads();
+    T before = 0, all = 0;
+    for (int k = 0; k < B / 64; k++) {
+        if (k < w) before += s_wave[k];
+        all += s_wave[k];
+    }
+    __syncthreads();  // s_wave may be reused
+    *total = all;
+    return before + inc - x;
 }
 
 // ---- device primitives (vt_prims.hip) -------------------------------------------------

@@ -1654,6 +1654,14 @@ __global__ void k_constant(const double* __restrict__ sums, const unsigned long 
     }
 }
 
+// A row's sweep list: its degree bucket, the wide bucket split by table size.
+__device__ __host__ __forceinline__ uint32_t list_bucket(int64_t d, int lpv_max, const BucketBounds& bb)
+{
+    const uint32_t b = (uint32_t)(d <= lpv_max ? kLpvBucket : degree_bucket(d, bb));
+    if (b == kHubBucket - 1) return d <= bb.wide[0] ? kWide512Bucket : d <= bb.wide[1] ? kWide1024Bucket : b;
+    return b;
+}
+
 // Sort keys for the sweep lists: (color bucket, degree bucket).
 // In a batch (gid), a vertex whose graph has left the phase gets key `excluded`, past every
 // list, so the sweeps no longer visit it.
@@ -1664,8 +1672,7 @@ __global__ void k_list_keys(const int64_t* __restrict__ offs, int64_t nv, const 
 {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nv; i += (int64_t)gridDim.x * blockDim.x) {
         const int64_t d = offs[i + 1] - offs[i];
-        uint32_t b = (uint32_t)(d <= lpv_max ? kLpvBucket : degree_bucket(d, bb));
-        if (b == kHubBucket - 1) b = d <= bb.wide[0] ? kWide512Bucket : d <= bb.wide[1] ? kWide1024Bucket : b;
+        const uint32_t b = list_bucket(d, lpv_max, bb);
         uint32_t c = 0;
         if (colors) c = (uint32_t)(colors[i] < 0 ? num_color - 1 : colors[i]);
         keys[i] = (gid && !gact[gid[i]]) ? excluded : c * kNumBuckets + b;
@@ -2183,6 +2190,54 @@ constexpr int kTailVerts = 8192;
 constexpr int kTailBlock = 1024;
 constexpr int kTailRun = 24;  // events a thread orders by insertion; longer runs take a wave each
 
+// tree_sum2's sums of a and of b squared (b may be null) over n <= kTailVerts values by one
+// workgroup: its blocks of 256 threads, four at a time, then its tree over the partials, in
+// thread 0's r.  lds: 2 * kTailBlock doubles.
+__device__ __forceinline__ void small_tree_sum2(const double* __restrict__ a, const double* __restrict__ b_sq, int n, int blocks,
+                                                int64_t chunk, double* lds, double (*part)[kTailVerts / (4 * 256)], double* r)
+{
+    const int t = threadIdx.x, sub = t & 255;
+    double *sa = lds, *sb = lds + kTailBlock;
+    for (int b0 = 0; b0 < blocks; b0 += kTailBlock / 256) {
+        const int b = b0 + (t >> 8);
+        const int64_t lo = (int64_t)b * chunk;
+        const int64_t hi = b < blocks ? min(lo + chunk, (int64_t)n) : lo;
+        double xa = 0.0, xb = 0.0;
+        for (int64_t i = lo + sub; i < hi; i += 256) {
+            xa = xa + a[i];
+            if (b_sq) {
+                const double v = b_sq[i];
+                xb = xb + v * v;
+            }
+        }
+        sa[t] = xa;
+        sb[t] = xb;
+        __syncthreads();
+        for (int h = 128; h > 0; h >>= 1) {
+            if (sub < h) {
+                sa[t] = sa[t] + sa[t + h];
+                sb[t] = sb[t] + sb[t + h];
+            }
+            __syncthreads();
+        }
+        if (sub == 0 && b < blocks) {
+            part[0][b] = sa[t];
+            part[1][b] = sb[t];
+        }
+        __syncthreads();
+    }
+    if (t == 0) {
+        // k_sum2_final's halving tree over the (at most 8) partials; its other entries are zeros
+        for (int q = 0; q < 2; q++) {
+            double y[8];
+            for (int k = 0; k < 8; k++) y[k] = 0.0 + (k < blocks ? part[q][k] : 0.0);
+            for (int h = 4; h > 0; h >>= 1)
+                for (int k = 0; k < h; k++) y[k] = y[k] + y[k + h];
+            r[q] = y[0];
+        }
+    }
+}
+
 struct TailArgs {
     MoverArgs m;
     int32_t nv;
@@ -2320,51 +2375,130 @@ __global__ void __launch_bounds__(kTailBlock) k_tail_small(TailArgs a)
         __syncthreads();
     }
     if (!a.cw) return;
-    // tree_sum2's blocks of 256 threads, four at a time, in ev's space
-    double* sa = (double*)ev;
-    double* sb = sa + kTailBlock;
-    const int sub = t & 255;
-    for (int b0 = 0; b0 < a.blocks; b0 += kTailBlock / 256) {
-        const int b = b0 + (t >> 8);
-        const int64_t lo = (int64_t)b * a.chunk;
-        const int64_t hi = b < a.blocks ? min(lo + a.chunk, (int64_t)a.nv) : lo;
-        double xa = 0.0, xb = 0.0;
-        for (int64_t i = lo + sub; i < hi; i += 256) {
-            xa = xa + a.cw[i];
-            const double v = a.cdeg[i];
-            xb = xb + v * v;
-        }
-        sa[t] = xa;
-        sb[t] = xb;
-        __syncthreads();
-        for (int h = 128; h > 0; h >>= 1) {
-            if (sub < h) {
-                sa[t] = sa[t] + sa[t + h];
-                sb[t] = sb[t] + sb[t + h];
-            }
-            __syncthreads();
-        }
-        if (sub == 0 && b < a.blocks) {
-            s_part[0][b] = sa[t];
-            s_part[1][b] = sb[t];
-        }
-        __syncthreads();
-    }
+    double r[2];
+    small_tree_sum2(a.cw, a.cdeg, a.nv, a.blocks, a.chunk, (double*)ev, s_part, r);
     if (t == 0) {
-        // k_sum2_final's halving tree over the (at most 8) partials; its other entries are zeros
-        double r[2];
-        for (int q = 0; q < 2; q++) {
-            double y[8];
-            for (int k = 0; k < 8; k++) y[k] = 0.0 + (k < a.blocks ? s_part[q][k] : 0.0);
-            for (int h = 4; h > 0; h >>= 1)
-                for (int k = 0; k < h; k++) y[k] = y[k] + y[k + h];
-            r[q] = y[0];
-            a.sums[q] = y[0];
-        }
+        a.sums[0] = r[0];
+        a.sums[1] = r[1];
         const double c = a.constant[0];
         a.out[0] = fabs((r[0] * c) - (r[1] * c * c));
         ((unsigned long long*)a.out)[1] = *a.movers;
         *a.movers = 0;
+    }
+}
+
+// The set-up of a phase on at most kTailVerts vertices, its degrees given, by one workgroup: the
+// state (k_init), 2m and 1/2m (tree_sum2, k_constant), the sweep's lists (vertices by degree
+// bucket, ascending inside) and the hub rows' offsets in the key array.  These were fourteen
+// launches and two host reads; the host reads all of it with one wait.
+struct SetupArgs {
+    const int64_t* offs;
+    const double* vdeg;
+    int32_t nv, blocks;
+    int64_t chunk;
+    double *cdeg, *sums, *constant, *out;  // out (pinned): [2] whole degrees, [16, 26) the buckets' sizes, [26] hub entries
+    int32_t *csize, *past, *curr, *target, *lists;
+    unsigned char* active;  // null when ET is off, with the three below
+    double *frozen, *pa, *pb;
+    int64_t* iscal;               // 4, cleared
+    unsigned long long* ucount;   // 6, cleared
+    int64_t* hoffs;               // nv + 1
+    BucketBounds bb;
+    int32_t lpv_max;
+};
+
+__global__ void __launch_bounds__(kTailBlock) k_setup_small(SetupArgs a)
+{
+    constexpr int kPer = kTailVerts / kTailBlock, kWaves = kTailBlock / 64;
+    __shared__ double lds[2 * kTailBlock];
+    __shared__ double s_part[2][kTailVerts / (4 * 256)];
+    __shared__ int s_cnt[kNumBuckets][kPer * kWaves];  // per bucket, by tile of vertices and wave
+    __shared__ int s_total[kNumBuckets];
+    __shared__ unsigned long long s_scan[kWaves];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const unsigned long long below = (1ull << lane) - 1;
+    if (t < 4) a.iscal[t] = 0;
+    if (t < 6) a.ucount[t] = 0;
+    bool fraction = false;
+    uint32_t bucket[kPer], rank[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        const int i = k * kTailBlock + t;
+        uint32_t b = kNumBuckets;
+        if (i < a.nv) {
+            const double d = a.vdeg[i];
+            fraction = fraction || !(whole_number(d) && d >= 0.0);
+            a.cdeg[i] = d;
+            a.csize[i] = 1;
+            a.past[i] = i;
+            a.curr[i] = i;
+            a.target[i] = 0;
+            if (a.active) {
+                a.active[i] = 1;
+                a.frozen[i] = 0.0;
+                a.pa[i] = 0.0;
+                a.pb[i] = 1.0;
+            }
+            b = list_bucket(a.offs[i + 1] - a.offs[i], a.lpv_max, a.bb);
+        }
+        bucket[k] = b;
+        rank[k] = 0;
+#pragma unroll
+        for (uint32_t q = 0; q < kNumBuckets; q++) {
+            const unsigned long long m = __ballot(b == q);
+            if (b == q) rank[k] = (uint32_t)__popcll(m & below);
+            if (lane == 0) s_cnt[q][k * kWaves + w] = __popcll(m);
+        }
+    }
+    const bool any_fraction = __syncthreads_or(fraction);
+    // each bucket's counts scanned by a wave, two a lane
+    static_assert(kPer * kWaves == 128 && kNumBuckets <= kWaves, "two counts per lane, a wave per bucket");
+    if (w < kNumBuckets) {
+        const int x0 = s_cnt[w][2 * lane], x1 = s_cnt[w][2 * lane + 1];
+        int inc = x0 + x1;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(inc, o);
+            if (lane >= o) inc += y;
+        }
+        s_cnt[w][2 * lane] = inc - x0 - x1;
+        s_cnt[w][2 * lane + 1] = inc - x1;
+        if (lane == 63) s_total[w] = inc;
+    }
+    __syncthreads();
+    int hub_off = 0;
+    for (int q = 0; q < kHubBucket; q++) hub_off += s_total[q];
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        const uint32_t b = bucket[k];
+        if (b >= kNumBuckets) continue;
+        int at = 0;
+        for (uint32_t q = 0; q < kNumBuckets; q++)
+            if (q < b) at += s_total[q];
+        a.lists[at + s_cnt[b][k * kWaves + w] + (int)rank[k]] = k * kTailBlock + t;
+    }
+    __syncthreads();
+    unsigned long long entries = 0;
+    const int nh = s_total[kHubBucket];
+    for (int j0 = 0; j0 < nh; j0 += kTailBlock) {
+        const int j = j0 + t;
+        const int32_t v = j < nh ? a.lists[hub_off + j] : 0;
+        unsigned long long sum = 0;
+        const unsigned long long x = j < nh ? (unsigned long long)(a.offs[v + 1] - a.offs[v]) : 0;
+        const unsigned long long at = entries + block_scan<kTailBlock>(x, s_scan, &sum);
+        if (j < nh) a.hoffs[j] = (int64_t)at;
+        entries += sum;
+    }
+    double r[2];
+    small_tree_sum2(a.vdeg, nullptr, a.nv, a.blocks, a.chunk, lds, s_part, r);
+    int64_t* out = (int64_t*)a.out;
+    if (t < kNumBuckets) out[16 + t] = s_total[t];
+    if (t == 0) {
+        a.hoffs[nh] = (int64_t)entries;
+        out[26] = (int64_t)entries;
+        a.sums[0] = r[0];
+        a.sums[1] = r[1];
+        a.constant[0] = 1.0 / r[0];
+        a.out[2] = !any_fraction && r[0] < 0x1p52 ? 1.0 : 0.0;
     }
 }
 
@@ -2761,11 +2895,15 @@ struct Phase {
         scal = DBuf<double>(ctx, 8);
         iscal = DBuf<int64_t>(ctx, 4);
         ucount = DBuf<unsigned long long>(ctx, 6);
+    }
+
+    void clear_counters()
+    {
         dzero(ctx, iscal.p, 32);
         dzero(ctx, ucount.p, 48);
     }
 
-    void init_state(bool with_et)
+    void row_degrees()
     {
         if (!tail32.p && nv && g->ne <= 48 * nv && g->max_degree <= kSfTile) {
             // short rows (a row's fold is one thread's, so no long ones): the split copy the
@@ -2787,6 +2925,12 @@ struct Phase {
                 VT_LAUNCH(ctx, "row_fold_long", k_row_fold_long, grid_for(nv, kFoldLongBlock, 4096), kFoldLongBlock, 0,
                           g->offs, g->edges, nv, vdeg.p, kFoldLongRow);
         }
+    }
+
+    void init_state(bool with_et)
+    {
+        clear_counters();
+        row_degrees();
         VT_LAUNCH(ctx, "init", k_init, grid_for(nv, 256, 8192), 256, 0, nv, (const double*)vdeg.p, cdeg.p, csize.p, past.p,
                   curr.p, target.p, with_et ? active.p : nullptr, with_et ? frozen.p : nullptr,
                   with_et ? pa.p : nullptr, with_et ? pb.p : nullptr, ucount.p + 5);
@@ -2799,6 +2943,46 @@ struct Phase {
         else tree_sum2(ctx, vdeg.p, nullptr, nv, sums());
         VT_LAUNCH(ctx, "constant", k_constant, 1, 64, 0, (const double*)sums(),
                   (const unsigned long long*)(ucount.p + 5), constant(), mail(ctx) + 2);
+    }
+
+    // alloc, init and build_lists of a plain phase on at most kTailVerts vertices (tree sums).
+    void setup_small()
+    {
+        lists = DBuf<int32_t>(ctx, (size_t)nv);
+        hub_offs.clear();
+        hub_offs.emplace_back(ctx, (size_t)nv + 1);
+        row_degrees();
+        SetupArgs a;
+        a.offs = g->offs;
+        a.vdeg = vdeg.p;
+        a.nv = (int32_t)nv;
+        int64_t blocks = 0;
+        sum2_plan(nv, &blocks, &a.chunk);
+        a.blocks = (int32_t)blocks;
+        a.cdeg = cdeg.p;
+        a.sums = sums();
+        a.constant = constant();
+        a.out = mail(ctx);
+        a.csize = csize.p;
+        a.past = past.p;
+        a.curr = curr.p;
+        a.target = target.p;
+        a.lists = lists.p;
+        a.active = et ? active.p : nullptr;
+        a.frozen = frozen.p;
+        a.pa = pa.p;
+        a.pb = pb.p;
+        a.iscal = iscal.p;
+        a.ucount = ucount.p;
+        a.hoffs = hub_offs[0].p;
+        a.bb = bounds();
+        a.lpv_max = lpv_max_degree();
+        VT_LAUNCH(ctx, "setup", k_setup_small, 1, kTailBlock, 0, a);
+        sync(ctx);
+        const int64_t* h = (const int64_t*)mail(ctx);
+        plan_sweeps(1, h + 16);
+        hub_total.assign(1, h[26]);
+        hub_sort = true;
     }
 
     // Sorts vertices into (color, degree bucket) lists and, with colors, the per-color event
@@ -2826,42 +3010,7 @@ struct Phase {
             if (alt) d2d(ctx, lists.p, v1, 4 * (size_t)nv);
             d2h(ctx, h.data(), hist, 8 * nkeys);
         }
-        sweeps.assign(ncol, ColorSweep{});
-        int64_t off = 0, max_hub = 0;
-        constexpr int kGroups[kFusedBuckets] = {256 / 4, 256 / 8, 256 / 16, 256 / 32};
-        for (int64_t c = 0; c < ncol; c++) {
-            ColorSweep& cs = sweeps[c];
-            int64_t blocks = 0;
-            for (int b = 0; b < kNumBuckets; b++) {
-                const int64_t cnt = h[c * kNumBuckets + b];
-                if (b < kFusedBuckets) {
-                    cs.plan.bbeg[b] = blocks;
-                    cs.plan.off[b] = off;
-                    cs.plan.n[b] = cnt;
-                    const int64_t nb = std::min<int64_t>((cnt + kGroups[b] - 1) / kGroups[b],
-                                                         ctx->tuning.blocks_per_bucket);
-                    blocks += (nb + kXcds - 1) / kXcds * kXcds;
-                } else if (b == kFusedBuckets) {
-                    cs.mid_off = off;
-                    cs.mid_n = cnt;
-                } else if (b == kWide512Bucket || b == kWide1024Bucket || b == kHubBucket - 1) {
-                    const int w = b == kWide512Bucket ? 0 : b == kWide1024Bucket ? 1 : 2;
-                    cs.wide_off[w] = off;
-                    cs.wide_n[w] = cnt;
-                } else if (b == kLpvBucket) {
-                    cs.lpv_off = off;
-                    cs.lpv_n = cnt;
-                } else {
-                    cs.hub_off = off;
-                    cs.hub_n = cnt;
-                    max_hub = std::max(max_hub, cnt);
-                }
-                off += cnt;
-            }
-            cs.plan.bbeg[kFusedBuckets] = blocks;
-            cs.fused_blocks = blocks;
-        }
-        for (int64_t c = 0; c < ncol; c++) sweeps[c].index = (int32_t)c;
+        const int64_t max_hub = plan_sweeps(ncol, h.data());
         // Hub rows: by sorting, unless the sweep must stay free of library sorts (a batch
         // replays its sweeps from captured graphs) or edge indexes exceed 32 bits.
         // the sorted path keeps run positions in 32 bits: hub entries (at most ne) below 2^31
@@ -2912,6 +3061,49 @@ struct Phase {
             color_ptr.assign(num_color + 1, 0);
             for (int64_t c = 0; c < num_color; c++) color_ptr[c + 1] = color_ptr[c] + hc[c];
         }
+    }
+
+    // The launch plan of every sweep from its lists' sizes h[sweep * kNumBuckets + bucket]; returns
+    // the largest number of hub rows in one.
+    int64_t plan_sweeps(int64_t ncol, const int64_t* h)
+    {
+        sweeps.assign(ncol, ColorSweep{});
+        int64_t off = 0, max_hub = 0;
+        constexpr int kGroups[kFusedBuckets] = {256 / 4, 256 / 8, 256 / 16, 256 / 32};
+        for (int64_t c = 0; c < ncol; c++) {
+            ColorSweep& cs = sweeps[c];
+            int64_t blocks = 0;
+            for (int b = 0; b < kNumBuckets; b++) {
+                const int64_t cnt = h[c * kNumBuckets + b];
+                if (b < kFusedBuckets) {
+                    cs.plan.bbeg[b] = blocks;
+                    cs.plan.off[b] = off;
+                    cs.plan.n[b] = cnt;
+                    const int64_t nb = std::min<int64_t>((cnt + kGroups[b] - 1) / kGroups[b],
+                                                         ctx->tuning.blocks_per_bucket);
+                    blocks += (nb + kXcds - 1) / kXcds * kXcds;
+                } else if (b == kFusedBuckets) {
+                    cs.mid_off = off;
+                    cs.mid_n = cnt;
+                } else if (b == kWide512Bucket || b == kWide1024Bucket || b == kHubBucket - 1) {
+                    const int w = b == kWide512Bucket ? 0 : b == kWide1024Bucket ? 1 : 2;
+                    cs.wide_off[w] = off;
+                    cs.wide_n[w] = cnt;
+                } else if (b == kLpvBucket) {
+                    cs.lpv_off = off;
+                    cs.lpv_n = cnt;
+                } else {
+                    cs.hub_off = off;
+                    cs.hub_n = cnt;
+                    max_hub = std::max(max_hub, cnt);
+                }
+                off += cnt;
+            }
+            cs.plan.bbeg[kFusedBuckets] = blocks;
+            cs.fused_blocks = blocks;
+        }
+        for (int64_t c = 0; c < ncol; c++) sweeps[c].index = (int32_t)c;
+        return max_hub;
     }
 
     void key_histogram(const uint32_t* keys, int64_t n, int64_t* hist, int nbins)
@@ -3259,6 +3451,14 @@ vt_phase* phase_begin(vt_ctx* ctx, vt_graph* g, const vt_phase_params* p)
         st->prevMod = p->lower;
         Phase& ph = st->ph;
         ph.alloc(et != 0);
+        if (mode == VT_MODE_PLAIN && nv > 0 && nv <= kTailVerts && g->ne < (int64_t(1) << 31) &&
+            !(p->flags & VT_FLAG_SEQUENTIAL_SUMS)) {
+            ph.setup_small();
+            ph.whole = mail(ctx)[2] == 1.0;
+            ctx->trace_q.clear();
+            ctx->trace_moves.clear();
+            return st;
+        }
         ph.init(p->flags);
         if (mode != VT_MODE_PLAIN) {
             for (int64_t i = 0; i < nv; i++)
@@ -3904,6 +4104,7 @@ int vt_sweep(vt_ctx* ctx, const vt_graph* g, const int64_t* curr, const int64_t*
             if (curr[i] < 0 || curr[i] >= nv) fail(ctx, VT_ERR_ARG, "vt_sweep: community of vertex %lld out of range", (long long)i);
         Phase ph(ctx, g);
         ph.alloc(false);
+        ph.clear_counters();
         const size_t b8 = 8 * (size_t)nv;
         DBuf<int64_t> wide(ctx, (size_t)std::max<int64_t>(nv, 1));
         auto ids = [&](const int64_t* src, int32_t* dst) {

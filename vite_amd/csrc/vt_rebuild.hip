@@ -193,14 +193,18 @@ constexpr int kCfMaxKeys = 128;           // distinct keys a community may hold 
 constexpr int kCfList = kCfMaxKeys + 64;  // a chunk adds at most 64 keys before the check
 constexpr uint32_t kNoKey = 0xffffffffu;
 
-// Per community c: its coarse row staged at rkey/rval[s0, s0 + rowlen[c]), with s0 its
-// offset in the concatenated rows; or, with more distinct keys than the table holds,
-// rowlen[c] = 0 and xcnt[c] = its entry count, for the sort path.
+// Per community c (there are *n_comm): its coarse row staged at rkey/rval[s0, s0 + rowlen[c]),
+// with s0 its offset in the concatenated rows; or, with more distinct keys than the table holds,
+// rowlen[c] = 0 and xcnt[c] = its entry count, for the sort path.  (A second pass over those
+// with a table of 512 or 1024 slots measured even with the sort on RGG n = 2^24: its 13 or 24 KB
+// of LDS per wave leave too few waves to hide a chunk's chain of LDS steps.)
 __global__ void __launch_bounds__(64 * kFoldWaves) k_comm_fold(
-    int64_t nc, const int64_t* __restrict__ cstart, const int64_t* __restrict__ moff, const int64_t* __restrict__ mrow,
-    const DEdge* __restrict__ edges, const uint32_t* __restrict__ newid,
+    const int64_t* __restrict__ n_comm, const int64_t* __restrict__ cstart, const int64_t* __restrict__ moff,
+    const int64_t* __restrict__ mrow, const DEdge* __restrict__ edges, const uint32_t* __restrict__ newid,
     uint32_t* __restrict__ rkey, double* __restrict__ rval, int64_t* __restrict__ rowlen, int64_t* __restrict__ xcnt)
 {
+    const int64_t nc = *n_comm;
+    if ((int64_t)blockIdx.x * kFoldWaves >= nc) return;
     __shared__ uint32_t tk[kFoldWaves][kCfCap];
     __shared__ double tv[kFoldWaves][kCfCap];
     __shared__ unsigned long long tm[kFoldWaves][kCfCap];
@@ -523,6 +527,162 @@ __global__ void k_pair_totals(const int64_t* __restrict__ a, const int64_t* __re
     }
 }
 
+// ---- small graphs (at most kSmallVerts vertices: the coarse levels, a caller's small graph) ---
+// Numbering, member lists and their offsets are some twenty launches of a few microseconds and
+// a host read; here one workgroup does them in LDS, and the row lengths' scans in another
+// launch, so that a rebuild is five launches and one host read.
+constexpr int kSmallVerts = 8192;
+constexpr int kSmallBlock = 1024;
+constexpr int kSmallPer = kSmallVerts / kSmallBlock;  // consecutive positions per thread in the scans
+
+// tot: [0] = the communities' number (0 with ids out of range), [1] = the ids out of range.
+__global__ void __launch_bounds__(kSmallBlock) k_members_small(const int64_t* __restrict__ cvect, int nv,
+                                                               const int64_t* __restrict__ offs, uint32_t* __restrict__ newid,
+                                                               int64_t* __restrict__ cstart, int64_t* __restrict__ moff,
+                                                               int64_t* __restrict__ mrow, int64_t* __restrict__ tot)
+{
+    __shared__ uint32_t first[kSmallVerts];  // each community's first vertex, then the sort's keys
+    __shared__ uint32_t rank[kSmallVerts];
+    __shared__ uint32_t s_wave[kSmallBlock / 64];
+    const int t = threadIdx.x;
+    for (int c = t; c < nv; c += kSmallBlock) first[c] = kNoKey;
+    __syncthreads();
+    int64_t bad = 0;
+    for (int i0 = 0; i0 < nv; i0 += kSmallBlock) {
+        const int i = i0 + t;
+        const int64_t c = i < nv ? cvect[i] : 0;
+        const bool out = c < 0 || c >= nv;
+        bad += __syncthreads_count(out);
+        if (i < nv && !out) atomicMin(&first[c], (uint32_t)i);
+    }
+    if (bad) {  // the same in every thread
+        if (t == 0) {
+            tot[0] = 0;
+            tot[1] = bad;
+        }
+        return;
+    }
+    __syncthreads();
+    uint32_t flags = 0, nc = 0;
+    for (int k = 0; k < kSmallPer; k++) {
+        const int i = t * kSmallPer + k;
+        if (i < nv && first[cvect[i]] == (uint32_t)i) flags |= 1u << k;
+    }
+    uint32_t r = block_scan<kSmallBlock, uint32_t>((uint32_t)__popc(flags), s_wave, &nc);
+    for (int k = 0; k < kSmallPer; k++)
+        if (flags >> k & 1) rank[t * kSmallPer + k] = r++;
+    __syncthreads();
+    uint32_t id[kSmallPer];
+#pragma unroll
+    for (int k = 0; k < kSmallPer; k++) {
+        const int i = k * kSmallBlock + t;
+        if (i < nv) newid[i] = id[k] = rank[first[cvect[i]]];
+    }
+    __syncthreads();
+    // members by community, ascending inside: a bitonic sort of (community, vertex), 13 bits each
+    static_assert(kSmallVerts == 1 << 13, "keys hold a vertex in 13 bits");
+    uint32_t* key = first;
+    int n2 = 64;
+    while (n2 < nv) n2 <<= 1;
+#pragma unroll
+    for (int k = 0; k < kSmallPer; k++) {
+        const int i = k * kSmallBlock + t;
+        if (i < n2) key[i] = i < nv ? id[k] << 13 | (uint32_t)i : kNoKey;
+    }
+    __syncthreads();
+    for (int k = 2; k <= n2; k <<= 1)
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            for (int p = t; p < n2 / 2; p += kSmallBlock) {
+                const int i = ((p & ~(j - 1)) << 1) | (p & (j - 1)), l = i + j;
+                const uint32_t a = key[i], b = key[l];
+                if ((a > b) == ((i & k) == 0)) {
+                    key[i] = b;
+                    key[l] = a;
+                }
+            }
+            // strides up to 64 stay inside the 128 keys that a wave's 64 pairs hold
+            if (j <= 64 && (j > 1 || k <= 64)) wave_lds_sync();
+            else __syncthreads();
+        }
+    __syncthreads();
+    uint32_t deg[kSmallPer], sum = 0, ne = 0;
+#pragma unroll
+    for (int k = 0; k < kSmallPer; k++) {
+        const int p = t * kSmallPer + k;
+        deg[k] = 0;
+        if (p < nv) {
+            const uint32_t x = key[p], c = x >> 13, m = x & (kSmallVerts - 1);
+            if (p == 0 || key[p - 1] >> 13 != c) cstart[c] = p;
+            const int64_t r0 = offs[m];
+            mrow[p] = r0;
+            deg[k] = (uint32_t)(offs[m + 1] - r0);
+        }
+        sum += deg[k];
+    }
+    uint32_t at = block_scan<kSmallBlock, uint32_t>(sum, s_wave, &ne);
+#pragma unroll
+    for (int k = 0; k < kSmallPer; k++) {
+        const int p = t * kSmallPer + k;
+        if (p < nv) moff[p] = at;
+        at += deg[k];
+    }
+    if (t == 0) {
+        cstart[nc] = nv;
+        moff[nv] = ne;
+        tot[0] = nc;
+        tot[1] = 0;
+    }
+}
+
+// The scans of the row lengths and of the overflowing communities' entries, and for the host
+// (out, pinned): communities, ids out of range, entries, overflowing entries, largest row, largest
+// overflowing community.
+__global__ void __launch_bounds__(kSmallBlock) k_rows_small(const int64_t* __restrict__ tot, const int64_t* __restrict__ rowlen,
+                                                            const int64_t* __restrict__ xcnt, int64_t* __restrict__ out_offs,
+                                                            int64_t* __restrict__ xoff, int64_t* __restrict__ out)
+{
+    __shared__ unsigned long long s_wave[kSmallBlock / 64];
+    const int t = threadIdx.x, nc = (int)tot[0];
+    unsigned long long len[kSmallPer], x[kSmallPer], la = 0, xa = 0, lmax = 0, xmax = 0, ltot = 0, xtot = 0;
+#pragma unroll
+    for (int k = 0; k < kSmallPer; k++) {
+        const int c = t * kSmallPer + k;
+        len[k] = c < nc ? (unsigned long long)rowlen[c] : 0;
+        x[k] = c < nc ? (unsigned long long)xcnt[c] : 0;
+        la += len[k];
+        xa += x[k];
+        lmax = len[k] > lmax ? len[k] : lmax;
+        xmax = x[k] > xmax ? x[k] : xmax;
+    }
+    unsigned long long lo = block_scan<kSmallBlock>(la, s_wave, &ltot), xo = block_scan<kSmallBlock>(xa, s_wave, &xtot);
+#pragma unroll
+    for (int k = 0; k < kSmallPer; k++) {
+        const int c = t * kSmallPer + k;
+        if (c < nc) {
+            out_offs[c] = (int64_t)lo;
+            xoff[c] = (int64_t)xo;
+        }
+        lo += len[k];
+        xo += x[k];
+    }
+    __shared__ unsigned long long s_max[2];
+    if (t < 2) s_max[t] = 0;
+    __syncthreads();
+    if (lmax) atomicMax(&s_max[0], lmax);
+    if (xmax) atomicMax(&s_max[1], xmax);
+    __syncthreads();
+    if (t == 0) {
+        out_offs[nc] = (int64_t)ltot;
+        xoff[nc] = (int64_t)xtot;
+        out[0] = nc;
+        out[1] = tot[1];
+        out[2] = (int64_t)ltot;
+        out[3] = (int64_t)xtot;
+        out[4] = (int64_t)s_max[0];
+        out[5] = (int64_t)s_max[1];
+    }
+}
+
 // Overflowing communities: their entries sorted stably by (C1, C2), runs folded left to
 // right, and each community's runs placed in its staged row.
 static void overflow_rows(vt_ctx* ctx, const vt_graph* g, const uint32_t* newid, int64_t nc, int bits,
@@ -598,67 +758,117 @@ static void overflow_rows(vt_ctx* ctx, const vt_graph* g, const uint32_t* newid,
               (const uint32_t*)rc2.p, (const double*)rw.p, nu, cstart, moff, (const int64_t*)run_first.p, rkey, rval);
 }
 
-static vt_graph* rebuild_fold(vt_ctx* ctx, const vt_graph* g, const uint32_t* newid, int64_t nc)
+// The members of each community in ascending vertex order (a stable sort by new id), and each
+// member's start in its community's concatenated row and row start in the CSR.
+static void member_lists(vt_ctx* ctx, const vt_graph* g, const uint32_t* newid, int64_t nc, int bits, int64_t* cstart,
+                         int64_t* moff, int64_t* mrow)
+{
+    const int64_t nv = g->nv;
+    const size_t n1 = (size_t)std::max<int64_t>(nv, 1);
+    DBuf<uint32_t> mk(ctx, n1), mv(ctx, n1), mk2(ctx, n1), mv2(ctx, n1);
+    d2d(ctx, mk.p, newid, 4 * (size_t)nv);
+    VT_LAUNCH(ctx, "rb_iota", k_iota_u32, grid_for(nv, 256, 8192), 256, 0, mv.p, nv);
+    bool malt = false;
+    sort_pairs_u32(ctx, mk.p, mv.p, nv, bits, mk2.p, mv2.p, &malt);
+    VT_LAUNCH(ctx, "rb_member_starts", k_member_starts, grid_for(nv, 256, 8192), 256, 0,
+              (const uint32_t*)(malt ? mk2.p : mk.p), nv, nc, cstart);
+    DBuf<int64_t> mdeg(ctx, n1 + 1);
+    VT_LAUNCH(ctx, "rb_mdeg", k_member_degrees, grid_for(nv + 1, 256, 8192), 256, 0,
+              (const uint32_t*)(malt ? mv2.p : mv.p), nv, (const int64_t*)g->offs, mdeg.p, mrow);
+    exclusive_scan_i64(ctx, mdeg.p, moff, nv + 1);
+}
+
+// New ids by first appearance; returns the number of communities, also at tot[0].
+static int64_t renumber(vt_ctx* ctx, const int64_t* d_cvect, int64_t nv, bool check_ids, uint32_t* newid, int64_t* tot)
+{
+    const size_t n1 = (size_t)std::max<int64_t>(nv, 1);
+    DBuf<unsigned long long> first(ctx, n1), bad(ctx, 2);
+    DBuf<int64_t> flag(ctx, n1), rank(ctx, n1);
+    dzero(ctx, bad.p, 16);
+    VT_LAUNCH(ctx, "rb_fill", k_fill_u64, grid_for(nv, 256, 8192), 256, 0, first.p, nv, ~0ull);
+    VT_LAUNCH(ctx, "rb_first", k_first_vertex, grid_for(nv, 256, 8192), 256, 0, d_cvect, nv, first.p, bad.p);
+    if (check_ids) {  // a caller's partition; a phase's own has every id in [0, nv)
+        unsigned long long nbad = 0;
+        d2h(ctx, &nbad, bad.p, 8);
+        if (nbad) fail(ctx, VT_ERR_ARG, "vt_rebuild: %llu community ids outside [0, nv)", nbad);
+    }
+    VT_LAUNCH(ctx, "rb_flags", k_first_flags, grid_for(nv, 256, 8192), 256, 0, d_cvect, nv,
+              (const unsigned long long*)first.p, flag.p);
+    exclusive_scan_i64(ctx, flag.p, rank.p, nv);
+    VT_LAUNCH(ctx, "rb_total", k_total, 1, 64, 0, (const int64_t*)flag.p, (const int64_t*)rank.p, nv, tot);
+    int64_t nc = 0;
+    d2h(ctx, &nc, tot, 8);
+    VT_LAUNCH(ctx, "rb_newid", k_vertex_newid, grid_for(nv, 256, 8192), 256, 0, d_cvect, nv,
+              (const unsigned long long*)first.p, (const int64_t*)rank.p, newid);
+    return nc;
+}
+
+vt_graph* rebuild(vt_ctx* ctx, const vt_graph* g, const int64_t* d_cvect, bool check_ids)
 {
     const int64_t nv = g->nv, ne = g->ne;
+    if (ne >= (int64_t(1) << 32)) fail(ctx, VT_ERR_LIMIT, "vt_rebuild: %lld edges; this build supports < 2^32", (long long)ne);
+    const size_t n1 = (size_t)std::max<int64_t>(nv, 1), e1 = (size_t)std::max<int64_t>(ne, 1);
+    const bool small = nv > 0 && nv <= kSmallVerts;
+    DBuf<uint32_t> newid(ctx, n1);
+    DBuf<int64_t> tot(ctx, 4);
+    int64_t nc = nv;  // small: known with the row lengths
+    if (!small) nc = renumber(ctx, d_cvect, nv, check_ids, newid.p, tot.p);
     const int bits = (int)bits_for(nc > 1 ? nc - 1 : 1);
-    const size_t c1n = (size_t)nc + 1, n1 = (size_t)std::max<int64_t>(nv, 1), e1 = (size_t)std::max<int64_t>(ne, 1);
-
-    // members of each community in ascending vertex order (stable sort by new id), and each
-    // member's start in its community's concatenated row
+    const size_t c1n = (size_t)nc + 1;
     DBuf<int64_t> cstart(ctx, c1n), moff(ctx, n1 + 1), mrow(ctx, n1);
-    {
-        DBuf<uint32_t> mk(ctx, n1), mv(ctx, n1), mk2(ctx, n1), mv2(ctx, n1);
-        d2d(ctx, mk.p, newid, 4 * (size_t)nv);
-        VT_LAUNCH(ctx, "rb_iota", k_iota_u32, grid_for(nv, 256, 8192), 256, 0, mv.p, nv);
-        bool malt = false;
-        sort_pairs_u32(ctx, mk.p, mv.p, nv, bits, mk2.p, mv2.p, &malt);
-        VT_LAUNCH(ctx, "rb_member_starts", k_member_starts, grid_for(nv, 256, 8192), 256, 0,
-                  (const uint32_t*)(malt ? mk2.p : mk.p), nv, nc, cstart.p);
-        DBuf<int64_t> mdeg(ctx, n1 + 1);
-        VT_LAUNCH(ctx, "rb_mdeg", k_member_degrees, grid_for(nv + 1, 256, 8192), 256, 0,
-                  (const uint32_t*)(malt ? mv2.p : mv.p), nv, (const int64_t*)g->offs, mdeg.p, mrow.p);
-        exclusive_scan_i64(ctx, mdeg.p, moff.p, nv + 1);
-    }
+    if (small)
+        VT_LAUNCH(ctx, "rb_members", k_members_small, 1, kSmallBlock, 0, d_cvect, (int)nv, (const int64_t*)g->offs, newid.p,
+                  cstart.p, moff.p, mrow.p, tot.p);
+    else member_lists(ctx, g, newid.p, nc, bits, cstart.p, moff.p, mrow.p);
 
     // every community's coarse row, staged at its offset in the concatenated rows
     DBuf<uint32_t> rkey(ctx, e1);
     DBuf<double> rval(ctx, e1);
-    DBuf<int64_t> rowlen(ctx, c1n), xcnt(ctx, c1n), out_offs(ctx, c1n), xoff(ctx, c1n), tot(ctx, 4);
-    dzero(ctx, rowlen.p + nc, 8);
-    dzero(ctx, xcnt.p + nc, 8);
+    DBuf<int64_t> rowlen(ctx, c1n), xcnt(ctx, c1n), out_offs(ctx, c1n), xoff(ctx, c1n);
     if (nc)
-        VT_LAUNCH(ctx, "rb_comm_fold", k_comm_fold, grid_for(nc, kFoldWaves, 262144), 64 * kFoldWaves, 0, nc,
-                  (const int64_t*)cstart.p, (const int64_t*)moff.p, (const int64_t*)mrow.p, (const DEdge*)g->edges, newid,
-                  rkey.p, rval.p, rowlen.p, xcnt.p);
-    exclusive_scan_i64(ctx, rowlen.p, out_offs.p, nc + 1);
-    exclusive_scan_i64(ctx, xcnt.p, xoff.p, nc + 1);
-    VT_LAUNCH(ctx, "rb_totals", k_pair_totals, 1, 64, 0, (const int64_t*)out_offs.p + nc, (const int64_t*)xoff.p + nc,
-              tot.p);
+        VT_LAUNCH(ctx, "rb_comm_fold", k_comm_fold, grid_for(nc, kFoldWaves, 262144), 64 * kFoldWaves, 0,
+                  (const int64_t*)tot.p, (const int64_t*)cstart.p, (const int64_t*)moff.p, (const int64_t*)mrow.p,
+                  (const DEdge*)g->edges, newid.p, rkey.p, rval.p, rowlen.p, xcnt.p);
     // the coarse graph's largest row is read with its entry count (the overflowing
     // communities' rows are added below, and the count and the largest row read again)
-    auto max_row = [&](const int64_t* offs, int64_t* out) {
-        if (nc)
-            VT_LAUNCH(ctx, "max_degree", k_max_degree, grid_for(nc, 256, 512), 256, 0, offs, nc, (unsigned long long*)out);
-    };
-    dzero(ctx, tot.p + 2, 16);
-    max_row(out_offs.p, tot.p + 2);
-    max_row(xoff.p, tot.p + 3);
     int64_t totals[4] = {0, 0, 0, 0};  // entries, overflowing entries, largest row, largest overflowing community
-    d2h(ctx, totals, tot.p, 32);
-    if (totals[1]) {
-        overflow_rows(ctx, g, newid, nc, bits, cstart.p, mrow.p, moff.p, xcnt.p, xoff.p, totals[1], totals[3], rkey.p,
-                      rval.p, rowlen.p);
+    auto read_totals = [&] {
+        if (small) {
+            const int64_t* out = (const int64_t*)(mail(ctx) + 8);
+            VT_LAUNCH(ctx, "rb_rows", k_rows_small, 1, kSmallBlock, 0, (const int64_t*)tot.p, (const int64_t*)rowlen.p,
+                      (const int64_t*)xcnt.p, out_offs.p, xoff.p, (int64_t*)(mail(ctx) + 8));
+            sync(ctx);
+            if (out[1])
+                fail(ctx, VT_ERR_ARG, "vt_rebuild: %llu community ids outside [0, nv)", (unsigned long long)out[1]);
+            nc = out[0];
+            std::memcpy(totals, out + 2, 32);
+            return;
+        }
+        dzero(ctx, rowlen.p + nc, 8);
+        dzero(ctx, xcnt.p + nc, 8);
         exclusive_scan_i64(ctx, rowlen.p, out_offs.p, nc + 1);
-        d2d(ctx, tot.p, out_offs.p + nc, 8);
-        dzero(ctx, tot.p + 2, 8);
-        max_row(out_offs.p, tot.p + 2);
-        d2h(ctx, totals, tot.p, 24);
+        exclusive_scan_i64(ctx, xcnt.p, xoff.p, nc + 1);
+        VT_LAUNCH(ctx, "rb_totals", k_pair_totals, 1, 64, 0, (const int64_t*)out_offs.p + nc, (const int64_t*)xoff.p + nc,
+                  tot.p);
+        dzero(ctx, tot.p + 2, 16);
+        if (nc) {
+            VT_LAUNCH(ctx, "max_degree", k_max_degree, grid_for(nc, 256, 512), 256, 0, (const int64_t*)out_offs.p, nc,
+                      (unsigned long long*)(tot.p + 2));
+            VT_LAUNCH(ctx, "max_degree", k_max_degree, grid_for(nc, 256, 512), 256, 0, (const int64_t*)xoff.p, nc,
+                      (unsigned long long*)(tot.p + 3));
+        }
+        d2h(ctx, totals, tot.p, 32);
+    };
+    read_totals();
+    if (totals[1]) {
+        overflow_rows(ctx, g, newid.p, nc, bits, cstart.p, mrow.p, moff.p, xcnt.p, xoff.p, totals[1], totals[3], rkey.p,
+                      rval.p, rowlen.p);
+        read_totals();
     }
 
     vt_graph* out = graph_new(ctx, nc, totals[0]);
     try {
-        d2d(ctx, out->offs, out_offs.p, 8 * c1n);
+        d2d(ctx, out->offs, out_offs.p, 8 * ((size_t)nc + 1));
         if (nc)
             VT_LAUNCH(ctx, "rb_row_copy", k_row_copy, grid_for(nc, kCfWaves, 65536), 64 * kCfWaves, 0, nc,
                       (const int64_t*)cstart.p, (const int64_t*)moff.p, (const int64_t*)rowlen.p,
@@ -681,36 +891,6 @@ static vt_graph* rebuild_fold(vt_ctx* ctx, const vt_graph* g, const uint32_t* ne
         throw;
     }
     return out;
-}
-
-vt_graph* rebuild(vt_ctx* ctx, const vt_graph* g, const int64_t* d_cvect, bool check_ids)
-{
-    const int64_t nv = g->nv, ne = g->ne;
-    if (ne >= (int64_t(1) << 32)) fail(ctx, VT_ERR_LIMIT, "vt_rebuild: %lld edges; this build supports < 2^32", (long long)ne);
-    const size_t n1 = (size_t)std::max<int64_t>(nv, 1);
-    DBuf<unsigned long long> first(ctx, n1), bad(ctx, 2);
-    DBuf<int64_t> flag(ctx, n1), rank(ctx, n1), tot(ctx, 2);
-    DBuf<uint32_t> newid(ctx, n1);
-    dzero(ctx, bad.p, 16);
-    VT_LAUNCH(ctx, "rb_fill", k_fill_u64, grid_for(nv, 256, 8192), 256, 0, first.p, nv, ~0ull);
-    VT_LAUNCH(ctx, "rb_first", k_first_vertex, grid_for(nv, 256, 8192), 256, 0, d_cvect, nv, first.p, bad.p);
-    if (check_ids) {  // a caller's partition; a phase's own has every id in [0, nv)
-        unsigned long long nbad = 0;
-        d2h(ctx, &nbad, bad.p, 8);
-        if (nbad) fail(ctx, VT_ERR_ARG, "vt_rebuild: %llu community ids outside [0, nv)", nbad);
-    }
-    VT_LAUNCH(ctx, "rb_flags", k_first_flags, grid_for(nv, 256, 8192), 256, 0, d_cvect, nv,
-              (const unsigned long long*)first.p, flag.p);
-    exclusive_scan_i64(ctx, flag.p, rank.p, nv);
-    VT_LAUNCH(ctx, "rb_total", k_total, 1, 64, 0, (const int64_t*)flag.p, (const int64_t*)rank.p, nv, tot.p);
-    int64_t nc = 0;
-    d2h(ctx, &nc, tot.p, 8);
-    VT_LAUNCH(ctx, "rb_newid", k_vertex_newid, grid_for(nv, 256, 8192), 256, 0, d_cvect, nv,
-              (const unsigned long long*)first.p, (const int64_t*)rank.p, newid.p);
-    first.reset();
-    flag.reset();
-    rank.reset();
-    return rebuild_fold(ctx, g, newid.p, nc);
 }
 
 }  // namespace vt
