@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <cstdarg>
 #include <mutex>
+#include <chrono>
 #include <cstring>
 #include <vector>
 
@@ -204,12 +205,32 @@ void d2h(vt_ctx* ctx, void* dst, const void* src, size_t bytes)
     ctx->stage_off = 0;  // the stream has drained: every staged copy has run
 }
 // Pinned host memory that kernels write a few scalars to (256 bytes; [0, 1]: an iteration's Q and
-// movers, [2]: a phase's whole degrees, [8, 14): a rebuild's totals): they are there when the
-// stream has drained, with no copy queued behind the kernel.
+// movers, [2]: a phase's whole degrees, [3]: the last post's number, [8, 14): a rebuild's totals,
+// [16, 27): a phase's list sizes), with no copy queued behind the kernel.
 double* mail(vt_ctx* ctx)
 {
-    if (!ctx->mail) VT_HIP(ctx, hipHostMalloc((void**)&ctx->mail, 256, hipHostMallocDefault));
+    if (!ctx->mail) {
+        VT_HIP(ctx, hipHostMalloc((void**)&ctx->mail, 256, hipHostMallocDefault));
+        std::memset(ctx->mail, 0, 256);
+    }
     return ctx->mail;
+}
+// Waits for the kernel that posts ctx->mail_seq.  The number is looked for in the pinned memory
+// first: waiting for the stream costs a marker behind the kernel and its interrupt (RGG n = 1000
+// upload and run, some 40 waits: 1.29 ms with stream waits, 1.10 so; RGG n = 65536: 3.85 and 3.55).  A kernel that takes longer than 200 us is
+// waited for with the stream, where that no longer matters and errors are reported.
+void mail_wait(vt_ctx* ctx)
+{
+    const unsigned long long* p = (const unsigned long long*)ctx->mail + 3;
+    const auto t0 = std::chrono::steady_clock::now();
+    for (;;) {
+        for (int k = 0; k < 64; k++) {
+            if (__atomic_load_n(p, __ATOMIC_ACQUIRE) == ctx->mail_seq) return;
+            __builtin_ia32_pause();
+        }
+        if (std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(200)) break;
+    }
+    sync(ctx);
 }
 void d2d(vt_ctx* ctx, void* dst, const void* src, size_t bytes)
 {

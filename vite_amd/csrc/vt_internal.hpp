@@ -64,6 +64,7 @@ struct vt_ctx {
     unsigned char* stage = nullptr;
     size_t stage_off = 0;
     double* mail = nullptr;  // pinned: Q and the movers of an iteration (vt::mail)
+    unsigned long long mail_seq = 0;  // the last number given to a kernel that posts there
     // sweep launch shape (performance only: every setting gives the same results)
     vt_tuning tuning = {{7, 15, 31, 63, 127, 1023}, 16384};  // replaced by default_tuning() at creation
 };
@@ -160,6 +161,13 @@ void h2d(vt_ctx* ctx, void* dst, const void* src, size_t bytes);
 void d2h(vt_ctx* ctx, void* dst, const void* src, size_t bytes);
 void d2d(vt_ctx* ctx, void* dst, const void* src, size_t bytes);
 double* mail(vt_ctx* ctx);
+// A kernel that writes to mail() ends with mail_post(out, seq), seq = ++ctx->mail_seq, and the host
+// waits for that number with mail_wait.
+void mail_wait(vt_ctx* ctx);
+__device__ __forceinline__ void mail_post(double* out, unsigned long long seq)
+{
+    __hip_atomic_store((unsigned long long*)out + 3, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 void dzero(vt_ctx* ctx, void* dst, size_t bytes);
 
 inline unsigned grid_for(int64_t n, int block, int64_t cap = 1 << 20)

@@ -879,7 +879,11 @@ struct SweepPlan {
     int64_t n[kFusedBuckets];         // list lengths
 };
 
-enum FusedPart { kPartRest = 1, kPartG16 = 2 };
+// One launch of all four buckets up to kOneLaunchBlocks blocks, where the launch costs about what it
+// does (RGG n = 65536, 4200 blocks: run 3.24 -> 3.14 ms; n = 2^20 is even); above, two, so that
+// each is timed by itself and the narrow groups' blocks do not wait behind bucket 2's.
+enum FusedPart { kPartRest = 1, kPartG16 = 2, kPartAll = 3 };
+constexpr int64_t kOneLaunchBlocks = 16384;
 
 template <bool BATCH, int PART, bool REC>
 __global__ void __launch_bounds__(kFusedBlock) __attribute__((amdgpu_waves_per_eu(8)))
@@ -902,6 +906,10 @@ k_local_move(MoveArgs a, const int32_t* __restrict__ lists, SweepPlan plan)
         switch (b) {
             case 0: run_bucket<4, 16, 256, true, BATCH, kNch[0], REC>(a, lds, list, plan.n[0], blk, nblk, &s_inactive); break;
             case 1: run_bucket<8, VT_CAP_G8, 256, true, BATCH, kNch[1], REC>(a, lds, list, plan.n[1], blk, nblk, &s_inactive); break;
+            case 2:
+                if constexpr (PART == kPartAll)
+                    run_bucket<16, 64, 256, true, BATCH, kNch[2], REC>(a, lds, list, plan.n[2], blk, nblk, &s_inactive);
+                break;
             default: run_bucket<32, 128, 256, true, BATCH, kNch[3], REC>(a, lds, list, plan.n[3], blk, nblk, &s_inactive); break;
         }
     }
@@ -2252,6 +2260,7 @@ struct TailArgs {
     int32_t blocks;
     double* sums;
     double* out;
+    unsigned long long seq;  // posted with out
 };
 
 __global__ void __launch_bounds__(kTailBlock) k_tail_small(TailArgs a)
@@ -2384,6 +2393,7 @@ __global__ void __launch_bounds__(kTailBlock) k_tail_small(TailArgs a)
         a.out[0] = fabs((r[0] * c) - (r[1] * c * c));
         ((unsigned long long*)a.out)[1] = *a.movers;
         *a.movers = 0;
+        mail_post(a.out, a.seq);
     }
 }
 
@@ -2405,6 +2415,7 @@ struct SetupArgs {
     int64_t* hoffs;               // nv + 1
     BucketBounds bb;
     int32_t lpv_max;
+    unsigned long long seq;       // posted with out
 };
 
 __global__ void __launch_bounds__(kTailBlock) k_setup_small(SetupArgs a)
@@ -2491,22 +2502,23 @@ __global__ void __launch_bounds__(kTailBlock) k_setup_small(SetupArgs a)
     double r[2];
     small_tree_sum2(a.vdeg, nullptr, a.nv, a.blocks, a.chunk, lds, s_part, r);
     int64_t* out = (int64_t*)a.out;
-    if (t < kNumBuckets) out[16 + t] = s_total[t];
     if (t == 0) {
+        for (int q = 0; q < kNumBuckets; q++) out[16 + q] = s_total[q];
         a.hoffs[nh] = (int64_t)entries;
         out[26] = (int64_t)entries;
         a.sums[0] = r[0];
         a.sums[1] = r[1];
         a.constant[0] = 1.0 / r[0];
         a.out[2] = !any_fraction && r[0] < 0x1p52 ? 1.0 : 0.0;
+        mail_post(a.out, a.seq);
     }
 }
 
 // currMod = |e_xx*c - a2_x*c*c| (louvain.cpp:2518-2524).
-// movers (or null): the iteration's mover count, copied to q[1] so that one read returns it
-// with the value, and cleared for the next iteration.
+// movers (or null): the iteration's mover count, copied to q[1] (q: the context's mail, where seq
+// is posted) so that one read returns it with the value, and cleared for the next iteration.
 __global__ void k_modularity(const double* __restrict__ sums, const double* __restrict__ constant,
-                             double* __restrict__ q, int64_t* __restrict__ movers)
+                             double* __restrict__ q, int64_t* __restrict__ movers, unsigned long long seq)
 {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
         const double c = constant[0];
@@ -2514,6 +2526,7 @@ __global__ void k_modularity(const double* __restrict__ sums, const double* __re
         if (movers) {
             ((int64_t*)q)[1] = movers[0];
             movers[0] = 0;
+            mail_post(q, seq);
         }
     }
 }
@@ -2525,7 +2538,7 @@ __global__ void __launch_bounds__(256) k_modularity_tree(const double* __restric
                                                          int64_t n, int64_t chunk, double2* __restrict__ part,
                                                          uint32_t* __restrict__ done, const double* __restrict__ constant,
                                                          double* __restrict__ sums, unsigned long long* __restrict__ movers,
-                                                         double* __restrict__ out)
+                                                         double* __restrict__ out, unsigned long long seq)
 {
     __shared__ double sa[256], sb[256];
     __shared__ bool s_last;
@@ -2575,6 +2588,7 @@ __global__ void __launch_bounds__(256) k_modularity_tree(const double* __restric
         ((unsigned long long*)out)[1] = *movers;
         *movers = 0;
         *done = 0;
+        mail_post(out, seq);
     }
 }
 
@@ -2977,8 +2991,9 @@ struct Phase {
         a.hoffs = hub_offs[0].p;
         a.bb = bounds();
         a.lpv_max = lpv_max_degree();
+        a.seq = ++ctx->mail_seq;
         VT_LAUNCH(ctx, "setup", k_setup_small, 1, kTailBlock, 0, a);
-        sync(ctx);
+        mail_wait(ctx);
         const int64_t* h = (const int64_t*)mail(ctx);
         plan_sweeps(1, h + 16);
         hub_total.assign(1, h[26]);
@@ -3233,13 +3248,17 @@ struct Phase {
         const bool batch = a.gid != nullptr;
         if (cs.fused_blocks) {
             const int64_t n16 = cs.plan.bbeg[3] - cs.plan.bbeg[2];
-            if (cs.fused_blocks > n16) {
+            const bool one = !batch && !a.rec && cs.fused_blocks <= kOneLaunchBlocks && n16 && cs.fused_blocks > n16;
+            if (one)
+                VT_LAUNCH(ctx, "local_move", (k_local_move<false, kPartAll, false>), (unsigned)cs.fused_blocks, kFusedBlock,
+                          0, a, (const int32_t*)lists.p, cs.plan);
+            if (!one && cs.fused_blocks > n16) {
                 auto kern = a.rec ? (batch ? k_local_move<true, kPartRest, true> : k_local_move<false, kPartRest, true>)
                                   : (batch ? k_local_move<true, kPartRest, false> : k_local_move<false, kPartRest, false>);
                 VT_LAUNCH(ctx, "local_move_rest", kern, (unsigned)(cs.fused_blocks - n16), kFusedBlock, 0, a,
                           (const int32_t*)lists.p, cs.plan);
             }
-            if (n16) {
+            if (!one && n16) {
                 auto kern = a.rec ? (batch ? k_local_move<true, kPartG16, true> : k_local_move<false, kPartG16, true>)
                                   : (batch ? k_local_move<true, kPartG16, false> : k_local_move<false, kPartG16, false>);
                 VT_LAUNCH(ctx, "local_move", kern, (unsigned)n16, kFusedBlock, 0, a, (const int32_t*)lists.p, cs.plan);
@@ -3355,6 +3374,7 @@ struct Phase {
         a.blocks = (int32_t)blocks;
         a.sums = sums();
         a.out = mail(ctx);
+        a.seq = 0;
         return a;
     }
 
@@ -3391,23 +3411,25 @@ struct Phase {
         double* out = mail(ctx);
         if (nv <= kTailVerts && nv && !seq) {
             const MoverArgs m{order, n, target.p, curr.p, et ? active.p : nullptr};
-            VT_LAUNCH(ctx, "tail", k_tail_small, 1, kTailBlock, 0, tail_args(m, cdeg.p, csize.p));
+            TailArgs a = tail_args(m, cdeg.p, csize.p);
+            a.seq = ++ctx->mail_seq;
+            VT_LAUNCH(ctx, "tail", k_tail_small, 1, kTailBlock, 0, a);
         } else {
             apply_moves(order, n, cdeg.p, csize.p);
             if (seq) {
                 seq_sum2(ctx, cw.p, cdeg.p, nv, sums());
                 VT_LAUNCH(ctx, "modularity", k_modularity, 1, 64, 0, (const double*)sums(), (const double*)constant(), out,
-                          iscal.p + 1);
+                          iscal.p + 1, ++ctx->mail_seq);
             } else {
                 int64_t grid = 0, chunk = 0;
                 sum2_plan(nv, &grid, &chunk);
                 double2* part = (double2*)scratch(ctx, "sum2_part", sizeof(double2) * 1024);
                 VT_LAUNCH(ctx, "modularity", k_modularity_tree, (unsigned)grid, 256, 0, (const double*)cw.p,
                           (const double*)cdeg.p, nv, chunk, part, (uint32_t*)(ucount.p + 4), (const double*)constant(),
-                          sums(), (unsigned long long*)(iscal.p + 1), out);
+                          sums(), (unsigned long long*)(iscal.p + 1), out, ++ctx->mail_seq);
             }
         }
-        sync(ctx);
+        mail_wait(ctx);
         std::memcpy(&movers_read, &out[1], 8);
         return out[0];
     }
@@ -3545,7 +3567,6 @@ double phase_end(vt_ctx* ctx, vt_phase* st, int64_t* cvect_out, int32_t* iters_o
     if (!g->part) g->part = (int64_t*)dalloc(ctx, 8 * (size_t)std::max<int64_t>(nv, 1));
     VT_LAUNCH(ctx, "widen_part", k_widen_ids, grid_for(nv, 256, 8192), 256, 0, (const int32_t*)ph.past.p, nv, g->part);
     if (cvect_out) d2h(ctx, cvect_out, g->part, 8 * (size_t)nv);
-    sync(ctx);
     if (iters_out) *iters_out = st->numIters;
     return st->prevMod;
 }
@@ -3797,6 +3818,7 @@ int vt_louvain_phase(vt_ctx* ctx, vt_graph* g, const vt_phase_params* p, int64_t
         VT_HIP(ctx, hipSetDevice(ctx->device));
         int32_t it = 0;
         const double q = run_phase(ctx, g, p, cvect_out, &it);
+        sync(ctx);
         if (iters_out) *iters_out = it;
         if (q_out) *q_out = q;
     });
@@ -4060,6 +4082,7 @@ int vt_phase_end(vt_ctx* ctx, vt_phase* st, int64_t* cvect_out, int32_t* iters_o
     const int rc = guarded(ctx, [&] {
         VT_HIP(ctx, hipSetDevice(ctx->device));
         const double q = phase_end(ctx, st, cvect_out, iters_out);
+        sync(ctx);
         if (q_out) *q_out = q;
     });
     delete st;
@@ -4150,7 +4173,7 @@ int vt_modularity(vt_ctx* ctx, int64_t nv, const double* cw, const double* cdeg,
         if (flags & VT_FLAG_SEQUENTIAL_SUMS) seq_sum2(ctx, a.p, b.p, nv, s.p);
         else tree_sum2(ctx, a.p, b.p, nv, s.p);
         VT_LAUNCH(ctx, "modularity", k_modularity, 1, 64, 0, (const double*)s.p, (const double*)(s.p + 2), s.p + 3,
-                  (int64_t*)nullptr);
+                  (int64_t*)nullptr, 0ull);
         double q = 0;
         d2h(ctx, &q, s.p + 3, 8);
         if (q_out) *q_out = q;

@@ -635,11 +635,12 @@ __global__ void __launch_bounds__(kSmallBlock) k_members_small(const int64_t* __
 }
 
 // The scans of the row lengths and of the overflowing communities' entries, and for the host
-// (out, pinned): communities, ids out of range, entries, overflowing entries, largest row, largest
+// (mail + 8, pinned): communities, ids out of range, entries, overflowing entries, largest row, largest
 // overflowing community.
 __global__ void __launch_bounds__(kSmallBlock) k_rows_small(const int64_t* __restrict__ tot, const int64_t* __restrict__ rowlen,
                                                             const int64_t* __restrict__ xcnt, int64_t* __restrict__ out_offs,
-                                                            int64_t* __restrict__ xoff, int64_t* __restrict__ out)
+                                                            int64_t* __restrict__ xoff, double* __restrict__ mail,
+                                                            unsigned long long seq)
 {
     __shared__ unsigned long long s_wave[kSmallBlock / 64];
     const int t = threadIdx.x, nc = (int)tot[0];
@@ -674,12 +675,14 @@ __global__ void __launch_bounds__(kSmallBlock) k_rows_small(const int64_t* __res
     if (t == 0) {
         out_offs[nc] = (int64_t)ltot;
         xoff[nc] = (int64_t)xtot;
+        int64_t* out = (int64_t*)(mail + 8);
         out[0] = nc;
         out[1] = tot[1];
         out[2] = (int64_t)ltot;
         out[3] = (int64_t)xtot;
         out[4] = (int64_t)s_max[0];
         out[5] = (int64_t)s_max[1];
+        mail_post(mail, seq);
     }
 }
 
@@ -836,8 +839,8 @@ vt_graph* rebuild(vt_ctx* ctx, const vt_graph* g, const int64_t* d_cvect, bool c
         if (small) {
             const int64_t* out = (const int64_t*)(mail(ctx) + 8);
             VT_LAUNCH(ctx, "rb_rows", k_rows_small, 1, kSmallBlock, 0, (const int64_t*)tot.p, (const int64_t*)rowlen.p,
-                      (const int64_t*)xcnt.p, out_offs.p, xoff.p, (int64_t*)(mail(ctx) + 8));
-            sync(ctx);
+                      (const int64_t*)xcnt.p, out_offs.p, xoff.p, mail(ctx), ++ctx->mail_seq);
+            mail_wait(ctx);
             if (out[1])
                 fail(ctx, VT_ERR_ARG, "vt_rebuild: %llu community ids outside [0, nv)", (unsigned long long)out[1]);
             nc = out[0];
