@@ -127,25 +127,19 @@ vt_graph* assemble(vt_ctx* ctx, const std::vector<Piece>& pcs, DBuf<int32_t>& gi
     }
     const int64_t nv = voff[ng], ne = eoff[ng];
     if (nv >= (int64_t(1) << 31) - 1) fail(ctx, VT_ERR_LIMIT, "batch: %lld vertices in all exceed 2^31 - 2", (long long)nv);
-    DBuf<int64_t> dvoff(ctx, ng + 1), deoff(ctx, ng + 1), dsv0(ctx, ng), dse0(ctx, ng);
-    DBuf<const int64_t*> dso(ctx, ng);
-    DBuf<const DEdge*> dse(ctx, ng);
-    h2d(ctx, dvoff.p, voff.data(), 8 * voff.size());
-    h2d(ctx, deoff.p, eoff.data(), 8 * eoff.size());
-    h2d(ctx, dsv0.p, sv0.data(), 8 * (size_t)ng);
-    h2d(ctx, dse0.p, se0.data(), 8 * (size_t)ng);
-    h2d(ctx, dso.p, so.data(), sizeof(void*) * (size_t)ng);
-    h2d(ctx, dse.p, se.data(), sizeof(void*) * (size_t)ng);
+    Packed in;
+    const size_t ovoff = in.add(voff), oeoff = in.add(eoff), ov0 = in.add(sv0), oe0 = in.add(se0), oso = in.add(so), ose = in.add(se);
+    in.send(ctx);
     vt_graph* u = graph_new(ctx, nv, ne);
     try {
         gid = DBuf<int32_t>(ctx, (size_t)std::max<int64_t>(nv, 1));
         VT_LAUNCH(ctx, "assemble_offs", k_assemble_offs, grid_for(std::max<int64_t>(nv, 1), 256, 8192), 256, 0, ng,
-                  (const int64_t*)dvoff.p, (const int64_t*)deoff.p, (const int64_t* const*)dso.p,
-                  (const int64_t*)dsv0.p, (const int64_t*)dse0.p, nv, u->offs, gid.p);
+                  in.at<int64_t>(ovoff), in.at<int64_t>(oeoff), in.at<const int64_t*>(oso), in.at<int64_t>(ov0),
+                  in.at<int64_t>(oe0), nv, u->offs, gid.p);
         if (ne)
             VT_LAUNCH(ctx, "assemble_edges", k_assemble_edges, grid_for(ne, 256, 16384), 256, 0, ng,
-                      (const int64_t*)dvoff.p, (const int64_t*)deoff.p, (const DEdge* const*)dse.p,
-                      (const int64_t*)dsv0.p, (const int64_t*)dse0.p, ne, u->edges);
+                      in.at<int64_t>(ovoff), in.at<int64_t>(oeoff), in.at<const DEdge*>(ose), in.at<int64_t>(ov0),
+                      in.at<int64_t>(oe0), ne, u->edges);
         graph_finalize(ctx, u);
     } catch (...) {
         graph_delete(ctx, u);

@@ -205,7 +205,8 @@ void d2h(vt_ctx* ctx, void* dst, const void* src, size_t bytes)
     ctx->stage_off = 0;  // the stream has drained: every staged copy has run
 }
 // Pinned host memory that kernels write a few scalars to (256 bytes; [0, 1]: an iteration's Q and
-// movers, [2]: a phase's whole degrees, [3]: the last post's number, [8, 14): a rebuild's totals,
+// movers, [2]: a phase's whole degrees, [3]: the last post's number,
+// [4, 8): a batch round's status, [8, 14): a rebuild's totals,
 // [16, 27): a phase's list sizes), with no copy queued behind the kernel.
 double* mail(vt_ctx* ctx)
 {
@@ -215,23 +216,29 @@ double* mail(vt_ctx* ctx)
     }
     return ctx->mail;
 }
-// Waits for the kernel that posts ctx->mail_seq.  The number is looked for in the pinned memory
+// Waits for the kernel that posts seq.  The number is looked for in the pinned memory
 // first: waiting for the stream costs a marker behind the kernel and its interrupt (RGG n = 1000
 // upload and run, some 40 waits: 1.29 ms with stream waits, 1.10 so; RGG n = 65536: 3.85 and 3.55).  A kernel that takes longer than 200 us is
 // waited for with the stream, where that no longer matters and errors are reported.
-void mail_wait(vt_ctx* ctx)
+void mail_wait(vt_ctx* ctx, unsigned long long seq)
 {
     const unsigned long long* p = (const unsigned long long*)ctx->mail + 3;
     const auto t0 = std::chrono::steady_clock::now();
     for (;;) {
         for (int k = 0; k < 64; k++) {
-            if (__atomic_load_n(p, __ATOMIC_ACQUIRE) == ctx->mail_seq) return;
+            if (__atomic_load_n(p, __ATOMIC_ACQUIRE) >= seq) return;
             __builtin_ia32_pause();
         }
         if (std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(200)) break;
     }
     sync(ctx);
 }
+void Packed::send(vt_ctx* ctx)
+{
+    dev = DBuf<unsigned char>(ctx, host.size());
+    h2d(ctx, dev.p, host.data(), host.size());
+}
+
 void d2d(vt_ctx* ctx, void* dst, const void* src, size_t bytes)
 {
     if (bytes) VT_HIP(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, ctx->stream));
@@ -459,18 +466,19 @@ void seg_sums_plan(vt_ctx* ctx, const std::vector<int64_t>& voff, SegSums& s)
         pbase[g + 1] = pbase[g] + grid;
     }
     s.ng = ng;
+    s.max_n = 0;
+    for (int32_t g = 0; g < ng; g++) s.max_n = std::max(s.max_n, voff[g + 1] - voff[g]);
     s.nblocks = (int64_t)bgraph.size();
-    s.voff = DBuf<int64_t>(ctx, voff.size());
-    s.bgraph = DBuf<int32_t>(ctx, bgraph.size());
-    s.bsub = DBuf<int32_t>(ctx, bsub.size());
-    s.chunk = DBuf<int64_t>(ctx, chunk.size());
-    s.pbase = DBuf<int64_t>(ctx, pbase.size());
     s.part = DBuf<double2>(ctx, bgraph.size());
-    h2d(ctx, s.voff.p, voff.data(), 8 * voff.size());
-    h2d(ctx, s.bgraph.p, bgraph.data(), 4 * bgraph.size());
-    h2d(ctx, s.bsub.p, bsub.data(), 4 * bsub.size());
-    h2d(ctx, s.chunk.p, chunk.data(), 8 * chunk.size());
-    h2d(ctx, s.pbase.p, pbase.data(), 8 * pbase.size());
+    s.data = Packed();
+    const size_t o0 = s.data.add(voff), o1 = s.data.add(chunk), o2 = s.data.add(pbase), o3 = s.data.add(bgraph),
+                 o4 = s.data.add(bsub);
+    s.data.send(ctx);
+    s.voff = s.data.at<int64_t>(o0);
+    s.chunk = s.data.at<int64_t>(o1);
+    s.pbase = s.data.at<int64_t>(o2);
+    s.bgraph = s.data.at<int32_t>(o3);
+    s.bsub = s.data.at<int32_t>(o4);
 }
 
 void seg_tree_sum2(vt_ctx* ctx, const SegSums& s, const double* a, const double* b, double* d_out,
@@ -478,17 +486,16 @@ void seg_tree_sum2(vt_ctx* ctx, const SegSums& s, const double* a, const double*
 {
     if (s.ng == 0) return;
     VT_LAUNCH(ctx, "seg_sum2_partial", k_seg_sum2_partial, (unsigned)s.nblocks, kSumBlock, 0, a, b,
-              (const int64_t*)s.voff.p, (const int32_t*)s.bgraph.p, (const int32_t*)s.bsub.p,
-              (const int64_t*)s.chunk.p, gact, s.part.p);
+              s.voff, s.bgraph, s.bsub, s.chunk, gact, s.part.p);
     VT_LAUNCH(ctx, "seg_sum2_final", k_seg_sum2_final, (unsigned)s.ng, kSumBlock, 0, (const double2*)s.part.p,
-              (const int64_t*)s.pbase.p, gact, d_out);
+              s.pbase, gact, d_out);
 }
 
 void seg_seq_sum2(vt_ctx* ctx, const SegSums& s, const double* a, const double* b, double* d_out,
                   const unsigned char* gact)
 {
     if (s.ng == 0) return;
-    VT_LAUNCH(ctx, "seg_seq_sum2", k_seg_seq_sum2, grid_for(s.ng, 64, 4096), 64, 0, a, b, (const int64_t*)s.voff.p,
+    VT_LAUNCH(ctx, "seg_seq_sum2", k_seg_seq_sum2, grid_for(s.ng, 64, 4096), 64, 0, a, b, s.voff,
               s.ng, gact, d_out);
 }
 

@@ -6,6 +6,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <map>
+#include <cstring>
 #include <string>
 #include <vector>
 
@@ -138,6 +139,26 @@ struct DBuf {
     ~DBuf() { reset(); }
 };
 
+// Host arrays sent to the device in one copy (a copy of a few hundred bytes costs its 4 us on the
+// device and as much on the host whatever it holds).
+struct Packed {
+    std::vector<unsigned char> host;
+    DBuf<unsigned char> dev;
+    template <class T>
+    size_t add(const T* src, size_t n)
+    {
+        const size_t off = (host.size() + 15) & ~size_t(15);
+        host.resize(off + n * sizeof(T));
+        if (n) std::memcpy(host.data() + off, src, n * sizeof(T));
+        return off;
+    }
+    template <class T>
+    size_t add(const std::vector<T>& v) { return add(v.data(), v.size()); }
+    void send(vt_ctx* ctx);
+    template <class T>
+    T* at(size_t off) const { return (T*)(dev.p + off); }
+};
+
 // ---- launches with optional event timing ---------------------------------------------
 struct TimedScope {
     vt_ctx* ctx;
@@ -162,8 +183,8 @@ void d2h(vt_ctx* ctx, void* dst, const void* src, size_t bytes);
 void d2d(vt_ctx* ctx, void* dst, const void* src, size_t bytes);
 double* mail(vt_ctx* ctx);
 // A kernel that writes to mail() ends with mail_post(out, seq), seq = ++ctx->mail_seq, and the host
-// waits for that number with mail_wait.
-void mail_wait(vt_ctx* ctx);
+// waits for that number, or a later one, with mail_wait.
+void mail_wait(vt_ctx* ctx, unsigned long long seq);
 __device__ __forceinline__ void mail_post(double* out, unsigned long long seq)
 {
     __hip_atomic_store((unsigned long long*)out + 3, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -339,9 +360,10 @@ void seq_sum2(vt_ctx* ctx, const double* a, const double* b_sq, int64_t n, doubl
 // each bit-identical to tree_sum2 / seq_sum2 on that graph alone.  d_out gets 2 per graph.
 struct SegSums {
     int32_t ng = 0;
-    int64_t nblocks = 0;
-    DBuf<int64_t> voff, chunk, pbase;
-    DBuf<int32_t> bgraph, bsub;
+    int64_t nblocks = 0, max_n = 0;  // max_n: the largest graph's vertices
+    Packed data;  // holds the arrays below
+    const int64_t *voff = nullptr, *chunk = nullptr, *pbase = nullptr;
+    const int32_t *bgraph = nullptr, *bsub = nullptr;
     DBuf<double2> part;
 };
 void seg_sums_plan(vt_ctx* ctx, const std::vector<int64_t>& voff, SegSums& s);

@@ -1665,7 +1665,7 @@ __global__ void k_constant(const double* __restrict__ sums, const unsigned long 
 // A row's sweep list: its degree bucket, the wide bucket split by table size.
 __device__ __host__ __forceinline__ uint32_t list_bucket(int64_t d, int lpv_max, const BucketBounds& bb)
 {
-    const uint32_t b = (uint32_t)(d <= lpv_max ? kLpvBucket : degree_bucket(d, bb));
+    const uint32_t b = (uint32_t)(lpv_max > 0 && d <= lpv_max ? kLpvBucket : degree_bucket(d, bb));
     if (b == kHubBucket - 1) return d <= bb.wide[0] ? kWide512Bucket : d <= bb.wide[1] ? kWide1024Bucket : b;
     return b;
 }
@@ -2196,17 +2196,18 @@ __global__ void __launch_bounds__(256) k_ev_fold_long(MoverArgs m, const uint32_
 // forms the modularity, in the order and with the trees of the separate kernels.
 constexpr int kTailVerts = 8192;
 constexpr int kTailBlock = 1024;
-constexpr int kTailRun = 24;  // events a thread orders by insertion; longer runs take a wave each
+constexpr int kTailRun = 64;  // events of a run folded by a thread; longer runs take a wave each
 
 // tree_sum2's sums of a and of b squared (b may be null) over n <= kTailVerts values by one
-// workgroup: its blocks of 256 threads, four at a time, then its tree over the partials, in
-// thread 0's r.  lds: 2 * kTailBlock doubles.
+// workgroup of B: its blocks of 256 threads, B / 256 at a time, then its tree over the partials,
+// in thread 0's r.  lds: 2 * B doubles; part[q]: room for `blocks`.
+template <int B, int P>
 __device__ __forceinline__ void small_tree_sum2(const double* __restrict__ a, const double* __restrict__ b_sq, int n, int blocks,
-                                                int64_t chunk, double* lds, double (*part)[kTailVerts / (4 * 256)], double* r)
+                                                int64_t chunk, double* lds, double (*part)[P], double* r)
 {
     const int t = threadIdx.x, sub = t & 255;
-    double *sa = lds, *sb = lds + kTailBlock;
-    for (int b0 = 0; b0 < blocks; b0 += kTailBlock / 256) {
+    double *sa = lds, *sb = lds + B;
+    for (int b0 = 0; b0 < blocks; b0 += B / 256) {
         const int b = b0 + (t >> 8);
         const int64_t lo = (int64_t)b * chunk;
         const int64_t hi = b < blocks ? min(lo + chunk, (int64_t)n) : lo;
@@ -2261,27 +2262,41 @@ struct TailArgs {
     double* sums;
     double* out;
     unsigned long long seq;  // posted with out
+    int32_t id0 = 0;         // the first vertex (all arrays start there, and ids are counted from it)
 };
 
-__global__ void __launch_bounds__(kTailBlock) k_tail_small(TailArgs a)
+template <int V, int B>
+struct TailLds {
+    uint32_t cur[V];                 // events per community, then the end of its run so far
+    alignas(16) uint16_t ev[2 * V];  // runs of positions, top bit: departure; then the sums' space
+    uint16_t lt[V], lc[V];
+    uint16_t longs[2 * V / kTailRun + 1];
+    uint32_t wave[B / 64];
+    uint32_t nlong;
+    double part[2][V / (4 * 256)];
+};
+
+// The folds, and with a.cw the sums in thread 0's r, for a.nv <= V vertices by a workgroup of B;
+// returns the movers.
+template <int V, int B>
+__device__ __forceinline__ unsigned tail_body(const TailArgs& a, TailLds<V, B>& l, double* r)
 {
-    __shared__ uint32_t cur[kTailVerts];     // events per community, then the end of its run so far
-    __shared__ uint16_t ev[2 * kTailVerts];  // runs of positions, top bit: departure
-    __shared__ uint16_t lt[kTailVerts], lc[kTailVerts];
-    __shared__ uint16_t s_long[2 * kTailVerts / kTailRun];
-    __shared__ uint32_t s_wave[kTailBlock / 64];
-    __shared__ uint32_t s_nlong;
-    __shared__ double s_part[2][kTailVerts / (4 * 256)];
+    static_assert(2 * B * 8 <= 2 * V * 2 && B % 256 == 0, "the sums' space is ev's");
+    uint32_t* cur = l.cur;
+    uint16_t *ev = l.ev, *lt = l.lt, *lc = l.lc, *s_long = l.longs;
+    uint32_t *s_wave = l.wave, &s_nlong = l.nlong;
     constexpr uint16_t kNone = 0xffff;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int n = (int)a.m.n;
-    for (int c = t; c < a.nv; c += kTailBlock) cur[c] = 0;
+    for (int c = t; c < a.nv; c += B) cur[c] = 0;
     if (t == 0) s_nlong = 0;
     __syncthreads();
     unsigned mine = 0;
-    for (int p = t; p < n; p += kTailBlock) {
+    for (int p = t; p < n; p += B) {
         int32_t v, tg, c;
         const bool mv = mover_at(a.m, p, v, tg, c);
+        tg -= a.id0;
+        c -= a.id0;
         lt[p] = mv ? (uint16_t)tg : kNone;
         lc[p] = mv ? (uint16_t)c : kNone;
         if (mv) {
@@ -2294,11 +2309,11 @@ __global__ void __launch_bounds__(kTailBlock) k_tail_small(TailArgs a)
     if (lane == 0) s_wave[w] = mine;
     __syncthreads();
     unsigned moved = 0;
-    for (int k = 0; k < kTailBlock / 64; k++) moved += s_wave[k];
+    for (int k = 0; k < B / 64; k++) moved += s_wave[k];
     __syncthreads();
     if (moved) {  // uniform
-        // exclusive scan of the counts: thread t takes kTailVerts / kTailBlock consecutive ones
-        constexpr int kPer = kTailVerts / kTailBlock;
+        // exclusive scan of the counts: thread t takes V / B consecutive ones
+        constexpr int kPer = V / B;
         uint32_t x[kPer], sum = 0;
 #pragma unroll
         for (int k = 0; k < kPer; k++) {
@@ -2322,43 +2337,72 @@ __global__ void __launch_bounds__(kTailBlock) k_tail_small(TailArgs a)
             run += x[k];
         }
         __syncthreads();
-        for (int p = t; p < n; p += kTailBlock) {
+        for (int p = t; p < n; p += B) {
             if (lt[p] == kNone) continue;
             ev[atomicAdd(&cur[lt[p]], 1u)] = (uint16_t)p;
             ev[atomicAdd(&cur[lc[p]], 1u)] = (uint16_t)(p | 0x8000);
         }
         __syncthreads();
-        for (int c = t; c < a.nv; c += kTailBlock) {
+        // each event's place in its run: the run's events of smaller positions, counted by a thread
+        // per event (independent reads; sorting a run by insertion was a chain of them)
+        constexpr int kEv = 2 * V / B;
+        const uint32_t ne = 2 * moved;
+        uint16_t e[kEv], at[kEv];
+#pragma unroll
+        for (int k = 0; k < kEv; k++) {
+            const uint32_t q = (uint32_t)(k * B + t);
+            at[k] = kNone;
+            e[k] = 0;
+            if (q < ne) {
+                const uint32_t x = ev[q], p = x & 0x7fff;
+                const int c = (x & 0x8000) ? lc[p] : lt[p];
+                const uint32_t b = c ? cur[c - 1] : 0, end = cur[c];
+                if (end - b <= (uint32_t)kTailRun && end - b > 1) {
+                    uint32_t r = b;
+                    for (uint32_t j = b; j < end; j++) r += (ev[j] & 0x7fffu) < p ? 1 : 0;
+                    at[k] = (uint16_t)r;
+                    e[k] = (uint16_t)x;
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kEv; k++)
+            if (at[k] != kNone) ev[at[k]] = e[k];
+        __syncthreads();
+        for (int c = t; c < a.nv; c += B) {
             const uint32_t b = c ? cur[c - 1] : 0, s = cur[c] - b;
             if (s == 0) continue;
             if (s > (uint32_t)kTailRun) {
                 s_long[atomicAdd(&s_nlong, 1u)] = (uint16_t)c;
                 continue;
             }
-            for (uint32_t k = 1; k < s; k++) {  // by position
-                const uint16_t e = ev[b + k];
-                uint32_t j = k;
-                while (j > 0 && (ev[b + j - 1] & 0x7fff) > (e & 0x7fff)) {
-                    ev[b + j] = ev[b + j - 1];
-                    j--;
-                }
-                ev[b + j] = e;
-            }
+            const double deg0 = a.cdeg[c];
+            const int32_t size0 = a.csize[c];
             double acc = 0.0;
             int change = 0;
-            for (uint32_t k = 0; k < s; k++) {
-                const uint16_t e = ev[b + k];
-                const int p = e & 0x7fff;
-                const double kv = a.vdeg[a.m.order ? a.m.order[p] : p];
-                acc = acc + ((e & 0x8000) ? -kv : kv);
-                change += (e & 0x8000) ? -1 : 1;
+            for (uint32_t k0 = 0; k0 < s; k0 += 8) {  // eight degrees in flight
+                double d[8];
+#pragma unroll
+                for (uint32_t u = 0; u < 8; u++) {
+                    d[u] = -0.0;  // leaves any sum unchanged
+                    if (k0 + u < s) {
+                        const uint16_t x = ev[b + k0 + u];
+                        const int p = x & 0x7fff;
+                        const double kv = a.vdeg[a.m.order ? a.m.order[p] : p];
+                        d[u] = (x & 0x8000) ? -kv : kv;
+                        change += (x & 0x8000) ? -1 : 1;
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < 8; u++) acc = acc + d[u];
             }
-            a.cdeg[c] = a.cdeg[c] + acc;
-            a.csize[c] += change;
+            a.cdeg[c] = deg0 + acc;
+            a.csize[c] = size0 + change;
         }
         __syncthreads();
         // long runs: a wave meets the community's events in order by walking the positions
-        for (uint32_t i = w; i < s_nlong; i += kTailBlock / 64) {
+        for (uint32_t i = w; i < s_nlong; i += B / 64) {
             const int c = s_long[i];
             double acc = 0.0;
             int change = 0;
@@ -2380,20 +2424,107 @@ __global__ void __launch_bounds__(kTailBlock) k_tail_small(TailArgs a)
                 a.csize[c] += change;
             }
         }
-        if (t == 0) *a.movers += moved;
         __syncthreads();
     }
-    if (!a.cw) return;
+    if (a.cw) small_tree_sum2<B>(a.cw, a.cdeg, a.nv, a.blocks, a.chunk, (double*)ev, l.part, r);
+    return moved;
+}
+
+// One graph's.
+__global__ void __launch_bounds__(kTailBlock) k_tail_small(TailArgs a)
+{
+    __shared__ TailLds<kTailVerts, kTailBlock> l;
     double r[2];
-    small_tree_sum2(a.cw, a.cdeg, a.nv, a.blocks, a.chunk, (double*)ev, s_part, r);
-    if (t == 0) {
-        a.sums[0] = r[0];
-        a.sums[1] = r[1];
-        const double c = a.constant[0];
-        a.out[0] = fabs((r[0] * c) - (r[1] * c * c));
-        ((unsigned long long*)a.out)[1] = *a.movers;
-        *a.movers = 0;
-        mail_post(a.out, a.seq);
+    const unsigned moved = tail_body(a, l, r);
+    if (threadIdx.x != 0) return;
+    const unsigned long long all = *a.movers + moved;
+    if (!a.cw) {
+        *a.movers = all;
+        return;
+    }
+    a.sums[0] = r[0];
+    a.sums[1] = r[1];
+    const double c = a.constant[0];
+    a.out[0] = fabs((r[0] * c) - (r[1] * c * c));
+    ((unsigned long long*)a.out)[1] = all;
+    *a.movers = 0;
+    mail_post(a.out, a.seq);
+}
+
+// A round of a batch whose graphs all have at most V vertices, after its sweep: a workgroup per
+// graph folds its moves, forms its Q, decides (k_batch_decide) and moves its communities on
+// (k_batch_rotate).  The last workgroup to finish posts the graphs that go on and their vertices.
+// The separate kernels are 22 launches a round, most of them a sort's.
+struct BatchTailArgs {
+    const int32_t* target;
+    int32_t *curr, *past, *csize;
+    const double *vdeg, *cw, *constant, *thresh, *lower;
+    double *cdeg, *prev;
+    const int64_t *voff, *chunk, *pbase;
+    unsigned char* act;
+    int32_t* iters;
+    unsigned long long* status;  // [0] graphs, [1] vertices, [2] finished workgroups; zero between rounds
+    double* out;                 // pinned: [slot], [slot + 1], and the number
+    int32_t slot;
+    unsigned long long seq;
+};
+
+// Up to 2048 vertices by 256 threads and 25 KB of LDS, six workgroups per CU; up to 4096 in 50 KB,
+// two (300 graphs of up to 4096 vertices took 64 us a round with 512 threads, 55 in the 98 KB of the
+// largest form, 51 so, and 36 with the ranks below).
+constexpr int kBatchTailSmall = 2048, kBatchTailMid = 4096;
+
+template <int V, int B>
+__global__ void __launch_bounds__(B) k_batch_tail(BatchTailArgs b)
+{
+    __shared__ TailLds<V, B> l;
+    __shared__ bool s_go;
+    const int32_t g = blockIdx.x;
+    const int64_t base = b.voff[g];
+    const int n = (int)(b.voff[g + 1] - base);
+    if (threadIdx.x == 0) s_go = false;
+    if (b.act[g]) {  // the same in every thread
+        TailArgs a;
+        a.m = MoverArgs{nullptr, n, b.target + base, b.curr + base, nullptr};
+        a.id0 = (int32_t)base;
+        a.nv = n;
+        a.vdeg = b.vdeg + base;
+        a.cdeg = b.cdeg + base;
+        a.csize = b.csize + base;
+        a.cw = b.cw + base;
+        a.chunk = b.chunk[g];
+        a.blocks = (int32_t)(b.pbase[g + 1] - b.pbase[g]);
+        double r[2];
+        tail_body(a, l, r);
+        if (threadIdx.x == 0) {
+            b.iters[g] += 1;
+            const double c = b.constant[g];
+            const double q = fabs((r[0] * c) - (r[1] * c * c));
+            if ((q - b.prev[g]) < b.thresh[g]) {
+                b.act[g] = 0;
+            } else {
+                b.prev[g] = q < b.lower[g] ? b.lower[g] : q;
+                s_go = true;
+                atomicAdd(b.status, 1ull);
+                atomicAdd(b.status + 1, (unsigned long long)n);
+            }
+        }
+        __syncthreads();
+        if (s_go)
+            for (int i = threadIdx.x; i < n; i += B) {
+                b.past[base + i] = b.curr[base + i];
+                b.curr[base + i] = b.target[base + i];
+            }
+    }
+    if (threadIdx.x == 0) {
+        __threadfence();
+        if (atomicAdd(b.status + 2, 1ull) + 1 == gridDim.x) {
+            unsigned long long* out = (unsigned long long*)b.out;
+            out[b.slot] = atomicExch(b.status, 0ull);
+            out[b.slot + 1] = atomicExch(b.status + 1, 0ull);
+            b.status[2] = 0;
+            mail_post(b.out, b.seq);
+        }
     }
 }
 
@@ -2500,7 +2631,7 @@ __global__ void __launch_bounds__(kTailBlock) k_setup_small(SetupArgs a)
         entries += sum;
     }
     double r[2];
-    small_tree_sum2(a.vdeg, nullptr, a.nv, a.blocks, a.chunk, lds, s_part, r);
+    small_tree_sum2<kTailBlock>(a.vdeg, nullptr, a.nv, a.blocks, a.chunk, lds, s_part, r);
     int64_t* out = (int64_t*)a.out;
     if (t == 0) {
         for (int q = 0; q < kNumBuckets; q++) out[16 + q] = s_total[q];
@@ -2993,7 +3124,7 @@ struct Phase {
         a.lpv_max = lpv_max_degree();
         a.seq = ++ctx->mail_seq;
         VT_LAUNCH(ctx, "setup", k_setup_small, 1, kTailBlock, 0, a);
-        mail_wait(ctx);
+        mail_wait(ctx, ctx->mail_seq);
         const int64_t* h = (const int64_t*)mail(ctx);
         plan_sweeps(1, h + 16);
         hub_total.assign(1, h[26]);
@@ -3248,10 +3379,12 @@ struct Phase {
         const bool batch = a.gid != nullptr;
         if (cs.fused_blocks) {
             const int64_t n16 = cs.plan.bbeg[3] - cs.plan.bbeg[2];
-            const bool one = !batch && !a.rec && cs.fused_blocks <= kOneLaunchBlocks && n16 && cs.fused_blocks > n16;
-            if (one)
-                VT_LAUNCH(ctx, "local_move", (k_local_move<false, kPartAll, false>), (unsigned)cs.fused_blocks, kFusedBlock,
-                          0, a, (const int32_t*)lists.p, cs.plan);
+            const bool one = !a.rec && cs.fused_blocks <= kOneLaunchBlocks && n16 && cs.fused_blocks > n16;
+            if (one) {
+                auto kern = batch ? k_local_move<true, kPartAll, false> : k_local_move<false, kPartAll, false>;
+                VT_LAUNCH(ctx, "local_move", kern, (unsigned)cs.fused_blocks, kFusedBlock, 0, a, (const int32_t*)lists.p,
+                          cs.plan);
+            }
             if (!one && cs.fused_blocks > n16) {
                 auto kern = a.rec ? (batch ? k_local_move<true, kPartRest, true> : k_local_move<false, kPartRest, true>)
                                   : (batch ? k_local_move<true, kPartRest, false> : k_local_move<false, kPartRest, false>);
@@ -3429,7 +3562,7 @@ struct Phase {
                           sums(), (unsigned long long*)(iscal.p + 1), out, ++ctx->mail_seq);
             }
         }
-        mail_wait(ctx);
+        mail_wait(ctx, ctx->mail_seq);
         std::memcpy(&movers_read, &out[1], 8);
         return out[0];
     }
@@ -3604,16 +3737,26 @@ void batch_phase(vt_ctx* ctx, vt_graph* u, const int32_t* d_gid, const SegSums& 
     const int64_t nv = u->nv;
     Phase ph(ctx, u);
     ph.alloc(false);
-    DBuf<double> gconst(ctx, ng), gsums(ctx, 2 * (size_t)ng), gprev(ctx, ng), gthr(ctx, ng), glow(ctx, ng);
-    DBuf<unsigned char> gact(ctx, ng), grot(ctx, ng);
-    DBuf<int32_t> giters(ctx, ng);
+    DBuf<double> gconst(ctx, ng), gsums(ctx, 2 * (size_t)ng);
+    DBuf<unsigned char> grot(ctx, ng);
     // [0] graphs still iterating, [1] their vertices (set by each round's decisions);
     // [2] the live list's length (the movers' flag scan runs over it); [3] movers (that
     // scan's total); [4] nv
-    DBuf<unsigned long long> status(ctx, 5);
+    const unsigned long long st0[5] = {(unsigned long long)ng, (unsigned long long)nv, (unsigned long long)nv, 0,
+                                       (unsigned long long)nv};
+    Packed in;
+    // each graph's modularity so far and iterations, read back together at the end
+    const size_t oprev = in.add(lower), oiters = in.add(std::vector<int32_t>((size_t)ng, 0)), oend = in.host.size();
+    const size_t olow = in.add(lower), othr = in.add(thresh), oact = in.add(std::vector<unsigned char>((size_t)ng, 1)),
+                 ostatus = in.add(st0, 5);
+    in.send(ctx);
+    double *gprev = in.at<double>(oprev), *glow = in.at<double>(olow), *gthr = in.at<double>(othr);
+    int32_t* giters = in.at<int32_t>(oiters);
+    unsigned char* gact = in.at<unsigned char>(oact);
+    unsigned long long* status = in.at<unsigned long long>(ostatus);
     DBuf<int32_t> live(ctx, (size_t)std::max<int64_t>(nv, 1));
     ph.gid = d_gid;
-    ph.gact = gact.p;
+    ph.gact = gact;
     ph.gconst = gconst.p;
     ph.hub_sort = false;  // the sweep is replayed from a captured graph: no library sort inside
     const bool seq = (flags & VT_FLAG_SEQUENTIAL_SUMS) != 0;
@@ -3622,18 +3765,71 @@ void batch_phase(vt_ctx* ctx, vt_graph* u, const int32_t* d_gid, const SegSums& 
     if (seq) seg_seq_sum2(ctx, seg, ph.vdeg.p, nullptr, gsums.p);
     else seg_tree_sum2(ctx, seg, ph.vdeg.p, nullptr, gsums.p);
     VT_LAUNCH(ctx, "seg_constant", k_seg_constant, grid_for(ng, 256, 64), 256, 0, (const double*)gsums.p, ng, gconst.p);
-    h2d(ctx, gthr.p, thresh.data(), 8 * (size_t)ng);
-    h2d(ctx, glow.p, lower.data(), 8 * (size_t)ng);
-    d2d(ctx, gprev.p, glow.p, 8 * (size_t)ng);
-    dzero(ctx, giters.p, 4 * (size_t)ng);
-    {
-        std::vector<unsigned char> ones((size_t)ng, 1);
-        h2d(ctx, gact.p, ones.data(), (size_t)ng);
-        const unsigned long long st0[5] = {(unsigned long long)ng, (unsigned long long)nv, (unsigned long long)nv, 0,
-                                           (unsigned long long)nv};
-        h2d(ctx, status.p, st0, sizeof(st0));
-    }
     ph.build_lists(nullptr, 1, false);
+
+    auto finish = [&](int rounds, int relists) {
+        if (!u->part) u->part = (int64_t*)dalloc(ctx, 8 * (size_t)std::max<int64_t>(nv, 1));
+        VT_LAUNCH(ctx, "widen_part", k_widen_ids, grid_for(nv, 256, 8192), 256, 0, (const int32_t*)ph.past.p, nv, u->part);
+        q_out.assign((size_t)ng, 0.0);
+        iters_out.assign((size_t)ng, 0);
+        std::vector<unsigned char> back(oend - oprev);
+        d2h(ctx, back.data(), gprev, back.size());
+        std::memcpy(q_out.data(), back.data(), 8 * (size_t)ng);
+        std::memcpy(iters_out.data(), back.data() + (oiters - oprev), 4 * (size_t)ng);
+        if (rounds_out) *rounds_out = rounds;
+        if (relists_out) *relists_out = relists;
+    };
+    // Small graphs: two or three launches a round, sent by the host one round ahead of the status
+    // that it reads (a captured graph's replay would cost more than they do).
+    if (!seq && nv && seg.max_n <= kTailVerts) {
+        BatchTailArgs b;
+        b.target = ph.target.p;
+        b.curr = ph.curr.p;
+        b.past = ph.past.p;
+        b.csize = ph.csize.p;
+        b.vdeg = ph.vdeg.p;
+        b.cw = ph.cw.p;
+        b.constant = gconst.p;
+        b.thresh = gthr;
+        b.lower = glow;
+        b.cdeg = ph.cdeg.p;
+        b.prev = gprev;
+        b.voff = seg.voff;
+        b.chunk = seg.chunk;
+        b.pbase = seg.pbase;
+        b.act = gact;
+        b.iters = giters;
+        b.status = status;
+        b.out = mail(ctx);
+        dzero(ctx, status, 24);
+        int64_t listed = nv;
+        int relists = 0;
+        for (int r = 0;; r++) {
+            ph.sweep(ph.sweeps[0]);
+            b.slot = 4 + 2 * (r & 1);
+            b.seq = ++ctx->mail_seq;
+            if (seg.max_n <= kBatchTailSmall)
+                VT_LAUNCH(ctx, "batch_tail", (k_batch_tail<kBatchTailSmall, 256>), (unsigned)ng, 256, 0, b);
+            else if (seg.max_n <= kBatchTailMid)
+                VT_LAUNCH(ctx, "batch_tail", (k_batch_tail<kBatchTailMid, kTailBlock>), (unsigned)ng, kTailBlock, 0, b);
+            else VT_LAUNCH(ctx, "batch_tail", (k_batch_tail<kTailVerts, kTailBlock>), (unsigned)ng, kTailBlock, 0, b);
+            if (r == 0) continue;
+            mail_wait(ctx, b.seq - 1);
+            const unsigned long long* prev = (const unsigned long long*)b.out + 4 + 2 * ((r - 1) & 1);
+            const int64_t active = (int64_t)prev[0], live_nv = (int64_t)prev[1];
+            if (active == 0) {  // rounds 0 .. r - 1 had graphs iterating; round r changes nothing
+                finish(r, relists);
+                return;
+            }
+            // the sweep lists without the finished graphs' vertices: a dozen launches and a wait, so
+            // rarely (a listed vertex of a finished graph costs the sweep its header alone)
+            if (8 * live_nv < listed) {
+                listed = live_nv;
+                relists++;
+                ph.build_lists(nullptr, 1, false);
+            }
+        }
+    }
 
     const int64_t nev = 2 * std::max<int64_t>(nv, 1);
     uint32_t* k0 = (uint32_t*)scratch(ctx, "bev_k0", 4 * (size_t)nev);
@@ -3644,9 +3840,9 @@ void batch_phase(vt_ctx* ctx, vt_graph* u, const int32_t* d_gid, const SegSums& 
     int32_t* mpos = (int32_t*)scratch(ctx, "bmv_pos", 4 * (size_t)std::max<int64_t>(nv, 1));
     const uint32_t none = (uint32_t)nv;
     const int bits = (int)bits_for(std::max<int64_t>(nv, 1));
-    int64_t* d_nlive = (int64_t*)(status.p + 2);
-    int64_t* d_movers = (int64_t*)(status.p + 3);
-    const int64_t* d_nv = (const int64_t*)(status.p + 4);
+    int64_t* d_nlive = (int64_t*)(status + 2);
+    int64_t* d_movers = (int64_t*)(status + 3);
+    const int64_t* d_nv = (const int64_t*)(status + 4);
     // The live list from the graphs' flags as they stand once the queued work has run; its
     // length is read back (the rounds captured after it take it as their launch size).
     int64_t nlive = nv;
@@ -3656,7 +3852,7 @@ void batch_phase(vt_ctx* ctx, vt_graph* u, const int32_t* d_gid, const SegSums& 
             return;
         }
         VT_LAUNCH(ctx, "live_flags", k_live_flags, grid_for(nv, 256, 8192), 256, 0, nv, d_gid,
-                  (const unsigned char*)gact.p, mflags);
+                  (const unsigned char*)gact, mflags);
         dev_scan_i32(ctx, mflags, mpos, d_nv, nv, d_nlive, "blive_part");
         VT_LAUNCH(ctx, "live_scatter", k_live_scatter, grid_for(nv, 256, 8192), 256, 0, nv, (const int32_t*)mflags,
                   (const int32_t*)mpos, live.p);
@@ -3678,7 +3874,7 @@ void batch_phase(vt_ctx* ctx, vt_graph* u, const int32_t* d_gid, const SegSums& 
         if (nlive) {
             VT_LAUNCH(ctx, "batch_flags", k_batch_flags, grid_for(nlive, 256, 8192), 256, 0, nlive,
                       (const int32_t*)live.p, (const int32_t*)ph.target.p, (const int32_t*)ph.curr.p, d_gid,
-                      (const unsigned char*)gact.p, mflags);
+                      (const unsigned char*)gact, mflags);
             dev_scan_i32(ctx, mflags, mpos, d_nlive, nlive, d_movers, "bmv_part");
             VT_LAUNCH(ctx, "emit_events", k_emit_events, grid_for(nlive, 256, 8192), 256, 0, (const int32_t*)live.p,
                       nlive, (const int32_t*)mflags, (const int32_t*)mpos, (const int32_t*)ph.target.p,
@@ -3688,12 +3884,12 @@ void batch_phase(vt_ctx* ctx, vt_graph* u, const int32_t* d_gid, const SegSums& 
         }
         const bool alt = dev_sort_pairs_u32(ctx, k0, v0, k1, v1, d_movers, 2, nev, bits);
         ph.fold_events(alt ? k1 : k0, alt ? v1 : v0, 2 * nv, none, ph.cdeg.p, ph.csize.p, d_movers);
-        if (seq) seg_seq_sum2(ctx, seg, ph.cw.p, ph.cdeg.p, gsums.p, (const unsigned char*)gact.p);
-        else seg_tree_sum2(ctx, seg, ph.cw.p, ph.cdeg.p, gsums.p, (const unsigned char*)gact.p);
-        dzero(ctx, status.p, 16);
+        if (seq) seg_seq_sum2(ctx, seg, ph.cw.p, ph.cdeg.p, gsums.p, (const unsigned char*)gact);
+        else seg_tree_sum2(ctx, seg, ph.cw.p, ph.cdeg.p, gsums.p, (const unsigned char*)gact);
+        dzero(ctx, status, 16);
         VT_LAUNCH(ctx, "batch_decide", k_batch_decide, grid_for(ng, 256, 64), 256, 0, ng, (const double*)gsums.p,
-                  (const double*)gconst.p, (const double*)gthr.p, (const double*)glow.p, gact.p, grot.p, gprev.p,
-                  giters.p, 0, (const int64_t*)seg.voff.p, status.p);
+                  (const double*)gconst.p, (const double*)gthr, (const double*)glow, gact, grot.p, gprev,
+                  giters, 0, seg.voff, status);
         if (nlive)
             VT_LAUNCH(ctx, "batch_rotate", k_batch_rotate, grid_for(nlive, 256, 8192), 256, 0, nlive,
                       (const int32_t*)live.p, d_gid, (const unsigned char*)grot.p, ph.past.p, ph.curr.p,
@@ -3747,7 +3943,7 @@ void batch_phase(vt_ctx* ctx, vt_graph* u, const int32_t* d_gid, const SegSums& 
             if (gexec) VT_HIP(ctx, hipGraphLaunch(gexec, ctx->stream));
             else round();
             unsigned long long* slot = pin + 2 * (r & 1);
-            VT_HIP(ctx, hipMemcpyAsync(slot, status.p, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost,
+            VT_HIP(ctx, hipMemcpyAsync(slot, status, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost,
                                        ctx->stream));
             VT_HIP(ctx, hipEventRecord(ev[r & 1], ctx->stream));
             if (use_graph && direct) capture();
@@ -3776,14 +3972,7 @@ void batch_phase(vt_ctx* ctx, vt_graph* u, const int32_t* d_gid, const SegSums& 
         throw;
     }
     release();
-    if (!u->part) u->part = (int64_t*)dalloc(ctx, 8 * (size_t)std::max<int64_t>(nv, 1));
-    VT_LAUNCH(ctx, "widen_part", k_widen_ids, grid_for(nv, 256, 8192), 256, 0, (const int32_t*)ph.past.p, nv, u->part);
-    q_out.assign((size_t)ng, 0.0);
-    iters_out.assign((size_t)ng, 0);
-    d2h(ctx, q_out.data(), gprev.p, 8 * (size_t)ng);
-    d2h(ctx, iters_out.data(), giters.p, 4 * (size_t)ng);
-    if (rounds_out) *rounds_out = rounds;
-    if (relists_out) *relists_out = relists;
+    finish(rounds, relists);
 }
 
 vt_tuning default_tuning()
