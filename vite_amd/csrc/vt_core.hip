@@ -206,8 +206,8 @@ void d2h(vt_ctx* ctx, void* dst, const void* src, size_t bytes)
 }
 // Pinned host memory that kernels write a few scalars to (256 bytes; [0, 1]: an iteration's Q and
 // movers, [2]: a phase's whole degrees, [3]: the last post's number,
-// [4, 8): a batch round's status, [8, 14): a rebuild's totals,
-// [16, 27): a phase's list sizes), with no copy queued behind the kernel.
+// [4, 8): a batch round's status, [8, 14): a rebuild's totals, [15]: whole hub rows,
+// [16, 29): a phase's list sizes), with no copy queued behind the kernel.
 double* mail(vt_ctx* ctx)
 {
     if (!ctx->mail) {

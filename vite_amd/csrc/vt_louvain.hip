@@ -51,16 +51,22 @@ __device__ __forceinline__ uint32_t slot_hash(int32_t c) { return (uint32_t)c * 
 
 // Degree buckets: (lanes per vertex G, table capacity CAP, max degree).  CAP >= 2*(deg+1)
 // keeps the table at most half full (a row has at most deg+1 distinct communities).
-constexpr int kNumBuckets = 10;
-constexpr int kLpvBucket = 7;      // lane per vertex (degree <= lpv_max)
+constexpr int kNumBuckets = 11;
+constexpr int kLpvBucket = 8;      // lane per vertex (degree <= lpv_max)
 // The wide bucket (one wave per row, up to 1023 entries) is split by degree so that each row
 // gets the smallest table that keeps it at most half full: 512 slots up to degree 255, 1024
 // up to 511, else 2048.  Smaller tables leave room for more resident waves per CU.
-constexpr int kWide512Bucket = 8;
-constexpr int kWide1024Bucket = 9;
+constexpr int kWide512Bucket = 9;
+constexpr int kWide1024Bucket = 10;
 constexpr int kLpvMaxDeg = 64;     // the largest row k_local_move_lpv is instantiated for
 constexpr int kLpvArena = 2560;
 constexpr int kHubBucket = 6;
+// Rows above the wide bucket's bound and of kHubLdsMin to kHubLdsMax entries: a workgroup each, in
+// LDS (k_hub_lds).  The hubs of kHubBucket are the longer ones, some hundreds on skewed graphs, and
+// shorter ones where a tuning's bounds send them there (the default bound is 511).  The two lists
+// are neighbours: a sweep that does not use the LDS form takes them as one.
+constexpr int kHubLdsBucket = 7;
+constexpr int kHubLdsMin = 512, kHubLdsMax = 4096;
 
 // Bucket of a row of degree d under per-bucket maximum degrees mx[0..5] (the tuning; the
 // default is 7, 15, 31, 63, 127, 1023): rows above mx[5] take the HBM-table kernel.
@@ -1509,6 +1515,394 @@ __global__ void __launch_bounds__(kHubBlock, 8) k_hub_move(MoveArgs a, const int
     if (threadIdx.x == 0 && inactive && a.inactive_count) atomicAdd(a.inactive_count, (unsigned long long)inactive);
 }
 
+// Hub rows of more than `above` and at most MAXD entries, a workgroup each, in one launch: the
+// row's communities are numbered by an LDS table, its entries placed by community (a counting
+// sort: counts, their scan, places by atomics), each run put in row order by counting, and folded
+// by a thread, runs of more than kHubLdsRun entries by a wave; then the gains and their argmax as
+// in k_hub_move.  The sorted form of the same rows was some twenty launches a sweep and three
+// radix passes over 12 bytes an entry in HBM.  What bounds it is the chain of its steps, some 20 us
+// a row: RGG n = 2^20 -i run 12.2 -> 10.8 ms, RGG n = 777001 -d 8 -t 1 run 17.7 -> 16.0.
+constexpr int kHubLdsRun = 64;
+
+template <int MAXD, int B, bool BATCH>
+__global__ void __launch_bounds__(B) k_hub_lds(MoveArgs a, const int32_t* __restrict__ hubs, int32_t nh, int above)
+{
+    constexpr int K = MAXD / B, kWaves = B / 64, kLongs = MAXD / kHubLdsRun;
+    __shared__ int32_t keys[2 * MAXD];   // -1 = empty
+    __shared__ uint32_t cur[2 * MAXD];   // entries per slot, then the end of its run so far
+    __shared__ uint16_t sid[MAXD];       // each entry's slot
+    __shared__ uint16_t placed[MAXD];    // entries by slot
+    __shared__ uint16_t occ[MAXD];       // occupied slots
+    __shared__ uint16_t longs[kLongs];
+    __shared__ double long_ey[kLongs];
+    __shared__ uint32_t s_wave[kWaves];
+    __shared__ int s_nocc, s_nlong;
+    __shared__ double s_ecc, s_self;
+    __shared__ double s_bg[kWaves];
+    __shared__ int32_t s_bc[kWaves];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    unsigned inactive = 0;
+    for (int32_t j = blockIdx.x; j < nh; j += gridDim.x) {
+        const int32_t v = hubs[j];
+        const int64_t e0 = a.offs[v];
+        const int64_t deg = a.offs[v + 1] - e0;
+        if (deg <= above || deg > MAXD) continue;  // another launch's
+        if constexpr (BATCH)
+            if (!a.gact[a.gid[v]]) continue;  // its graph has left the phase
+        if (a.active && !a.active[v]) {
+            if (t == 0) {
+                a.cw[v] = a.frozen[v];  // louvain.cpp:101-104
+                inactive++;
+            }
+            continue;
+        }
+        const int d = (int)deg;
+        const int32_t* tail = a.tail32 + e0;
+        const double* wgt = a.wgt + e0;
+        const int32_t cc = a.curr[v];
+        const uint32_t cap = 2u << (d > 1 ? 32 - __builtin_clz((unsigned)(d - 1)) : 0);  // 2 * the power of two >= d
+        for (uint32_t i = t; i < cap; i += B) {
+            keys[i] = -1;
+            cur[i] = 0;
+        }
+        if (t == 0) {
+            s_nocc = s_nlong = 0;
+            s_ecc = s_self = 0.0;
+        }
+        int32_t c[K];
+        bool loops = false;
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const int i = k * B + t;
+            c[k] = i < d ? tail[i] : -1;
+            loops = loops || c[k] == v;
+        }
+#pragma unroll
+        for (int k = 0; k < K; k++)
+            if (c[k] >= 0) c[k] = a.curr[c[k]];
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            if (c[k] < 0) continue;
+            uint32_t h = (slot_hash(c[k]) >> 7) & (cap - 1);
+            for (;;) {  // ends: at most half of the slots are ever taken
+                const int32_t old = atomicCAS(&keys[h], -1, c[k]);
+                if (old == -1) occ[atomicAdd(&s_nocc, 1)] = (uint16_t)h;
+                if (old == -1 || old == c[k]) break;
+                h = (h + 1) & (cap - 1);
+            }
+            sid[k * B + t] = (uint16_t)h;
+            atomicAdd(&cur[h], 1u);
+        }
+        const bool any_loop = __syncthreads_or(loops);
+        const uint32_t per = cap > (uint32_t)B ? cap / B : 1;
+        uint32_t sum = 0, all = 0;
+        for (uint32_t k = 0; k < per; k++)
+            if (t * per + k < cap) sum += cur[t * per + k];
+        uint32_t run = block_scan<B, uint32_t>(sum, s_wave, &all);
+        for (uint32_t k = 0; k < per; k++)
+            if (t * per + k < cap) {
+                const uint32_t x = cur[t * per + k];
+                cur[t * per + k] = run;
+                run += x;
+            }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const int i = k * B + t;
+            if (i < d) placed[atomicAdd(&cur[sid[i]], 1u)] = (uint16_t)i;
+        }
+        __syncthreads();
+        // each entry's place in its run: the run's entries before it in the row
+        constexpr uint16_t kNone = 0xffff;
+        uint16_t e[K], at[K];
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const int q = k * B + t;
+            at[k] = kNone;
+            e[k] = 0;
+            if (q < d) {
+                const uint32_t i = placed[q], sl = sid[i];
+                const uint32_t b = sl ? cur[sl - 1] : 0, end = cur[sl];
+                if (end - b <= (uint32_t)kHubLdsRun && end - b > 1) {
+                    uint32_t r = b;
+                    for (uint32_t x = b; x < end; x++) r += placed[x] < i ? 1 : 0;
+                    at[k] = (uint16_t)r;
+                    e[k] = (uint16_t)i;
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < K; k++)
+            if (at[k] != kNone) placed[at[k]] = e[k];
+        __syncthreads();
+        // the runs' folds, the first weight as is, the own community's from 0.0
+        double ey[K], ay[K];
+        const int m = s_nocc;
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const int p = k * B + t;
+            c[k] = cc;
+            ey[k] = ay[k] = 0.0;
+            if (p >= m) continue;
+            const uint32_t sl = occ[p], b = sl ? cur[sl - 1] : 0, end = cur[sl];
+            if (end - b > (uint32_t)kHubLdsRun) {
+                longs[atomicAdd(&s_nlong, 1)] = (uint16_t)sl;
+                continue;
+            }
+            c[k] = keys[sl];
+            ay[k] = a.cdeg[c[k]];
+            double acc = c[k] == cc ? 0.0 : -0.0;
+            for (uint32_t x0 = b; x0 < end; x0 += 8) {
+                double y[8];
+#pragma unroll
+                for (uint32_t u = 0; u < 8; u++) y[u] = x0 + u < end ? wgt[placed[x0 + u]] : -0.0;
+#pragma unroll
+                for (int u = 0; u < 8; u++) acc = acc + y[u];
+            }
+            ey[k] = acc;
+            if (c[k] == cc) s_ecc = acc;
+        }
+        __syncthreads();
+        const int nl = s_nlong;
+        for (int x = w; x < nl; x += kWaves) {
+            const uint16_t sl = longs[x];
+            const bool own = keys[sl] == cc;
+            const uint32_t b = sl ? cur[sl - 1] : 0, end = cur[sl];
+            uint32_t q = b;  // the run's entries in row order
+            for (int i0 = 0; i0 < d; i0 += 64) {
+                const bool in = i0 + lane < d && sid[i0 + lane] == sl;
+                const unsigned long long hits = __ballot(in);
+                if (in) placed[q + __popcll(hits & ((1ull << lane) - 1))] = (uint16_t)(i0 + lane);
+                q += (uint32_t)__popcll(hits);
+            }
+            wave_sync();
+            const double acc = wave_left_fold<2>(own ? 0.0 : -0.0, end - b, [&](int64_t i) { return wgt[placed[b + i]]; });
+            if (lane == 0) {
+                long_ey[x] = acc;
+                if (own) s_ecc = acc;
+            }
+        }
+        if (any_loop && w == kWaves - 1) {
+            const double self = wave_left_fold<2>(0.0, d, [&](int64_t i) { return tail[i] == v ? wgt[i] : -0.0; });
+            if (lane == 0) s_self = self;
+        }
+        __syncthreads();
+        const double constant = BATCH ? a.constant[a.gid[v]] : *a.constant;
+        const double ecc = s_ecc, kv = a.vdeg[v];
+        const double eix = ecc - s_self, ax = a.cdeg[cc] - kv;
+        double bg = 0.0;
+        int32_t bc = INT_MAX;
+        auto consider = [&](int32_t cand, double eyc, double ayc) {
+            const double gain = 2.0 * (eyc - eix) - 2.0 * kv * (ayc - ax) * constant;
+            argmax_take(bg, bc, gain > 0.0 ? gain : 0.0, gain > 0.0 ? cand : INT_MAX);
+        };
+#pragma unroll
+        for (int k = 0; k < K; k++)
+            if (c[k] != cc) consider(c[k], ey[k], ay[k]);
+        for (int x = t; x < nl; x += B) {
+            const int32_t cand = keys[longs[x]];
+            if (cand != cc) consider(cand, long_ey[x], a.cdeg[cand]);
+        }
+        for (int o = 32; o > 0; o >>= 1) argmax_take(bg, bc, __shfl_xor(bg, o), __shfl_xor(bc, o));
+        if (lane == 0) {
+            s_bg[w] = bg;
+            s_bc[w] = bc;
+        }
+        __syncthreads();
+        if (t == 0) {
+            for (int x = 1; x < kWaves; x++) argmax_take(bg, bc, s_bg[x], s_bc[x]);
+            int32_t tgt = cc;
+            if (bg > 0.0) {
+                tgt = bc;
+                if (a.csize[cc] == 1 && tgt > cc && a.csize[tgt] == 1) tgt = cc;  // louvain.cpp:2275-2276
+            }
+            a.target[v] = tgt;
+            a.cw[v] = ecc;
+            if (a.frozen) a.frozen[v] = ecc;
+        }
+        __syncthreads();
+    }
+    if (t == 0 && inactive && a.inactive_count) atomicAdd(a.inactive_count, (unsigned long long)inactive);
+}
+
+// Hub rows of more than kHubLdsMax entries whose weights are whole numbers (their totals below
+// 2^51): any order of adding a community's weights has the bits of the fold, so nothing is
+// sorted.  A workgroup adds a chunk of a row in an LDS table, and each community of the chunk once
+// to one table in HBM, keyed by (hub, community); a pass over that table forms the gains, one
+// picks the smallest community of the largest and clears it.  Four launches, where the sorted form
+// has some twenty: BA n = 300007 -i run 7.04 -> 6.19 ms with k_hub_lds beside it.
+struct HubWhole {
+    const int32_t* hubs;
+    int32_t nh;
+    const int64_t* hoffs;
+    unsigned long long cap;     // slots, twice the entries
+    unsigned long long* key;    // (hub << 32 | community) + 1; 0 = empty
+    double* val;                // the weights' sum, then the gain
+    double *self, *ecc;         // per hub
+    unsigned long long* best;   // per hub: the largest gain's bits
+    unsigned long long* cand;   // per hub: 2^32 - 1 - the smallest community that holds it (0: none)
+};
+constexpr int kHubwChunk = 1024;  // shorter than a row: a chunk is of one hub or two
+
+__device__ __forceinline__ unsigned long long hubw_slot(unsigned long long key, unsigned long long cap)
+{
+    return __umul64hi(key * 0x9E3779B97F4A7C15ull, cap);
+}
+
+__global__ void __launch_bounds__(256) k_hubw_insert(MoveArgs a, HubWhole h)
+{
+    constexpr int kSlots = 2 * kHubwChunk;
+    __shared__ uint32_t s_key[kSlots];  // community, top bit: the chunk's second hub
+    __shared__ double s_val[kSlots];
+    constexpr uint32_t kEmpty = 0xffffffffu;
+    const int64_t total = h.hoffs[h.nh];
+    for (int64_t lo = (int64_t)blockIdx.x * kHubwChunk; lo < total; lo += (int64_t)gridDim.x * kHubwChunk) {
+        for (int i = threadIdx.x; i < kSlots; i += 256) {
+            s_key[i] = kEmpty;
+            s_val[i] = 0.0;
+        }
+        int32_t x = 0, y = h.nh - 1;  // the hub of the first entry
+        while (x < y) {
+            const int32_t mid = (x + y + 1) >> 1;
+            if (h.hoffs[mid] <= lo) x = mid;
+            else y = mid - 1;
+        }
+        const int64_t bound = h.hoffs[x + 1];
+        const int64_t at0 = a.offs[h.hubs[x]] - h.hoffs[x];
+        const int64_t at1 = x + 1 < h.nh ? a.offs[h.hubs[x + 1]] - bound : 0;
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kHubwChunk / 256; k++) {
+            const int64_t q = lo + k * 256 + threadIdx.x;
+            if (q >= total) continue;
+            const bool second = q >= bound;
+            const int64_t e = q + (second ? at1 : at0);
+            const int32_t tail = a.tail32[e];
+            const double wt = a.wgt[e];
+            const int32_t j = x + (second ? 1 : 0);
+            if (tail == h.hubs[j]) unsafeAtomicAdd(&h.self[j], wt);
+            const int32_t c = a.curr[tail];
+            const uint32_t key = (uint32_t)c | (second ? 0x80000000u : 0u);
+            uint32_t p = ((uint32_t)slot_hash(c) ^ (second ? 0x55555555u : 0u)) & (kSlots - 1);
+            for (;;) {  // ends: at most half of the slots are ever taken
+                const uint32_t old = atomicCAS(&s_key[p], kEmpty, key);
+                if (old == kEmpty || old == key) break;
+                p = (p + 1) & (kSlots - 1);
+            }
+            __hip_atomic_fetch_add(&s_val[p], wt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < kSlots; i += 256) {
+            const uint32_t k = s_key[i];
+            if (k == kEmpty) continue;
+            const int32_t j = x + (int32_t)(k >> 31);
+            const unsigned long long key = (((unsigned long long)j << 32) | (k & 0x7fffffffu)) + 1;
+            unsigned long long p = hubw_slot(key, h.cap);
+            for (;;) {  // ends: the table has two slots for every entry
+                const unsigned long long old = atomicCAS(&h.key[p], 0ull, key);
+                if (old == 0 || old == key) break;
+                p = p + 1 < h.cap ? p + 1 : 0;
+            }
+            unsafeAtomicAdd(&h.val[p], s_val[i]);
+        }
+        __syncthreads();  // the table is reused
+    }
+}
+
+// Gains (louvain.cpp:2246-2273) in place of the sums, but for the hubs' own communities.
+__global__ void k_hubw_gain(MoveArgs a, HubWhole h)
+{
+    const double constant = *a.constant;
+    for (unsigned long long i = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x; i < h.cap;
+         i += (unsigned long long)gridDim.x * blockDim.x) {
+        const unsigned long long key = h.key[i];
+        if (!key) continue;
+        const int32_t j = (int32_t)((key - 1) >> 32), c = (int32_t)(uint32_t)(key - 1);
+        const int32_t v = h.hubs[j];
+        if (a.active && !a.active[v]) continue;
+        const int32_t cc = a.curr[v];
+        if (c == cc) {
+            h.ecc[j] = h.val[i];
+            continue;
+        }
+        const unsigned long long own = (((unsigned long long)j << 32) | (uint32_t)cc) + 1;
+        double ecc = 0.0;
+        for (unsigned long long p = hubw_slot(own, h.cap);;) {
+            const unsigned long long k = h.key[p];
+            if (k == own) ecc = h.val[p];
+            if (k == own || k == 0) break;
+            p = p + 1 < h.cap ? p + 1 : 0;
+        }
+        const double kv = a.vdeg[v];
+        const double eix = ecc - h.self[j];
+        const double ax = a.cdeg[cc] - kv;
+        const double gain = 2.0 * (h.val[i] - eix) - 2.0 * kv * (a.cdeg[c] - ax) * constant;
+        h.val[i] = gain;
+        // Most gains lose to one that is there already; of those that do not, the largest of each hub's
+        // lanes (four hubs at most, then each lane its own).
+        unsigned long long bits = gain > 0.0 ? (unsigned long long)__double_as_longlong(gain) : 0ull;
+        if (bits && bits <= __hip_atomic_load(&h.best[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) bits = 0;
+        for (int round = 0; round < 4 && bits; round++) {
+            if (j != __builtin_amdgcn_readfirstlane(j)) continue;
+            unsigned long long m = 0;
+            for (unsigned long long x = __ballot(1); x; x &= x - 1) {
+                const int l = __builtin_ctzll(x);
+                const unsigned long long o =
+                    ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(bits >> 32), l) << 32) |
+                    (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)bits, l);
+                m = o > m ? o : m;
+            }
+            if (bits == m) atomicMax(&h.best[j], m);
+            bits = 0;
+        }
+        if (bits) atomicMax(&h.best[j], bits);
+    }
+}
+
+__global__ void k_hubw_pick(MoveArgs a, HubWhole h)
+{
+    for (unsigned long long i = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x; i < h.cap;
+         i += (unsigned long long)gridDim.x * blockDim.x) {
+        const unsigned long long key = h.key[i];
+        if (!key) continue;
+        const int32_t j = (int32_t)((key - 1) >> 32), c = (int32_t)(uint32_t)(key - 1);
+        const int32_t v = h.hubs[j];
+        if (!(a.active && !a.active[v]) && c != a.curr[v]) {
+            const double gain = h.val[i];
+            if (gain > 0.0 && (unsigned long long)__double_as_longlong(gain) == h.best[j])
+                atomicMax(&h.cand[j], 0xffffffffull - (uint32_t)c);
+        }
+        h.key[i] = 0;
+        h.val[i] = 0.0;
+    }
+}
+
+__global__ void k_hubw_final(MoveArgs a, HubWhole h)
+{
+    for (int32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < h.nh; j += gridDim.x * blockDim.x) {
+        const int32_t v = h.hubs[j];
+        if (a.active && !a.active[v]) {
+            a.cw[v] = a.frozen[v];  // louvain.cpp:101-104
+            if (a.inactive_count) atomicAdd(a.inactive_count, 1ull);
+        } else {
+            const int32_t cc = a.curr[v];
+            const double ecc = h.ecc[j];
+            int32_t tgt = cc;
+            if (h.cand[j]) {
+                tgt = (int32_t)(0xffffffffull - h.cand[j]);
+                if (a.csize[cc] == 1 && tgt > cc && a.csize[tgt] == 1) tgt = cc;  // louvain.cpp:2275-2276
+            }
+            a.target[v] = tgt;
+            a.cw[v] = ecc;
+            if (a.frozen) a.frozen[v] = ecc;
+        }
+        h.self[j] = h.ecc[j] = 0.0;
+        h.best[j] = h.cand[j] = 0;
+    }
+}
+
 // Per hub: target (with the singleton rule, louvain.cpp:2275-2276) and clusterWeight, or the
 // frozen weight of a hub early termination froze (louvain.cpp:101-104).
 __global__ void k_hub_final(MoveArgs a, const int32_t* __restrict__ hubs, int32_t nh, const double* __restrict__ own,
@@ -1580,12 +1974,14 @@ __global__ void __launch_bounds__(kFoldRows) k_row_fold(const int64_t* __restric
 // kFoldBlockRow and more a workgroup each where their weights are whole numbers: a skewed
 // graph's giant coarse row (half a million entries) held the launch for 4.5 ms as one wave's
 // chain of lane reads on BA n = 2^22.  A workgroup's rows are gridDim apart, so that hubs
-// with neighbouring ids spread over the chip.
+// with neighbouring ids spread over the chip.  fraction (or null) is set where a row of
+// kFoldBlockRow entries and more is no such sum.
 constexpr int kFoldLongBlock = 256;
-constexpr int64_t kFoldBlockRow = 8192;
+constexpr int64_t kFoldBlockRow = kHubLdsMax + 1;
 __global__ void __launch_bounds__(kFoldLongBlock) k_row_fold_long(const int64_t* __restrict__ offs,
                                                                  const DEdge* __restrict__ edges, int64_t nv,
-                                                                 double* __restrict__ vdeg, int64_t long_min)
+                                                                 double* __restrict__ vdeg, int64_t long_min,
+                                                                 unsigned long long* __restrict__ fraction)
 {
     __shared__ int32_t s_row[kFoldLongBlock];
     __shared__ int32_t s_n, s_big;
@@ -1615,7 +2011,10 @@ __global__ void __launch_bounds__(kFoldLongBlock) k_row_fold_long(const int64_t*
                 if (threadIdx.x == 0) vdeg[v] = 0.0 + sum;
             } else if (w == 0) {
                 sum = wave_left_fold<4>(0.0, d, weight);
-                if (lane == 0) vdeg[v] = sum;
+                if (lane == 0) {
+                    vdeg[v] = sum;
+                    if (fraction) *fraction = 1;  // any workgroup's store
+                }
             }
         }
         for (int k = w; k < n; k += kFoldLongBlock / 64) {
@@ -1654,18 +2053,28 @@ __global__ void k_init(int64_t nv, const double* __restrict__ vdeg, double* __re
 // whole (pinned host memory): 1.0 where every degree is a whole number >= 0 and they total
 // less than 2^52.
 __global__ void k_constant(const double* __restrict__ sums, const unsigned long long* __restrict__ fraction,
-                           double* __restrict__ constant, double* __restrict__ whole)
+                           const unsigned long long* __restrict__ hub_fraction, double* __restrict__ constant,
+                           double* __restrict__ whole, double* __restrict__ hub_whole)
 {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
         constant[0] = 1.0 / sums[0];
         *whole = *fraction == 0 && sums[0] < 0x1p52 ? 1.0 : 0.0;
+        *hub_whole = hub_fraction && *hub_fraction == 0 ? 1.0 : 0.0;
     }
+}
+
+// Whether a sweep's `lds` rows take k_hub_lds: not too many, and no sorted path beside them (which
+// costs its launches however few rows it has).
+__device__ __host__ __forceinline__ bool hub_lds_used(int64_t hubs, int64_t lds, int64_t limit, bool whole)
+{
+    return lds <= limit && (hubs == 0 || whole || limit == INT32_MAX);
 }
 
 // A row's sweep list: its degree bucket, the wide bucket split by table size.
 __device__ __host__ __forceinline__ uint32_t list_bucket(int64_t d, int lpv_max, const BucketBounds& bb)
 {
     const uint32_t b = (uint32_t)(lpv_max > 0 && d <= lpv_max ? kLpvBucket : degree_bucket(d, bb));
+    if (b == kHubBucket && d >= kHubLdsMin && d <= kHubLdsMax) return kHubLdsBucket;
     if (b == kHubBucket - 1) return d <= bb.wide[0] ? kWide512Bucket : d <= bb.wide[1] ? kWide1024Bucket : b;
     return b;
 }
@@ -1698,13 +2107,14 @@ __global__ void k_color_keys(int64_t nv, const int64_t* __restrict__ colors, int
 }
 
 // Histogram of small keys: per-block counts in LDS, one global atomic per touched bin.
-__global__ void k_key_histogram(const uint32_t* __restrict__ keys, int64_t n, int64_t* __restrict__ hist, int nbins)
+// Counts of the keys in [lo, lo + nbins).
+__global__ void k_key_histogram(const uint32_t* __restrict__ keys, int64_t n, int64_t* __restrict__ hist, uint32_t lo, int nbins)
 {
     extern __shared__ unsigned s_bins[];
     for (int i = threadIdx.x; i < nbins; i += blockDim.x) s_bins[i] = 0;
     __syncthreads();
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        if (keys[i] < (uint32_t)nbins) atomicAdd(&s_bins[keys[i]], 1u);  // larger keys: excluded
+        if (keys[i] - lo < (uint32_t)nbins) atomicAdd(&s_bins[keys[i] - lo], 1u);
     __syncthreads();
     for (int i = threadIdx.x; i < nbins; i += blockDim.x)
         if (s_bins[i]) atomicAdd((unsigned long long*)&hist[i], (unsigned long long)s_bins[i]);
@@ -2537,7 +2947,7 @@ struct SetupArgs {
     const double* vdeg;
     int32_t nv, blocks;
     int64_t chunk;
-    double *cdeg, *sums, *constant, *out;  // out (pinned): [2] whole degrees, [16, 26) the buckets' sizes, [26] hub entries
+    double *cdeg, *sums, *constant, *out;  // out (pinned): [2] whole degrees, [16, 27) the buckets' sizes, [28] hub entries
     int32_t *csize, *past, *curr, *target, *lists;
     unsigned char* active;  // null when ET is off, with the three below
     double *frozen, *pa, *pb;
@@ -2546,7 +2956,9 @@ struct SetupArgs {
     int64_t* hoffs;               // nv + 1
     BucketBounds bb;
     int32_t lpv_max;
-    unsigned long long seq;       // posted with out
+    int64_t hub_limit;                       // hub_lds_limit()
+    const unsigned long long* hub_fraction;  // row_degrees' (or null: no long hub rows)
+    unsigned long long seq;                  // posted with out
 };
 
 __global__ void __launch_bounds__(kTailBlock) k_setup_small(SetupArgs a)
@@ -2620,7 +3032,9 @@ __global__ void __launch_bounds__(kTailBlock) k_setup_small(SetupArgs a)
     }
     __syncthreads();
     unsigned long long entries = 0;
-    const int nh = s_total[kHubBucket];
+    const bool whole = a.hub_fraction && *a.hub_fraction == 0;
+    const int nh = s_total[kHubBucket] +
+                   (hub_lds_used(s_total[kHubBucket], s_total[kHubLdsBucket], a.hub_limit, whole) ? 0 : s_total[kHubLdsBucket]);
     for (int j0 = 0; j0 < nh; j0 += kTailBlock) {
         const int j = j0 + t;
         const int32_t v = j < nh ? a.lists[hub_off + j] : 0;
@@ -2636,7 +3050,8 @@ __global__ void __launch_bounds__(kTailBlock) k_setup_small(SetupArgs a)
     if (t == 0) {
         for (int q = 0; q < kNumBuckets; q++) out[16 + q] = s_total[q];
         a.hoffs[nh] = (int64_t)entries;
-        out[26] = (int64_t)entries;
+        out[28] = (int64_t)entries;
+        a.out[15] = whole ? 1.0 : 0.0;
         a.sums[0] = r[0];
         a.sums[1] = r[1];
         a.constant[0] = 1.0 / r[0];
@@ -2931,9 +3346,11 @@ __global__ void k_batch_rotate(int64_t n, const int32_t* __restrict__ live, cons
 struct ColorSweep {
     SweepPlan plan{};
     int64_t fused_blocks = 0;
-    int64_t mid_off = 0, mid_n = 0, hub_off = 0, hub_n = 0, lpv_off = 0, lpv_n = 0;
+    int64_t mid_off = 0, mid_n = 0, hub_off = 0, hub_n = 0, hubl_off = 0, hubl_n = 0;
+    int64_t lpv_off = 0, lpv_n = 0;
     int64_t wide_off[3] = {0, 0, 0}, wide_n[3] = {0, 0, 0};  // 512-, 1024- and 2048-slot tables
-    int32_t index = 0;  // position in Phase::sweeps
+    int32_t index = 0;   // position in Phase::sweeps
+    bool whole = false;  // the hubs of hub_n take k_hubw_*
 };
 
 // Rows up to this degree take the lane-per-vertex kernel when VITE_AMD_LPV_MAXDEG is set
@@ -2965,6 +3382,14 @@ struct Phase {
     // that is no whole number
     DBuf<unsigned long long> ucount;
     DBuf<uint32_t> ev_cnt;   // events per community, zero between uses
+    // Set by row_degrees where a hub row's weights are no whole numbers (null: not looked for, or
+    // read), the host's reading of it, and whether the sweeps add the hubs' weights in any order
+    // (k_hubw_*).
+    unsigned long long* hub_fraction = nullptr;
+    bool hub_exact = false, hub_whole = false;
+    DBuf<unsigned long long> hw_key;  // zero between sweeps, with the three below
+    DBuf<double> hw_val, hw_hub;
+    DBuf<unsigned long long> hw_best;
     bool whole = false;      // whole degrees, so that any order of adding events gives the same bits
     std::vector<ColorSweep> sweeps;      // per color (one entry in plain/vorder)
     std::vector<int64_t> color_ptr;      // colorPtr (louvain.cpp:647-661)
@@ -3050,6 +3475,11 @@ struct Phase {
 
     void row_degrees()
     {
+        hub_fraction = nullptr;
+        if (hub_whole_possible()) {
+            hub_fraction = (unsigned long long*)scratch(ctx, "hub_fraction", 8);
+            dzero(ctx, hub_fraction, 8);
+        }
         if (!tail32.p && nv && g->ne <= 48 * nv && g->max_degree <= kSfTile) {
             // short rows (a row's fold is one thread's, so no long ones): the split copy the
             // local move reads and the degrees in one pass
@@ -3060,7 +3490,7 @@ struct Phase {
                       tail32.p, wgt.p, vdeg.p);
         } else if (nv && nv < 65536 && g->ne > 48 * nv) {  // few, long rows: a thread per row would leave the GPU idle
             VT_LAUNCH(ctx, "row_fold", k_row_fold_long, grid_for(nv, kFoldLongBlock / 64, 65536), kFoldLongBlock, 0, g->offs,
-                      g->edges, nv, vdeg.p, (int64_t)0);
+                      g->edges, nv, vdeg.p, (int64_t)0, hub_fraction);
         } else if (nv) {
             // a thread per row, and a wave per row for the rows of kFoldLongRow or more
             const bool split = g->max_degree >= kFoldLongRow;
@@ -3068,7 +3498,7 @@ struct Phase {
                       vdeg.p, split ? kFoldLongRow : INT64_MAX);
             if (split)
                 VT_LAUNCH(ctx, "row_fold_long", k_row_fold_long, grid_for(nv, kFoldLongBlock, 4096), kFoldLongBlock, 0,
-                          g->offs, g->edges, nv, vdeg.p, kFoldLongRow);
+                          g->offs, g->edges, nv, vdeg.p, kFoldLongRow, hub_fraction);
         }
     }
 
@@ -3087,7 +3517,8 @@ struct Phase {
         if (flags & VT_FLAG_SEQUENTIAL_SUMS) seq_sum2(ctx, vdeg.p, nullptr, nv, sums());
         else tree_sum2(ctx, vdeg.p, nullptr, nv, sums());
         VT_LAUNCH(ctx, "constant", k_constant, 1, 64, 0, (const double*)sums(),
-                  (const unsigned long long*)(ucount.p + 5), constant(), mail(ctx) + 2);
+                  (const unsigned long long*)(ucount.p + 5), (const unsigned long long*)hub_fraction, constant(),
+                  mail(ctx) + 2, mail(ctx) + 15);
     }
 
     // alloc, init and build_lists of a plain phase on at most kTailVerts vertices (tree sums).
@@ -3122,12 +3553,15 @@ struct Phase {
         a.hoffs = hub_offs[0].p;
         a.bb = bounds();
         a.lpv_max = lpv_max_degree();
+        a.hub_limit = hub_lds_limit();
+        a.hub_fraction = hub_fraction;
         a.seq = ++ctx->mail_seq;
         VT_LAUNCH(ctx, "setup", k_setup_small, 1, kTailBlock, 0, a);
         mail_wait(ctx, ctx->mail_seq);
         const int64_t* h = (const int64_t*)mail(ctx);
+        hub_whole = hub_exact = mail(ctx)[15] == 1.0;
         plan_sweeps(1, h + 16);
-        hub_total.assign(1, h[26]);
+        hub_total.assign(1, h[28]);
         hub_sort = true;
     }
 
@@ -3142,6 +3576,8 @@ struct Phase {
         uint32_t* k0 = (uint32_t*)scratch(ctx, "lk0", 4 * n1);
         uint32_t* k1 = (uint32_t*)scratch(ctx, "lk1", 4 * n1);
         uint32_t* v1 = (uint32_t*)scratch(ctx, "lv1", 4 * n1);
+        if (ncol > 1638 || (d_colors && num_color > 16384))
+            fail(ctx, VT_ERR_LIMIT, "too many sweep lists (%lld colors)", (long long)num_color);
         const int64_t nkeys = ncol * kNumBuckets;
         int64_t* hist = (int64_t*)scratch(ctx, "lhist", 8 * (size_t)(nkeys + 1));
         std::vector<int64_t> h(nkeys, 0);
@@ -3155,7 +3591,10 @@ struct Phase {
             sort_pairs_u32(ctx, k0, (uint32_t*)lists.p, nv, (int)bits_for(nkeys), k1, v1, &alt);
             if (alt) d2d(ctx, lists.p, v1, 4 * (size_t)nv);
             d2h(ctx, h.data(), hist, 8 * nkeys);
+            if (hub_fraction) hub_exact = mail(ctx)[15] == 1.0;  // k_constant's, there by now
+            hub_fraction = nullptr;
         }
+        hub_whole = hub_exact && hub_whole_possible();
         const int64_t max_hub = plan_sweeps(ncol, h.data());
         // Hub rows: by sorting, unless the sweep must stay free of library sorts (a batch
         // replays its sweeps from captured graphs) or edge indexes exceed 32 bits.
@@ -3209,6 +3648,26 @@ struct Phase {
         }
     }
 
+    // How many rows k_hub_lds takes at most (-1: none).  It saves the sorted form's twenty launches
+    // (RGG n = 2^20 -i run 12.2 -> 10.8 ms) but its rows of up to 4096 entries run one or two per CU:
+    // on RGG n = 2^24, with 4000 to 15000 such rows a sweep, it took 14.0 ms of a run and the sorted
+    // form 10.5.  (From 2^17 vertices the sorted form's keys of 17 K hubs pass 32 bits and take the
+    // library's sort: BA n = 2^22, device time of a run 71.0 -> 64.1 ms with the larger limit.)  A tuning that forces a form of the sorted path gets it; a batch's only other form
+    // is a wave per row.
+    int64_t hub_lds_limit() const
+    {
+        if (gid) return INT32_MAX;
+        if (ctx->tuning.hub_block_min <= 0 || ctx->tuning.hub_block_min >= (1 << 30)) return -1;
+        if (bits_for(nv) >= 18) return 32768;
+        return g->max_degree <= 1024 ? 8192 : 1536;
+    }
+    // Whether the sweeps may use k_hubw_* for the hubs of kHubBucket: all longer than kHubLdsMax.
+    bool hub_whole_possible() const
+    {
+        return !gid && hub_lds_limit() >= 0 && ctx->tuning.bucket_max_degree[5] >= kHubLdsMin - 1 &&
+               g->max_degree > kHubLdsMax && g->ne < (int64_t(1) << 31);
+    }
+
     // The launch plan of every sweep from its lists' sizes h[sweep * kNumBuckets + bucket]; returns
     // the largest number of hub rows in one.
     int64_t plan_sweeps(int64_t ncol, const int64_t* h)
@@ -3238,15 +3697,24 @@ struct Phase {
                 } else if (b == kLpvBucket) {
                     cs.lpv_off = off;
                     cs.lpv_n = cnt;
+                } else if (b == kHubLdsBucket) {
+                    cs.hubl_off = off;
+                    cs.hubl_n = cnt;
                 } else {
                     cs.hub_off = off;
                     cs.hub_n = cnt;
-                    max_hub = std::max(max_hub, cnt);
                 }
                 off += cnt;
             }
             cs.plan.bbeg[kFusedBuckets] = blocks;
             cs.fused_blocks = blocks;
+            cs.whole = hub_whole;
+            if (cs.hubl_n && !hub_lds_used(cs.hub_n, cs.hubl_n, hub_lds_limit(), hub_whole)) {
+                cs.hub_n += cs.hubl_n;
+                cs.hubl_n = 0;
+                cs.whole = false;  // k_hubw_* takes long rows only
+            }
+            max_hub = std::max(max_hub, cs.hub_n);
         }
         for (int64_t c = 0; c < ncol; c++) sweeps[c].index = (int32_t)c;
         return max_hub;
@@ -3254,9 +3722,12 @@ struct Phase {
 
     void key_histogram(const uint32_t* keys, int64_t n, int64_t* hist, int nbins)
     {
-        if (nbins > 16384) fail(ctx, VT_ERR_LIMIT, "too many sweep lists (%d)", nbins);
-        VT_LAUNCH(ctx, "key_hist", k_key_histogram, grid_for(n, 256, 2048), 256, sizeof(unsigned) * nbins, keys, n, hist,
-                  nbins);
+        constexpr int kBins = 16384;  // 64 KB of LDS
+        for (int lo = 0; lo < nbins; lo += kBins) {
+            const int here = std::min(kBins, nbins - lo);
+            VT_LAUNCH(ctx, "key_hist", k_key_histogram, grid_for(n, 256, 2048), 256, sizeof(unsigned) * here, keys, n, hist + lo,
+                      (uint32_t)lo, here);
+        }
     }
 
     MoveArgs move_args()
@@ -3365,6 +3836,33 @@ struct Phase {
                   (const unsigned long long*)best, (const int32_t*)bestc);
     }
 
+    void hub_sweep_whole(const MoveArgs& a, const ColorSweep& cs, int64_t total)
+    {
+        int64_t most = 0, hubs = 0;
+        for (const ColorSweep& x : sweeps) {
+            most = std::max(most, hub_total[x.index]);
+            hubs = std::max(hubs, x.hub_n);
+        }
+        if (hw_key.n < 2 * (size_t)most || hw_hub.n < 2 * (size_t)hubs) {
+            hw_key = DBuf<unsigned long long>(ctx, 2 * (size_t)most);
+            hw_val = DBuf<double>(ctx, 2 * (size_t)most);
+            hw_hub = DBuf<double>(ctx, 2 * (size_t)hubs);
+            hw_best = DBuf<unsigned long long>(ctx, 2 * (size_t)hubs);
+            dzero(ctx, hw_key.p, 16 * (size_t)most);
+            dzero(ctx, hw_val.p, 16 * (size_t)most);
+            dzero(ctx, hw_hub.p, 16 * (size_t)hubs);
+            dzero(ctx, hw_best.p, 16 * (size_t)hubs);
+        }
+        const HubWhole hw{(const int32_t*)(lists.p + cs.hub_off), (int32_t)cs.hub_n, hub_offs[cs.index].p,
+                          2 * (unsigned long long)total, hw_key.p, hw_val.p, hw_hub.p, hw_hub.p + hubs, hw_best.p,
+                          hw_best.p + hubs};
+        TimedScope ts(ctx, "local_move_hub");
+        VT_LAUNCH(ctx, "hubw_insert", k_hubw_insert, grid_for(total, kHubwChunk, 1 << 21), 256, 0, a, hw);
+        VT_LAUNCH(ctx, "hubw_gain", k_hubw_gain, grid_for(2 * total, 256, 8192), 256, 0, a, hw);
+        VT_LAUNCH(ctx, "hubw_pick", k_hubw_pick, grid_for(2 * total, 256, 8192), 256, 0, a, hw);
+        VT_LAUNCH(ctx, "hubw_final", k_hubw_final, grid_for(cs.hub_n, 64, 4096), 64, 0, a, hw);
+    }
+
     void sweep(const ColorSweep& cs)
     {
         prepare_sweep();
@@ -3410,7 +3908,23 @@ struct Phase {
             VT_LAUNCH(ctx, "local_move_wide", kern, (unsigned)std::min<int64_t>(cs.wide_n[w], 16384), 64, 0, a,
                       (const int32_t*)(lists.p + cs.wide_off[w]), cs.wide_n[w]);
         }
-        if (cs.hub_n && hub_sort) {
+        if (cs.hubl_n) {
+            const int32_t* hubs = (const int32_t*)(lists.p + cs.hubl_off);
+            const unsigned nb = (unsigned)std::min<int64_t>(cs.hubl_n, 16384);
+            const int32_t n = (int32_t)cs.hubl_n;
+            // 22, 44 and 88 KB of LDS: 28, 24 and 16 waves per CU.  Where every row has a CU to itself,
+            // one launch of the largest: each takes some 20 us for any number of rows.
+            auto k1 = batch ? k_hub_lds<1024, 256, true> : k_hub_lds<1024, 256, false>;
+            auto k2 = batch ? k_hub_lds<2048, 512, true> : k_hub_lds<2048, 512, false>;
+            auto k4 = batch ? k_hub_lds<4096, 1024, true> : k_hub_lds<4096, 1024, false>;
+            const bool one = n <= 256, only1 = g->max_degree <= 1024, only2 = g->max_degree <= 2048;
+            if (only1 || !one) VT_LAUNCH(ctx, "local_move_hub", k1, nb, 256, 0, a, hubs, n, 0);
+            if (!only1 && (only2 || !one)) VT_LAUNCH(ctx, "local_move_hub", k2, nb, 512, 0, a, hubs, n, one ? 0 : 1024);
+            if (!only2) VT_LAUNCH(ctx, "local_move_hub", k4, nb, 1024, 0, a, hubs, n, one ? 0 : 2048);
+        }
+        if (cs.hub_n && cs.whole && hub_sort && hub_total[cs.index] < (int64_t(1) << 31)) {
+            hub_sweep_whole(a, cs, hub_total[cs.index]);
+        } else if (cs.hub_n && hub_sort) {
             const int64_t total = hub_total[cs.index];
             const int cbits = (int)bits_for(nv > 1 ? nv - 1 : 1);  // community ids < nv
             const int kbits = cbits + (int)bits_for(cs.hub_n);
