@@ -211,6 +211,7 @@ __global__ void __launch_bounds__(64 * kFoldWaves) k_comm_fold(
     __shared__ uint32_t tl[kFoldWaves][kCfList];  // keys in insertion order
     __shared__ uint16_t ts[kFoldWaves][kCfList];  // and their slots
     __shared__ double wst[kFoldWaves][65];        // [0] = -0.0, then the chunk's weights
+    __shared__ alignas(16) double own[kFoldWaves][72];  // the chunk's internal weights
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const unsigned long long below = (1ull << lane) - 1;
     for (int i = lane; i < kCfCap; i += 64) {
@@ -250,13 +251,27 @@ __global__ void __launch_bounds__(64 * kFoldWaves) k_comm_fold(
                 const int64_t kn = mr.csr_index(p + 128, moff, mrow);
                 if (p + 128 < mr.s1) enn = edges[kn];
             }
-            // internal entries (about half after a phase) form one long run per chunk: add
-            // them in lane order with the lane read as a scalar, without the table
+            // internal entries (about half after a phase) form one long run per chunk: packed in
+            // lane order and filled up to eight with -0.0, every lane reads them back and adds them,
+            // an LDS read for two and an add each (a lane read as a scalar took two reads, an add and
+            // the steps of the mask: 8.4 ms for the 563 M entries of RGG n = 2^24, this 7.0)
             const bool in = valid && c2 == (uint32_t)c;
             const bool ext = valid && !in;
             const unsigned long long im = __ballot(in);
-            any_self = any_self || im != 0;
-            for (unsigned long long mm = im; mm; mm &= mm - 1) self = self + readlane_f64(wt, __builtin_ctzll(mm));
+            if (im) {
+                any_self = true;
+                const int cnt = __popcll(im);
+                if (in) own[w][__popcll(im & below)] = wt;
+                if (lane < 8) own[w][cnt + lane] = -0.0;
+                wave_lds_sync();
+                for (int k = 0; k < cnt; k += 8) {
+                    double y[8];
+#pragma unroll
+                    for (int u = 0; u < 8; u++) y[u] = own[w][k + u];
+#pragma unroll
+                    for (int u = 0; u < 8; u++) self = self + y[u];
+                }
+            }
             int slot = 0;
             bool fresh = false;
             if (ext) {
