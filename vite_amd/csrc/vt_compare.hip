@@ -5,9 +5,8 @@
 // also puts them together (same-same) or not (same-diff), and for every pair inside one
 // community of C2 whether C1 separates them (diff-same), by walking all pairs: O(sum of
 // squared community sizes).  The counts are integers, so any order gives the same values:
-// here every vertex adds, with one atomic increment each, the number of vertices before it
-// that share its C1 community, its C2 community, and its (C1, C2) pair, which sums to
-// C(n,2) over each group.  The pair groups live in an open-addressed HBM table of 64-bit
+// here every vertex adds one, with an atomic increment, to its (C1, C2) pair, the pairs add their
+// counts to the sizes of C1 and C2, and C(k, 2) is summed over each group.  The pair groups live in an open-addressed HBM table of 64-bit
 // keys (C1 * nC2 + C2) at most half full.  Then
 //   same-same = sum over (a,b) of C(n_ab, 2),
 //   same-diff = sum over a of C(n_a, 2) - same-same,
@@ -16,6 +15,7 @@
 // (a left fold over the sorted community sizes, zero-size ids included) are formed on the
 // host with the reference's expressions and order.
 #include <hip/hip_runtime.h>
+#include <rocprim/device/device_radix_sort.hpp>
 
 #include <algorithm>
 #include <cstring>
@@ -60,54 +60,74 @@ __global__ void __launch_bounds__(kCmpBlock) k_cmp_range(const int64_t* __restri
     if (threadIdx.x < 4) part[4 * blockIdx.x + threadIdx.x] = s[threadIdx.x][0];
 }
 
-__global__ void k_cmp_fill(unsigned long long* __restrict__ p, int64_t n, unsigned long long v)
+// A pair of communities and its vertices, in one line of memory.
+struct __align__(16) PairSlot {
+    unsigned long long key, cnt;
+};
+
+__global__ void k_cmp_clear(PairSlot* __restrict__ t, int64_t n)
 {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        p[i] = v;
+        t[i] = PairSlot{kEmptyKey, 0};
 }
 
-// Every vertex: increments of its C1 size, its C2 size and its (C1, C2) pair count; the
-// old values summed give the three pair totals (sums[0..2]).
+// Every vertex: its (C1, C2) pair's count.  Bound by the memory's atomics, so a pair that is there
+// already is found with a load, and the communities' sizes are left to the pairs, fewer than the
+// vertices where the partitions resemble each other (three increments and an exchange per vertex
+// took 220 us for n = 1000003 with 180 K pairs, this and k_cmp_sizes 121).
 __global__ void __launch_bounds__(kCmpBlock) k_cmp_count(const int64_t* __restrict__ c1, const int64_t* __restrict__ c2,
-                                                         int64_t n, uint64_t nc2, unsigned long long* __restrict__ size1,
-                                                         unsigned long long* __restrict__ size2,
-                                                         unsigned long long* __restrict__ keys,
-                                                         unsigned long long* __restrict__ cnt, int logcap,
-                                                         unsigned long long* __restrict__ sums)
+                                                         int64_t n, uint64_t nc2, PairSlot* __restrict__ pairs, int logcap)
 {
-    __shared__ unsigned long long s[3][kCmpBlock];
-    unsigned long long p1 = 0, p2 = 0, p12 = 0;
     const unsigned long long mask = (1ull << logcap) - 1;
     for (int64_t i = blockIdx.x * (int64_t)kCmpBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kCmpBlock) {
-        const uint64_t a = (uint64_t)c1[i], b = (uint64_t)c2[i];
-        p1 += atomicAdd(&size1[a], 1ull);
-        p2 += atomicAdd(&size2[b], 1ull);
-        const unsigned long long key = a * nc2 + b;
+        const unsigned long long key = (uint64_t)c1[i] * nc2 + (uint64_t)c2[i];
         unsigned long long h = (key * 0x9E3779B97F4A7C15ull) >> (64 - logcap);
         for (;;) {  // ends: at most n distinct keys in a table of at least 2n slots
-            const unsigned long long old = atomicCAS(&keys[h], kEmptyKey, key);
+            unsigned long long old = __hip_atomic_load(&pairs[h].key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (old == kEmptyKey) old = atomicCAS(&pairs[h].key, kEmptyKey, key);
             if (old == kEmptyKey || old == key) break;
             h = (h + 1) & mask;
         }
-        p12 += atomicAdd(&cnt[h], 1ull);
+        atomicAdd(&pairs[h].cnt, 1ull);
     }
-    s[0][threadIdx.x] = p1;
-    s[1][threadIdx.x] = p2;
-    s[2][threadIdx.x] = p12;
+}
+
+// The communities' sizes from the pairs' counts, and *same += C(count, 2) over the pairs.
+__global__ void __launch_bounds__(kCmpBlock) k_cmp_sizes(const PairSlot* __restrict__ pairs, int64_t cap, uint64_t nc2,
+                                                         unsigned long long* __restrict__ size1,
+                                                         unsigned long long* __restrict__ size2,
+                                                         unsigned long long* __restrict__ same)
+{
+    unsigned long long p = 0;
+    for (int64_t i = blockIdx.x * (int64_t)kCmpBlock + threadIdx.x; i < cap; i += (int64_t)gridDim.x * kCmpBlock) {
+        const PairSlot x = pairs[i];
+        if (x.key == kEmptyKey) continue;
+        atomicAdd(&size1[x.key / nc2], x.cnt);
+        atomicAdd(&size2[x.key % nc2], x.cnt);
+        p += x.cnt * (x.cnt - 1) / 2;
+    }
+    __shared__ unsigned long long s;
+    if (threadIdx.x == 0) s = 0;
     __syncthreads();
-    for (int o = kCmpBlock / 2; o > 0; o >>= 1) {
-        if (threadIdx.x < o)
-            for (int k = 0; k < 3; k++) s[k][threadIdx.x] += s[k][threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x < 3) atomicAdd(&sums[threadIdx.x], s[threadIdx.x][0]);
+    for (int o = 32; o > 0; o >>= 1) p += __shfl_xor(p, o);
+    if ((threadIdx.x & 63) == 0 && p) atomicAdd(&s, p);
+    __syncthreads();
+    if (threadIdx.x == 0 && s) atomicAdd(same, s);
+}
+
+// The pairs of vertices inside communities of these sizes.
+uint64_t pairs_inside(const uint64_t* size, int64_t n)
+{
+    uint64_t p = 0;
+    for (int64_t i = 0; i < n; i++) p += size[i] * (size[i] - 1) / 2;
+    return p;
 }
 
 // compute_gini_coeff (compare.cpp:310-337) on sizes already sorted ascending: the one-thread
 // left folds of (i+1)*size[i] and size[i], then the reference's closing expression.
-double gini_sorted(const std::vector<uint64_t>& sorted)
+double gini_sorted(const uint64_t* sorted, int64_t n)
 {
-    const int numColors = (int)sorted.size();
+    const int numColors = (int)n;
     double numFunc = 0.0, denFunc = 0.0;
     for (int64_t i = 0; i < numColors; i++) {
         numFunc = numFunc + (double)((i + 1) * (int64_t)sorted[i]);
@@ -116,16 +136,12 @@ double gini_sorted(const std::vector<uint64_t>& sorted)
     return ((2 * numFunc) / (numColors * denFunc)) - ((double)(numColors + 1) / (double)numColors);
 }
 
-// Community sizes sorted ascending on the device, then read back.
-std::vector<uint64_t> sorted_sizes(vt_ctx* ctx, unsigned long long* d_size, int64_t nc, int64_t n)
+// Both partitions' community sizes, each sorted ascending, in one sort: C2's carry the bit above
+// the sizes.
+__global__ void k_cmp_mark(unsigned long long* __restrict__ size, int64_t n, unsigned long long bit)
 {
-    std::vector<uint64_t> h((size_t)nc);
-    DBuf<uint64_t> kalt(ctx, (size_t)nc);
-    DBuf<uint32_t> v(ctx, (size_t)nc), valt(ctx, (size_t)nc);
-    bool alt = false;
-    sort_pairs_u64(ctx, (uint64_t*)d_size, v.p, nc, (int)bits_for(n), kalt.p, valt.p, &alt);
-    d2h(ctx, h.data(), alt ? (const void*)kalt.p : (const void*)d_size, 8 * (size_t)nc);
-    return h;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+        size[i] |= bit;
 }
 
 }  // namespace
@@ -170,35 +186,45 @@ extern "C" int vt_compare_communities(vt_ctx* ctx, int64_t n, const int64_t* tru
         int logcap = 1;
         while ((1ll << logcap) < 2 * n) logcap++;
         const int64_t cap = 1ll << logcap;
-        DBuf<unsigned long long> size1(ctx, (size_t)nc1), size2(ctx, (size_t)nc2), keys(ctx, (size_t)cap),
-            cnt(ctx, (size_t)cap), sums(ctx, 3);
-        dzero(ctx, size1.p, 8 * (size_t)nc1);
-        dzero(ctx, size2.p, 8 * (size_t)nc2);
-        dzero(ctx, cnt.p, 8 * (size_t)cap);
-        dzero(ctx, sums.p, 24);
-        VT_LAUNCH(ctx, "cmp_fill", k_cmp_fill, grid_for(cap, 256, 8192), 256, 0, keys.p, cap, kEmptyKey);
+        const int64_t nc = nc1 + nc2;
+        // [0, nc1) the sizes of C1, then those of C2, then the pairs that both put together
+        DBuf<unsigned long long> size(ctx, (size_t)nc + 1);
+        DBuf<PairSlot> pairs(ctx, (size_t)cap);
+        unsigned long long *size1 = size.p, *size2 = size.p + nc1, *same = size.p + nc;
+        dzero(ctx, size.p, 8 * (size_t)(nc + 1));
+        VT_LAUNCH(ctx, "cmp_clear", k_cmp_clear, grid_for(cap, 256, 8192), 256, 0, pairs.p, cap);
         VT_LAUNCH(ctx, "cmp_count", k_cmp_count, grid_for(n, kCmpBlock, 8192), kCmpBlock, 0, (const int64_t*)c1.p,
-                  (const int64_t*)c2.p, n, (uint64_t)nc2, size1.p, size2.p, keys.p, cnt.p, logcap, sums.p);
-        unsigned long long s[3];
-        d2h(ctx, s, sums.p, sizeof(s));
-        const std::vector<uint64_t> z1 = sorted_sizes(ctx, size1.p, nc1, n);
-        const std::vector<uint64_t> z2 = sorted_sizes(ctx, size2.p, nc2, n);
-        sync(ctx);
+                  (const int64_t*)c2.p, n, (uint64_t)nc2, pairs.p, logcap);
+        VT_LAUNCH(ctx, "cmp_sizes", k_cmp_sizes, grid_for(cap, kCmpBlock, 2048), kCmpBlock, 0, (const PairSlot*)pairs.p, cap,
+                  (uint64_t)nc2, size1, size2, same);
+        const int bits = (int)bits_for(n);
+        VT_LAUNCH(ctx, "cmp_mark", k_cmp_mark, grid_for(nc2, 256, 8192), 256, 0, size2, nc2, 1ull << bits);
+        DBuf<unsigned long long> alt(ctx, (size_t)nc);
+        rocprim::double_buffer<unsigned long long> kb(size.p, alt.p);
+        size_t tb = 0;
+        VT_HIP(ctx, rocprim::radix_sort_keys(nullptr, tb, kb, (size_t)nc, 0, bits + 1, ctx->stream));
+        void* tmp = scratch(ctx, "sort_tmp", tb);
+        VT_HIP(ctx, rocprim::radix_sort_keys(tmp, tb, kb, (size_t)nc, 0, bits + 1, ctx->stream));
+        if (kb.current() != size.p) d2d(ctx, size.p, kb.current(), 8 * (size_t)nc);
+        std::vector<uint64_t> z((size_t)nc + 1);
+        d2h(ctx, z.data(), size.p, 8 * z.size());
+        for (int64_t i = nc1; i < nc; i++) z[i] -= 1ull << bits;
+        const uint64_t ss = z[(size_t)nc], p1 = pairs_inside(z.data(), nc1), p2 = pairs_inside(z.data() + nc1, nc2);
 
         vt_compare_stats r;
         std::memset(&r, 0, sizeof(r));
         r.n = n;
         r.nc_truth = nc1;
         r.nc_found = nc2;
-        r.same_same = (int64_t)s[2];
-        r.same_diff = (int64_t)(s[0] - s[2]);
-        r.diff_same = (int64_t)(s[1] - s[2]);
+        r.same_same = (int64_t)ss;
+        r.same_diff = (int64_t)(p1 - ss);
+        r.diff_same = (int64_t)(p2 - ss);
         // compare.cpp:267-272, term by term
         r.precision = (double)r.same_same / (double)(r.same_same + r.diff_same);
         r.recall = (double)r.same_same / (double)(r.same_same + r.same_diff);
         r.f_score = 2.0 * ((r.precision * r.recall) / (r.precision + r.recall));
-        r.gini_truth = gini_sorted(z1);
-        r.gini_found = gini_sorted(z2);
+        r.gini_truth = gini_sorted(z.data(), nc1);
+        r.gini_found = gini_sorted(z.data() + nc1, nc2);
         *out = r;
     });
 }
