@@ -12,7 +12,8 @@
 
 namespace vt {
 
-double run_phase(vt_ctx* ctx, vt_graph* g, const vt_phase_params* p, int64_t* cvect_out, int32_t* iters_out);
+double run_phase(vt_ctx* ctx, vt_graph* g, const vt_phase_params* p, int64_t* cvect_out, int32_t* iters_out,
+                 const int64_t* d_colors);
 int64_t color_graph(vt_ctx* ctx, const vt_graph* g, int64_t nHash, int target_percent, bool single, int64_t* d_colors);
 
 static double now_s()
@@ -65,22 +66,19 @@ void run_loop(vt_ctx* ctx, const vt_graph* g0, const vt_run_params* rp, vt_run_r
             pp.et_type = rp->et_type;
             pp.et_delta = rp->et_delta;
             pp.flags = rp->flags;
-            std::vector<int64_t> colors;
+            DBuf<int64_t> colors;  // they stay on the device
             const double t1 = now_s();
             if ((rp->coloring || rp->vertex_order) && phase == 0) {
-                DBuf<int64_t> dc(ctx, (size_t)std::max<int64_t>(dg->nv, 1));
-                const int64_t numColors = color_graph(ctx, dg, rp->max_colors / 2, 70, rp->single_color_iter != 0, dc.p);
-                colors.resize(dg->nv);
-                d2h(ctx, colors.data(), dc.p, 8 * (size_t)dg->nv);
+                colors = DBuf<int64_t>(ctx, (size_t)std::max<int64_t>(dg->nv, 1));
+                const int64_t numColors = color_graph(ctx, dg, rp->max_colors / 2, 70, rp->single_color_iter != 0, colors.p);
                 res->num_colors = numColors;
                 pp.mode = rp->coloring ? VT_MODE_COLOR : VT_MODE_VORDER;
                 pp.num_color = numColors + 1;
-                pp.colors = colors.data();
             }
             const int lvl = std::min(res->nlevels, VT_MAX_LEVELS - 1);
             res->level_nv[lvl] = dg->nv;
             res->level_ne[lvl] = dg->ne;
-            currMod = run_phase(ctx, dg, &pp, nullptr, &iters);
+            currMod = run_phase(ctx, dg, &pp, nullptr, &iters, colors.p);
             if (res->ncalls <= VT_MAX_LEVELS) {
                 res->call_q[res->ncalls] = currMod;
                 res->call_iters[res->ncalls] = iters;
@@ -106,7 +104,7 @@ void run_loop(vt_ctx* ctx, const vt_graph* g0, const vt_run_params* rp, vt_run_r
                     pp.thresh = 1.0E-6;
                     pp.flags = rp->flags;
                     const double tx = now_s();
-                    currMod = run_phase(ctx, dg, &pp, nullptr, &iters);
+                    currMod = run_phase(ctx, dg, &pp, nullptr, &iters, nullptr);
                     ctime += now_s() - tx;
                     if (res->ncalls <= VT_MAX_LEVELS) {
                         res->call_q[res->ncalls] = currMod;

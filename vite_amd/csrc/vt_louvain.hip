@@ -4100,7 +4100,8 @@ struct vt_phase {
 
 namespace vt {
 
-vt_phase* phase_begin(vt_ctx* ctx, vt_graph* g, const vt_phase_params* p)
+// d_colors (or null): the colors in device memory, known to be in range, instead of p->colors.
+vt_phase* phase_begin(vt_ctx* ctx, vt_graph* g, const vt_phase_params* p, const int64_t* d_colors = nullptr)
 {
     int mode = p->mode, et = p->et_type;
     if (mode < 0 || mode > 2) fail(ctx, VT_ERR_ARG, "vt_louvain_phase: bad mode %d", mode);
@@ -4108,7 +4109,7 @@ vt_phase* phase_begin(vt_ctx* ctx, vt_graph* g, const vt_phase_params* p)
     if (mode != VT_MODE_PLAIN) {
         if (p->num_color < 1) fail(ctx, VT_ERR_ARG, "vt_louvain_phase: num_color must be >= 1");
         if (p->num_color == 1) { mode = VT_MODE_PLAIN; et = 0; }  // louvain.cpp:601-605
-        else if (!p->colors) fail(ctx, VT_ERR_ARG, "vt_louvain_phase: colors required for mode %d", mode);
+        else if (!p->colors && !d_colors) fail(ctx, VT_ERR_ARG, "vt_louvain_phase: colors required for mode %d", mode);
     }
     const int64_t nv = g->nv;
     vt_phase* st = new vt_phase(ctx, g);
@@ -4129,16 +4130,17 @@ vt_phase* phase_begin(vt_ctx* ctx, vt_graph* g, const vt_phase_params* p)
             return st;
         }
         ph.init(p->flags);
-        if (mode != VT_MODE_PLAIN) {
+        if (mode != VT_MODE_PLAIN && !d_colors) {
             for (int64_t i = 0; i < nv; i++)
                 if (p->colors[i] > p->num_color - 1 || p->colors[i] < -1)
                     fail(ctx, VT_ERR_ARG, "vt_louvain_phase: color %lld of vertex %lld outside [-1, num_color-1]",
                          (long long)p->colors[i], (long long)i);
             st->dcolors = DBuf<int64_t>(ctx, (size_t)std::max<int64_t>(nv, 1));
             h2d(ctx, st->dcolors.p, p->colors, 8 * (size_t)nv);
+            d_colors = st->dcolors.p;
         }
         // Sweep lists per color for COLOR; one Jacobi sweep (event order = colorIndex) for VORDER.
-        ph.build_lists(mode != VT_MODE_PLAIN ? st->dcolors.p : nullptr, p->num_color, mode == VT_MODE_VORDER);
+        ph.build_lists(mode != VT_MODE_PLAIN ? d_colors : nullptr, p->num_color, mode == VT_MODE_VORDER);
         ph.whole = nv && mail(ctx)[2] == 1.0;  // k_constant's, there since build_lists read the lists' sizes
     } catch (...) {
         delete st;
@@ -4218,9 +4220,10 @@ double phase_end(vt_ctx* ctx, vt_phase* st, int64_t* cvect_out, int32_t* iters_o
     return st->prevMod;
 }
 
-double run_phase(vt_ctx* ctx, vt_graph* g, const vt_phase_params* p, int64_t* cvect_out, int32_t* iters_out)
+double run_phase(vt_ctx* ctx, vt_graph* g, const vt_phase_params* p, int64_t* cvect_out, int32_t* iters_out,
+                 const int64_t* d_colors)
 {
-    vt_phase* st = phase_begin(ctx, g, p);
+    vt_phase* st = phase_begin(ctx, g, p, d_colors);
     try {
         while (!st->done) phase_step(ctx, st);
         const double q = phase_end(ctx, st, cvect_out, iters_out);
@@ -4520,7 +4523,7 @@ int vt_louvain_phase(vt_ctx* ctx, vt_graph* g, const vt_phase_params* p, int64_t
     return guarded(ctx, [&] {
         VT_HIP(ctx, hipSetDevice(ctx->device));
         int32_t it = 0;
-        const double q = run_phase(ctx, g, p, cvect_out, &it);
+        const double q = run_phase(ctx, g, p, cvect_out, &it, nullptr);
         sync(ctx);
         if (iters_out) *iters_out = it;
         if (q_out) *q_out = q;
