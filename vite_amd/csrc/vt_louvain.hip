@@ -69,7 +69,7 @@ constexpr int kHubLdsBucket = 7;
 constexpr int kHubLdsMin = 512, kHubLdsMax = 4096;
 
 // Bucket of a row of degree d under per-bucket maximum degrees mx[0..5] (the tuning; the
-// default is 7, 15, 31, 63, 127, 1023): rows above mx[5] take the HBM-table kernel.
+// default is 7, 15, 47, 63, 191, 511): rows above mx[5] are hubs.
 struct BucketBounds {
     int32_t mx[6];
     int32_t wide[2];  // rows of bucket 5 up to wide[0] take the 512-slot table, up to wide[1] the 1024-slot one
