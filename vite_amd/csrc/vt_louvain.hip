@@ -2143,12 +2143,6 @@ __global__ void k_add_i64(int64_t* __restrict__ acc, const int64_t* __restrict__
     if (threadIdx.x == 0 && blockIdx.x == 0) *acc += *x;
 }
 
-__global__ void k_scan_total(const int32_t* __restrict__ flags, const int32_t* __restrict__ pos, int64_t n,
-                             int64_t* __restrict__ total)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0) total[0] = n ? (int64_t)pos[n - 1] + flags[n - 1] : 0;
-}
-
 __global__ void k_emit_events(const int32_t* __restrict__ order, int64_t n, const int32_t* __restrict__ flags,
                               const int32_t* __restrict__ pos, const int32_t* __restrict__ target,
                               const int32_t* __restrict__ curr, uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
