@@ -147,7 +147,7 @@ __global__ void k_dsort_sizes(const int64_t* __restrict__ d_count, int64_t mult,
                               int64_t* __restrict__ sizes)
 {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
-        const int64_t n = *d_count * mult;
+        const int64_t n = d_count ? *d_count * mult : mult;
         const int64_t nt = ceil_div(n, kTile);
         const int64_t per = ceil_div(nt, grid);
         const int64_t nb = per ? ceil_div(nt, per) : 0;
