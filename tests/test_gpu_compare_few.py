@@ -54,3 +54,20 @@ def test_counting_time_with_few_communities(ctx):
         us[k] = 1e3 * best
     # one atomic per vertex on four lines of memory took 25 times as long as on a thousand communities'
     assert us[2] < 4 * us[1024], us
+
+
+@pytest.mark.parametrize("n", [70001, 300007])
+def test_singletons(ctx, n):
+    """As many communities as vertices: the sizes' host loop at its longest."""
+    rng = np.random.default_rng(n)
+    ids, half = rng.permutation(n), np.arange(n) // 2
+    for a, b in ((ids, ids), (ids, half), (half, ids)):
+        s = ctx.compare_communities(a, b)
+        pairs = {True: n // 2, False: 0}
+        assert s["same_same"] == 0
+        assert (s["same_diff"], s["diff_same"]) == (pairs[a is half], pairs[b is half])
+        for part, gini in ((a, s["gini_truth"]), (b, s["gini_found"])):
+            size = np.sort(np.bincount(part)).astype(float)
+            k = len(size)
+            num = float(((np.arange(k) + 1) * size).sum())  # whole numbers below 2^53
+            assert gini == (2 * num) / (k * size.sum()) - (k + 1.0) / k
