@@ -1811,6 +1811,8 @@ __global__ void __launch_bounds__(256) k_hubw_insert(MoveArgs a, HubWhole h)
     }
 }
 
+constexpr int kHubwHubs = 4096;  // hubs of a sweep, at most
+
 // Gains (louvain.cpp:2246-2273) in place of the sums, but for the hubs' own communities.
 __global__ void k_hubw_gain(MoveArgs a, HubWhole h)
 {
@@ -2063,11 +2065,28 @@ __global__ void k_constant(const double* __restrict__ sums, const unsigned long 
     }
 }
 
+// Whether a sweep's `hubs`, all longer than kHubLdsMax, take k_hubw_* (`whole`: their weights allow
+// it).  What it saves is the sort of the LDS rows beside them, so there have to be several times as
+// many: with 8 to 30 beside each, 4 hubs of 10000 entries took a sweep 109-145 us and sorted with
+// the others 132-151 (BA n = 300007: 198 and 263), but without any 16 hubs of 10000 took 252 us and
+// sorted 162, 6000 of 5500 12 ms and sorted 1.4.
+__device__ __host__ __forceinline__ bool hub_whole_used(int64_t hubs, int64_t lds, bool whole)
+{
+    return whole && hubs > 0 && hubs <= kHubwHubs && 8 * hubs <= lds;
+}
+
+// Nor where those hubs have many entries and none much of them: an entry costs the table two random
+// atomics, until the vertices move to few communities, as a giant row's do.
+__device__ __host__ __forceinline__ bool hub_whole_pays(int64_t entries, int64_t max_degree)
+{
+    return entries <= (1 << 20) || 16 * max_degree >= entries;
+}
+
 // Whether a sweep's `lds` rows take k_hub_lds: not too many, and no sorted path beside them (which
 // costs its launches however few rows it has).
 __device__ __host__ __forceinline__ bool hub_lds_used(int64_t hubs, int64_t lds, int64_t limit, bool whole)
 {
-    return lds <= limit && (hubs == 0 || whole || limit == INT32_MAX);
+    return lds <= limit && (hubs == 0 || hub_whole_used(hubs, lds, whole) || limit == INT32_MAX);
 }
 
 // A row's sweep list: its degree bucket, the wide bucket split by table size.
@@ -2941,7 +2960,8 @@ struct SetupArgs {
     const double* vdeg;
     int32_t nv, blocks;
     int64_t chunk;
-    double *cdeg, *sums, *constant, *out;  // out (pinned): [2] whole degrees, [16, 27) the buckets' sizes, [28] hub entries
+    double *cdeg, *sums, *constant, *out;  // out (pinned): [2] whole degrees, [16, 27) the buckets' sizes, [27] the
+    // LDS rows take k_hub_lds, [28] hub entries
     int32_t *csize, *past, *curr, *target, *lists;
     unsigned char* active;  // null when ET is off, with the three below
     double *frozen, *pa, *pb;
@@ -2950,7 +2970,7 @@ struct SetupArgs {
     int64_t* hoffs;               // nv + 1
     BucketBounds bb;
     int32_t lpv_max;
-    int64_t hub_limit;                       // hub_lds_limit()
+    int64_t hub_limit, max_degree;           // hub_lds_limit(), the graph's
     const unsigned long long* hub_fraction;  // row_degrees' (or null: no long hub rows)
     unsigned long long seq;                  // posted with out
 };
@@ -3027,23 +3047,29 @@ __global__ void __launch_bounds__(kTailBlock) k_setup_small(SetupArgs a)
     __syncthreads();
     unsigned long long entries = 0;
     const bool whole = a.hub_fraction && *a.hub_fraction == 0;
-    const int nh = s_total[kHubBucket] +
-                   (hub_lds_used(s_total[kHubBucket], s_total[kHubLdsBucket], a.hub_limit, whole) ? 0 : s_total[kHubLdsBucket]);
-    for (int j0 = 0; j0 < nh; j0 += kTailBlock) {
-        const int j = j0 + t;
-        const int32_t v = j < nh ? a.lists[hub_off + j] : 0;
-        unsigned long long sum = 0;
-        const unsigned long long x = j < nh ? (unsigned long long)(a.offs[v + 1] - a.offs[v]) : 0;
-        const unsigned long long at = entries + block_scan<kTailBlock>(x, s_scan, &sum);
-        if (j < nh) a.hoffs[j] = (int64_t)at;
-        entries += sum;
-    }
+    auto scan_hubs = [&](int from, int to) {  // the offsets of the hub rows [from, to)
+        for (int j0 = from; j0 < to; j0 += kTailBlock) {
+            const int j = j0 + t;
+            const int32_t v = j < to ? a.lists[hub_off + j] : 0;
+            unsigned long long sum = 0;
+            const unsigned long long x = j < to ? (unsigned long long)(a.offs[v + 1] - a.offs[v]) : 0;
+            const unsigned long long at = entries + block_scan<kTailBlock>(x, s_scan, &sum);
+            if (j < to) a.hoffs[j] = (int64_t)at;
+            entries += sum;
+        }
+    };
+    const int hubs = s_total[kHubBucket], in_lds = s_total[kHubLdsBucket];
+    scan_hubs(0, hubs);
+    const bool apart = hub_lds_used(hubs, in_lds, a.hub_limit, whole) && (hubs == 0 || hub_whole_pays((int64_t)entries, a.max_degree));
+    const int nh = apart ? hubs : hubs + in_lds;  // the LDS rows follow the hubs in the lists
+    scan_hubs(hubs, nh);
     double r[2];
     small_tree_sum2<kTailBlock>(a.vdeg, nullptr, a.nv, a.blocks, a.chunk, lds, s_part, r);
     int64_t* out = (int64_t*)a.out;
     if (t == 0) {
         for (int q = 0; q < kNumBuckets; q++) out[16 + q] = s_total[q];
         a.hoffs[nh] = (int64_t)entries;
+        out[27] = apart;
         out[28] = (int64_t)entries;
         a.out[15] = whole ? 1.0 : 0.0;
         a.sums[0] = r[0];
@@ -3548,6 +3574,7 @@ struct Phase {
         a.bb = bounds();
         a.lpv_max = lpv_max_degree();
         a.hub_limit = hub_lds_limit();
+        a.max_degree = g->max_degree;
         a.hub_fraction = hub_fraction;
         a.seq = ++ctx->mail_seq;
         VT_LAUNCH(ctx, "setup", k_setup_small, 1, kTailBlock, 0, a);
@@ -3555,6 +3582,7 @@ struct Phase {
         const int64_t* h = (const int64_t*)mail(ctx);
         hub_whole = hub_exact = mail(ctx)[15] == 1.0;
         plan_sweeps(1, h + 16);
+        if (!h[27]) sort_all_hubs(sweeps[0]);
         hub_total.assign(1, h[28]);
         hub_sort = true;
     }
@@ -3598,14 +3626,20 @@ struct Phase {
         hub_total.assign(ncol, 0);
         if (hub_sort) {
             for (int64_t c = 0; c < ncol; c++) {
-                const ColorSweep& cs = sweeps[c];
-                hub_offs.emplace_back(ctx, (size_t)cs.hub_n + 1);
+                ColorSweep& cs = sweeps[c];
+                hub_offs.emplace_back(ctx, (size_t)(cs.hub_n + cs.hubl_n) + 1);
+                auto scan_hubs = [&] {
+                    DBuf<int64_t> deg(ctx, (size_t)cs.hub_n + 1);
+                    VT_LAUNCH(ctx, "hub_degrees", k_hub_degrees, grid_for(cs.hub_n + 1, 256, 1024), 256, 0,
+                              (const int32_t*)(lists.p + cs.hub_off), (int32_t)cs.hub_n, (const int64_t*)g->offs, deg.p);
+                    exclusive_scan_i64(ctx, deg.p, hub_offs.back().p, cs.hub_n + 1);
+                    d2h(ctx, &hub_total[c], hub_offs.back().p + cs.hub_n, 8);
+                };
                 if (!cs.hub_n) continue;
-                DBuf<int64_t> deg(ctx, (size_t)cs.hub_n + 1);
-                VT_LAUNCH(ctx, "hub_degrees", k_hub_degrees, grid_for(cs.hub_n + 1, 256, 1024), 256, 0,
-                          (const int32_t*)(lists.p + cs.hub_off), (int32_t)cs.hub_n, (const int64_t*)g->offs, deg.p);
-                exclusive_scan_i64(ctx, deg.p, hub_offs.back().p, cs.hub_n + 1);
-                d2h(ctx, &hub_total[c], hub_offs.back().p + cs.hub_n, 8);
+                scan_hubs();
+                if (!cs.whole || hub_whole_pays(hub_total[c], g->max_degree)) continue;
+                sort_all_hubs(cs);
+                scan_hubs();
             }
         }
         // Hub tables: one HBM table per resident wave, sized for the largest row.
@@ -3662,6 +3696,14 @@ struct Phase {
                g->max_degree > kHubLdsMax && g->ne < (int64_t(1) << 31);
     }
 
+    // A sweep's LDS rows join its hubs, which are sorted (k_hubw_* takes long rows only).
+    static void sort_all_hubs(ColorSweep& cs)
+    {
+        cs.hub_n += cs.hubl_n;
+        cs.hubl_n = 0;
+        cs.whole = false;
+    }
+
     // The launch plan of every sweep from its lists' sizes h[sweep * kNumBuckets + bucket]; returns
     // the largest number of hub rows in one.
     int64_t plan_sweeps(int64_t ncol, const int64_t* h)
@@ -3702,12 +3744,8 @@ struct Phase {
             }
             cs.plan.bbeg[kFusedBuckets] = blocks;
             cs.fused_blocks = blocks;
-            cs.whole = hub_whole;
-            if (cs.hubl_n && !hub_lds_used(cs.hub_n, cs.hubl_n, hub_lds_limit(), hub_whole)) {
-                cs.hub_n += cs.hubl_n;
-                cs.hubl_n = 0;
-                cs.whole = false;  // k_hubw_* takes long rows only
-            }
+            cs.whole = hub_whole_used(cs.hub_n, cs.hubl_n, hub_whole);
+            if (cs.hubl_n && !hub_lds_used(cs.hub_n, cs.hubl_n, hub_lds_limit(), hub_whole)) sort_all_hubs(cs);
             max_hub = std::max(max_hub, cs.hub_n);
         }
         for (int64_t c = 0; c < ncol; c++) sweeps[c].index = (int32_t)c;
