@@ -61,3 +61,21 @@ def test_phases(ctx):
         q_o, cv_o, it_o = po.louvain_phase(g, **kw)
         q, cv, it = dg.louvain_phase(sequential=True, **kw)
         assert (q, it) == (q_o, it_o) and np.array_equal(cv, cv_o), kw
+
+
+def test_gains_of_few_hubs_with_many_communities(ctx):
+    """Sixteen hubs with a community per entry: forming the gains may not take a multiple of the adding."""
+    g = _graph(20000, [10000] * 16, [560] * 128, 3)
+    dg = ctx.upload(vite_amd.CSR(g.offs, g.edges))
+    st = dg.phase_begin(thresh=-1.0)
+    best = {}
+    for _ in range(5):
+        ctx.set_profiling(True)
+        ctx.reset_stats()
+        st.sweep()
+        for k in ("hubw_insert", "hubw_gain"):
+            best[k] = min(best.get(k, np.inf), ctx.kernel_stats(k)[2])
+        ctx.set_profiling(False)
+    st.end(want_cvect=False)
+    # an atomic per wave and hub on one line of memory took 11 times as long
+    assert 0 < best["hubw_gain"] < 3 * best["hubw_insert"], best

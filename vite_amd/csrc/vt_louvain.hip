@@ -1811,14 +1811,21 @@ __global__ void __launch_bounds__(256) k_hubw_insert(MoveArgs a, HubWhole h)
     }
 }
 
-constexpr int kHubwHubs = 4096;  // hubs of a sweep, at most
+// Gains (louvain.cpp:2246-2273) in place of the sums, but for the hubs' own communities.  A
+// workgroup keeps the hubs' largest gains in LDS and ends with an atomic per hub: an atomic per wave and
+// hub, on a line of memory for sixteen hubs, took 299 us for 16 hubs of 10000 entries where the rest
+// of the sweep took 80.
+constexpr int kHubwHubs = 4096;  // 32 KB
+constexpr int kHubwGainBlock = 1024;
 
-// Gains (louvain.cpp:2246-2273) in place of the sums, but for the hubs' own communities.
-__global__ void k_hubw_gain(MoveArgs a, HubWhole h)
+__global__ void __launch_bounds__(kHubwGainBlock) k_hubw_gain(MoveArgs a, HubWhole h)
 {
+    __shared__ unsigned long long s_best[kHubwHubs];
+    for (int32_t j = threadIdx.x; j < h.nh; j += kHubwGainBlock) s_best[j] = 0;
+    __syncthreads();
     const double constant = *a.constant;
-    for (unsigned long long i = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x; i < h.cap;
-         i += (unsigned long long)gridDim.x * blockDim.x) {
+    for (unsigned long long i = blockIdx.x * (unsigned long long)kHubwGainBlock + threadIdx.x; i < h.cap;
+         i += (unsigned long long)gridDim.x * kHubwGainBlock) {
         const unsigned long long key = h.key[i];
         if (!key) continue;
         const int32_t j = (int32_t)((key - 1) >> 32), c = (int32_t)(uint32_t)(key - 1);
@@ -1842,25 +1849,12 @@ __global__ void k_hubw_gain(MoveArgs a, HubWhole h)
         const double ax = a.cdeg[cc] - kv;
         const double gain = 2.0 * (h.val[i] - eix) - 2.0 * kv * (a.cdeg[c] - ax) * constant;
         h.val[i] = gain;
-        // Most gains lose to one that is there already; of those that do not, the largest of each hub's
-        // lanes (four hubs at most, then each lane its own).
-        unsigned long long bits = gain > 0.0 ? (unsigned long long)__double_as_longlong(gain) : 0ull;
-        if (bits && bits <= __hip_atomic_load(&h.best[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) bits = 0;
-        for (int round = 0; round < 4 && bits; round++) {
-            if (j != __builtin_amdgcn_readfirstlane(j)) continue;
-            unsigned long long m = 0;
-            for (unsigned long long x = __ballot(1); x; x &= x - 1) {
-                const int l = __builtin_ctzll(x);
-                const unsigned long long o =
-                    ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(bits >> 32), l) << 32) |
-                    (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)bits, l);
-                m = o > m ? o : m;
-            }
-            if (bits == m) atomicMax(&h.best[j], m);
-            bits = 0;
-        }
-        if (bits) atomicMax(&h.best[j], bits);
+        const unsigned long long bits = gain > 0.0 ? (unsigned long long)__double_as_longlong(gain) : 0ull;
+        if (bits > __hip_atomic_load(&s_best[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) atomicMax(&s_best[j], bits);
     }
+    __syncthreads();
+    for (int32_t j = threadIdx.x; j < h.nh; j += kHubwGainBlock)
+        if (s_best[j]) atomicMax(&h.best[j], s_best[j]);
 }
 
 __global__ void k_hubw_pick(MoveArgs a, HubWhole h)
@@ -2067,9 +2061,9 @@ __global__ void k_constant(const double* __restrict__ sums, const unsigned long 
 
 // Whether a sweep's `hubs`, all longer than kHubLdsMax, take k_hubw_* (`whole`: their weights allow
 // it).  What it saves is the sort of the LDS rows beside them, so there have to be several times as
-// many: with 8 to 30 beside each, 4 hubs of 10000 entries took a sweep 109-145 us and sorted with
-// the others 132-151 (BA n = 300007: 198 and 263), but without any 16 hubs of 10000 took 252 us and
-// sorted 162, 6000 of 5500 12 ms and sorted 1.4.
+// many: a sweep with 4 hubs of 10000 entries and 8 to 30 LDS rows beside each took 54-66 us and
+// sorted with the others 134-142 (64 such hubs 157-213 and 188-258, BA n = 300007 183 and 263), but
+// 1000 hubs of 10000 alone 2.1 ms and sorted 1.0, 6000 of 5500 4 ms and sorted 0.4.
 __device__ __host__ __forceinline__ bool hub_whole_used(int64_t hubs, int64_t lds, bool whole)
 {
     return whole && hubs > 0 && hubs <= kHubwHubs && 8 * hubs <= lds;
@@ -3890,7 +3884,7 @@ struct Phase {
                           hw_best.p + hubs};
         TimedScope ts(ctx, "local_move_hub");
         VT_LAUNCH(ctx, "hubw_insert", k_hubw_insert, grid_for(total, kHubwChunk, 1 << 21), 256, 0, a, hw);
-        VT_LAUNCH(ctx, "hubw_gain", k_hubw_gain, grid_for(2 * total, 256, 8192), 256, 0, a, hw);
+        VT_LAUNCH(ctx, "hubw_gain", k_hubw_gain, grid_for(2 * total, kHubwGainBlock, 512), kHubwGainBlock, 0, a, hw);
         VT_LAUNCH(ctx, "hubw_pick", k_hubw_pick, grid_for(2 * total, 256, 8192), 256, 0, a, hw);
         VT_LAUNCH(ctx, "hubw_final", k_hubw_final, grid_for(cs.hub_n, 64, 4096), 64, 0, a, hw);
     }
