@@ -1225,17 +1225,33 @@ __device__ __forceinline__ double hub_run_fold(const double* __restrict__ wgt, c
     return acc;
 }
 
-// The runs of this many entries and more that a wave's lanes hold (`mine`), one after another by
-// the whole wave; every lane calls it, and a lane with `mine` gets its run's fold in ey.
+// The runs of this many entries and more that a wave's lanes hold (`mine`): one after another by the
+// whole wave, or, where they are many of about one length, by their lanes side by side.  A term takes
+// a lane some 480 cycles (two reads that wait for each other, four in flight) and a wave 33, of whole
+// numbers 19, so the lines lie at 12 and 24 times the longest run (16 hubs of 10000 entries in 10
+// communities: by waves 890 us, of whole numbers 501, by lanes 206).  Every lane calls it, and a lane with
+// `mine` gets its run's fold in ey.
 constexpr int32_t kHubLongRun = 256;
-// Runs of this many by a workgroup, where their launch has whole tiles of runs to a workgroup.
+// Runs of whole weights of this many by a workgroup, where their launch has whole tiles of runs
+// to a workgroup.
 constexpr int32_t kHubBlockRun = 8192;
 
 template <int R>
 __device__ __forceinline__ void hub_long_runs(const double* __restrict__ wgt, const uint32_t* __restrict__ vals, bool mine,
                                               int32_t b, int32_t e, double& ey)
 {
-    for (unsigned long long m = __ballot(mine); m; m &= m - 1) {
+    const unsigned long long runs = __ballot(mine);
+    if (!runs) return;
+    int32_t all = mine ? e - b : 0, longest = all;  // a sweep's hub entries are below 2^31
+    for (int o = 32; o > 0; o >>= 1) {
+        all += __shfl_xor(all, o);
+        longest = max(longest, __shfl_xor(longest, o));
+    }
+    if (all / (__ballot(mine && !whole_number(wgt[vals[b]])) ? 12 : 24) > longest) {
+        if (mine) ey = hub_run_fold(wgt, vals, b, e);
+        return;
+    }
+    for (unsigned long long m = runs; m; m &= m - 1) {
         const int l = __builtin_ctzll(m);
         const uint32_t* q = vals + __builtin_amdgcn_readlane(b, l);
         const int64_t n = __builtin_amdgcn_readlane(e, l) - __builtin_amdgcn_readlane(b, l);
@@ -1340,8 +1356,10 @@ __global__ void __launch_bounds__(kHubBlock) k_hub_own(MoveArgs a, const int32_t
 // Per run of another community: its counter (the run's weights folded left to right, the
 // first as is) and its gain (louvain.cpp:2246-2273); best[j] = the largest positive gain's
 // bits (non-negative doubles order as their bit patterns).
+// One term in flight per lane in a wave's folds: with four the kernel held 102 registers and 4 waves
+// per SIMD instead of 7, and 256 hubs of 40000 entries with a run each took 444 us instead of 400.
 template <class K>
-__global__ void __launch_bounds__(kHubBlock) k_hub_runs(MoveArgs a, const int32_t* __restrict__ hubs, int32_t nh, const int64_t* __restrict__ hoffs,
+__global__ void __launch_bounds__(kHubBlock, 7) k_hub_runs(MoveArgs a, const int32_t* __restrict__ hubs, int32_t nh, const int64_t* __restrict__ hoffs,
                            const K* __restrict__ keys, const uint32_t* __restrict__ vals, const int32_t* __restrict__ pos,
                            const int32_t* __restrict__ head, const int32_t* __restrict__ starts, int cbits,
                            const double* __restrict__ own, double* __restrict__ gains,
@@ -1371,9 +1389,9 @@ __global__ void __launch_bounds__(kHubBlock) k_hub_runs(MoveArgs a, const int32_
             other = !(a.active && !a.active[v]) && c != cc;
         }
         const int32_t len = e - b;
-        const bool big = other && len >= kHubBlockRun;
+        const bool big = other && len >= kHubBlockRun && whole_number(a.wgt[vals[b]]);
         if (other && len < kHubLongRun) ey = hub_run_fold(a.wgt, vals, b, e);
-        hub_long_runs<4>(a.wgt, vals, other && len >= kHubLongRun && !big, b, e, ey);
+        hub_long_runs<1>(a.wgt, vals, other && len >= kHubLongRun && !big, b, e, ey);
         if (__syncthreads_or(big)) {  // runs between a hub and a giant community: by the workgroup
             s_run[threadIdx.x] = big ? make_int2(b, e) : make_int2(0, 0);
             __syncthreads();
@@ -1382,8 +1400,8 @@ __global__ void __launch_bounds__(kHubBlock) k_hub_runs(MoveArgs a, const int32_
                 if (q.x == q.y) continue;
                 auto weight = [&](int64_t k) { return a.wgt[vals[q.x + k]]; };
                 double sum = 0.0;
-                if (!block_exact_sum<kHubBlock, 8>(q.y - q.x, weight, s_red, &sum) && threadIdx.x < 64)
-                    sum = wave_left_fold<4>(-0.0, q.y - q.x, weight);
+                if (!block_exact_sum<kHubBlock, 4>(q.y - q.x, weight, s_red, &sum) && threadIdx.x < 64)
+                    sum = wave_left_fold<1>(-0.0, q.y - q.x, weight);
                 if (threadIdx.x == 0) s_ey[t] = sum;
             }
             __syncthreads();
