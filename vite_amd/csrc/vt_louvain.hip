@@ -1985,11 +1985,11 @@ __global__ void __launch_bounds__(kFoldRows) k_row_fold(const int64_t* __restric
 }
 
 // The rows of long_min entries and more (hubs, the coarse levels), a wave each, and those of
-// kFoldBlockRow and more a workgroup each where their weights are whole numbers: a skewed
-// graph's giant coarse row (half a million entries) held the launch for 4.5 ms as one wave's
-// chain of lane reads on BA n = 2^22.  A workgroup's rows are gridDim apart, so that hubs
-// with neighbouring ids spread over the chip.  fraction (or null) is set where a row of
-// kFoldBlockRow entries and more is no such sum.
+// kFoldBlockRow and more that begin with whole weights a workgroup each: a skewed graph's giant
+// coarse row (half a million entries) held the launch for 4.5 ms as one wave's chain of lane reads
+// on BA n = 2^22.  A workgroup's rows are gridDim apart, so that hubs with neighbouring ids spread over
+// the chip.  fraction (or null) is set where a row of kFoldBlockRow entries and more is no sum of
+// whole numbers.
 constexpr int kFoldLongBlock = 256;
 constexpr int64_t kFoldBlockRow = kHubLdsMax + 1;
 __global__ void __launch_bounds__(kFoldLongBlock) k_row_fold_long(const int64_t* __restrict__ offs,
@@ -1997,26 +1997,36 @@ __global__ void __launch_bounds__(kFoldLongBlock) k_row_fold_long(const int64_t*
                                                                  double* __restrict__ vdeg, int64_t long_min,
                                                                  unsigned long long* __restrict__ fraction)
 {
-    __shared__ int32_t s_row[kFoldLongBlock];
-    __shared__ int32_t s_n, s_big;
+    __shared__ int32_t s_row[kFoldLongBlock], s_block[kFoldLongBlock];
+    __shared__ int32_t s_n, s_nblock;
     __shared__ double s_red[kFoldLongBlock / 64];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int64_t step = (int64_t)gridDim.x * kFoldLongBlock;
     for (int64_t base = 0; base < nv; base += step) {
-        if (threadIdx.x == 0) s_n = s_big = 0;
+        if (threadIdx.x == 0) s_n = s_nblock = 0;
         __syncthreads();
         const int64_t i = base + (int64_t)threadIdx.x * gridDim.x + blockIdx.x;
-        if (i < nv) {
-            const int64_t d = offs[i + 1] - offs[i];
-            if (d >= long_min) {  // the workgroup's rows from the list's end
-                if (d >= kFoldBlockRow) s_row[kFoldLongBlock - 1 - atomicAdd(&s_big, 1)] = (int32_t)i;
-                else s_row[atomicAdd(&s_n, 1)] = (int32_t)i;
+        if (i < nv && offs[i + 1] - offs[i] >= long_min) s_row[atomicAdd(&s_n, 1)] = (int32_t)i;
+        __syncthreads();
+        const int n = s_n;
+        for (int k = w; k < n; k += kFoldLongBlock / 64) {
+            const int64_t v = s_row[k];
+            const DEdge* e = edges + offs[v];
+            const int64_t d = offs[v + 1] - offs[v];
+            if (d >= kFoldBlockRow) {
+                if (__ballot(!whole_number(e[lane].weight)) == 0) {
+                    if (lane == 0) s_block[atomicAdd(&s_nblock, 1)] = (int32_t)v;
+                    continue;
+                }
+                if (lane == 0 && fraction) *fraction = 1;  // any wave's store
             }
+            const double sum = wave_left_fold<4>(0.0, d, [=](int64_t j) { return e[j].weight; });
+            if (lane == 0) vdeg[v] = sum;
         }
         __syncthreads();
-        const int n = s_n, nbig = s_big;
-        for (int k = 0; k < nbig; k++) {
-            const int64_t v = s_row[kFoldLongBlock - 1 - k];
+        const int nblock = s_nblock;
+        for (int k = 0; k < nblock; k++) {
+            const int64_t v = s_block[k];
             const DEdge* e = edges + offs[v];
             const int64_t d = offs[v + 1] - offs[v];
             auto weight = [=](int64_t j) { return e[j].weight; };
@@ -2027,17 +2037,11 @@ __global__ void __launch_bounds__(kFoldLongBlock) k_row_fold_long(const int64_t*
                 sum = wave_left_fold<4>(0.0, d, weight);
                 if (lane == 0) {
                     vdeg[v] = sum;
-                    if (fraction) *fraction = 1;  // any workgroup's store
+                    if (fraction) *fraction = 1;
                 }
             }
         }
-        for (int k = w; k < n; k += kFoldLongBlock / 64) {
-            const int64_t v = s_row[k];
-            const DEdge* e = edges + offs[v];
-            const double sum = wave_left_fold<4>(0.0, offs[v + 1] - offs[v], [=](int64_t j) { return e[j].weight; });
-            if (lane == 0) vdeg[v] = sum;
-        }
-        __syncthreads();  // the list is reused
+        __syncthreads();  // the lists are reused
     }
 }
 
@@ -3525,12 +3529,13 @@ struct Phase {
                       g->edges, nv, vdeg.p, (int64_t)0, hub_fraction);
         } else if (nv) {
             // a thread per row, and a wave per row for the rows of kFoldLongRow or more
-            const bool split = g->max_degree >= kFoldLongRow;
+            const int64_t min_len = kFoldLongRow;
+            const bool split = g->max_degree >= min_len;
             VT_LAUNCH(ctx, "row_fold", k_row_fold, grid_for(nv, kFoldRows, 16384), kFoldRows, 0, g->offs, g->edges, nv,
-                      vdeg.p, split ? kFoldLongRow : INT64_MAX);
+                      vdeg.p, split ? min_len : INT64_MAX);
             if (split)
-                VT_LAUNCH(ctx, "row_fold_long", k_row_fold_long, grid_for(nv, kFoldLongBlock, 4096), kFoldLongBlock, 0,
-                          g->offs, g->edges, nv, vdeg.p, kFoldLongRow, hub_fraction);
+                VT_LAUNCH(ctx, "row_fold_long", k_row_fold_long, grid_for(nv, kFoldLongBlock / 4, 8192), kFoldLongBlock, 0,
+                          g->offs, g->edges, nv, vdeg.p, min_len, hub_fraction);
         }
     }
 
