@@ -1962,7 +1962,7 @@ __global__ void k_hbm_table_init(int32_t* keys, double* vals, int64_t n)
 constexpr int kFoldRows = 256;
 // Rows at least this long get a wave each when a graph has them (a hub of degree 36 K
 // folded by one thread held the whole launch for 3 ms).
-constexpr int64_t kFoldLongRow = 512;
+constexpr int64_t kFoldLongRow = 512, kFoldLongMany = 2048;
 
 __global__ void __launch_bounds__(kFoldRows) k_row_fold(const int64_t* __restrict__ offs, const DEdge* __restrict__ edges,
                                                         int64_t nv, double* __restrict__ vdeg, int64_t long_min)
@@ -3528,8 +3528,10 @@ struct Phase {
             VT_LAUNCH(ctx, "row_fold", k_row_fold_long, grid_for(nv, kFoldLongBlock / 64, 65536), kFoldLongBlock, 0, g->offs,
                       g->edges, nv, vdeg.p, (int64_t)0, hub_fraction);
         } else if (nv) {
-            // a thread per row, and a wave per row for the rows of kFoldLongRow or more
-            const int64_t min_len = kFoldLongRow;
+            // A thread per row, and a wave per long row: from kFoldLongRow entries where those are few,
+            // from kFoldLongMany where the average row is long (70000 rows of 600 real weights by
+            // threads 279 us, by waves 377, which add one term at a time for 64 lanes).
+            const int64_t min_len = g->ne > 48 * nv ? kFoldLongMany : kFoldLongRow;
             const bool split = g->max_degree >= min_len;
             VT_LAUNCH(ctx, "row_fold", k_row_fold, grid_for(nv, kFoldRows, 16384), kFoldRows, 0, g->offs, g->edges, nv,
                       vdeg.p, split ? min_len : INT64_MAX);
