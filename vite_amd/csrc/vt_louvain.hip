@@ -2053,7 +2053,7 @@ __global__ void k_init(int64_t nv, const double* __restrict__ vdeg, double* __re
 {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nv; i += (int64_t)gridDim.x * blockDim.x) {
         const double d = vdeg[i];
-        if (!(whole_number(d) && d >= 0.0)) *fraction = 1;  // any thread's store
+        if (fraction && !(whole_number(d) && d >= 0.0)) *fraction = 1;  // any thread's store
         cdeg[i] = d;
         csize[i] = 1;
         past[i] = (int32_t)i;
@@ -2068,14 +2068,15 @@ __global__ void k_init(int64_t nv, const double* __restrict__ vdeg, double* __re
     }
 }
 
-// whole (pinned host memory): 1.0 where every degree is a whole number >= 0 and they total
-// less than 2^52.
+// whole (pinned host memory, or null where no moves follow): 1.0 where every degree is a whole
+// number >= 0 and they total less than 2^52.
 __global__ void k_constant(const double* __restrict__ sums, const unsigned long long* __restrict__ fraction,
                            const unsigned long long* __restrict__ hub_fraction, double* __restrict__ constant,
                            double* __restrict__ whole, double* __restrict__ hub_whole)
 {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
         constant[0] = 1.0 / sums[0];
+        if (!whole) return;
         *whole = *fraction == 0 && sums[0] < 0x1p52 ? 1.0 : 0.0;
         *hub_whole = hub_fraction && *hub_fraction == 0 ? 1.0 : 0.0;
     }
@@ -3509,10 +3510,10 @@ struct Phase {
         dzero(ctx, ucount.p, 48);
     }
 
-    void row_degrees()
+    void row_degrees(bool moves = true)
     {
         hub_fraction = nullptr;
-        if (hub_whole_possible()) {
+        if (moves && hub_whole_possible()) {
             hub_fraction = (unsigned long long*)scratch(ctx, "hub_fraction", 8);
             dzero(ctx, hub_fraction, 8);
         }
@@ -3541,23 +3542,24 @@ struct Phase {
         }
     }
 
-    void init_state(bool with_et)
+    // moves: a phase's, which counts its moves and asks whether the degrees are whole numbers.
+    void init_state(bool with_et, bool moves = true)
     {
-        clear_counters();
-        row_degrees();
+        if (moves) clear_counters();
+        row_degrees(moves);
         VT_LAUNCH(ctx, "init", k_init, grid_for(nv, 256, 8192), 256, 0, nv, (const double*)vdeg.p, cdeg.p, csize.p, past.p,
                   curr.p, target.p, with_et ? active.p : nullptr, with_et ? frozen.p : nullptr,
-                  with_et ? pa.p : nullptr, with_et ? pb.p : nullptr, ucount.p + 5);
+                  with_et ? pa.p : nullptr, with_et ? pb.p : nullptr, moves ? ucount.p + 5 : nullptr);
     }
 
-    void init(int flags)
+    void init(int flags, bool moves = true)
     {
-        init_state(et);
+        init_state(et, moves);
         if (flags & VT_FLAG_SEQUENTIAL_SUMS) seq_sum2(ctx, vdeg.p, nullptr, nv, sums());
         else tree_sum2(ctx, vdeg.p, nullptr, nv, sums());
         VT_LAUNCH(ctx, "constant", k_constant, 1, 64, 0, (const double*)sums(),
                   (const unsigned long long*)(ucount.p + 5), (const unsigned long long*)hub_fraction, constant(),
-                  mail(ctx) + 2, mail(ctx) + 15);
+                  moves ? mail(ctx) + 2 : nullptr, mail(ctx) + 15);
     }
 
     // alloc, init and build_lists of a plain phase on at most kTailVerts vertices (tree sums).
@@ -4865,7 +4867,7 @@ int vt_init_degrees(vt_ctx* ctx, const vt_graph* g, int32_t flags, double* vdeg_
         VT_HIP(ctx, hipSetDevice(ctx->device));
         Phase ph(ctx, g);
         ph.alloc(false);
-        ph.init(flags);
+        ph.init(flags, false);
         if (vdeg_out) d2h(ctx, vdeg_out, ph.vdeg.p, 8 * (size_t)g->nv);
         if (constant_out) d2h(ctx, constant_out, ph.constant(), 8);
         sync(ctx);
