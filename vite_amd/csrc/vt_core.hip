@@ -525,7 +525,15 @@ void exclusive_scan_i32(vt_ctx* ctx, const int32_t* in, int32_t* out, int64_t n)
                                         ctx->stream));
 }
 
+// Up to 2^20 pairs the library sorts blocks and merges them, two launches for every doubling; the
+// device sort takes one launch and three per 8 bits, whatever n.  The line lies where their times
+// cross, by the passes (us, library and device: 8 bits 13 and 22 at 4096 pairs, 24 and 22 at 5000, 120 and 25
+// at 2^20; 16 bits 37 and 46 at 65536, 48 and 47 at 131072; 20 bits 50 and 66 at 131072, 82 and 67 at 262144).
 constexpr int64_t kDevSortPairs = 1 << 20;
+static bool dev_sort_pays(int64_t n, int bits)
+{
+    return n <= kDevSortPairs && n > (bits <= 8 ? 4096 : bits <= 16 ? 65536 : 131072);
+}
 
 void sort_pairs_u32(vt_ctx* ctx, uint32_t* keys, uint32_t* vals, int64_t n, int bits, uint32_t* keys_alt,
                     uint32_t* vals_alt, bool* result_in_alt)
@@ -533,10 +541,7 @@ void sort_pairs_u32(vt_ctx* ctx, uint32_t* keys, uint32_t* vals, int64_t n, int 
     *result_in_alt = false;
     if (n <= 1) return;
     TimedScope ts(ctx, "sort_u32");
-    // Up to 2^20 pairs the library merges, two launches for every doubling from a few thousand pairs;
-    // the device sort takes one and three per 8 bits (300 RGGs of 256 to 4096 vertices in a
-    // batch 6.01 -> 5.64 ms, RGG n = 2^20 -i run 10.62 -> 10.39).
-    if (n <= kDevSortPairs) {
+    if (dev_sort_pays(n, bits)) {
         *result_in_alt = dev_sort_pairs_u32(ctx, keys, vals, keys_alt, vals_alt, nullptr, n, n, bits);
         return;
     }
