@@ -193,18 +193,27 @@ constexpr int kCfMaxKeys = 128;           // distinct keys a community may hold 
 constexpr int kCfList = kCfMaxKeys + 64;  // a chunk adds at most 64 keys before the check
 constexpr uint32_t kNoKey = 0xffffffffu;
 
-// Per community c (there are *n_comm): its coarse row staged at rkey/rval[s0, s0 + rowlen[c]),
+// A rebuild's device scalars: [0] communities, [1] ids out of range (small graphs), later [0] the
+// coarse entries, [1] the overflowing communities' entries, [2, 3] the largest of their rows and
+// communities, [4, 5] work items of the overflow (32 bits each).
+constexpr int kTotals = 6;
+
+// Per community c (there are tot[0]): its coarse row staged at rkey/rval[s0, s0 + rowlen[c]),
 // with s0 its offset in the concatenated rows; or, with more distinct keys than the table holds,
 // rowlen[c] = 0 and xcnt[c] = its entry count, for the sort path.  (A second pass over those
 // with a table of 512 or 1024 slots measured even with the sort on RGG n = 2^24: its 13 or 24 KB
 // of LDS per wave leave too few waves to hide a chunk's chain of LDS steps.)
 __global__ void __launch_bounds__(64 * kFoldWaves) k_comm_fold(
-    const int64_t* __restrict__ n_comm, const int64_t* __restrict__ cstart, const int64_t* __restrict__ moff,
+    int64_t* __restrict__ tot, const int64_t* __restrict__ cstart, const int64_t* __restrict__ moff,
     const int64_t* __restrict__ mrow, const DEdge* __restrict__ edges, const uint32_t* __restrict__ newid,
     uint32_t* __restrict__ rkey, double* __restrict__ rval, int64_t* __restrict__ rowlen, int64_t* __restrict__ xcnt)
 {
-    const int64_t nc = *n_comm;
+    const int64_t nc = tot[0];
     if ((int64_t)blockIdx.x * kFoldWaves >= nc) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        rowlen[nc] = xcnt[nc] = 0;  // the scans' last terms
+        for (int k = 2; k < kTotals; k++) tot[k] = 0;
+    }
     __shared__ uint32_t tk[kFoldWaves][kCfCap];
     __shared__ double tv[kFoldWaves][kCfCap];
     __shared__ unsigned long long tm[kFoldWaves][kCfCap];
@@ -534,11 +543,33 @@ __global__ void __launch_bounds__(256) k_row_copy_long(const uint32_t* __restric
     }
 }
 
-__global__ void k_pair_totals(const int64_t* __restrict__ a, const int64_t* __restrict__ b, int64_t* __restrict__ out)
+// The two scans' totals, and the largest row and overflowing community, in one launch (xoff null:
+// the rows alone, once the overflowing communities have theirs; the others' stay).
+__global__ void __launch_bounds__(256) k_totals(const int64_t* __restrict__ offs, const int64_t* __restrict__ xoff, int64_t nc,
+                                                int64_t* __restrict__ tot)
 {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        out[0] = *a;
-        out[1] = *b;
+    long long row = 0, x = 0;
+    for (int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x; i < nc; i += (int64_t)gridDim.x * 256) {
+        row = max(row, (long long)(offs[i + 1] - offs[i]));
+        if (xoff) x = max(x, (long long)(xoff[i + 1] - xoff[i]));
+    }
+    __shared__ unsigned long long s_max[2];
+    if (threadIdx.x < 2) s_max[threadIdx.x] = 0;
+    __syncthreads();
+    for (int o = 32; o > 0; o >>= 1) {
+        row = max(row, __shfl_xor(row, o));
+        x = max(x, __shfl_xor(x, o));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        atomicMax(&s_max[0], (unsigned long long)row);
+        atomicMax(&s_max[1], (unsigned long long)x);
+    }
+    __syncthreads();
+    // one atomic per block: every block's atomics go to the one address
+    if (threadIdx.x < 2 && s_max[threadIdx.x]) atomicMax((unsigned long long*)tot + 2 + threadIdx.x, s_max[threadIdx.x]);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        tot[0] = offs[nc];
+        if (xoff) tot[1] = xoff[nc];
     }
 }
 
@@ -734,22 +765,21 @@ __global__ void __launch_bounds__(kSmallBlock) k_rows_small(const int64_t* __res
 // right, and each community's runs placed in its staged row.
 static void overflow_rows(vt_ctx* ctx, const vt_graph* g, const uint32_t* newid, int64_t nc, int bits,
                           const int64_t* cstart, const int64_t* mrow, const int64_t* moff, const int64_t* xcnt,
-                          const int64_t* xoff, int64_t nx, int64_t xmax, uint32_t* rkey, double* rval, int64_t* rowlen)
+                          const int64_t* xoff, int64_t nx, int64_t xmax, uint32_t* counts, uint32_t* rkey, double* rval,
+                          int64_t* rowlen)
 {
     const size_t x1 = (size_t)std::max<int64_t>(nx, 1), c1n = (size_t)nc + 1;
     DBuf<unsigned long long> k0(ctx, x1), k1(ctx, x1);
     DBuf<double> v0(ctx, x1), v1(ctx, x1);
-    DBuf<uint32_t> counts(ctx, 2);
-    dzero(ctx, counts.p, 8);
     {
         // an overflowing community has more than kCfMaxKeys entries
         const int64_t cap = nx / kCfMaxKeys + nx / kItemLen + 1;
         DBuf<Item> items(ctx, (size_t)cap);
-        VT_LAUNCH(ctx, "rb_ovf_items", k_split_items, grid_for(nc, 256, 4096), 256, 0, nc, xcnt, (int64_t)1, counts.p,
+        VT_LAUNCH(ctx, "rb_ovf_items", k_split_items, grid_for(nc, 256, 4096), 256, 0, nc, xcnt, (int64_t)1, counts,
                   items.p);
         // timed under a name of its own where a giant community is among them
         const char* name = xmax > (1 << 16) ? "rb_ovf_emit_big" : "rb_ovf_emit";
-        VT_LAUNCH(ctx, name, k_ovf_emit, (unsigned)std::min<int64_t>(cap, 65536), 64, 0, (const uint32_t*)counts.p,
+        VT_LAUNCH(ctx, name, k_ovf_emit, (unsigned)std::min<int64_t>(cap, 65536), 64, 0, (const uint32_t*)counts,
                   (const Item*)items.p, cstart, moff, mrow, (const DEdge*)g->edges, newid, xoff, bits, k0.p, v0.p);
     }
     const unsigned long long* ks = k0.p;
@@ -795,9 +825,10 @@ static void overflow_rows(vt_ctx* ctx, const vt_graph* g, const uint32_t* newid,
     DBuf<double> rw(ctx, (size_t)nu);
     DBuf<uint32_t> longs(ctx, (size_t)(nx / kExtLongRun + 1));
     VT_LAUNCH(ctx, "rb_fold", k_ext_runs, grid_for(nu, 256, 16384), 256, 0, ks, vs, (const int64_t*)starts.p, nu, bits,
-              rc1.p, rc2.p, rw.p, counts.p + 1, longs.p);
-    VT_LAUNCH(ctx, "rb_fold_long", k_ext_runs_long, (unsigned)std::min<int64_t>(nx / kExtLongRun + 1, 16384), 64, 0,
-              (const uint32_t*)(counts.p + 1), (const uint32_t*)longs.p, vs, (const int64_t*)starts.p, rw.p);
+              rc1.p, rc2.p, rw.p, counts + 1, longs.p);
+    if (xmax >= kExtLongRun)  // a run lies in one community
+        VT_LAUNCH(ctx, "rb_fold_long", k_ext_runs_long, (unsigned)std::min<int64_t>(nx / kExtLongRun + 1, 16384), 64, 0,
+                  (const uint32_t*)(counts + 1), (const uint32_t*)longs.p, vs, (const int64_t*)starts.p, rw.p);
     DBuf<int64_t> run_first(ctx, c1n);
     VT_LAUNCH(ctx, "rb_ovf_rows", k_ovf_rows, grid_for(nc, 256, 16384), 256, 0, nc, xcnt, (const uint32_t*)rc1.p, nu,
               run_first.p, rowlen);
@@ -857,7 +888,7 @@ vt_graph* rebuild(vt_ctx* ctx, const vt_graph* g, const int64_t* d_cvect, bool c
     const size_t n1 = (size_t)std::max<int64_t>(nv, 1), e1 = (size_t)std::max<int64_t>(ne, 1);
     const bool small = nv > 0 && nv <= kSmallVerts;
     DBuf<uint32_t> newid(ctx, n1);
-    DBuf<int64_t> tot(ctx, 4);
+    DBuf<int64_t> tot(ctx, kTotals);
     int64_t nc = nv;  // small: known with the row lengths
     if (!small) nc = renumber(ctx, d_cvect, nv, check_ids, newid.p, tot.p);
     const int bits = (int)bits_for(nc > 1 ? nc - 1 : 1);
@@ -874,12 +905,17 @@ vt_graph* rebuild(vt_ctx* ctx, const vt_graph* g, const int64_t* d_cvect, bool c
     DBuf<int64_t> rowlen(ctx, c1n), xcnt(ctx, c1n), out_offs(ctx, c1n), xoff(ctx, c1n);
     if (nc)
         VT_LAUNCH(ctx, "rb_comm_fold", k_comm_fold, grid_for(nc, kFoldWaves, 262144), 64 * kFoldWaves, 0,
-                  (const int64_t*)tot.p, (const int64_t*)cstart.p, (const int64_t*)moff.p, (const int64_t*)mrow.p,
-                  (const DEdge*)g->edges, newid.p, rkey.p, rval.p, rowlen.p, xcnt.p);
+                  tot.p, (const int64_t*)cstart.p, (const int64_t*)moff.p, (const int64_t*)mrow.p, (const DEdge*)g->edges,
+                  newid.p, rkey.p, rval.p, rowlen.p, xcnt.p);
+    else {
+        dzero(ctx, rowlen.p, 8);
+        dzero(ctx, xcnt.p, 8);
+        dzero(ctx, tot.p, 8 * kTotals);
+    }
     // the coarse graph's largest row is read with its entry count (the overflowing
     // communities' rows are added below, and the count and the largest row read again)
     int64_t totals[4] = {0, 0, 0, 0};  // entries, overflowing entries, largest row, largest overflowing community
-    auto read_totals = [&] {
+    auto read_totals = [&](bool first) {
         if (small) {
             const int64_t* out = (const int64_t*)(mail(ctx) + 8);
             VT_LAUNCH(ctx, "rb_rows", k_rows_small, 1, kSmallBlock, 0, (const int64_t*)tot.p, (const int64_t*)rowlen.p,
@@ -891,26 +927,17 @@ vt_graph* rebuild(vt_ctx* ctx, const vt_graph* g, const int64_t* d_cvect, bool c
             std::memcpy(totals, out + 2, 32);
             return;
         }
-        dzero(ctx, rowlen.p + nc, 8);
-        dzero(ctx, xcnt.p + nc, 8);
         exclusive_scan_i64(ctx, rowlen.p, out_offs.p, nc + 1);
-        exclusive_scan_i64(ctx, xcnt.p, xoff.p, nc + 1);
-        VT_LAUNCH(ctx, "rb_totals", k_pair_totals, 1, 64, 0, (const int64_t*)out_offs.p + nc, (const int64_t*)xoff.p + nc,
-                  tot.p);
-        dzero(ctx, tot.p + 2, 16);
-        if (nc) {
-            VT_LAUNCH(ctx, "max_degree", k_max_degree, grid_for(nc, 256, 512), 256, 0, (const int64_t*)out_offs.p, nc,
-                      (unsigned long long*)(tot.p + 2));
-            VT_LAUNCH(ctx, "max_degree", k_max_degree, grid_for(nc, 256, 512), 256, 0, (const int64_t*)xoff.p, nc,
-                      (unsigned long long*)(tot.p + 3));
-        }
+        if (first) exclusive_scan_i64(ctx, xcnt.p, xoff.p, nc + 1);
+        VT_LAUNCH(ctx, "rb_totals", k_totals, grid_for(std::max<int64_t>(nc, 1), 256, 512), 256, 0, (const int64_t*)out_offs.p,
+                  first ? (const int64_t*)xoff.p : nullptr, nc, tot.p);
         d2h(ctx, totals, tot.p, 32);
     };
-    read_totals();
+    read_totals(true);
     if (totals[1]) {
-        overflow_rows(ctx, g, newid.p, nc, bits, cstart.p, mrow.p, moff.p, xcnt.p, xoff.p, totals[1], totals[3], rkey.p,
-                      rval.p, rowlen.p);
-        read_totals();
+        overflow_rows(ctx, g, newid.p, nc, bits, cstart.p, mrow.p, moff.p, xcnt.p, xoff.p, totals[1], totals[3], (uint32_t*)(tot.p + 4),
+                      rkey.p, rval.p, rowlen.p);
+        read_totals(false);
     }
 
     vt_graph* out = graph_new(ctx, nc, totals[0]);
