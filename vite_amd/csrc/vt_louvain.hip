@@ -2571,16 +2571,20 @@ __global__ void __launch_bounds__(256) k_ev_fold(int64_t nv, uint32_t* __restric
     }
 }
 
-// The long runs, a workgroup each: the run's events set their bits in LDS, every thread reads
-// back a stretch of the bits, and a scan of the threads' counts gives each its place in the
-// sorted run, which overwrites the unsorted one; wave 0 then folds it.
+// The long runs, a workgroup each.  Up to kEvRunRank events are held in LDS and each takes the place
+// that the smaller ones leave it.  In a longer run the events set their bits in LDS, every thread
+// reads back a stretch of the bits, and a scan of the threads' counts gives each its place: two
+// walks of 2n bits, whatever the run's length (7000 runs of 70 events at n = 490000 took 380 us so, by
+// their ranks 127).  The sorted run overwrites the unsorted one, and wave 0 folds it.
+constexpr uint32_t kEvRunRank = 1024;
+
 __global__ void __launch_bounds__(256) k_ev_fold_long(MoverArgs m, const uint32_t* __restrict__ ctl,
                                                       const int32_t* __restrict__ longs, uint32_t* __restrict__ cnt,
                                                       const uint32_t* __restrict__ base, uint32_t* __restrict__ ev,
                                                       const double* __restrict__ vdeg, double* __restrict__ cdeg,
                                                       int32_t* __restrict__ csize)
 {
-    __shared__ uint32_t bits[2 * kEvVerts / 32];
+    __shared__ alignas(16) uint32_t bits[2 * kEvVerts / 32];
     __shared__ uint32_t s_wave[4];
     const uint32_t nl = ctl[1];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -2588,27 +2592,33 @@ __global__ void __launch_bounds__(256) k_ev_fold_long(MoverArgs m, const uint32_
     for (uint32_t i = blockIdx.x; i < nl; i += gridDim.x) {
         const int32_t c = longs[i];
         const uint32_t s = cnt[c], b = base[c];
-        for (int k = threadIdx.x; k < per * 256; k += 256) bits[k] = 0;
-        __syncthreads();
-        for (uint32_t k = threadIdx.x; k < s; k += 256) {
-            const uint32_t e = ev[b + k];
-            atomicOr(&bits[e >> 5], 1u << (e & 31));
+        if (s <= kEvRunRank) {  // the same in every thread
+            for (uint32_t k = threadIdx.x; k < ((s + 3) & ~3u); k += 256) bits[k] = k < s ? ev[b + k] : 0xffffffffu;
+            __syncthreads();
+            for (uint32_t k = threadIdx.x; k < s; k += 256) {
+                const uint32_t e = bits[k];
+                uint32_t at = b;
+                for (uint32_t q = 0; q < s; q += 4) {
+                    const uint4 x = *(const uint4*)&bits[q];
+                    at += (x.x < e) + (x.y < e) + (x.z < e) + (x.w < e);
+                }
+                ev[at] = e;
+            }
+        } else {
+            for (int k = threadIdx.x; k < per * 256; k += 256) bits[k] = 0;
+            __syncthreads();
+            for (uint32_t k = threadIdx.x; k < s; k += 256) {
+                const uint32_t e = ev[b + k];
+                atomicOr(&bits[e >> 5], 1u << (e & 31));
+            }
+            __syncthreads();
+            uint32_t sum = 0, all = 0;
+            for (int k = 0; k < per; k++) sum += __popc(bits[threadIdx.x * per + k]);
+            uint32_t at = b + block_scan<256, uint32_t>(sum, s_wave, &all);
+            for (int k = 0; k < per; k++)
+                for (uint32_t x = bits[threadIdx.x * per + k]; x; x &= x - 1)
+                    ev[at++] = (uint32_t)(threadIdx.x * per + k) * 32 + (uint32_t)__builtin_ctz(x);
         }
-        __syncthreads();
-        uint32_t sum = 0;
-        for (int k = 0; k < per; k++) sum += __popc(bits[threadIdx.x * per + k]);
-        uint32_t inc = sum;
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t y = __shfl_up(inc, o);
-            if (lane >= o) inc += y;
-        }
-        if (lane == 63) s_wave[w] = inc;
-        __syncthreads();
-        uint32_t at = b + inc - sum;
-        for (int k = 0; k < w; k++) at += s_wave[k];
-        for (int k = 0; k < per; k++)
-            for (uint32_t x = bits[threadIdx.x * per + k]; x; x &= x - 1)
-                ev[at++] = (uint32_t)(threadIdx.x * per + k) * 32 + (uint32_t)__builtin_ctz(x);
         __syncthreads();
         if (w == 0) {
             double acc = 0.0;
