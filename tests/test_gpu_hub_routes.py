@@ -79,3 +79,25 @@ def test_gains_of_few_hubs_with_many_communities(ctx):
     st.end(want_cvect=False)
     # an atomic per wave and hub on one line of memory took 11 times as long
     assert 0 < best["hubw_gain"] < 3 * best["hubw_insert"], best
+
+
+@pytest.mark.parametrize("n", [8000, 9000])
+@pytest.mark.parametrize("rows,lds", [([1500] * 1023, True), ([1500] * 1024, False), ([600] * 1024 + [1500] * 400, True)])
+def test_many_rows_in_lds(ctx, n, rows, lds):
+    """Rows that go to LDS, up to a thousand of any length, more where they are short on average."""
+    g = _graph(n, [], rows, n + len(rows), whole=False)
+    dg = ctx.upload(vite_amd.CSR(g.offs, g.edges))
+    st = dg.phase_begin(thresh=-1.0)
+    for it in range(2):
+        ctx.set_profiling(True)
+        ctx.reset_stats()
+        st.sweep()
+        used = ctx.kernel_stats("local_move_hub_sort")[1]
+        ctx.set_profiling(False)
+        assert used == (0 if lds else 1)
+        s = st.state()
+        t_o, cw_o, _, _ = po.sweep(g, s["curr"], s["csize"], s["cdeg"].copy(), s["vdeg"], s["constant"])
+        assert np.array_equal(s["target"], t_o), it
+        assert np.array_equal(s["cw"].view(np.uint64), cw_o.view(np.uint64)), it
+        st.step()
+    st.end(want_cvect=False)

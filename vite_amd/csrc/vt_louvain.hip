@@ -68,6 +68,7 @@ constexpr int kHubBucket = 6;
 // are neighbours: a sweep that does not use the LDS form takes them as one.
 constexpr int kHubLdsBucket = 7;
 constexpr int kHubLdsMin = 512, kHubLdsMax = 4096;
+constexpr int kHubLdsMany = 1024;
 
 // Bucket of a row of degree d under per-bucket maximum degrees mx[0..5] (the tuning; the
 // default is 7, 15, 47, 63, 191, 511): rows above mx[5] are hubs.
@@ -2107,6 +2108,16 @@ __device__ __host__ __forceinline__ bool hub_lds_used(int64_t hubs, int64_t lds,
     return lds <= limit && (hubs == 0 || hub_whole_used(hubs, lds, whole) || limit == INT32_MAX);
 }
 
+// Nor long LDS rows, where they are many (from the count at which the sorted form has a workgroup
+// sort each): rows of more than 1024 entries run two and one to a CU, and where their runs have
+// some sixty entries, too many to be put in order and folded by a thread and few for a wave, 1400 rows
+// of 2000 took 277 us, sorted 215, 8000 1273 and 820.  Rows of 560 to 1100 were 1.1 to 2.7 times as
+// fast as sorted at all counts and runs.
+__device__ __host__ __forceinline__ bool hub_lds_pays(int64_t lds, int64_t entries)
+{
+    return lds < kHubLdsMany || entries <= 1100 * lds;
+}
+
 // A row's sweep list: its degree bucket, the wide bucket split by table size.
 __device__ __host__ __forceinline__ uint32_t list_bucket(int64_t d, int lpv_max, const BucketBounds& bb)
 {
@@ -3088,9 +3099,12 @@ __global__ void __launch_bounds__(kTailBlock) k_setup_small(SetupArgs a)
     };
     const int hubs = s_total[kHubBucket], in_lds = s_total[kHubLdsBucket];
     scan_hubs(0, hubs);
-    const bool apart = hub_lds_used(hubs, in_lds, a.hub_limit, whole) && (hubs == 0 || hub_whole_pays((int64_t)entries, a.max_degree));
-    const int nh = apart ? hubs : hubs + in_lds;  // the LDS rows follow the hubs in the lists
-    scan_hubs(hubs, nh);
+    const unsigned long long hub_entries = entries;
+    bool apart = hub_lds_used(hubs, in_lds, a.hub_limit, whole) && (hubs == 0 || hub_whole_pays((int64_t)entries, a.max_degree));
+    if (!apart || in_lds >= kHubLdsMany) scan_hubs(hubs, hubs + in_lds);  // the LDS rows follow the hubs in the lists
+    apart = apart && hub_lds_pays(in_lds, (int64_t)(entries - hub_entries));
+    const int nh = apart ? hubs : hubs + in_lds;
+    if (apart) entries = hub_entries;
     double r[2];
     small_tree_sum2<kTailBlock>(a.vdeg, nullptr, a.nv, a.blocks, a.chunk, lds, s_part, r);
     int64_t* out = (int64_t*)a.out;
@@ -3660,18 +3674,22 @@ struct Phase {
             for (int64_t c = 0; c < ncol; c++) {
                 ColorSweep& cs = sweeps[c];
                 hub_offs.emplace_back(ctx, (size_t)(cs.hub_n + cs.hubl_n) + 1);
-                auto scan_hubs = [&] {
-                    DBuf<int64_t> deg(ctx, (size_t)cs.hub_n + 1);
-                    VT_LAUNCH(ctx, "hub_degrees", k_hub_degrees, grid_for(cs.hub_n + 1, 256, 1024), 256, 0,
-                              (const int32_t*)(lists.p + cs.hub_off), (int32_t)cs.hub_n, (const int64_t*)g->offs, deg.p);
-                    exclusive_scan_i64(ctx, deg.p, hub_offs.back().p, cs.hub_n + 1);
-                    d2h(ctx, &hub_total[c], hub_offs.back().p + cs.hub_n, 8);
+                auto entries_of = [&](int64_t off, int64_t n) {  // and their offsets
+                    int64_t total = 0;
+                    if (!n) return total;
+                    DBuf<int64_t> deg(ctx, (size_t)n + 1);
+                    VT_LAUNCH(ctx, "hub_degrees", k_hub_degrees, grid_for(n + 1, 256, 1024), 256, 0,
+                              (const int32_t*)(lists.p + off), (int32_t)n, (const int64_t*)g->offs, deg.p);
+                    exclusive_scan_i64(ctx, deg.p, hub_offs.back().p, n + 1);
+                    d2h(ctx, &total, hub_offs.back().p + n, 8);
+                    return total;
                 };
-                if (!cs.hub_n) continue;
-                scan_hubs();
-                if (!cs.whole || hub_whole_pays(hub_total[c], g->max_degree)) continue;
-                sort_all_hubs(cs);
-                scan_hubs();
+                if (cs.hubl_n >= kHubLdsMany && !hub_lds_pays(cs.hubl_n, entries_of(cs.hubl_off, cs.hubl_n))) sort_all_hubs(cs);
+                hub_total[c] = entries_of(cs.hub_off, cs.hub_n);
+                if (cs.whole && !hub_whole_pays(hub_total[c], g->max_degree)) {
+                    sort_all_hubs(cs);
+                    hub_total[c] = entries_of(cs.hub_off, cs.hub_n);
+                }
             }
         }
         // Hub tables: one HBM table per resident wave, sized for the largest row.
@@ -3709,11 +3727,11 @@ struct Phase {
     }
 
     // How many rows k_hub_lds takes at most (-1: none).  It saves the sorted form's twenty launches
-    // (RGG n = 2^20 -i run 12.2 -> 10.8 ms) but its rows of up to 4096 entries run one or two per CU:
-    // on RGG n = 2^24, with 4000 to 15000 such rows a sweep, it took 14.0 ms of a run and the sorted
-    // form 10.5.  (From 2^17 vertices the sorted form's keys of 17 K hubs pass 32 bits and take the
-    // library's sort: BA n = 2^22, device time of a run 71.0 -> 64.1 ms with the larger limit.)  A tuning that forces a form of the sorted path gets it; a batch's only other form
-    // is a wave per row.
+    // (RGG n = 2^20 -i run 12.2 -> 10.8 ms).  On coarse levels the rows' neighbours lie in few
+    // communities, and the form of thousands of rows is even or behind there: sweeps of RGG n = 2^24's levels
+    // take 1150 us with 22573 rows of 59376 vertices in LDS and 1088 sorted, 430 and 278 with 2492 rows of
+    // 2537 vertices, but 825 and 900 with 6449 rows of 230287.  A tuning that forces a form of the
+    // sorted path gets it; a batch's only other form is a wave per row.
     int64_t hub_lds_limit() const
     {
         if (gid) return INT32_MAX;
@@ -3976,8 +3994,9 @@ struct Phase {
             const int32_t* hubs = (const int32_t*)(lists.p + cs.hubl_off);
             const unsigned nb = (unsigned)std::min<int64_t>(cs.hubl_n, 16384);
             const int32_t n = (int32_t)cs.hubl_n;
-            // 22, 44 and 88 KB of LDS: 28, 24 and 16 waves per CU.  Where every row has a CU to itself,
-            // one launch of the largest: each takes some 20 us for any number of rows.
+            // 22, 45 and 89 KB of LDS and 121 to 128 registers: four, two and one workgroup of 4, 8 and 16
+            // waves per CU.  Where every row has a CU to itself, one launch of the largest: each takes
+            // some 20 us for any number of rows.
             auto k1 = batch ? k_hub_lds<1024, 256, true> : k_hub_lds<1024, 256, false>;
             auto k2 = batch ? k_hub_lds<2048, 512, true> : k_hub_lds<2048, 512, false>;
             auto k4 = batch ? k_hub_lds<4096, 1024, true> : k_hub_lds<4096, 1024, false>;
