@@ -32,14 +32,15 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_GBS = 8000.0
 # Rows of bucket 2 (16-lane groups; degree <= 47 with the default bounds) run in the
 # launch named "local_move", the dominant one on random geometric graphs; buckets 0, 1
-# and 3 run in "local_move_rest" and larger degree classes in their own launches.
+# and 3 run in "local_move_rest" and larger degree classes in their own launches.  On graphs of
+# some hundred thousand rows and fewer, buckets 0 to 3 run in one launch, "local_move_all".
 G16_BUCKET = 2
 
 
-def g16_kernel(tuning):
-    """The bucket-2 launch's kernel as rocprof names it: single graph, part 2, and whether it
-    reads the per-vertex community records (the vertex_records tuning)."""
-    return f"k_local_move<false, 2, {'true' if tuning.get('vertex_records') else 'false'}>"
+def g16_kernel(tuning, all_buckets=False):
+    """The bucket-2 launch's kernel as rocprof names it: single graph, part 2 (3 where it takes
+    buckets 0 to 3), and whether it reads the per-vertex community records (the vertex_records tuning)."""
+    return f"k_local_move<false, {3 if all_buckets else 2}, {'true' if tuning.get('vertex_records') else 'false'}>"
 # rocprofv3 FETCH_SIZE / WRITE_SIZE (KiB per dispatch) against the bytes a plain 1 GiB
 # device copy really moves: FETCH_SIZE reads half of them, WRITE_SIZE all of them.
 FETCH_SCALE = 2.0
@@ -415,7 +416,7 @@ def skewed_form(ctx, args):
     for _ in range(reps):
         st.sweep()
     kernels = {}
-    for k in ("local_move", "local_move_rest", "local_move_mid", "local_move_wide", "local_move_hub_sort",
+    for k in ("local_move", "local_move_rest", "local_move_all", "local_move_mid", "local_move_wide", "local_move_hub_sort",
               "local_move_hub"):
         avg, cnt, _ = ctx.kernel_stats(k)
         if cnt:
@@ -686,6 +687,9 @@ def main():
     wall = time.perf_counter() - t0
     ms_per_step = 1e3 * wall / args.steps
     kavg, kcount, ktot = ctx.kernel_stats("local_move")
+    all_buckets = kcount == 0  # a small graph: one launch for buckets 0 to 3
+    if all_buckets:
+        kavg, kcount, ktot = ctx.kernel_stats("local_move_all")
     ctx.set_profiling(False)
     state = st.state()
     per_iter = None
@@ -695,9 +699,10 @@ def main():
             f"({100 * per_iter['hbm_frac']:.1f}% of HBM peak in algorithmic bytes)")
     st.end(want_cvect=False)
 
-    # the dominant kernel's own share: the rows of bucket 2 under the tuning in force
+    # the dominant kernel's own share: the rows of bucket 2 (or 0 to 3) under the tuning in force
     deg = np.diff(dg.offsets())
-    fused = degree_buckets(deg, tuning["bucket_max_degree"]) == G16_BUCKET
+    bucket = degree_buckets(deg, tuning["bucket_max_degree"])
+    fused = bucket <= 3 if all_buckets else bucket == G16_BUCKET
     Vf, Ef = int(np.count_nonzero(fused)), int(deg[fused].sum())
     alg_bytes = 24 * Ef + 56 * Vf
     achieved = alg_bytes / (kavg * 1e-3) / 1e9 if kavg > 0 else 0.0
@@ -706,7 +711,7 @@ def main():
         f"({Vf} of {V} rows, {Ef} of {E} entries), {achieved:.1f} GB/s algorithmic "
         f"({100 * achieved / HBM_PEAK_GBS:.1f}% of peak), {value / 1e9:.2f} G edges/s")
     tag = f"rgg_n{V}"
-    traffic, traffic_src = measured_traffic("local_move", tag, g16_kernel(tuning))
+    traffic, traffic_src = measured_traffic("local_move", tag, g16_kernel(tuning, all_buckets))
 
     out = {
         "metric": METRIC, "value": value, "unit": "edges/s", "n_gpus": 1, "steps": args.steps,
@@ -718,8 +723,9 @@ def main():
                    "threshold": 1e-3, "tuning": tuning},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                     "kernel": g16_kernel(tuning), "kernel_avg_ms": kavg, "algorithmic_bytes_per_launch": alg_bytes,
-                     "bytes_formula": "24E + 56V over the kernel's rows (bucket 2: 16-lane groups)",
+                     "kernel": g16_kernel(tuning, all_buckets), "kernel_avg_ms": kavg, "algorithmic_bytes_per_launch": alg_bytes,
+                     "bytes_formula": "24E + 56V over the kernel's rows "
+                                      + ("(buckets 0 to 3)" if all_buckets else "(bucket 2: 16-lane groups)"),
                      "sweep_achieved": (24 * E + 56 * V) / (ms_per_step * 1e-3) / 1e9,
                      "sweep_formula": "24E + 56V over all rows / wall time of the whole sweep (every launch)",
                      "kernel_rows": Vf, "kernel_entries": Ef,

@@ -32,4 +32,4 @@ def test_routes(ctx, n, parts, device):
     launch()
     sorts, passes = ctx.kernel_stats("sort_u32")[1], ctx.kernel_stats("dsort_scatter")[1]
     ctx.set_profiling(False)
-    assert sorts == 1 and (passes > 0) == device
+    assert sorts == (0 if device else 1) and (passes > 0) == device

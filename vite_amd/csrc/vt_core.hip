@@ -540,11 +540,11 @@ void sort_pairs_u32(vt_ctx* ctx, uint32_t* keys, uint32_t* vals, int64_t n, int 
 {
     *result_in_alt = false;
     if (n <= 1) return;
-    TimedScope ts(ctx, "sort_u32");
-    if (dev_sort_pays(n, bits)) {
+    if (dev_sort_pays(n, bits)) {  // timed launch by launch (dsort_*)
         *result_in_alt = dev_sort_pairs_u32(ctx, keys, vals, keys_alt, vals_alt, nullptr, n, n, bits);
         return;
     }
+    TimedScope ts(ctx, "sort_u32");
     rocprim::double_buffer<uint32_t> kb(keys, keys_alt);
     rocprim::double_buffer<uint32_t> vb(vals, vals_alt);
     size_t tb = 0;

@@ -3938,7 +3938,6 @@ struct Phase {
         const HubWhole hw{(const int32_t*)(lists.p + cs.hub_off), (int32_t)cs.hub_n, hub_offs[cs.index].p,
                           2 * (unsigned long long)total, hw_key.p, hw_val.p, hw_hub.p, hw_hub.p + hubs, hw_best.p,
                           hw_best.p + hubs};
-        TimedScope ts(ctx, "local_move_hub");
         VT_LAUNCH(ctx, "hubw_insert", k_hubw_insert, grid_for(total, kHubwChunk, 1 << 21), 256, 0, a, hw);
         VT_LAUNCH(ctx, "hubw_gain", k_hubw_gain, grid_for(2 * total, kHubwGainBlock, 512), kHubwGainBlock, 0, a, hw);
         VT_LAUNCH(ctx, "hubw_pick", k_hubw_pick, grid_for(2 * total, 256, 8192), 256, 0, a, hw);
@@ -3962,7 +3961,7 @@ struct Phase {
             const bool one = !a.rec && cs.fused_blocks <= kOneLaunchBlocks && n16 && cs.fused_blocks > n16;
             if (one) {
                 auto kern = batch ? k_local_move<true, kPartAll, false> : k_local_move<false, kPartAll, false>;
-                VT_LAUNCH(ctx, "local_move", kern, (unsigned)cs.fused_blocks, kFusedBlock, 0, a, (const int32_t*)lists.p,
+                VT_LAUNCH(ctx, "local_move_all", kern, (unsigned)cs.fused_blocks, kFusedBlock, 0, a, (const int32_t*)lists.p,
                           cs.plan);
             }
             if (!one && cs.fused_blocks > n16) {
@@ -3990,35 +3989,48 @@ struct Phase {
             VT_LAUNCH(ctx, "local_move_wide", kern, (unsigned)std::min<int64_t>(cs.wide_n[w], 16384), 64, 0, a,
                       (const int32_t*)(lists.p + cs.wide_off[w]), cs.wide_n[w]);
         }
-        if (cs.hubl_n) {
-            const int32_t* hubs = (const int32_t*)(lists.p + cs.hubl_off);
-            const unsigned nb = (unsigned)std::min<int64_t>(cs.hubl_n, 16384);
-            const int32_t n = (int32_t)cs.hubl_n;
-            // 22, 45 and 89 KB of LDS and 121 to 128 registers: four, two and one workgroup of 4, 8 and 16
-            // waves per CU.  Where every row has a CU to itself, one launch of the largest: each takes
-            // some 20 us for any number of rows.
-            auto k1 = batch ? k_hub_lds<1024, 256, true> : k_hub_lds<1024, 256, false>;
-            auto k2 = batch ? k_hub_lds<2048, 512, true> : k_hub_lds<2048, 512, false>;
-            auto k4 = batch ? k_hub_lds<4096, 1024, true> : k_hub_lds<4096, 1024, false>;
-            const bool one = n <= 256, only1 = g->max_degree <= 1024, only2 = g->max_degree <= 2048;
-            if (only1 || !one) VT_LAUNCH(ctx, "local_move_hub", k1, nb, 256, 0, a, hubs, n, 0);
-            if (!only1 && (only2 || !one)) VT_LAUNCH(ctx, "local_move_hub", k2, nb, 512, 0, a, hubs, n, one ? 0 : 1024);
-            if (!only2) VT_LAUNCH(ctx, "local_move_hub", k4, nb, 1024, 0, a, hubs, n, one ? 0 : 2048);
+        if (!cs.hubl_n && !cs.hub_n) return;
+        if (cs.hub_n && hub_sort && !cs.whole) {
+            hub_sweep_sorted(a, cs);  // its rows are all of the sweep's hub rows
+            return;
         }
-        if (cs.hub_n && cs.whole && hub_sort && hub_total[cs.index] < (int64_t(1) << 31)) {
+        TimedScope ts(ctx, "local_move_hub");
+        if (cs.hubl_n) hub_sweep_lds(a, cs);
+        if (cs.hub_n && cs.whole) {
             hub_sweep_whole(a, cs, hub_total[cs.index]);
-        } else if (cs.hub_n && hub_sort) {
-            const int64_t total = hub_total[cs.index];
-            const int cbits = (int)bits_for(nv > 1 ? nv - 1 : 1);  // community ids < nv
-            const int kbits = cbits + (int)bits_for(cs.hub_n);
-            if (kbits <= 32 && total < (int64_t(1) << 31)) hub_sweep<uint32_t>(a, cs, total, cbits, kbits);
-            else hub_sweep<unsigned long long>(a, cs, total, cbits, kbits);
         } else if (cs.hub_n) {
             const int blocks = (int)std::min<int64_t>(cs.hub_n, hub_blocks);
-            VT_LAUNCH(ctx, "local_move_hub", k_move_hbm, (unsigned)blocks, 64, 0, a, (const int32_t*)(lists.p + cs.hub_off),
+            VT_LAUNCH(ctx, "hub_hbm", k_move_hbm, (unsigned)blocks, 64, 0, a, (const int32_t*)(lists.p + cs.hub_off),
                       cs.hub_n, (int32_t*)scratch(ctx, "hub_keys", 0), (double*)scratch(ctx, "hub_vals", 0),
                       (int32_t*)scratch(ctx, "hub_occ", 0), (uint32_t)hub_cap);
         }
+    }
+
+    void hub_sweep_lds(const MoveArgs& a, const ColorSweep& cs)
+    {
+        const int32_t* hubs = (const int32_t*)(lists.p + cs.hubl_off);
+        const unsigned nb = (unsigned)std::min<int64_t>(cs.hubl_n, 16384);
+        const int32_t n = (int32_t)cs.hubl_n;
+        const bool batch = a.gid != nullptr;
+        // 22, 45 and 89 KB of LDS and 121 to 128 registers: four, two and one workgroup of 4, 8 and 16
+        // waves per CU.  Where every row has a CU to itself, one launch of the largest: each takes
+        // some 20 us for any number of rows.
+        auto k1 = batch ? k_hub_lds<1024, 256, true> : k_hub_lds<1024, 256, false>;
+        auto k2 = batch ? k_hub_lds<2048, 512, true> : k_hub_lds<2048, 512, false>;
+        auto k4 = batch ? k_hub_lds<4096, 1024, true> : k_hub_lds<4096, 1024, false>;
+        const bool one = n <= 256, only1 = g->max_degree <= 1024, only2 = g->max_degree <= 2048;
+        if (only1 || !one) VT_LAUNCH(ctx, "hub_lds", k1, nb, 256, 0, a, hubs, n, 0);
+        if (!only1 && (only2 || !one)) VT_LAUNCH(ctx, "hub_lds", k2, nb, 512, 0, a, hubs, n, one ? 0 : 1024);
+        if (!only2) VT_LAUNCH(ctx, "hub_lds", k4, nb, 1024, 0, a, hubs, n, one ? 0 : 2048);
+    }
+
+    void hub_sweep_sorted(const MoveArgs& a, const ColorSweep& cs)
+    {
+        const int64_t total = hub_total[cs.index];
+        const int cbits = (int)bits_for(nv > 1 ? nv - 1 : 1);  // community ids < nv
+        const int kbits = cbits + (int)bits_for(cs.hub_n);
+        if (kbits <= 32 && total < (int64_t(1) << 31)) hub_sweep<uint32_t>(a, cs, total, cbits, kbits);
+        else hub_sweep<unsigned long long>(a, cs, total, cbits, kbits);
     }
 
     // Folds the sweep's moves into localCinfo in processing order, with no host read: the
