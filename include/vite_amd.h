@@ -85,14 +85,18 @@ typedef struct {
      * with the neighbour's line.  Pays on graphs whose neighbours are scattered (random
      * reads); 0 (the default): separate arrays. */
     int32_t vertex_records;
-    /* Rows above bucket_max_degree[5] (hubs): those of 512 to 4096 entries take a workgroup each
-     * in LDS where a sweep does not have too many, longer ones of whole weights one table; the
-     * others are grouped by neighbour community with a sort per sweep.  There a sweep with at least this many hubs gives each hub a workgroup, which
-     * sorts the hub's row (a segmented sort) and moves the hub, unless its largest hub holds
-     * more than 1/64 of the hub entries; otherwise it sorts all hub entries at once and runs
-     * every community run in a flat launch (a few large hubs would leave most of the chip
-     * idle).  0 <= hub_block_min <= 2^30; 0 sorts every hub row and gives every sweep the per-hub
-     * form, 2^30 sorts them all and runs the flat form. */
+    /* Rows above bucket_max_degree[5] (hubs) are moved in one of three ways.
+     *   In LDS, a workgroup each: rows of 512 to 4096 entries, where a sweep does not have too many
+     *   of them and no hub row beside them has to be sorted.
+     *   One table of (hub, community) sums: longer rows of whole weights, where they are few beside
+     *   the rows in LDS.
+     *   Sorted by neighbour community, every other sweep's hub rows together: a sweep with at least
+     *   hub_block_min of them sorts each hub's row by a workgroup (a segmented sort), which then
+     *   moves the hub, unless the largest holds more than 1/64 of the hub entries; any other
+     *   sweep sorts all hub entries at once and takes every community run in a flat launch (a
+     *   few large hubs would leave most of the chip idle).
+     * 0 <= hub_block_min <= 2^30; 0 sorts every hub row and gives every sweep the per-hub form,
+     * 2^30 sorts them all and runs the flat form. */
     int32_t hub_block_min;
 } vt_tuning;
 int vt_ctx_get_tuning(const vt_ctx* ctx, vt_tuning* out);

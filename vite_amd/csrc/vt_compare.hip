@@ -5,9 +5,9 @@
 // also puts them together (same-same) or not (same-diff), and for every pair inside one
 // community of C2 whether C1 separates them (diff-same), by walking all pairs: O(sum of
 // squared community sizes).  The counts are integers, so any order gives the same values:
-// here every vertex adds one, with an atomic increment, to its (C1, C2) pair, the pairs add their
-// counts to the sizes of C1 and C2, and C(k, 2) is summed over each group.  The pair groups live in an open-addressed HBM table of 64-bit
-// keys (C1 * nC2 + C2) at most half full.  Then
+// here every vertex adds one to its (C1, C2) pair, the pairs add their counts to the sizes of C1
+// and C2, and C(k, 2) is summed over each group.  The pairs live in an open-addressed HBM table
+// of 64-bit keys (C1 * nC2 + C2) at most half full.  Then
 //   same-same = sum over (a,b) of C(n_ab, 2),
 //   same-diff = sum over a of C(n_a, 2) - same-same,
 //   diff-same = sum over b of C(n_b, 2) - same-same,
@@ -72,7 +72,8 @@ __global__ void k_cmp_clear(PairSlot* __restrict__ t, int64_t n)
 }
 
 // cnt vertices of the pair `key`, in the table.
-__device__ __forceinline__ void pair_add(PairSlot* __restrict__ pairs, int logcap, unsigned long long key, unsigned long long cnt)
+__device__ __forceinline__ void pair_add(PairSlot* __restrict__ pairs, int logcap, unsigned long long key,
+                                         unsigned long long cnt)
 {
     const unsigned long long mask = (1ull << logcap) - 1;
     unsigned long long h = (key * 0x9E3779B97F4A7C15ull) >> (64 - logcap);
@@ -95,8 +96,8 @@ constexpr int kCmpSlots = 1024;
 constexpr int64_t kCmpChunk = 1024;  // vertices per workgroup, at least
 
 __global__ void __launch_bounds__(kCmpBlock) k_cmp_count(const int64_t* __restrict__ c1, const int64_t* __restrict__ c2,
-                                                         int64_t n, int64_t chunk, uint64_t nc2, PairSlot* __restrict__ pairs,
-                                                         int logcap)
+                                                         int64_t n, int64_t chunk, uint64_t nc2,
+                                                         PairSlot* __restrict__ pairs, int logcap)
 {
     __shared__ unsigned long long s_key[kCmpSlots];
     __shared__ unsigned s_cnt[kCmpSlots];

@@ -204,25 +204,22 @@ void d2h(vt_ctx* ctx, void* dst, const void* src, size_t bytes)
     }
     ctx->stage_off = 0;  // the stream has drained: every staged copy has run
 }
-// Pinned host memory that kernels write a few scalars to (256 bytes; [0, 1]: an iteration's Q and
-// movers, [2]: a phase's whole degrees, [3]: the last post's number,
-// [4, 8): a batch round's status, [8, 14): a rebuild's totals, [15]: whole hub rows,
-// [16, 29): a phase's list sizes), with no copy queued behind the kernel.
 double* mail(vt_ctx* ctx)
 {
     if (!ctx->mail) {
-        VT_HIP(ctx, hipHostMalloc((void**)&ctx->mail, 256, hipHostMallocDefault));
-        std::memset(ctx->mail, 0, 256);
+        VT_HIP(ctx, hipHostMalloc((void**)&ctx->mail, 8 * kMailSlots, hipHostMallocDefault));
+        std::memset(ctx->mail, 0, 8 * kMailSlots);
     }
     return ctx->mail;
 }
-// Waits for the kernel that posts seq.  The number is looked for in the pinned memory
-// first: waiting for the stream costs a marker behind the kernel and its interrupt (RGG n = 1000
-// upload and run, some 40 waits: 1.29 ms with stream waits, 1.10 so; RGG n = 65536: 3.85 and 3.55).  A kernel that takes longer than 200 us is
-// waited for with the stream, where that no longer matters and errors are reported.
+// Waits for the kernel that posts seq.  The number is looked for in the pinned memory first: waiting
+// for the stream costs a marker behind the kernel and its interrupt (RGG n = 1000 upload and run, some
+// 40 waits: 1.29 ms with stream waits, 1.10 so; RGG n = 65536: 3.85 and 3.55).  A kernel that takes
+// longer than 200 us is waited for with the stream, where that no longer matters and errors are
+// reported.
 void mail_wait(vt_ctx* ctx, unsigned long long seq)
 {
-    const unsigned long long* p = (const unsigned long long*)ctx->mail + 3;
+    const unsigned long long* p = (const unsigned long long*)ctx->mail + kMailSeq;
     const auto t0 = std::chrono::steady_clock::now();
     for (;;) {
         for (int k = 0; k < 64; k++) {

@@ -64,7 +64,7 @@ struct vt_ctx {
     // ring restarts whenever the stream has drained (sync, d2h).
     unsigned char* stage = nullptr;
     size_t stage_off = 0;
-    double* mail = nullptr;  // pinned: Q and the movers of an iteration (vt::mail)
+    double* mail = nullptr;  // pinned (vt::mail)
     unsigned long long mail_seq = 0;  // the last number given to a kernel that posts there
     // sweep launch shape (performance only: every setting gives the same results)
     vt_tuning tuning = {{7, 15, 31, 63, 127, 1023}, 16384};  // replaced by default_tuning() at creation
@@ -181,13 +181,28 @@ void sync(vt_ctx* ctx);
 void h2d(vt_ctx* ctx, void* dst, const void* src, size_t bytes);
 void d2h(vt_ctx* ctx, void* dst, const void* src, size_t bytes);
 void d2d(vt_ctx* ctx, void* dst, const void* src, size_t bytes);
+// Pinned host memory that kernels write a few scalars to, with no copy queued behind the kernel: doubles
+// or 64-bit integers at these places.
+enum MailSlot : int {
+    kMailQ = 0,           // an iteration's Q, and its movers behind it
+    kMailWhole = 2,       // 1.0 where a phase's degrees are whole numbers
+    kMailSeq = 3,         // the last post's number
+    kMailBatch = 4,       // a batch round's graphs and vertices that go on, two rounds in turn
+    kMailRebuild = 8,     // a small rebuild's communities, ids out of range and four totals
+    kMailHubWhole = 15,   // 1.0 where the hub rows' weights are whole numbers
+    kMailLists = 16,      // a small phase's list sizes, kMailListSlots at most
+    kMailHubsApart = 27,  // 1 where its LDS rows are not sorted with the hubs
+    kMailHubEntries = 28,
+    kMailSlots = 32
+};
+constexpr int kMailListSlots = kMailHubsApart - kMailLists;
 double* mail(vt_ctx* ctx);
 // A kernel that writes to mail() ends with mail_post(out, seq), seq = ++ctx->mail_seq, and the host
 // waits for that number, or a later one, with mail_wait.
 void mail_wait(vt_ctx* ctx, unsigned long long seq);
 __device__ __forceinline__ void mail_post(double* out, unsigned long long seq)
 {
-    __hip_atomic_store((unsigned long long*)out + 3, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store((unsigned long long*)out + kMailSeq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 void dzero(vt_ctx* ctx, void* dst, size_t bytes);
 

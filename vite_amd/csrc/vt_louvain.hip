@@ -53,6 +53,7 @@ __device__ __forceinline__ uint32_t slot_hash(int32_t c) { return (uint32_t)c * 
 // Degree buckets: (lanes per vertex G, table capacity CAP, max degree).  CAP >= 2*(deg+1)
 // keeps the table at most half full (a row has at most deg+1 distinct communities).
 constexpr int kNumBuckets = 11;
+static_assert(kNumBuckets <= kMailListSlots, "a small phase posts its lists' sizes");
 constexpr int kLpvBucket = 8;      // lane per vertex (degree <= lpv_max)
 // The wide bucket (one wave per row, up to 1023 entries) is split by degree so that each row
 // gets the smallest table that keeps it at most half full: 512 slots up to degree 255, 1024
@@ -530,8 +531,8 @@ __device__ __forceinline__ void fold_chunk(const GroupTable<G>& t, double* ecc_c
 
 // Per-vertex header, prefetched one vertex ahead.
 // A vertex as the fused buckets see it: row start, degree (< 0 for a vertex early
-// termination froze), own community and weighted degree.  Rows here have degree <= 127 and
-// community ids fit 32 bits (vt_graph_upload rejects nv >= 2^31).
+// termination froze), own community and weighted degree.  Rows here have degree <= 191 (the
+// default bound of bucket 4) and community ids fit 32 bits (vt_graph_upload rejects nv >= 2^31).
 // In a batch, degree -2 marks a vertex whose graph has left the phase (nothing is written)
 // and `cst` carries its graph's 1/2m.
 struct VHeaderBase {
@@ -868,11 +869,11 @@ __device__ __forceinline__ void run_bucket(const MoveArgs& a, char* lds, const i
     }
 }
 
-// Buckets 0-3 (degree <= 63) of one sweep in two launches over one block plan: blocks
-// [bbeg[b], bbeg[b+1]) run bucket b over its list range.  Bucket 2 (16-lane groups) runs
-// alone and buckets 0, 1 and 3 share the other launch: each kernel then fits 64 VGPRs,
-// so a SIMD holds eight waves (one kernel for all four needs 70 and holds seven).
-// Bucket 4 (64 <= degree <= 127) has its own launch so that its larger tables do not set
+// Buckets 0-3 (degree <= 63) of one sweep over one block plan: blocks [bbeg[b], bbeg[b+1]) run
+// bucket b over its list range.  Up to kOneLaunchBlocks they are one launch; above, bucket 2
+// (16-lane groups) runs alone and buckets 0, 1 and 3 share the other.  Every form is held to 64
+// VGPRs, so a SIMD holds eight waves.
+// Bucket 4 (degrees 64 to 191 by default) has its own launch so that its larger tables do not set
 // the LDS footprint, and so the occupancy, of these.
 constexpr int kFusedBuckets = 4;
 constexpr int kFusedBlock = 256;
@@ -925,7 +926,7 @@ k_local_move(MoveArgs a, const int32_t* __restrict__ lists, SweepPlan plan)
     if (threadIdx.x == 0 && s_inactive && a.inactive_count) atomicAdd(a.inactive_count, (unsigned long long)s_inactive);
 }
 
-// Bucket 4 (64 <= degree <= 127): four 64-lane groups per block, 256-slot tables.
+// Bucket 4 (degrees 64 to 191 by default): four 64-lane groups per block, 256-slot tables.
 template <bool BATCH, bool REC>
 __global__ void __launch_bounds__(256) k_local_move_mid(MoveArgs a, const int32_t* __restrict__ list, int64_t n)
 {
@@ -1361,11 +1362,14 @@ __global__ void __launch_bounds__(kHubBlock) k_hub_own(MoveArgs a, const int32_t
 // One term in flight per lane in a wave's folds: with four the kernel held 102 registers and 4 waves
 // per SIMD instead of 7, and 256 hubs of 40000 entries with a run each took 444 us instead of 400.
 template <class K>
-__global__ void __launch_bounds__(kHubBlock, 7) k_hub_runs(MoveArgs a, const int32_t* __restrict__ hubs, int32_t nh, const int64_t* __restrict__ hoffs,
-                           const K* __restrict__ keys, const uint32_t* __restrict__ vals, const int32_t* __restrict__ pos,
-                           const int32_t* __restrict__ head, const int32_t* __restrict__ starts, int cbits,
-                           const double* __restrict__ own, double* __restrict__ gains,
-                           unsigned long long* __restrict__ best)
+__global__ void __launch_bounds__(kHubBlock, 7) k_hub_runs(MoveArgs a, const int32_t* __restrict__ hubs, int32_t nh,
+                                                           const int64_t* __restrict__ hoffs, const K* __restrict__ keys,
+                                                           const uint32_t* __restrict__ vals,
+                                                           const int32_t* __restrict__ pos,
+                                                           const int32_t* __restrict__ head,
+                                                           const int32_t* __restrict__ starts, int cbits,
+                                                           const double* __restrict__ own, double* __restrict__ gains,
+                                                           unsigned long long* __restrict__ best)
 {
     __shared__ double s_red[kHubBlock / 64], s_ey[kHubBlock];
     __shared__ int2 s_run[kHubBlock];
@@ -2154,9 +2158,10 @@ __global__ void k_color_keys(int64_t nv, const int64_t* __restrict__ colors, int
     }
 }
 
-// Histogram of small keys: per-block counts in LDS, one global atomic per touched bin.
-// Counts of the keys in [lo, lo + nbins).
-__global__ void k_key_histogram(const uint32_t* __restrict__ keys, int64_t n, int64_t* __restrict__ hist, uint32_t lo, int nbins)
+// Histogram of the keys in [lo, lo + nbins): per-block counts in LDS, one global atomic per touched
+// bin.
+__global__ void k_key_histogram(const uint32_t* __restrict__ keys, int64_t n, int64_t* __restrict__ hist, uint32_t lo,
+                                int nbins)
 {
     extern __shared__ unsigned s_bins[];
     for (int i = threadIdx.x; i < nbins; i += blockDim.x) s_bins[i] = 0;
@@ -2907,8 +2912,8 @@ __global__ void __launch_bounds__(kTailBlock) k_tail_small(TailArgs a)
     a.sums[0] = r[0];
     a.sums[1] = r[1];
     const double c = a.constant[0];
-    a.out[0] = fabs((r[0] * c) - (r[1] * c * c));
-    ((unsigned long long*)a.out)[1] = all;
+    a.out[kMailQ] = fabs((r[0] * c) - (r[1] * c * c));
+    ((unsigned long long*)a.out)[kMailQ + 1] = all;
     *a.movers = 0;
     mail_post(a.out, a.seq);
 }
@@ -2926,7 +2931,7 @@ struct BatchTailArgs {
     unsigned char* act;
     int32_t* iters;
     unsigned long long* status;  // [0] graphs, [1] vertices, [2] finished workgroups; zero between rounds
-    double* out;                 // pinned: [slot], [slot + 1], and the number
+    double* out;                 // the mail: [slot], [slot + 1], and the number
     int32_t slot;
     unsigned long long seq;
 };
@@ -2999,8 +3004,7 @@ struct SetupArgs {
     const double* vdeg;
     int32_t nv, blocks;
     int64_t chunk;
-    double *cdeg, *sums, *constant, *out;  // out (pinned): [2] whole degrees, [16, 27) the buckets' sizes, [27] the
-    // LDS rows take k_hub_lds, [28] hub entries
+    double *cdeg, *sums, *constant, *out;  // out: the mail
     int32_t *csize, *past, *curr, *target, *lists;
     unsigned char* active;  // null when ET is off, with the three below
     double *frozen, *pa, *pb;
@@ -3109,15 +3113,15 @@ __global__ void __launch_bounds__(kTailBlock) k_setup_small(SetupArgs a)
     small_tree_sum2<kTailBlock>(a.vdeg, nullptr, a.nv, a.blocks, a.chunk, lds, s_part, r);
     int64_t* out = (int64_t*)a.out;
     if (t == 0) {
-        for (int q = 0; q < kNumBuckets; q++) out[16 + q] = s_total[q];
+        for (int q = 0; q < kNumBuckets; q++) out[kMailLists + q] = s_total[q];
         a.hoffs[nh] = (int64_t)entries;
-        out[27] = apart;
-        out[28] = (int64_t)entries;
-        a.out[15] = whole ? 1.0 : 0.0;
+        out[kMailHubsApart] = apart;
+        out[kMailHubEntries] = (int64_t)entries;
+        a.out[kMailHubWhole] = whole ? 1.0 : 0.0;
         a.sums[0] = r[0];
         a.sums[1] = r[1];
         a.constant[0] = 1.0 / r[0];
-        a.out[2] = !any_fraction && r[0] < 0x1p52 ? 1.0 : 0.0;
+        a.out[kMailWhole] = !any_fraction && r[0] < 0x1p52 ? 1.0 : 0.0;
         mail_post(a.out, a.seq);
     }
 }
@@ -3192,8 +3196,8 @@ __global__ void __launch_bounds__(256) k_modularity_tree(const double* __restric
         sums[0] = sa[0];
         sums[1] = sb[0];
         const double c = constant[0];
-        out[0] = fabs((sa[0] * c) - (sb[0] * c * c));
-        ((unsigned long long*)out)[1] = *movers;
+        out[kMailQ] = fabs((sa[0] * c) - (sb[0] * c * c));
+        ((unsigned long long*)out)[kMailQ + 1] = *movers;
         *movers = 0;
         *done = 0;
         mail_post(out, seq);
@@ -3584,7 +3588,7 @@ struct Phase {
         else tree_sum2(ctx, vdeg.p, nullptr, nv, sums());
         VT_LAUNCH(ctx, "constant", k_constant, 1, 64, 0, (const double*)sums(),
                   (const unsigned long long*)(ucount.p + 5), (const unsigned long long*)hub_fraction, constant(),
-                  moves ? mail(ctx) + 2 : nullptr, mail(ctx) + 15);
+                  moves ? mail(ctx) + kMailWhole : nullptr, mail(ctx) + kMailHubWhole);
     }
 
     // alloc, init and build_lists of a plain phase on at most kTailVerts vertices (tree sums).
@@ -3626,16 +3630,16 @@ struct Phase {
         VT_LAUNCH(ctx, "setup", k_setup_small, 1, kTailBlock, 0, a);
         mail_wait(ctx, ctx->mail_seq);
         const int64_t* h = (const int64_t*)mail(ctx);
-        hub_whole = hub_exact = mail(ctx)[15] == 1.0;
-        plan_sweeps(1, h + 16);
-        if (!h[27]) sort_all_hubs(sweeps[0]);
-        hub_total.assign(1, h[28]);
+        hub_whole = hub_exact = mail(ctx)[kMailHubWhole] == 1.0;
+        plan_sweeps(1, h + kMailLists);
+        if (!h[kMailHubsApart]) sort_all_hubs(sweeps[0]);
+        hub_total.assign(1, h[kMailHubEntries]);
         hub_sort = true;
     }
 
     // Sorts vertices into (color, degree bucket) lists and, with colors, the per-color event
-    // order; per color, plans one block range for buckets 0-3 (run as two launches: bucket 2
-    // alone, buckets 0, 1 and 3 together).
+    // order; per color, plans one block range for buckets 0-3 (one launch up to kOneLaunchBlocks,
+    // else two: bucket 2 alone, buckets 0, 1 and 3 together).
     void build_lists(const int64_t* d_colors, int64_t num_color, bool want_corder)
     {
         const int64_t ncol = d_colors && !want_corder ? num_color : 1;
@@ -3659,7 +3663,7 @@ struct Phase {
             sort_pairs_u32(ctx, k0, (uint32_t*)lists.p, nv, (int)bits_for(nkeys), k1, v1, &alt);
             if (alt) d2d(ctx, lists.p, v1, 4 * (size_t)nv);
             d2h(ctx, h.data(), hist, 8 * nkeys);
-            if (hub_fraction) hub_exact = mail(ctx)[15] == 1.0;  // k_constant's, there by now
+            if (hub_fraction) hub_exact = mail(ctx)[kMailHubWhole] == 1.0;  // k_constant's, there by now
             hub_fraction = nullptr;
         }
         hub_whole = hub_exact && hub_whole_possible();
@@ -4172,8 +4176,8 @@ struct Phase {
             }
         }
         mail_wait(ctx, ctx->mail_seq);
-        std::memcpy(&movers_read, &out[1], 8);
-        return out[0];
+        std::memcpy(&movers_read, &out[kMailQ + 1], 8);
+        return out[kMailQ];
     }
 };
 
@@ -4219,7 +4223,7 @@ vt_phase* phase_begin(vt_ctx* ctx, vt_graph* g, const vt_phase_params* p, const 
         if (mode == VT_MODE_PLAIN && nv > 0 && nv <= kTailVerts && g->ne < (int64_t(1) << 31) &&
             !(p->flags & VT_FLAG_SEQUENTIAL_SUMS)) {
             ph.setup_small();
-            ph.whole = mail(ctx)[2] == 1.0;
+            ph.whole = mail(ctx)[kMailWhole] == 1.0;
             ctx->trace_q.clear();
             ctx->trace_moves.clear();
             return st;
@@ -4236,7 +4240,7 @@ vt_phase* phase_begin(vt_ctx* ctx, vt_graph* g, const vt_phase_params* p, const 
         }
         // Sweep lists per color for COLOR; one Jacobi sweep (event order = colorIndex) for VORDER.
         ph.build_lists(mode != VT_MODE_PLAIN ? d_colors : nullptr, p->num_color, mode == VT_MODE_VORDER);
-        ph.whole = nv && mail(ctx)[2] == 1.0;  // k_constant's, there since build_lists read the lists' sizes
+        ph.whole = nv && mail(ctx)[kMailWhole] == 1.0;  // k_constant's, there since build_lists read the lists' sizes
     } catch (...) {
         delete st;
         throw;
@@ -4418,7 +4422,7 @@ void batch_phase(vt_ctx* ctx, vt_graph* u, const int32_t* d_gid, const SegSums& 
         int relists = 0;
         for (int r = 0;; r++) {
             ph.sweep(ph.sweeps[0]);
-            b.slot = 4 + 2 * (r & 1);
+            b.slot = kMailBatch + 2 * (r & 1);
             b.seq = ++ctx->mail_seq;
             if (seg.max_n <= kBatchTailSmall)
                 VT_LAUNCH(ctx, "batch_tail", (k_batch_tail<kBatchTailSmall, 256>), (unsigned)ng, 256, 0, b);
@@ -4427,7 +4431,7 @@ void batch_phase(vt_ctx* ctx, vt_graph* u, const int32_t* d_gid, const SegSums& 
             else VT_LAUNCH(ctx, "batch_tail", (k_batch_tail<kTailVerts, kTailBlock>), (unsigned)ng, kTailBlock, 0, b);
             if (r == 0) continue;
             mail_wait(ctx, b.seq - 1);
-            const unsigned long long* prev = (const unsigned long long*)b.out + 4 + 2 * ((r - 1) & 1);
+            const unsigned long long* prev = (const unsigned long long*)b.out + kMailBatch + 2 * ((r - 1) & 1);
             const int64_t active = (int64_t)prev[0], live_nv = (int64_t)prev[1];
             if (active == 0) {  // rounds 0 .. r - 1 had graphs iterating; round r changes nothing
                 finish(r, relists);

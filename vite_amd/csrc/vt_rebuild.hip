@@ -709,8 +709,8 @@ __global__ void __launch_bounds__(kSmallBlock) k_members_small(const int64_t* __
     }
 }
 
-// The scans of the row lengths and of the overflowing communities' entries, and for the host
-// (mail + 8, pinned): communities, ids out of range, entries, overflowing entries, largest row, largest
+// The scans of the row lengths and of the overflowing communities' entries, and for the host (in
+// the mail): communities, ids out of range, entries, overflowing entries, largest row, largest
 // overflowing community.
 __global__ void __launch_bounds__(kSmallBlock) k_rows_small(const int64_t* __restrict__ tot, const int64_t* __restrict__ rowlen,
                                                             const int64_t* __restrict__ xcnt, int64_t* __restrict__ out_offs,
@@ -750,7 +750,7 @@ __global__ void __launch_bounds__(kSmallBlock) k_rows_small(const int64_t* __res
     if (t == 0) {
         out_offs[nc] = (int64_t)ltot;
         xoff[nc] = (int64_t)xtot;
-        int64_t* out = (int64_t*)(mail + 8);
+        int64_t* out = (int64_t*)(mail + kMailRebuild);
         out[0] = nc;
         out[1] = tot[1];
         out[2] = (int64_t)ltot;
@@ -777,7 +777,8 @@ static void overflow_rows(vt_ctx* ctx, const vt_graph* g, const uint32_t* newid,
         DBuf<Item> items(ctx, (size_t)cap);
         VT_LAUNCH(ctx, "rb_ovf_items", k_split_items, grid_for(nc, 256, 4096), 256, 0, nc, xcnt, (int64_t)1, counts,
                   items.p);
-        // timed under a name of its own where a giant community is among them
+        // the same launch, timed under a name of its own where a community of more than 2^16 entries is
+        // among them
         const char* name = xmax > (1 << 16) ? "rb_ovf_emit_big" : "rb_ovf_emit";
         VT_LAUNCH(ctx, name, k_ovf_emit, (unsigned)std::min<int64_t>(cap, 65536), 64, 0, (const uint32_t*)counts,
                   (const Item*)items.p, cstart, moff, mrow, (const DEdge*)g->edges, newid, xoff, bits, k0.p, v0.p);
@@ -917,7 +918,7 @@ vt_graph* rebuild(vt_ctx* ctx, const vt_graph* g, const int64_t* d_cvect, bool c
     int64_t totals[4] = {0, 0, 0, 0};  // entries, overflowing entries, largest row, largest overflowing community
     auto read_totals = [&](bool first) {
         if (small) {
-            const int64_t* out = (const int64_t*)(mail(ctx) + 8);
+            const int64_t* out = (const int64_t*)(mail(ctx) + kMailRebuild);
             VT_LAUNCH(ctx, "rb_rows", k_rows_small, 1, kSmallBlock, 0, (const int64_t*)tot.p, (const int64_t*)rowlen.p,
                       (const int64_t*)xcnt.p, out_offs.p, xoff.p, mail(ctx), ++ctx->mail_seq);
             mail_wait(ctx, ctx->mail_seq);
