@@ -66,6 +66,7 @@ struct vt_ctx {
     size_t stage_off = 0;
     double* mail = nullptr;  // pinned (vt::mail)
     unsigned long long mail_seq = 0;  // the last number given to a kernel that posts there
+    int queued = 0;                   // launches since the host last waited for the stream
     // sweep launch shape (performance only: every setting gives the same results)
     vt_tuning tuning = {{7, 15, 31, 63, 127, 1023}, 16384};  // replaced by default_tuning() at creation
 };
@@ -173,6 +174,7 @@ void flush_timings(vt_ctx* ctx);
 #define VT_LAUNCH(ctx, name, kernel, grid, block, shmem, ...)                                  \
     do {                                                                                      \
         ::vt::TimedScope ts_(ctx, name);                                                      \
+        (ctx)->queued++;                                                                      \
         hipLaunchKernelGGL(kernel, dim3(grid), dim3(block), shmem, (ctx)->stream, __VA_ARGS__); \
         VT_HIP(ctx, hipGetLastError());                                                       \
     } while (0)
