@@ -206,6 +206,38 @@ void d2h(vt_ctx* ctx, void* dst, const void* src, size_t bytes)
     ctx->queued = 0;
     ctx->stage_off = 0;  // the stream has drained: every staged copy has run
 }
+// Where they all fit the staging ring, the copies are queued there and waited for together; a copy
+// and its wait cost some 10 us each.
+void d2h_all(vt_ctx* ctx, const std::vector<HostRead>& reads)
+{
+    size_t all = 0;
+    for (const HostRead& r : reads) all += r.dst ? (r.bytes + 255) & ~size_t(255) : 0;
+    if (all > kStageMax) {
+        for (const HostRead& r : reads)
+            if (r.dst) d2h(ctx, r.dst, r.src, r.bytes);
+        return;
+    }
+    if (!ctx->stage) {
+        VT_HIP(ctx, hipHostMalloc((void**)&ctx->stage, kStageCap, hipHostMallocDefault));
+        ctx->stage_off = 0;
+    }
+    if (ctx->stage_off + all > kStageCap) sync(ctx);
+    size_t off = ctx->stage_off;
+    for (const HostRead& r : reads) {
+        if (!r.dst || !r.bytes) continue;
+        VT_HIP(ctx, hipMemcpyAsync(ctx->stage + off, r.src, r.bytes, hipMemcpyDeviceToHost, ctx->stream));
+        off += (r.bytes + 255) & ~size_t(255);
+    }
+    VT_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    off = ctx->stage_off;
+    for (const HostRead& r : reads) {
+        if (!r.dst || !r.bytes) continue;
+        std::memcpy(r.dst, ctx->stage + off, r.bytes);
+        off += (r.bytes + 255) & ~size_t(255);
+    }
+    ctx->queued = 0;
+    ctx->stage_off = 0;
+}
 double* mail(vt_ctx* ctx)
 {
     if (!ctx->mail) {

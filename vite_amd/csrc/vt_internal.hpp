@@ -182,6 +182,13 @@ void flush_timings(vt_ctx* ctx);
 void sync(vt_ctx* ctx);
 void h2d(vt_ctx* ctx, void* dst, const void* src, size_t bytes);
 void d2h(vt_ctx* ctx, void* dst, const void* src, size_t bytes);
+// Several reads with one wait (dst null: none).
+struct HostRead {
+    void* dst;
+    const void* src;
+    size_t bytes;
+};
+void d2h_all(vt_ctx* ctx, const std::vector<HostRead>& reads);
 void d2d(vt_ctx* ctx, void* dst, const void* src, size_t bytes);
 // Pinned host memory that kernels write a few scalars to, with no copy queued behind the kernel: doubles
 // or 64-bit integers at these places.

@@ -24,7 +24,6 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-#include <memory>
 #include <vector>
 
 #include "vt_internal.hpp"
@@ -4591,14 +4590,27 @@ void batch_phase(vt_ctx* ctx, vt_graph* u, const int32_t* d_gid, const SegSums& 
     finish(rounds, relists);
 }
 
-// A phase's 32-bit ids as a caller's 64-bit ones (dst may be null), widened on the host: half the
-// bytes to copy, and no launch.
+// A phase's 32-bit ids as a caller's 64-bit ones, widened on the host: half the bytes to copy, and no
+// launch.  The ids are read into the upper half of dst, from where each moves down to its place.
+static HostRead ids_read(int64_t* dst, const int32_t* src, int64_t n)
+{
+    return HostRead{dst ? (int32_t*)dst + n : nullptr, src, 4 * (size_t)n};
+}
+static void widen_on_host(int64_t* dst, int64_t n)
+{
+    if (!dst) return;
+    constexpr int64_t kBlock = 1024;
+    int32_t x[kBlock];
+    for (int64_t i = 0; i < n; i += kBlock) {  // writes end before the next block's ids
+        const int64_t m = std::min(kBlock, n - i);
+        std::memcpy(x, (const unsigned char*)dst + 4 * (n + i), 4 * (size_t)m);
+        for (int64_t k = 0; k < m; k++) dst[i + k] = x[k];
+    }
+}
 static void ids_to_host(vt_ctx* ctx, int64_t* dst, const int32_t* src, int64_t n)
 {
-    if (!dst || !n) return;
-    std::unique_ptr<int32_t[]> ids(new int32_t[(size_t)n]);
-    d2h(ctx, ids.get(), src, 4 * (size_t)n);
-    for (int64_t i = 0; i < n; i++) dst[i] = ids[(size_t)i];
+    d2h_all(ctx, {ids_read(dst, src, n)});
+    widen_on_host(dst, n);
 }
 
 vt_tuning default_tuning()
@@ -4875,13 +4887,9 @@ int vt_phase_get_state(vt_ctx* ctx, const vt_phase* st, int64_t* curr, int64_t* 
         VT_HIP(ctx, hipSetDevice(ctx->device));
         const Phase& ph = st->ph;
         const size_t b8 = 8 * (size_t)ph.nv;
-        ids_to_host(ctx, curr, ph.curr.p, ph.nv);
-        ids_to_host(ctx, csize, ph.csize.p, ph.nv);
-        ids_to_host(ctx, target, ph.target.p, ph.nv);
-        if (cdeg) d2h(ctx, cdeg, ph.cdeg.p, b8);
-        if (vdeg) d2h(ctx, vdeg, ph.vdeg.p, b8);
-        if (cw) d2h(ctx, cw, ph.cw.p, b8);
-        if (constant) d2h(ctx, constant, ph.scal.p + 2, 8);
+        d2h_all(ctx, {ids_read(curr, ph.curr.p, ph.nv), ids_read(csize, ph.csize.p, ph.nv), ids_read(target, ph.target.p, ph.nv),
+                      {cdeg, ph.cdeg.p, b8}, {vdeg, ph.vdeg.p, b8}, {cw, ph.cw.p, b8}, {constant, ph.scal.p + 2, 8}});
+        for (int64_t* ids : {curr, csize, target}) widen_on_host(ids, ph.nv);
     });
 }
 
