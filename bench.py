@@ -32,8 +32,8 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_GBS = 8000.0
 # Rows of bucket 2 (16-lane groups; degree <= 47 with the default bounds) run in the
 # launch named "local_move", the dominant one on random geometric graphs; buckets 0, 1
-# and 3 run in "local_move_rest" and larger degree classes in their own launches.  On graphs of
-# some hundred thousand rows and fewer, buckets 0 to 3 run in one launch, "local_move_all".
+# and 3 run in "local_move_rest" and larger degree classes in their own launches.  Where a sweep has few
+# workgroups (a small graph, or a tuning with a small cap), buckets 0 to 3 run in one, "local_move_all".
 G16_BUCKET = 2
 
 
@@ -687,7 +687,7 @@ def main():
     wall = time.perf_counter() - t0
     ms_per_step = 1e3 * wall / args.steps
     kavg, kcount, ktot = ctx.kernel_stats("local_move")
-    all_buckets = kcount == 0  # a small graph: one launch for buckets 0 to 3
+    all_buckets = kcount == 0  # few workgroups: one launch for buckets 0 to 3
     if all_buckets:
         kavg, kcount, ktot = ctx.kernel_stats("local_move_all")
     ctx.set_profiling(False)
