@@ -29,7 +29,7 @@ def _expected(a, b):
                 precision=ss / (ss + ds), recall=ss / (ss + sd))
 
 
-@pytest.mark.parametrize("n", [1023, 1024, 1025, 4097, 300007, 2048 * 1024 + 1])
+@pytest.mark.parametrize("n", [255, 256, 257, 1023, 1025, 4097, 65537, 300007, 1024 * 1024 + 1, 2048 * 1024 + 1])
 def test_few_communities(ctx, n):
     for k in (1, 2, 3, 40, 700):
         truth, found = _partitions(n, k, n + k)

@@ -91,9 +91,8 @@ __device__ __forceinline__ void pair_add(PairSlot* __restrict__ pairs, int logca
 // each on one line, and where the communities are few a few pairs hold most of the vertices: a
 // workgroup counts its chunk in an LDS table first, one slot per hash, and adds each slot once; a
 // pair whose slot another one has goes to memory directly (n = 1000003 with 2, 64, 1024 and 30011
-// communities: 45, 144, 187 and 79 us; an atomic per vertex took 10023, 1542, 402 and 84).
+// communities: 48, 148, 183 and 81 us; an atomic per vertex took 10023, 1542, 402 and 84).
 constexpr int kCmpSlots = 1024;
-constexpr int64_t kCmpChunk = 1024;  // vertices per workgroup, at least
 
 __global__ void __launch_bounds__(kCmpBlock) k_cmp_count(const int64_t* __restrict__ c1, const int64_t* __restrict__ c2,
                                                          int64_t n, int64_t chunk, uint64_t nc2,
@@ -220,7 +219,10 @@ extern "C" int vt_compare_communities(vt_ctx* ctx, int64_t n, const int64_t* tru
         unsigned long long *size1 = size.p, *size2 = size.p + nc1, *same = size.p + nc;
         dzero(ctx, size.p, 8 * (size_t)(nc + 1));
         VT_LAUNCH(ctx, "cmp_clear", k_cmp_clear, grid_for(cap, 256, 8192), 256, 0, pairs.p, cap);
-        const int64_t chunk = std::max(kCmpChunk, (n + 2047) / 2048);
+        // a vertex per thread until there is a workgroup per CU, 1024 vertices until there are four, then
+        // those four (n = 30000 with 3750 communities: 16 us, with 1024 a workgroup 24; n = 4 * 10^6 with 2
+        // communities 66, with 2048 workgroups 125)
+        const int64_t chunk = std::max(std::min<int64_t>(std::max<int64_t>(256, n / 256), 1024), (n + 1023) / 1024);
         VT_LAUNCH(ctx, "cmp_count", k_cmp_count, (unsigned)((n + chunk - 1) / chunk), kCmpBlock, 0, (const int64_t*)c1.p,
                   (const int64_t*)c2.p, n, chunk, (uint64_t)nc2, pairs.p, logcap);
         VT_LAUNCH(ctx, "cmp_sizes", k_cmp_sizes, grid_for(cap, kCmpBlock, 2048), kCmpBlock, 0, (const PairSlot*)pairs.p, cap,
