@@ -1,5 +1,5 @@
 """The end of an iteration: the moves folded into the communities and the modularity.  Three
-forms by vertex count (one workgroup up to 8192 vertices, atomics up to 2^20, a sort above), and
+forms by vertex count (one workgroup up to 8192 vertices, atomics up to 2^19, a sort above), and
 in each the event runs take different folds by their length; all give the bits of the oracle's
 in-order folds, and the modularity the bits of vt_modularity on the same arrays."""
 import numpy as np

@@ -1,7 +1,7 @@
 """GPU parity at larger sizes: a 2^20-vertex RGG (29 M directed entries) swept from a
 mid-run device state, a hub-heavy Barabasi-Albert graph (2^17 vertices, m = 8, rows up to
-a few thousand entries, so the sorted hub path runs) through whole phases, runs (also with
-coloring and early termination) and a rebuild with a giant community, and the benchmark's
+a few thousand entries, which go to LDS and, the longest, to the table of whole weights)
+through whole phases, runs (also with coloring and early termination) and a rebuild with a giant community, and the benchmark's
 two RGGs (n = 65,536 and n = 2^24 + 1%) and its skewed-degree BA graph (n = 2^22, m = 8,
 -c 8 -t 2 -a 0.25) through whole runs against the compiled reference's main()
 (tests/golden/reference_large.json).  The graphs are generated on the
@@ -129,8 +129,9 @@ def test_ba_2p22_hub_key_widths_and_forms(ctx):
 
 def test_ba_giant_community_of_few_hubs_rebuild(ctx):
     """A community of at most 64 members holding more than 2^16 entries: the rebuild's
-    overflow path emits it with every wave (k_ovf_emit_big), each lane finding its member by
-    wave shuffles.  On BA n = 2^20, m = 8 the largest hubs have several thousand entries each,
+    overflow path emits it a wave per 4096 entries (k_ovf_emit, timed as rb_ovf_emit_big where
+    such a community is among them), each lane finding its member by wave shuffles.  On BA
+    n = 2^20, m = 8 the largest hubs have several thousand entries each,
     so a few dozen of them pass 2^16.  The coarse CSR equals the oracle's byte for byte."""
     dg = ctx.gen_ba(79, 1 << 20, 8)
     g = _host(dg)
