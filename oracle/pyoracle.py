@@ -2,7 +2,7 @@
 to the compiled reference harness (oracle/_ref/libvite_ref.so).
 
 TEST INFRASTRUCTURE ONLY: imported by tests/, the smoke check and the bench's
-CPU-baseline leg as the checker.  Nothing in the product imports it.
+CPU-baseline leg as the oracle.  Nothing in the product imports it.
 """
 from __future__ import annotations
 
